@@ -1,0 +1,1120 @@
+// The projection as a contraction on the matrix cores (included by ekv_lut.hip).
+//
+// A branch current depends on x - w alone, and the thresholds of a layer lie in an interval
+// [w_lo, w_hi] that is narrow against the width 2 n U_T over which the current changes. On it
+//     f(x - w) = sum_j c_j(x) T_j(t),   t = (w - w_c) / w_h in [-1, 1],
+// with Chebyshev polynomials T_j converges geometrically, whatever x is: the current's nearest
+// singularities lie at (x - w) / (2 n U_T) = +-i pi, so the terms fall like rho^-j with
+// rho = z + sqrt(z^2 + 1), z = pi * 2 n U_T / w_h (Trefethen, Approximation Theory and
+// Approximation Practice, ch. 8). Both sums over cells become products of matrices whose inner
+// index is (input, j):
+//     Idiff[m, o]  = sum_(k, j) (c_j r)[m, k] (T_j(t+) - T_j(t-))[o, k]
+//     dX[m, k]     = sum_j g_j(x[m, k]) H_j[m, k],  H_j = sum_o G[m, o] (T_j(t+) - T_j(t-))[o, k]
+//     dVth+-[o, k] = -+ sum_j T_j(t+-[o, k]) S_j,   S_j = sum_m G[m, o] (d_j r)[m, k]
+// with f' = sum_j d_j T_j and g_j = r (d_j - (r / V_sat) c_j): j = 0 cancels in the difference
+// of the branches. R terms cost R products per cell and direction where the cell itself costs
+// 32 (forward) or 52 (backward) VALU instructions, four or eight of them transcendental.
+//
+// Precision. Operands are kept to 22 bits as the sum of two f16 (hi + lo, scaled by a power of
+// two per row so that the row's largest value is near 2^12), and every product is formed as
+// hi hi + hi lo + lo hi in fp32 accumulators; the differences T_j(t+) - T_j(t-) are formed in
+// fp64 before they are rounded, so that a cell no longer loses the bits in which its two
+// branches agree. c_j, d_j and g_j come from tables over x built per call in fp64 (cubic
+// interpolation, step at most kSepStep of 2 n U_T: 2e-8 relative; the step is a power of two,
+// so that a position within a step is exact in fp32).
+//
+// Measured (GPT-L layer 768 x 3072 at 2048 tokens, initial thresholds, R = 8): forward 4.30 ms
+// by the per-cell kernels, 0.30 ms here; backward 8.17 and 0.74 ms; error against float64 of
+// the forward 2.8e-6 and 2.6e-7, of dX 2.3e-6 and 3.4e-7, of dVth 3.5e-7 and 2.7e-7 (2-norm).
+//
+// R is chosen per call on the device from the thresholds' spread (sep_terms); a call whose
+// operands do not suit (non-finite values, x near -V_sat or spread over more than the table
+// holds, thresholds spread too far) runs the per-cell kernels, which return at once otherwise.
+
+typedef _Float16 sep_h8 __attribute__((ext_vector_type(8)));
+typedef _Float16 sep_h2 __attribute__((ext_vector_type(2)));
+typedef float sep_f16 __attribute__((ext_vector_type(16)));
+typedef unsigned sep_u4 __attribute__((ext_vector_type(4)));
+
+constexpr int kSepStatBlocks = 256;     // blocks of each statistics pass (partials each)
+constexpr int kSepColChunks = 64;       // row chunks of a column pass, at most
+constexpr int kSepGridMax = 16384;      // x-table points, at most
+constexpr double kSepStep = 0.0148;     // x-table step in units of 2 n U_T
+constexpr int kSepMaxTerms = 64;
+constexpr float kSepQScale = 256.0f;    // of the threshold-side operand (values in [-2, 2])
+
+// Widest threshold spread, in units of 2 n U_T, that R = 8, 16, 32, 64 terms take: there the
+// truncation is 1e-7 of the gradients (the forward's is ten times smaller), below the fp32
+// sums' own rounding (float64 evaluation of the truncated series against the formula).
+__host__ __device__ inline int sep_terms(float spread_u) {
+    return spread_u <= 1.12f ? 8 : spread_u <= 4.4f ? 16 : spread_u <= 11.0f ? 32 : spread_u <= 24.0f ? 64 : 0;
+}
+
+// What the passes of a call share, in its workspace.
+struct SepHead {
+    int terms;    // 0: the per-cell kernels run
+    int n_grid;
+    float x0, step, inv_step; // table point i stands for x0 + i * step; step a power of two, x0 a multiple of it
+    double wc, inv_wh, wh;   // t = (w - wc) * inv_wh
+};
+
+__device__ inline bool sep_gate(const SepHead* head, bool want) {
+    return head == nullptr || (head->terms != 0) == want;
+}
+
+struct SepArgs {
+    const float* x;
+    const float* wp;
+    const float* wn;
+    const float* g;          // backward: [M][ldg]
+    int64_t M, K, O, ldg;
+    const float* in_affine;
+    float in_lo, in_hi;
+    // formula
+    double a, v_d;           // 1 / (2 n U_T), V_D
+    double v_sat;
+    int max_terms;
+    // workspace
+    SepHead* head;
+    float2* xpart;           // [kSepStatBlocks]
+    float2* wpart;           // [kSepStatBlocks]
+    unsigned* gpart;         // [kSepStatBlocks]
+    float2* xrow;            // forward: [M] row ranges of x
+    float2* xcol;            // backward: [kSepColChunks][K]
+    unsigned* grow;          // backward: [M] largest |G| of a row (bits)
+    unsigned* gcol;          // backward: [kSepColChunks][O]
+    float* tab;              // forward c_j r (j = 1..R), backward d_j r (j = 0..R-1): [n_grid][R]
+    float* tab2;             // backward g_j (j = 1..R)
+    _Float16* xop;           // forward [M][Kd], backward [K R][Md]: hi/lo pairs, 32 + 32
+    _Float16* wop;           // forward [O][Kd], backward [K R][Od]
+    _Float16* gop;           // backward [M][Od]
+    _Float16* gopT;          // backward [O][Md]
+    float* xscale;           // forward [M], backward [K]: inverse scale of xop's rows
+    float* gscale;           // backward [M]
+    float* gscaleT;          // backward [O]
+    float2* tT;              // backward [K][Op]: {t+, t-}
+    int64_t Op;
+    int need_x, need_w;
+};
+
+__device__ inline float sep_input(const SepArgs& a, float x, float s, float b) {
+    return a.in_affine ? input_map(x, s, b, a.in_lo, a.in_hi) : x;
+}
+
+// Inner lengths in f16 pairs' slabs of 32: the forward's (j / 8, k, j % 8) index, each eight
+// terms of four inputs a slab (K padded to fours), tokens and outputs of the backward.
+__host__ __device__ inline int64_t sep_slabs_kj(int64_t K, int terms) { return (K + 3) / 4 * (terms / 8); }
+__host__ __device__ inline int64_t sep_slabs(int64_t n) { return (n + 31) / 32; }
+
+// ----------------------------------------------------------------------------------
+// Statistics: ranges of x (per row forward, per column backward), of the thresholds, and the
+// largest |G| of each row and column. NaN makes a range infinite and a maximum non-finite.
+// HBM-bound: x, the thresholds and G are read once (G and, with both gradients, twice).
+// ----------------------------------------------------------------------------------
+
+__device__ inline void sep_minmax(float v, float& lo, float& hi) {
+    const bool bad = v != v;
+    lo = fminf(lo, bad ? -INFINITY : v);
+    hi = fmaxf(hi, bad ? INFINITY : v);
+}
+
+__device__ inline void sep_wave_minmax(float& lo, float& hi) {
+    for (int d = 32; d > 0; d >>= 1) {
+        lo = fminf(lo, __shfl_xor(lo, d));
+        hi = fmaxf(hi, __shfl_xor(hi, d));
+    }
+}
+
+__device__ inline unsigned sep_bits(float v) { return __float_as_uint(v) & 0x7fffffffu; }
+
+// Blocks of 16 waves: kSepStatBlocks of x, kSepStatBlocks of the thresholds, then (g)
+// kSepStatBlocks of G's rows and kSepColChunks / 4 x ceil(O / 256) of its columns, and (xcol)
+// kSepColChunks / 4 x ceil(K / 256) of x's columns. Four loads in flight per thread.
+__global__ __launch_bounds__(1024) void sep_stat_kernel(SepArgs a) {
+    int b = blockIdx.x;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const float as = a.in_affine ? a.in_affine[0] : 1.0f, ab = a.in_affine ? a.in_affine[1] : 0.0f;
+    if (b < kSepStatBlocks) {
+        float lo = INFINITY, hi = -INFINITY;
+        if (a.xrow) {  // a wave per row
+            for (int64_t m = (int64_t)b * 16 + wave; m < a.M; m += (int64_t)kSepStatBlocks * 16) {
+                float l = INFINITY, h = -INFINITY;
+                const float* row = a.x + m * a.K;
+                for (int64_t k = lane; k < a.K; k += 256) {
+                    float v[4];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) v[q] = row[k + q * 64 < a.K ? k + q * 64 : k];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) sep_minmax(sep_input(a, v[q], as, ab), l, h);
+                }
+                sep_wave_minmax(l, h);
+                if (lane == 0) a.xrow[m] = make_float2(l, h);
+                lo = fminf(lo, l);
+                hi = fmaxf(hi, h);
+            }
+        } else {
+            const int64_t n = a.M * a.K, stride = (int64_t)kSepStatBlocks * 1024;
+            for (int64_t e = (int64_t)b * 1024 + t; e < n; e += 4 * stride) {
+                float v[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) v[q] = a.x[e + q * stride < n ? e + q * stride : e];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) sep_minmax(sep_input(a, v[q], as, ab), lo, hi);
+            }
+        }
+        block_minmax(lo, hi, &a.xpart[b]);
+        return;
+    }
+    b -= kSepStatBlocks;
+    if (b < kSepStatBlocks) {
+        float lo = INFINITY, hi = -INFINITY;
+        const int64_t n = a.O * a.K, stride = (int64_t)kSepStatBlocks * 1024;
+        for (int64_t e = (int64_t)b * 1024 + t; e < n; e += 2 * stride) {
+            const int64_t f = e + stride < n ? e + stride : e;
+            const float v[4] = {a.wp[e], a.wn[e], a.wp[f], a.wn[f]};
+#pragma unroll
+            for (int q = 0; q < 4; ++q) sep_minmax(v[q], lo, hi);
+        }
+        block_minmax(lo, hi, &a.wpart[b]);
+        return;
+    }
+    b -= kSepStatBlocks;
+    if (b < kSepStatBlocks) {
+        unsigned all = 0;
+        for (int64_t m = (int64_t)b * 16 + wave; m < a.M; m += (int64_t)kSepStatBlocks * 16) {
+            unsigned h = 0;
+            const float* row = a.g + m * a.ldg;
+            for (int64_t o = lane; o < a.O; o += 256) {
+                unsigned v[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) v[q] = sep_bits(row[o + q * 64 < a.O ? o + q * 64 : o]);
+                h = max(h, max(max(v[0], v[1]), max(v[2], v[3])));
+            }
+            for (int d = 32; d > 0; d >>= 1) h = max(h, (unsigned)__shfl_xor((int)h, d));
+            if (lane == 0) a.grow[m] = h;
+            all = max(all, h);
+        }
+        __shared__ unsigned s_all;
+        if (t == 0) s_all = 0;
+        __syncthreads();
+        if (lane == 0) atomicMax(&s_all, all);
+        __syncthreads();
+        if (t == 0) a.gpart[b] = s_all;
+        return;
+    }
+    b -= kSepStatBlocks;
+    const int gcols = a.need_w ? kSepColChunks / 4 * (int)((a.O + 255) / 256) : 0;
+    const int64_t rows = (a.M + kSepColChunks - 1) / kSepColChunks;
+    const bool of_g = b < gcols;
+    if (!of_g) b -= gcols;
+    const int chunk = b % (kSepColChunks / 4) * 4 + (t >> 8);
+    const int64_t col = (int64_t)(b / (kSepColChunks / 4)) * 256 + (t & 255);
+    const int64_t m0 = chunk * rows, m1 = m0 + rows < a.M ? m0 + rows : a.M;
+    if (of_g) {
+        if (col >= a.O) return;
+        unsigned h = 0;
+#pragma unroll 8
+        for (int64_t m = m0; m < m1; ++m) h = max(h, sep_bits(a.g[m * a.ldg + col]));
+        a.gcol[(int64_t)chunk * a.O + col] = h;
+    } else {
+        if (col >= a.K) return;
+        float lo = INFINITY, hi = -INFINITY;
+#pragma unroll 8
+        for (int64_t m = m0; m < m1; ++m) sep_minmax(sep_input(a, a.x[m * a.K + col], as, ab), lo, hi);
+        a.xcol[(int64_t)chunk * a.K + col] = make_float2(lo, hi);
+    }
+}
+
+// ----------------------------------------------------------------------------------
+// Mode and coefficient tables. Every block reduces the partials itself and block 0 records the
+// result; a thread builds one table point: the slope at R Chebyshev points of the threshold
+// interval, its coefficients d_j (Trefethen ch. 3: a discrete cosine sum), and c_j by
+// integration, c_j = -(w_h / 2j) (d_(j-1) - d_(j+1)), which needs no difference of currents.
+// ----------------------------------------------------------------------------------
+
+__device__ inline double sep_slope(double v, double a, double v_d) {  // f'(v) of f = sp(u1)^2 - sp(u2)^2
+    const double u1 = v * a, u2 = (v - v_d) * a;
+    const double e1 = exp(-fabs(u1)), e2 = exp(-fabs(u2));
+    const double s1 = log1p(e1) + fmax(u1, 0.0), s2 = log1p(e2) + fmax(u2, 0.0);
+    const double g1 = (u1 >= 0.0 ? 1.0 : e1) / (1.0 + e1), g2 = (u2 >= 0.0 ? 1.0 : e2) / (1.0 + e2);
+    return 2.0 * a * (s1 * g1 - s2 * g2);
+}
+
+__global__ __launch_bounds__(256) void sep_table_kernel(SepArgs a) {
+    __shared__ float2 s_x, s_w;
+    __shared__ unsigned s_g;
+    __shared__ SepHead s_head;
+    __shared__ double s_cos[4 * kSepMaxTerms], s_val[256], s_d[256];
+    const int t = threadIdx.x;
+    block_minmax(a.xpart[t].x, a.xpart[t].y, &s_x);
+    __syncthreads();
+    block_minmax(a.wpart[t].x, a.wpart[t].y, &s_w);
+    if (t == 0) s_g = 0;
+    __syncthreads();
+    if (a.g) atomicMax(&s_g, a.gpart[t]);
+    __syncthreads();
+    if (t == 0) {
+        SepHead h{};
+        const float xlo = s_x.x, xhi = s_x.y, wlo = s_w.x, whi = s_w.y;
+        const double step = exp2(floor(log2(kSepStep / a.a)));
+        const double rlo = 1.0 + (double)xlo / a.v_sat, rhi = 1.0 + (double)xhi / a.v_sat;
+        const double first = floor((double)xlo / step) - 1.0;
+        const double points = floor((double)xhi / step) - first + 3.0;
+        const bool finite = xlo > -1e30f && xhi < 1e30f && wlo > -1e30f && whi < 1e30f && s_g < 0x7f800000u;
+        const float spread = (float)(((double)whi - (double)wlo) * a.a);
+        const int terms = sep_terms(spread);
+        // |u| far below the exponent range of fp64, r and the table over x well behaved
+        if (finite && terms > 0 && terms <= a.max_terms && rlo > 0.1 && rhi > 0.1 && points <= (double)kSepGridMax &&
+            fmax(fabs((double)xlo), fabs((double)xhi)) < step * (1 << 23) &&
+            fmax(fabs((double)xlo), fabs((double)xhi)) * a.a < 300.0 &&
+            fmax(fabs((double)wlo), fabs((double)whi)) * a.a < 300.0) {
+            h.terms = terms;
+            h.n_grid = (int)points;
+            h.x0 = (float)(first * step);
+            h.step = (float)step;
+            h.inv_step = (float)(1.0 / step);
+            h.wc = 0.5 * ((double)wlo + (double)whi);
+            h.wh = fmax(0.5 * ((double)whi - (double)wlo), 1e-3 / a.a);
+            h.inv_wh = 1.0 / h.wh;
+        }
+        s_head = h;
+        if (blockIdx.x == 0) *a.head = h;
+    }
+    __syncthreads();
+    const SepHead h = s_head;
+    const int R = h.terms;
+    if (R == 0) return;
+    for (int q = t; q < 4 * R; q += 256) s_cos[q] = cospi((double)q / (2.0 * R));
+    // a block takes 256 / R points at a time: a thread per (point, Chebyshev point), then per
+    // (point, j)
+    const int per = 256 / R, pl = t / R, n = t - pl * R;
+    for (int i0 = blockIdx.x * per; i0 < h.n_grid; i0 += gridDim.x * per) {
+        const double x = (double)h.x0 + (double)(i0 + pl) * (double)h.step;
+        const double r = 1.0 / (1.0 + x / a.v_sat);
+        __syncthreads();
+        s_val[t] = sep_slope(x - (h.wc + h.wh * s_cos[2 * n + 1]), a.a, a.v_d);
+        __syncthreads();
+        double d = 0.0;
+        for (int q = 0; q < R; ++q) d += s_val[pl * R + q] * s_cos[(n * (2 * q + 1)) % (4 * R)];
+        d *= 2.0 / R;
+        s_d[t] = d;
+        __syncthreads();
+        if (i0 + pl < h.n_grid) {
+            const int j = n + 1;  // c_j from d_(j-1) = d and d_(j+1)
+            const double d_next = j < R ? s_d[t + 1] : 0.0, d_after = j + 1 < R ? s_d[t + 2] : 0.0;
+            const double c = -h.wh / (2.0 * j) * (d - d_after);
+            const size_t e = (size_t)(i0 + pl) * R + n;
+            if (a.tab2) {
+                a.tab[e] = (float)((n == 0 ? 0.5 * d : d) * r);
+                a.tab2[e] = (float)(r * (d_next - r / a.v_sat * c));
+            } else {
+                a.tab[e] = (float)(c * r);
+            }
+        }
+    }
+}
+
+// Position of x in a table: the first of its four points and their cubic weights.
+struct SepAt {
+    int i;
+    float w[4];
+};
+
+__device__ inline SepAt sep_at(const SepHead& h, float x) {
+    int i = (int)((x - h.x0) * h.inv_step);
+    i = i < 1 ? 1 : i > h.n_grid - 3 ? h.n_grid - 3 : i;
+    // x0 + i step is exact, and so is x's distance from it
+    const float f = (x - (h.x0 + (float)i * h.step)) * h.inv_step, g = 1.0f - f;
+    SepAt at;
+    at.i = i - 1;
+    at.w[0] = -f * g * (1.0f + g) * (1.0f / 6.0f);
+    at.w[1] = g * (1.0f + f) * (1.0f + g) * 0.5f;
+    at.w[2] = f * (1.0f + f) * (1.0f + g) * 0.5f;
+    at.w[3] = -f * g * (1.0f + f) * (1.0f / 6.0f);
+    return at;
+}
+
+__device__ inline float4 sep_eval4(const float* tab, int R, const SepAt& at, int j) {
+    const float* p = tab + (size_t)at.i * R + j;
+    const float4 v0 = *reinterpret_cast<const float4*>(p), v1 = *reinterpret_cast<const float4*>(p + R);
+    const float4 v2 = *reinterpret_cast<const float4*>(p + 2 * R), v3 = *reinterpret_cast<const float4*>(p + 3 * R);
+    float4 s;
+    s.x = fmaf(at.w[3], v3.x, fmaf(at.w[2], v2.x, fmaf(at.w[1], v1.x, at.w[0] * v0.x)));
+    s.y = fmaf(at.w[3], v3.y, fmaf(at.w[2], v2.y, fmaf(at.w[1], v1.y, at.w[0] * v0.y)));
+    s.z = fmaf(at.w[3], v3.z, fmaf(at.w[2], v2.z, fmaf(at.w[1], v1.z, at.w[0] * v0.z)));
+    s.w = fmaf(at.w[3], v3.w, fmaf(at.w[2], v2.w, fmaf(at.w[1], v1.w, at.w[0] * v0.w)));
+    return s;
+}
+
+// The power of two that brings a largest value to [2^11, 2^12), and its inverse.
+__device__ inline float sep_scale_of(float largest, float* inverse) {
+    int e = 12;
+    if (largest > 0.0f) e = 12 - (ilogbf(largest) + 1);
+    e = e > 120 ? 120 : e < -120 ? -120 : e;
+    *inverse = ldexpf(1.0f, -e);
+    return ldexpf(1.0f, e);
+}
+
+// A row's largest |c_j r| or |d_j r|, from above: the first coefficient grows with x and
+// dominates the others, r falls with x.
+__device__ inline float sep_bound(const SepHead& h, const float* tab, int j, float2 range, float v_sat) {
+    const SepAt at = sep_at(h, range.y);
+    const float* p = tab + (size_t)at.i * h.terms + j;
+    float s = 0.0f;
+    for (int q = 0; q < 4; ++q) s = fmaf(at.w[q], p[q * h.terms], s);
+    return fabsf(s) * (1.0f + range.y / v_sat) / (1.0f + range.x / v_sat) * 1.001f;
+}
+
+__device__ inline void sep_split(float v, _Float16& hi, _Float16& lo) {
+    hi = (_Float16)v;
+    lo = (_Float16)(v - (float)hi);
+}
+
+// Stores a pair of neighbouring inner elements (e, e + 1; e even) of a row of hi/lo slabs.
+__device__ inline void sep_store2(_Float16* row, int64_t e, float v0, float v1) {
+    sep_h2 hi, lo;
+    _Float16 h0, l0, h1, l1;
+    sep_split(v0, h0, l0);
+    sep_split(v1, h1, l1);
+    hi.x = h0; hi.y = h1; lo.x = l0; lo.y = l1;
+    _Float16* p = row + (e >> 5) * 64 + (e & 31);
+    *reinterpret_cast<sep_h2*>(p) = hi;
+    *reinterpret_cast<sep_h2*>(p + 32) = lo;
+}
+
+// ----------------------------------------------------------------------------------
+// Forward operands: xop[m][(j / 8, k, j % 8)] = c_j r (a wave per row, lanes along k) and
+// wop[o][(j / 8, k, j % 8)] = T_j(t+) - T_j(t-), each (row, k) R values in 16-byte stores. HBM-bound: four
+// bytes per value written.
+// ----------------------------------------------------------------------------------
+
+constexpr int kSepExpandBlocks = 2048;
+
+__device__ inline void sep_store8(_Float16* row, int64_t e, const float v[8]) {
+    sep_h8 hi, lo;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        _Float16 h, l;
+        sep_split(v[q], h, l);
+        hi[q] = h;
+        lo[q] = l;
+    }
+    _Float16* p = row + (e >> 5) * 64 + (e & 31);
+    *reinterpret_cast<sep_h8*>(p) = hi;
+    *reinterpret_cast<sep_h8*>(p + 32) = lo;
+}
+
+// Walks T_1, T_2, ... of both branches and hands out blocks of eight differences.
+struct SepChebPair {
+    double p0 = 1.0, p1, n0 = 1.0, n1, tp, tn;
+    __device__ SepChebPair(double a, double b) : p1(a), n1(b), tp(2.0 * a), tn(2.0 * b) {}
+    __device__ void next8(float* v, float scale) {  // T_j(t+) - T_j(t-) of the next eight j
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            v[q] = (float)(p1 - n1) * scale;
+            const double p2 = tp * p1 - p0, n2 = tn * n1 - n0;
+            p0 = p1;
+            p1 = p2;
+            n0 = n1;
+            n1 = n2;
+        }
+    }
+};
+
+// Where the per-cell kernels take the call: their prep, in the same launch.
+__global__ __launch_bounds__(256) void sep_expand_fwd_kernel(SepArgs a, PrepArgs prep) {
+    const SepHead h = *a.head;
+    const int R = h.terms;
+    if (R == 0) {
+        if (blockIdx.x < kPrepBlocksX + kPrepBlocksW) prep_block(prep, blockIdx.x);
+        return;
+    }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t slabs = sep_slabs_kj(a.K, R);
+    const int64_t kc = (a.K + 3) / 4 * 4;  // inputs with their padding
+    const int64_t row_waves = (int64_t)gridDim.x * 4;
+    const float as = a.in_affine ? a.in_affine[0] : 1.0f, ab = a.in_affine ? a.in_affine[1] : 0.0f;
+    float v[8];
+    for (int64_t row = (int64_t)blockIdx.x * 4 + wave; row < a.M + a.O; row += row_waves) {
+        if (row < a.M) {
+            float inv;
+            const float scale = sep_scale_of(sep_bound(h, a.tab, 0, a.xrow[row], (float)a.v_sat), &inv);
+            if (lane == 0) a.xscale[row] = inv / kSepQScale;
+            _Float16* dst = a.xop + row * slabs * 64;
+            for (int64_t k = lane; k < kc; k += 64) {
+                if (k < a.K) {
+                    const SepAt at = sep_at(h, sep_input(a, a.x[row * a.K + k], as, ab));
+                    for (int j = 0; j < R; j += 8) {
+                        const float4 lo = sep_eval4(a.tab, R, at, j), hi = sep_eval4(a.tab, R, at, j + 4);
+                        v[0] = lo.x * scale; v[1] = lo.y * scale; v[2] = lo.z * scale; v[3] = lo.w * scale;
+                        v[4] = hi.x * scale; v[5] = hi.y * scale; v[6] = hi.z * scale; v[7] = hi.w * scale;
+                        sep_store8(dst, kc * j + k * 8, v);
+                    }
+                } else {
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) v[q] = 0.0f;
+                    for (int j = 0; j < R; j += 8) sep_store8(dst, kc * j + k * 8, v);
+                }
+            }
+        } else {
+            const int64_t o = row - a.M;
+            _Float16* dst = a.wop + o * slabs * 64;
+            for (int64_t k = lane; k < kc; k += 64) {
+                const bool real = k < a.K;
+                const double tp = real ? ((double)a.wp[o * a.K + k] - h.wc) * h.inv_wh : 0.0;
+                const double tn = real ? ((double)a.wn[o * a.K + k] - h.wc) * h.inv_wh : 0.0;
+                SepChebPair c(tp, tn);
+                for (int j = 0; j < R; j += 8) {
+                    c.next8(v, kSepQScale);
+                    sep_store8(dst, kc * j + k * 8, v);
+                }
+            }
+        }
+    }
+}
+
+// ----------------------------------------------------------------------------------
+// Backward operands, inner index contiguous: xop[(k, j)][m] = d_j r, wop[(k, j)][o] = T_j(t+) -
+// T_j(t-) with tT[k][o] = {t+, t-}, gop[m][o] and gopT[o][m]. Tiles of 32 inputs (or rows of G)
+// by 128 inner elements go through LDS, so that reads run along the tensors' rows and writes
+// along the inner index. HBM-bound.
+// ----------------------------------------------------------------------------------
+
+__global__ __launch_bounds__(256) void sep_expand_bwd_kernel(SepArgs a, int x_blocks, int w_blocks, PrepArgs prep) {
+    const SepHead h = *a.head;
+    const int R = h.terms;
+    if (R == 0) {  // the per-cell kernels take the call: their prep
+        if (blockIdx.x < kPrepBlocksX + kPrepBlocksW) prep_block(prep, blockIdx.x);
+        return;
+    }
+    __shared__ float s_a[32][130], s_b[32][130];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int64_t m_slabs = sep_slabs(a.M), o_slabs = sep_slabs(a.O);
+    int b = blockIdx.x;
+    if (b < x_blocks) {
+        const int n_mt = (int)((a.M + 127) / 128);
+        const int64_t m0 = (int64_t)(b % n_mt) * 128, k0 = (int64_t)(b / n_mt) * 32;
+        const float as = a.in_affine ? a.in_affine[0] : 1.0f, ab = a.in_affine ? a.in_affine[1] : 0.0f;
+        for (int q = t; q < 32 * 128; q += 256) {
+            const int64_t m = m0 + (q >> 5), k = k0 + (q & 31);
+            s_a[q & 31][q >> 5] = m < a.M && k < a.K ? sep_input(a, a.x[m * a.K + k], as, ab) : 0.0f;
+        }
+        __syncthreads();
+        for (int kk = wave; kk < 32 && k0 + kk < a.K; kk += 4) {
+            const int64_t k = k0 + kk;
+            static_assert(kSepColChunks == 64, "a lane per chunk");
+            float2 range = a.xcol[(int64_t)lane * a.K + k];
+            sep_wave_minmax(range.x, range.y);
+            float inv;
+            const float scale = sep_scale_of(2.0f * sep_bound(h, a.tab, 0, range, (float)a.v_sat), &inv);
+            if (m0 == 0 && lane == 0) a.xscale[k] = inv;
+            const int ml = 2 * lane;
+            const int64_t m = m0 + ml;
+            if (m >= m_slabs * 32) continue;
+            const float s0 = m < a.M ? scale : 0.0f, s1 = m + 1 < a.M ? scale : 0.0f;
+            const SepAt p0 = sep_at(h, m < a.M ? s_a[kk][ml] : range.y);
+            const SepAt p1 = sep_at(h, m + 1 < a.M ? s_a[kk][ml + 1] : range.y);
+            for (int j = 0; j < R; j += 4) {
+                const float4 u = sep_eval4(a.tab, R, p0, j), v = sep_eval4(a.tab, R, p1, j);
+                _Float16* dst = a.xop + (k * R + j) * m_slabs * 64;
+                sep_store2(dst, m, u.x * s0, v.x * s1);
+                sep_store2(dst + m_slabs * 64, m, u.y * s0, v.y * s1);
+                sep_store2(dst + 2 * m_slabs * 64, m, u.z * s0, v.z * s1);
+                sep_store2(dst + 3 * m_slabs * 64, m, u.w * s0, v.w * s1);
+            }
+        }
+        return;
+    }
+    b -= x_blocks;
+    if (b < w_blocks) {
+        const int n_ot = (int)((a.O + 127) / 128);
+        const int64_t o0 = (int64_t)(b % n_ot) * 128, k0 = (int64_t)(b / n_ot) * 32;
+        for (int q = t; q < 32 * 128; q += 256) {
+            const int64_t o = o0 + (q >> 5), k = k0 + (q & 31);
+            const bool real = o < a.O && k < a.K;
+            s_a[q & 31][q >> 5] = real ? a.wp[o * a.K + k] : (float)h.wc;
+            s_b[q & 31][q >> 5] = real ? a.wn[o * a.K + k] : (float)h.wc;
+        }
+        __syncthreads();
+        for (int kk = wave; kk < 32 && k0 + kk < a.K; kk += 4) {
+            const int64_t k = k0 + kk;
+            const int ol = 2 * lane;
+            const int64_t o = o0 + ol;
+            if (o >= o_slabs * 32) continue;
+            double t_[4];
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                t_[2 * q] = ((double)s_a[kk][ol + q] - h.wc) * h.inv_wh;
+                t_[2 * q + 1] = ((double)s_b[kk][ol + q] - h.wc) * h.inv_wh;
+            }
+            if (a.need_w) {
+                reinterpret_cast<float4*>(a.tT + k * a.Op)[o >> 1] =
+                    make_float4((float)t_[0], (float)t_[1], (float)t_[2], (float)t_[3]);
+            }
+            if (!a.need_x) continue;
+            const bool r0 = o < a.O, r1 = o + 1 < a.O;
+            SepChebPair c0(r0 ? t_[0] : 0.0, r0 ? t_[1] : 0.0), c1(r1 ? t_[2] : 0.0, r1 ? t_[3] : 0.0);
+            float u[8], v[8];
+            for (int j = 0; j < R; j += 8) {
+                c0.next8(u, kSepQScale);
+                c1.next8(v, kSepQScale);
+                _Float16* dst = a.wop + (k * R + j) * o_slabs * 64;
+#pragma unroll
+                for (int q = 0; q < 8; ++q) sep_store2(dst + q * o_slabs * 64, o, u[q], v[q]);
+            }
+        }
+        return;
+    }
+    b -= w_blocks;
+    if (b >= (int)((a.O + 127) / 128 * ((a.M + 31) / 32))) return;  // blocks that only the prep needs
+    // G: tiles of 32 rows by 128 outputs
+    const int n_ot = (int)((a.O + 127) / 128);
+    const int64_t o0 = (int64_t)(b % n_ot) * 128, m0 = (int64_t)(b / n_ot) * 32;
+    for (int q = t; q < 32 * 128; q += 256) {
+        const int64_t m = m0 + (q >> 7), o = o0 + (q & 127);
+        s_a[q >> 7][q & 127] = m < a.M && o < a.O ? a.g[m * a.ldg + o] : 0.0f;
+    }
+    __syncthreads();
+    if (a.need_x) {
+        for (int mm = wave; mm < 32 && m0 + mm < a.M; mm += 4) {
+            const int64_t m = m0 + mm, o = o0 + 2 * lane;
+            float inv;
+            const float scale = sep_scale_of(__uint_as_float(a.grow[m]), &inv);
+            if (o0 == 0 && lane == 0) a.gscale[m] = inv / kSepQScale;
+            if (o < o_slabs * 32)
+                sep_store2(a.gop + m * o_slabs * 64, o, s_a[mm][2 * lane] * scale, s_a[mm][2 * lane + 1] * scale);
+        }
+    }
+    if (a.need_w) {
+        // 16 lanes hold the 32 tokens of one output: 16 outputs at a time
+        for (int q = t >> 4; q < 128 && o0 + q < a.O; q += 16) {
+            const int64_t o = o0 + q;
+            unsigned big = 0;
+            for (int c = t & 15; c < kSepColChunks; c += 16) big = max(big, a.gcol[(int64_t)c * a.O + o]);
+            for (int d = 8; d > 0; d >>= 1) big = max(big, (unsigned)__shfl_xor((int)big, d, 16));
+            float inv;
+            const float scale = sep_scale_of(__uint_as_float(big), &inv);
+            if (m0 == 0 && (t & 15) == 0) a.gscaleT[o] = inv;
+            const int mm = 2 * (t & 15);
+            sep_store2(a.gopT + o * m_slabs * 64, m0 + mm, s_a[mm][q] * scale, s_a[mm + 1][q] * scale);
+        }
+    }
+}
+
+// ----------------------------------------------------------------------------------
+// The product of two operands of hi/lo slabs, C[i][j] = sum_e A[i][e] B[j][e]: tiles of
+// (WM MI 32) x (WN NI 32), one slab (32 inner elements, 128 bytes per row) of both operands at
+// a time in two LDS buffers. A slab's loads are issued before the arithmetic of the one
+// before it, which takes three products per pair of fragments (hi hi, hi lo, lo hi):
+// 3072 matrix-core cycles per 64 KB of operands for the 256 x 256 tile, so that one buffer
+// ahead covers the memory's latency and the operands need ~21 bytes per cycle and CU. Rows are
+// 128 bytes and their eight 16-byte parts are stored at part ^ (row / 2 % 8), so that the 16
+// rows that a quarter-wave reads lie on different banks. Rows past the operand's end read its
+// last row (their results are dropped).
+// Blocks are dealt so that each XCD works on neighbouring tiles (whose operands its L2 holds).
+// ----------------------------------------------------------------------------------
+
+enum SepEpilogue { kSepForward, kSepDx, kSepDv };
+
+struct SepGemm {
+    const uint4* a;
+    const uint4* b;
+    const SepHead* head;
+    int64_t a_rows, b_rows;   // a_rows: per term where it depends on R (rows_of_terms)
+    int rows_of_terms;        // 1: the A operand has a_rows * R rows
+    int64_t inner;            // inner elements; with inner_of_terms the (k, j) index of a_rows... K inputs
+    int inner_of_terms;
+    int n_split;
+    int tiles_a, tiles_b;     // at the most terms
+    float* out;               // forward: planes [n_split][M][O]; dX: [n_split][M][K]; dVth: [n_split][2][Kp][Op]
+    int64_t M, K, O, Kp, Op;
+    const float* scale_a;     // forward [M], dVth [K]
+    const float* scale_b;     // dX [M], dVth [O]
+    // dX
+    const float* x;
+    const float* in_affine;
+    float in_lo, in_hi;
+    const float* tab2;
+    // dVth
+    const float2* tT;
+};
+
+template <int WM, int WN, int MI, int NI, SepEpilogue EPI>
+__global__ __launch_bounds__(WM * WN * 64, 2) void sep_gemm_kernel(SepGemm g) {
+    constexpr int kThreads = WM * WN * 64, TM = WM * MI * 32, TN = WN * NI * 32;
+    constexpr int kLoadA = TM * 8 / kThreads, kLoadB = TN * 8 / kThreads, kRowStep = kThreads / 8;
+    extern __shared__ __attribute__((aligned(16))) char s_sep[];
+    const SepHead* head = g.head;
+    const int R = __builtin_amdgcn_readfirstlane(head->terms);
+    if (R == 0) return;
+    const int64_t a_rows = g.rows_of_terms ? g.a_rows * R : g.a_rows;
+    const int slabs = (int)(g.inner_of_terms ? sep_slabs_kj(g.inner, R) : sep_slabs(g.inner));
+    const int ta = (int)((a_rows + TM - 1) / TM), tb = g.tiles_b;
+    // blocks run over the XCDs round robin: give XCD c the tiles [c n / 8, (c + 1) n / 8)
+    const int n = ta * tb * g.n_split;
+    int id = blockIdx.x;
+    if (id >= n) return;
+    {
+        const int per = n / 8, rest = n % 8, xcd = id & 7;
+        id = xcd * per + (xcd < rest ? xcd : rest) + (id >> 3);
+    }
+    // tiles of one split in groups of four along A: neighbours share both operands
+    const int split = id / (ta * tb);
+    id -= split * (ta * tb);
+    const int group = id / (4 * tb), in_group = id - group * 4 * tb;
+    const int height = min(4, ta - group * 4);
+    const int tile_a = group * 4 + in_group % height, tile_b = in_group / height;
+    const int64_t a0 = (int64_t)tile_a * TM, b0 = (int64_t)tile_b * TN;
+    const int s_begin = (int)((int64_t)slabs * split / g.n_split), s_end = (int)((int64_t)slabs * (split + 1) / g.n_split);
+
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int wr = wave / WN, wc = wave % WN;
+    const int part = t & 7, row0 = t >> 3;
+    unsigned pa[kLoadA], pb[kLoadB];  // byte offsets (an operand holds less than 4 GiB)
+#pragma unroll
+    for (int q = 0; q < kLoadA; ++q) {
+        const int64_t row = a0 + row0 + q * kRowStep;
+        pa[q] = (unsigned)(((row < a_rows ? row : a_rows - 1) * slabs * 8 + part) * 16);
+    }
+#pragma unroll
+    for (int q = 0; q < kLoadB; ++q) {
+        const int64_t row = b0 + row0 + q * kRowStep;
+        pb[q] = (unsigned)(((row < g.b_rows ? row : g.b_rows - 1) * slabs * 8 + part) * 16);
+    }
+    constexpr int kBuf = (TM + TN) * 128;
+    // kRowStep rows further on the swizzle is the same: kRowStep is a multiple of 16
+    static_assert(kRowStep % 16 == 0, "");
+    const int st_off = row0 * 128 + ((part ^ ((row0 >> 1) & 7)) << 4);
+    const int fl = lane & 31, fh = lane >> 5;
+    const int frag = fl * 128 + ((fh ^ ((fl >> 1) & 7)) << 4);
+    const int fa = wr * MI * 32 * 128, fb = TM * 128 + wc * NI * 32 * 128;
+
+    sep_f16 acc[MI][NI];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NI; ++j)
+#pragma unroll
+            for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.0f;
+
+    const char* abase = reinterpret_cast<const char*>(g.a);
+    const char* bbase = reinterpret_cast<const char*>(g.b);
+    sep_u4 ra[kLoadA], rb[kLoadB];
+    auto load = [&](int s) {
+#pragma unroll
+        for (int q = 0; q < kLoadA; ++q) ra[q] = *reinterpret_cast<const sep_u4*>(abase + (pa[q] + (unsigned)s * 128u));
+#pragma unroll
+        for (int q = 0; q < kLoadB; ++q) rb[q] = *reinterpret_cast<const sep_u4*>(bbase + (pb[q] + (unsigned)s * 128u));
+    };
+    auto store = [&](int buf) {
+        char* base = s_sep + buf * kBuf + st_off;
+#pragma unroll
+        for (int q = 0; q < kLoadA; ++q) *reinterpret_cast<sep_u4*>(base + q * kRowStep * 128) = ra[q];
+#pragma unroll
+        for (int q = 0; q < kLoadB; ++q) *reinterpret_cast<sep_u4*>(base + TM * 128 + q * kRowStep * 128) = rb[q];
+    };
+    if (s_begin < s_end) {
+        load(s_begin);
+        store(0);
+    }
+    __syncthreads();
+    for (int s = s_begin; s < s_end; ++s) {
+        const int buf = (s - s_begin) & 1;
+        const bool more = s + 1 < s_end;
+        if (more) load(s + 1);
+        const char* base = s_sep + buf * kBuf;
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            sep_h8 ah[MI], al[MI], bh[NI], bl[NI];
+            const int off = frag ^ (ks << 5);  // parts ks * 2 + fh (hi), + 4 (lo)
+#pragma unroll
+            for (int i = 0; i < MI; ++i) {
+                ah[i] = *reinterpret_cast<const sep_h8*>(base + fa + i * 4096 + off);
+                al[i] = *reinterpret_cast<const sep_h8*>(base + fa + i * 4096 + (off ^ 64));
+            }
+#pragma unroll
+            for (int j = 0; j < NI; ++j) {
+                bh[j] = *reinterpret_cast<const sep_h8*>(base + fb + j * 4096 + off);
+                bl[j] = *reinterpret_cast<const sep_h8*>(base + fb + j * 4096 + (off ^ 64));
+            }
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int j = 0; j < NI; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i], bl[j], acc[i][j], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int j = 0; j < NI; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[i], bh[j], acc[i][j], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int j = 0; j < NI; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i], bh[j], acc[i][j], 0, 0, 0);
+        }
+        if (more) store(buf ^ 1);
+        __syncthreads();
+    }
+
+    // lane (fl, fh) holds rows q % 4 + 8 (q / 4) + 4 fh of column fl of each 32 x 32 tile
+    if constexpr (EPI == kSepForward) {
+        float* out = g.out + (int64_t)split * g.M * g.O;
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                const int64_t m = a0 + (wr * MI + i) * 32 + (q & 3) + 8 * (q >> 2) + 4 * fh;
+                if (m >= g.M) continue;
+                const float sc = g.scale_a[m];
+#pragma unroll
+                for (int j = 0; j < NI; ++j) {
+                    const int64_t o = b0 + (wc * NI + j) * 32 + fl;
+                    if (o < g.O) out[m * g.O + o] = acc[i][j][q] * sc;
+                }
+            }
+        }
+    } else if constexpr (EPI == kSepDx) {
+        const SepHead h = *head;
+        const float as = g.in_affine ? g.in_affine[0] : 1.0f, ab = g.in_affine ? g.in_affine[1] : 0.0f;
+        float* out = g.out + (int64_t)split * g.M * g.K;
+        const int nb = R / 8, sh = __builtin_ctz(nb);
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+            const int64_t m = b0 + (wc * NI + j) * 32 + fl;
+            const int64_t mc = m < g.M ? m : g.M - 1;
+            const float sc = g.scale_b[mc];
+            float sum = 0.0f;
+#pragma unroll
+            for (int i = 0; i < MI; ++i) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {  // eight rows (k, 8 jb ..)
+                    const int64_t block = (a0 + (wr * MI + i) * 32) / 8 + q;
+                    const int64_t k = block >> sh;
+                    const int jb = (int)block & (nb - 1);
+                    const int64_t kc = k < g.K ? k : g.K - 1;
+                    const float xr = g.x[mc * g.K + kc];
+                    const SepAt at = sep_at(h, g.in_affine ? input_map(xr, as, ab, g.in_lo, g.in_hi) : xr);
+                    const float4 v = sep_eval4(g.tab2, R, at, jb * 8 + 4 * fh);
+                    float s = acc[i][j][4 * q] * v.x;
+                    s = fmaf(acc[i][j][4 * q + 1], v.y, s);
+                    s = fmaf(acc[i][j][4 * q + 2], v.z, s);
+                    s = fmaf(acc[i][j][4 * q + 3], v.w, s);
+                    sum += s;
+                    if (jb == nb - 1) {
+                        sum += __shfl_xor(sum, 32);
+                        if (fh == 0 && m < g.M && k < g.K) out[m * g.K + k] = sum * sc;
+                        sum = 0.0f;
+                    }
+                }
+            }
+        }
+    } else {
+        float* out = g.out + (int64_t)split * 2 * g.Kp * g.Op;
+        const int nb = R / 8, sh = __builtin_ctz(nb);
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+            const int64_t o = b0 + (wc * NI + j) * 32 + fl;
+            const int64_t oc = o < g.O ? o : g.O - 1;
+            const float sb = g.scale_b[oc];
+            float sp = 0.0f, sn = 0.0f, p0 = 0.0f, p1 = 0.0f, n0 = 0.0f, n1 = 0.0f;
+            float2 tt = make_float2(0.0f, 0.0f);
+#pragma unroll
+            for (int i = 0; i < MI; ++i) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int64_t block = (a0 + (wr * MI + i) * 32) / 8 + q;
+                    const int64_t k = block >> sh;
+                    const int jb = (int)block & (nb - 1);
+                    const int64_t kc = k < g.K ? k : g.K - 1;
+                    if (jb == 0) {
+                        tt = g.tT[kc * g.Op + oc];
+                        p0 = n0 = 1.0f;  // T_0, T_1
+                        p1 = tt.x;
+                        n1 = tt.y;
+                    }
+                    float vp[4], vn[4];  // this lane's four of the eight polynomials
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        vp[e & 3] = e < 4 || fh ? p0 : vp[e & 3];
+                        vn[e & 3] = e < 4 || fh ? n0 : vn[e & 3];
+                        const float p2 = fmaf(2.0f * tt.x, p1, -p0), n2 = fmaf(2.0f * tt.y, n1, -n0);
+                        p0 = p1;
+                        p1 = p2;
+                        n0 = n1;
+                        n1 = n2;
+                    }
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        sp = fmaf(acc[i][j][4 * q + e], vp[e], sp);
+                        sn = fmaf(acc[i][j][4 * q + e], vn[e], sn);
+                    }
+                    if (jb == nb - 1) {
+                        sp += __shfl_xor(sp, 32);
+                        sn += __shfl_xor(sn, 32);
+                        if (o < g.O && k < g.K)
+                            out[((int64_t)fh * g.Kp + k) * g.Op + o] = (fh ? sn : sp) * sb * g.scale_a[k];
+                        sp = sn = 0.0f;
+                    }
+                }
+            }
+        }
+    }
+}
+
+__device__ bool sep_takes(const SepHead* head) {
+    return head != nullptr && __builtin_amdgcn_readfirstlane(head->terms) != 0;
+}
+
+// Finishes the forward (split_reduce_body) from the planes of whichever path took the call; a
+// per-cell plan without a split (cell.n_split <= 1) has written its outputs itself.
+template <int VEC>
+__global__ __launch_bounds__(256) void sep_reduce_fwd_kernel(FwdArgs sep, FwdArgs cell, const SepHead* head,
+                                                             int clamp_out) {
+    if (sep_takes(head))
+        split_reduce_body<VEC>(sep, clamp_out);
+    else if (cell.n_split > 1)
+        split_reduce_body<VEC>(cell, clamp_out);
+}
+
+// grad_reduce_kernel's dX and dVth parts from the planes of whichever path took the call.
+__global__ __launch_bounds__(256) void sep_reduce_bwd_kernel(DxReduceArgs dx, DxReduceArgs dx_cell, int dx_blocks,
+                                                             DvReduceArgs dv, DvReduceArgs dv_cell, int dv_blocks,
+                                                             const SepHead* head) {
+    const int b = blockIdx.x;
+    if (sep_takes(head)) {
+        if (b < dx_blocks)
+            dx_reduce_block(dx, b, dx_blocks);
+        else
+            dv_reduce_block(dv, b - dx_blocks, dv_blocks);
+    } else {
+        if (b < dx_blocks)
+            dx_reduce_block(dx_cell, b, dx_blocks);
+        else
+            dv_reduce_block(dv_cell, b - dx_blocks, dv_blocks);
+    }
+}
+
+// ----------------------------------------------------------------------------------
+// Host side: plans and launches.
+// ----------------------------------------------------------------------------------
+
+// Exact-formula calls of fewer cells M K O run the per-cell kernels; larger ones consider 16 terms
+// at most, 32 from 2^28 cells and 64 from 2^30. The operands' passes cost R bytes x 4 per input
+// of x and of the thresholds whatever the other side's length is, so many terms need a long
+// other side. Measured (one box, forward and backward, us, per-cell kernels against the
+// contraction, K x O at M tokens): 8 terms 192 x 768 at 256 (2^25.2 cells) 66 / 104 against
+// 51 / 90, at 128 43 / 87 against 50 / 84; 16 terms at 256 66 / 104 against 60 / 103, at 512
+// 97 / 165 against 64 / 114; 32 terms 768 x 3072 at 128 (2^28.2) 317 / 625 against 281 / 436,
+// at 64 225 / 359 against 261 / 347; 64 terms at 512 (2^30.2) 1120 / 2202 against 798 / 1435,
+// at 256 592 / 1216 against 570 / 936. A call that turns out not to suit pays the statistics
+// and the launches that return: 13-20 us.
+#ifndef ISA_EKV_CONTRACT_MIN_CELLS
+#define ISA_EKV_CONTRACT_MIN_CELLS (1 << 25)
+#endif
+
+struct SepPlan {
+    int max_terms;  // 0: not considered
+    bool big;       // 256 x 256 tiles instead of 128 x 128
+    int split, split_dx, split_dv;
+    int64_t Kp, Op;
+    size_t off_head, off_part, off_row, off_col, off_grow, off_gcol, off_tab, off_tab2, off_xop, off_wop, off_gop,
+        off_gopT, off_scale, off_gscale, off_gscaleT, off_tT, off_planes, off_planes_dv, bytes;
+};
+
+constexpr int64_t kSepOperandBytes = (int64_t)2 << 30;  // of one operand, at most (32-bit byte offsets)
+
+// Splits of a product's inner length: the count (each at least 8 slabs) that makes the launch's
+// time least, in slabs of one tile: rounds of blocks over the CUs (one 256 x 256 block each,
+// two of 128 x 128), each the split's slabs and about 5 more of prologue and epilogue, and for
+// every further plane its write and read back against ~1.4 us a slab.
+inline int sep_splits(int64_t tiles, int64_t slabs, bool big, double plane_bytes) {
+    int best = 1;
+    double best_cost = 0.0;
+    const int64_t at_once = big ? kCUs : 2 * kCUs;
+    for (int s = 1; s <= 16 && (s == 1 || slabs / s >= 8); ++s) {
+        const double rounds = (double)((tiles * s + at_once - 1) / at_once);
+        const double cost = rounds * ((double)(slabs + s - 1) / s + 5.0) + s * plane_bytes / 4e12 / (big ? 1.4e-6 : 0.7e-6);
+        if (s == 1 || cost < best_cost) {
+            best = s;
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
+inline bool sep_big(int64_t rows_a, int64_t rows_b, int64_t slabs) {
+    // 256 x 256 tiles halve the operand reads per product; they need enough of them
+    return ((rows_a + 255) / 256) * ((rows_b + 255) / 256) * (slabs / 16 + 1) >= 2 * kCUs && rows_a >= 192 && rows_b >= 192;
+}
+
+SepPlan plan_sep(int64_t M, int64_t K, int64_t O, bool backward, bool need_x, bool need_w, size_t base) {
+    SepPlan p{};
+    p.bytes = base;
+    const double cells = (double)M * (double)K * (double)O;
+    if (M < 16 || O < 16 || K < 8 || cells < (double)ISA_EKV_CONTRACT_MIN_CELLS) return p;
+    p.Kp = round_up(K, 8);
+    p.Op = round_up(O, 256);
+    const int64_t Mr = round_up(M, 32), Or = round_up(O, 32), Kr = round_up(K, 4);
+    int terms = cells >= 1 << 30 ? 64 : cells >= 1 << 28 ? 32 : 16;
+    while (terms >= 8 && (Mr * Kr * terms * 4 >= kSepOperandBytes || Or * Kr * terms * 4 >= kSepOperandBytes)) terms /= 2;
+    if (terms < 8 || Mr * Or * 4 >= kSepOperandBytes) return p;
+    p.max_terms = terms;
+    size_t off = (size_t)round_up((int64_t)base, 256);
+    auto take = [&](int64_t bytes) {
+        const size_t at = off;
+        off += (size_t)round_up(bytes, 256);
+        return at;
+    };
+    p.off_head = take(sizeof(SepHead));
+    p.off_part = take(kSepStatBlocks * 24);
+    p.off_tab = take((int64_t)kSepGridMax * 8 * 4 * (terms / 8));
+    p.off_xop = take(Mr * Kr * terms * 4);
+    p.off_wop = take(Or * Kr * terms * 4);
+    if (!backward) {
+        p.off_row = take(M * 8);
+        p.off_scale = take(M * 4);
+        const int64_t slabs = (K + 3) / 4;
+        p.big = sep_big(M, O, slabs);
+        const int64_t tile = p.big ? 256 : 128;
+        p.split = sep_splits(((M + tile - 1) / tile) * ((O + tile - 1) / tile), slabs, p.big, 8.0 * M * O);
+        p.off_planes = take((int64_t)p.split * M * O * 4);
+    } else {
+        p.off_tab2 = take((int64_t)kSepGridMax * 8 * 4 * (terms / 8));
+        p.off_col = take(kSepColChunks * K * 8);
+        p.off_grow = take(M * 4);
+        p.off_gcol = take(kSepColChunks * O * 4);
+        p.off_gop = take(Mr * Or * 4);
+        p.off_gopT = take(Mr * Or * 4);
+        p.off_scale = take(K * 4);
+        p.off_gscale = take(M * 4);
+        p.off_gscaleT = take(O * 4);
+        p.off_tT = take(K * p.Op * 8);
+        p.big = sep_big(8 * K, std::min(M, O), std::min(M, O) / 32);
+        const int64_t tile = p.big ? 256 : 128, tk = (8 * K + tile - 1) / tile;
+        p.split_dx = sep_splits(tk * ((M + tile - 1) / tile), (O + 31) / 32, p.big, 8.0 * M * K);
+        p.split_dv = sep_splits(tk * ((O + tile - 1) / tile), (M + 31) / 32, p.big, 16.0 * p.Kp * p.Op);
+        if (need_x) p.off_planes = take((int64_t)p.split_dx * M * K * 4);
+        if (need_w) p.off_planes_dv = take((int64_t)p.split_dv * 2 * p.Kp * p.Op * 4);
+    }
+    p.bytes = off;
+    return p;
+}
+
+template <SepEpilogue EPI>
+void launch_sep_gemm(bool big, int max_terms, SepGemm g, hipStream_t s) {
+    const int64_t tile = big ? 256 : 128;
+    const int64_t rows_a = g.rows_of_terms ? g.a_rows * max_terms : g.a_rows;
+    g.tiles_b = (int)((g.b_rows + tile - 1) / tile);
+    const dim3 grid((unsigned)((rows_a + tile - 1) / tile * g.tiles_b * g.n_split));
+    if (big)
+        hipLaunchKernelGGL((sep_gemm_kernel<2, 4, 4, 2, EPI>), grid, dim3(512), 131072, s, g);
+    else
+        hipLaunchKernelGGL((sep_gemm_kernel<2, 2, 2, 2, EPI>), grid, dim3(256), 65536, s, g);
+}
+
+constexpr int kSepTableBlocks = 256;
+
+// The forward up to its planes (statistics, tables, operands, product).
+hipError_t sep_forward(const SepPlan& p, SepArgs a, const PrepArgs& prep, char* ws, hipStream_t s) {
+    a.head = reinterpret_cast<SepHead*>(ws + p.off_head);
+    a.xpart = reinterpret_cast<float2*>(ws + p.off_part);
+    a.wpart = a.xpart + kSepStatBlocks;
+    a.xrow = reinterpret_cast<float2*>(ws + p.off_row);
+    a.tab = reinterpret_cast<float*>(ws + p.off_tab);
+    a.xop = reinterpret_cast<_Float16*>(ws + p.off_xop);
+    a.wop = reinterpret_cast<_Float16*>(ws + p.off_wop);
+    a.xscale = reinterpret_cast<float*>(ws + p.off_scale);
+    a.max_terms = p.max_terms;
+    hipLaunchKernelGGL(sep_stat_kernel, dim3(2 * kSepStatBlocks), dim3(1024), 0, s, a);
+    hipLaunchKernelGGL(sep_table_kernel, dim3(kSepTableBlocks), dim3(256), 0, s, a);
+    const int64_t expand = std::min<int64_t>((a.M + a.O + 3) / 4, kSepExpandBlocks);
+    hipLaunchKernelGGL(sep_expand_fwd_kernel, dim3((unsigned)std::max<int64_t>(expand, kPrepBlocksX + kPrepBlocksW)),
+                       dim3(256), 0, s, a, prep);
+    SepGemm g{};
+    g.a = reinterpret_cast<const uint4*>(a.xop);
+    g.b = reinterpret_cast<const uint4*>(a.wop);
+    g.head = a.head;
+    g.a_rows = a.M;
+    g.b_rows = a.O;
+    g.inner = a.K;
+    g.inner_of_terms = 1;
+    g.n_split = p.split;
+    g.out = reinterpret_cast<float*>(ws + p.off_planes);
+    g.M = a.M;
+    g.K = a.K;
+    g.O = a.O;
+    g.scale_a = a.xscale;
+    launch_sep_gemm<kSepForward>(p.big, p.max_terms, g, s);
+    return hipGetLastError();
+}
+
+// The backward up to its dX and dVth planes.
+hipError_t sep_backward(const SepPlan& p, SepArgs a, const PrepArgs& prep, char* ws, hipStream_t s) {
+    a.head = reinterpret_cast<SepHead*>(ws + p.off_head);
+    a.xpart = reinterpret_cast<float2*>(ws + p.off_part);
+    a.wpart = a.xpart + kSepStatBlocks;
+    a.gpart = reinterpret_cast<unsigned*>(a.wpart + kSepStatBlocks);
+    a.xcol = reinterpret_cast<float2*>(ws + p.off_col);
+    a.grow = reinterpret_cast<unsigned*>(ws + p.off_grow);
+    a.gcol = reinterpret_cast<unsigned*>(ws + p.off_gcol);
+    a.tab = reinterpret_cast<float*>(ws + p.off_tab);
+    a.tab2 = reinterpret_cast<float*>(ws + p.off_tab2);
+    a.xop = reinterpret_cast<_Float16*>(ws + p.off_xop);
+    a.wop = reinterpret_cast<_Float16*>(ws + p.off_wop);
+    a.gop = reinterpret_cast<_Float16*>(ws + p.off_gop);
+    a.gopT = reinterpret_cast<_Float16*>(ws + p.off_gopT);
+    a.xscale = reinterpret_cast<float*>(ws + p.off_scale);
+    a.gscale = reinterpret_cast<float*>(ws + p.off_gscale);
+    a.gscaleT = reinterpret_cast<float*>(ws + p.off_gscaleT);
+    a.tT = reinterpret_cast<float2*>(ws + p.off_tT);
+    a.Op = p.Op;
+    a.max_terms = p.max_terms;
+    const int64_t col_blocks = kSepColChunks / 4 * ((a.need_w ? (a.O + 255) / 256 : 0) + (a.K + 255) / 256);
+    hipLaunchKernelGGL(sep_stat_kernel, dim3((unsigned)(3 * kSepStatBlocks + col_blocks)), dim3(1024), 0, s, a);
+    hipLaunchKernelGGL(sep_table_kernel, dim3(kSepTableBlocks), dim3(256), 0, s, a);
+    const int64_t kt = (a.K + 31) / 32, ot = (a.O + 127) / 128;
+    const int64_t x_blocks = a.need_w ? kt * ((a.M + 127) / 128) : 0, w_blocks = kt * ot, g_blocks = ot * ((a.M + 31) / 32);
+    const int64_t expand = x_blocks + w_blocks + g_blocks;
+    hipLaunchKernelGGL(sep_expand_bwd_kernel, dim3((unsigned)std::max<int64_t>(expand, kPrepBlocksX + kPrepBlocksW)),
+                       dim3(256), 0, s, a, (int)x_blocks, (int)w_blocks, prep);
+    SepGemm g{};
+    g.head = a.head;
+    g.M = a.M;
+    g.K = a.K;
+    g.O = a.O;
+    g.Kp = p.Kp;
+    g.Op = p.Op;
+    g.a_rows = a.K;
+    g.rows_of_terms = 1;
+    if (a.need_x) {
+        SepGemm d = g;
+        d.a = reinterpret_cast<const uint4*>(a.wop);
+        d.b = reinterpret_cast<const uint4*>(a.gop);
+        d.b_rows = a.M;
+        d.inner = a.O;
+        d.n_split = p.split_dx;
+        d.out = reinterpret_cast<float*>(ws + p.off_planes);
+        d.scale_b = a.gscale;
+        d.x = a.x;
+        d.in_affine = a.in_affine;
+        d.in_lo = a.in_lo;
+        d.in_hi = a.in_hi;
+        d.tab2 = a.tab2;
+        launch_sep_gemm<kSepDx>(p.big, p.max_terms, d, s);
+    }
+    if (a.need_w) {
+        SepGemm d = g;
+        d.a = reinterpret_cast<const uint4*>(a.xop);
+        d.b = reinterpret_cast<const uint4*>(a.gopT);
+        d.b_rows = a.O;
+        d.inner = a.M;
+        d.n_split = p.split_dv;
+        d.out = reinterpret_cast<float*>(ws + p.off_planes_dv);
+        d.scale_a = a.xscale;
+        d.scale_b = a.gscaleT;
+        d.tT = a.tT;
+        launch_sep_gemm<kSepDv>(p.big, p.max_terms, d, s);
+    }
+    return hipGetLastError();
+}

@@ -368,6 +368,9 @@ __global__ void lut_pack_kernel(const void* ti, const void* td, int n, int src_b
 // Token records: {c, r} (forward) or {c, r, -r / z_div, 0} (backward), r = 1/(1 + x/V_sat).
 // ----------------------------------------------------------------------------------
 
+struct SepHead;
+__device__ bool sep_takes(const SepHead* head);  // whether the contraction takes the call (null: no)
+
 struct PrepArgs {
     const float* x;
     const float* wp;
@@ -963,6 +966,7 @@ struct FwdArgs {
     int copy_window;        // LUT: > 0: the copies hold only the coordinate window, of at most this many records
     int mc_budget, mc_max;  // LUT: mc_budget > 0: the launch may hold up to mc_max windowed copies in this many LDS records
     unsigned long long* clock_acc;  // profiling: {cycles, wall ticks, blocks} of this kernel (BlockClock), or null
+    const SepHead* skip;    // the contraction's head: nothing to do where it takes the call
 };
 
 // The work of one forward wave.
@@ -1616,6 +1620,7 @@ __global__ __launch_bounds__(kFwdWaves * 64) void fwd_global_kernel(FwdArgs a) {
 // Exact-formula forward (reference: ekv_triton.py:69-91): same tiling, no table.
 template <int MR, bool SPLITS>
 __global__ __launch_bounds__(kFwdWaves * 64) void fwd_exact_kernel(FwdArgs a) {
+    if (sep_takes(a.skip)) return;
     const bool fast = exact_operands_in_fast_range(a.partials);
     FwdTile t;
     if (!fwd_tile<SPLITS>(a, MR, t)) return;
@@ -1654,6 +1659,7 @@ struct BwdArgs {
     int mc_budget, mc_max;  // split tables: the two-copy launch may hold up to mc_max windowed copies
     unsigned long long* clock_acc;  // profiling: {cycles, wall ticks, blocks} of this kernel (BlockClock), or null
     int xcd_order;          // ranked launch: 1 runs each token split's blocks on one XCD (xcd_work_index)
+    const SepHead* skip;    // the contraction's head: nothing to do where it takes the call
 };
 
 // LDS table views for the backward. Interleaved: one 16-byte record {A_I, dI, A_D, dD} per
@@ -2764,6 +2770,7 @@ __global__ __launch_bounds__(1024, ISA_EKV_BWD_MIN_BLOCKS) void bwd_global_kerne
 // holds only the dX transpose buffers.
 template <bool NEED_X, bool NEED_W>
 __global__ __launch_bounds__(1024) void bwd_exact_kernel(BwdArgs a) {
+    if (sep_takes(a.skip)) return;
     extern __shared__ float4 s_red_exact[];
     const bool fast = exact_operands_in_fast_range(a.partials);
     const int waves = blockDim.x >> 6;
@@ -3574,6 +3581,72 @@ __global__ __launch_bounds__(1024, 8) void valu_probe_kernel(int iters, const fl
     }
 }
 
+// Finishes a K-split forward (fwd_body wrote each split's partial sums): the splits are summed
+// in split order, then clamped (LUT) or scaled (exact, measured) and given the layer glue
+// exactly as fwd_body's epilogue does. Grid-stride over the [M][O] outputs, VEC of them per
+// thread (VEC = 4 when O and every pointer allow 16-byte accesses).
+template <int VEC>
+__device__ inline void split_reduce_body(const FwdArgs& a, int clamp_out) {
+    const int64_t n = (int64_t)a.M * a.O;
+    const int64_t nv = n / VEC;
+    const bool has_r = a.glue && a.r_tia != nullptr;
+    const float r = has_r ? tia_gain(a.r_tia, a.r_log_scale, a.r_log_lo, a.r_log_hi) : 1.0f;
+    unsigned ymax = 0;
+    for (int64_t ev = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; ev < nv; ev += (int64_t)gridDim.x * blockDim.x) {
+        float v[VEC], id[VEC];
+        if constexpr (VEC == 4) {
+            float4 t = reinterpret_cast<const float4*>(a.split_part)[ev];
+            for (int sp = 1; sp < a.n_split; ++sp) {
+                const float4 u = reinterpret_cast<const float4*>(a.split_part + (size_t)sp * n)[ev];
+                t.x += u.x;
+                t.y += u.y;
+                t.z += u.z;
+                t.w += u.w;
+            }
+            v[0] = t.x;
+            v[1] = t.y;
+            v[2] = t.z;
+            v[3] = t.w;
+        } else {
+            v[0] = a.split_part[ev];
+            for (int sp = 1; sp < a.n_split; ++sp) v[0] += a.split_part[(size_t)sp * n + ev];
+        }
+#pragma unroll
+        for (int i = 0; i < VEC; ++i)
+            id[i] = clamp_out ? fminf(fmaxf(v[i], a.out_min), a.out_max) : v[i] * a.out_scale;
+        const int64_t e = ev * VEC;
+        if (!a.glue) {
+            if constexpr (VEC == 4)
+                reinterpret_cast<float4*>(a.out)[ev] = make_float4(id[0], id[1], id[2], id[3]);
+            else
+                a.out[e] = id[0];
+            continue;
+        }
+        const int o0 = (int)(e % a.O);  // VEC divides O: the VEC outputs share a row
+        float y[VEC];
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) {
+            const float yt = layer_tia(id[i], r, has_r, a.y_lo, a.y_hi);
+            ymax = max(ymax, layer_stat_bits(yt));
+            y[i] = layer_adc(yt, a.adc_scale, a.adc_shift, o0 + i);
+        }
+        if constexpr (VEC == 4) {
+            if (a.idiff) reinterpret_cast<float4*>(a.idiff)[ev] = make_float4(id[0], id[1], id[2], id[3]);
+            reinterpret_cast<float4*>(a.out)[ev] = make_float4(y[0], y[1], y[2], y[3]);
+        } else {
+            if (a.idiff) a.idiff[e] = id[0];
+            a.out[e] = y[0];
+        }
+    }
+    if (a.stat_bits) {  // every lane of the wave is here: the loop has no early exit
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) ymax = max(ymax, (unsigned)__shfl_xor((int)ymax, d, 64));
+        if ((threadIdx.x & 63) == 0) atomicMax(a.stat_bits, ymax);
+    }
+}
+
+#include "contraction.hpp"
+
 // ----------------------------------------------------------------------------------
 // Host-side planning shared by the workspace queries and the launches.
 // ----------------------------------------------------------------------------------
@@ -4097,6 +4170,7 @@ struct CallSetup {
     float k2, c2;     // exact: 2^(-V_D a_log2), V_D a_log2
     double cur_scale; // exact: I_S ln2^2 (current constant of the cells)
     double der_scale; // exact: 2 I_S ln2 / (2 n U_T) (derivative constant of the cells)
+    double inv_2nut, i_s, v_d;  // exact: the formula's constants
 };
 
 CallSetup lut_setup(const void* lut, int n_entries, float delta_min, float delta_max) {
@@ -4123,6 +4197,9 @@ int exact_setup(const double* params, CallSetup* cs) {
     cs->k2 = (float)std::exp2(-v_d * cs->a_log2);
     cs->cur_scale = i_s * ln2 * ln2;
     cs->der_scale = 2.0 * i_s * inv_2nut * ln2;
+    cs->inv_2nut = inv_2nut;
+    cs->i_s = i_s;
+    cs->v_d = v_d;
     if (!(cs->a_log2 < 1e30)) return fail(ISA_EKV_EINVAL, "2 n U_T too small");
     return 0;
 }
@@ -4186,68 +4263,9 @@ __global__ void stat_merge_kernel(const unsigned* bits, float* abs_max, double* 
     if (total) *total += count;
 }
 
-// Finishes a K-split forward (fwd_body wrote each split's partial sums): the splits are summed
-// in split order, then clamped (LUT) or scaled (exact, measured) and given the layer glue
-// exactly as fwd_body's epilogue does. Grid-stride over the [M][O] outputs, VEC of them per
-// thread (VEC = 4 when O and every pointer allow 16-byte accesses).
 template <int VEC>
 __global__ __launch_bounds__(256) void split_reduce_kernel(FwdArgs a, int clamp_out) {
-    const int64_t n = (int64_t)a.M * a.O;
-    const int64_t nv = n / VEC;
-    const bool has_r = a.glue && a.r_tia != nullptr;
-    const float r = has_r ? tia_gain(a.r_tia, a.r_log_scale, a.r_log_lo, a.r_log_hi) : 1.0f;
-    unsigned ymax = 0;
-    for (int64_t ev = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; ev < nv; ev += (int64_t)gridDim.x * blockDim.x) {
-        float v[VEC], id[VEC];
-        if constexpr (VEC == 4) {
-            float4 t = reinterpret_cast<const float4*>(a.split_part)[ev];
-            for (int sp = 1; sp < a.n_split; ++sp) {
-                const float4 u = reinterpret_cast<const float4*>(a.split_part + (size_t)sp * n)[ev];
-                t.x += u.x;
-                t.y += u.y;
-                t.z += u.z;
-                t.w += u.w;
-            }
-            v[0] = t.x;
-            v[1] = t.y;
-            v[2] = t.z;
-            v[3] = t.w;
-        } else {
-            v[0] = a.split_part[ev];
-            for (int sp = 1; sp < a.n_split; ++sp) v[0] += a.split_part[(size_t)sp * n + ev];
-        }
-#pragma unroll
-        for (int i = 0; i < VEC; ++i)
-            id[i] = clamp_out ? fminf(fmaxf(v[i], a.out_min), a.out_max) : v[i] * a.out_scale;
-        const int64_t e = ev * VEC;
-        if (!a.glue) {
-            if constexpr (VEC == 4)
-                reinterpret_cast<float4*>(a.out)[ev] = make_float4(id[0], id[1], id[2], id[3]);
-            else
-                a.out[e] = id[0];
-            continue;
-        }
-        const int o0 = (int)(e % a.O);  // VEC divides O: the VEC outputs share a row
-        float y[VEC];
-#pragma unroll
-        for (int i = 0; i < VEC; ++i) {
-            const float yt = layer_tia(id[i], r, has_r, a.y_lo, a.y_hi);
-            ymax = max(ymax, layer_stat_bits(yt));
-            y[i] = layer_adc(yt, a.adc_scale, a.adc_shift, o0 + i);
-        }
-        if constexpr (VEC == 4) {
-            if (a.idiff) reinterpret_cast<float4*>(a.idiff)[ev] = make_float4(id[0], id[1], id[2], id[3]);
-            reinterpret_cast<float4*>(a.out)[ev] = make_float4(y[0], y[1], y[2], y[3]);
-        } else {
-            if (a.idiff) a.idiff[e] = id[0];
-            a.out[e] = y[0];
-        }
-    }
-    if (a.stat_bits) {  // every lane of the wave is here: the loop has no early exit
-#pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) ymax = max(ymax, (unsigned)__shfl_xor((int)ymax, d, 64));
-        if ((threadIdx.x & 63) == 0) atomicMax(a.stat_bits, ymax);
-    }
+    split_reduce_body<VEC>(a, clamp_out);
 }
 
 // Points a forward launch at the plan's K split (no-op without one).
@@ -4258,6 +4276,18 @@ void set_split(const FwdPlan& p, char* ws, FwdArgs& fa) {
 }
 
 bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
+
+hipError_t finish_sep(const FwdArgs& sep, const FwdArgs& cell, const SepHead* head, bool clamp_out, hipStream_t s) {
+    const int64_t n = (int64_t)sep.M * sep.O;
+    const bool vec4 = sep.O % 4 == 0 && aligned16(sep.out) && (!sep.glue || !sep.idiff || aligned16(sep.idiff));
+    const int64_t work = vec4 ? n / 4 : n;
+    const unsigned blocks = (unsigned)std::min<int64_t>((work + 255) / 256, 8192);
+    if (vec4)
+        hipLaunchKernelGGL(sep_reduce_fwd_kernel<4>, dim3(blocks), dim3(256), 0, s, sep, cell, head, clamp_out ? 1 : 0);
+    else
+        hipLaunchKernelGGL(sep_reduce_fwd_kernel<1>, dim3(blocks), dim3(256), 0, s, sep, cell, head, clamp_out ? 1 : 0);
+    return hipGetLastError();
+}
 
 hipError_t finish_split(const FwdPlan& p, const FwdArgs& fa, bool clamp_out, hipStream_t s) {
     if (p.n_split <= 1) return hipSuccess;
@@ -4332,6 +4362,26 @@ FwdTableCfg fwd_table_cfg(int n_entries, int wpb, bool copies) {
     return t;
 }
 
+SepArgs make_sep(const CallSetup& cs, const float* x, const float* wp, const float* wn, int64_t M, int64_t K, int64_t O,
+                 float v_sat, const isa_ekv_glue* glue) {
+    SepArgs a{};
+    a.x = x;
+    a.wp = wp;
+    a.wn = wn;
+    a.M = M;
+    a.K = K;
+    a.O = O;
+    if (glue && glue->in_affine) {
+        a.in_affine = glue->in_affine;
+        a.in_lo = glue->in_lo;
+        a.in_hi = glue->in_hi;
+    }
+    a.a = cs.inv_2nut;
+    a.v_d = cs.v_d;
+    a.v_sat = v_sat;
+    return a;
+}
+
 int run_forward(const CallSetup& cs, const float* x, const float* vth_pos, const float* vth_neg, int64_t M,
                 int64_t K, int64_t O, float v_sat, float out_min, float out_max, float* out, void* workspace,
                 size_t workspace_bytes, hipStream_t s, const isa_ekv_glue* glue = nullptr,
@@ -4339,8 +4389,11 @@ int run_forward(const CallSetup& cs, const float* x, const float* vth_pos, const
     if (M == 0 || O == 0) return 0;
     if (!out) return fail(ISA_EKV_EINVAL, "out is null");
     const FwdPlan p = plan_forward_call(cs.exact, cs.n_entries, M, K, O);
-    if (!workspace || workspace_bytes < p.bytes)
-        return fail(ISA_EKV_EINVAL, "forward workspace too small (%zu < %zu bytes)", workspace_bytes, p.bytes);
+    SepPlan sp{};
+    sp.bytes = p.bytes;
+    if (cs.exact) sp = plan_sep(M, K, O, false, false, false, p.bytes);
+    if (!workspace || workspace_bytes < sp.bytes)
+        return fail(ISA_EKV_EINVAL, "forward workspace too small (%zu < %zu bytes)", workspace_bytes, sp.bytes);
     char* ws = static_cast<char*>(workspace);
     CallTimer call_timer(s, 2, timed);
     PrepArgs pa = make_prep(cs, x, vth_pos, vth_neg, M, K, O, p.Kp, p.Op, v_sat, 2, ws, p.off_xrec, p.off_wsT,
@@ -4348,7 +4401,14 @@ int run_forward(const CallSetup& cs, const float* x, const float* vth_pos, const
     const bool stats = glue && (glue->stat_abs_max || glue->stat_total);
     unsigned* stat_bits = stats ? reinterpret_cast<unsigned*>(ws + p.off_stat) : nullptr;
     pa.stat_bits = stat_bits;
-    hipLaunchKernelGGL(prep_kernel, dim3(kPrepBlocksX + kPrepBlocksW), dim3(256), 0, s, pa);
+    const SepHead* sep_head = nullptr;
+    if (sp.max_terms > 0) {  // its launches hold the prep for the case that it does not take the call
+        const hipError_t e = sep_forward(sp, make_sep(cs, x, vth_pos, vth_neg, M, K, O, v_sat, glue), pa, ws, s);
+        if (e != hipSuccess) return hip_fail(e, "forward contraction launch");
+        sep_head = reinterpret_cast<const SepHead*>(ws + sp.off_head);
+    } else {
+        hipLaunchKernelGGL(prep_kernel, dim3(kPrepBlocksX + kPrepBlocksW), dim3(256), 0, s, pa);
+    }
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return hip_fail(err, "forward prep launch");
     FwdArgs fa{};
@@ -4364,6 +4424,7 @@ int run_forward(const CallSetup& cs, const float* x, const float* vth_pos, const
     fa.Op = (int)p.Op;
     fa.n_mt = p.n_mt;
     fa.n_ot = p.n_ot;
+    fa.skip = sep_head;
     fa.out_min = out_min;
     fa.out_max = out_max;
     if (glue) {
@@ -4427,7 +4488,14 @@ int run_forward(const CallSetup& cs, const float* x, const float* vth_pos, const
     if (timed && !cs.exact) fa.clock_acc = clock_acc(0);
     launch_forward(cs.exact, gtab, p.mr, p.wpb, dim3(p.blocks), lds, s, fa);
     err = hipGetLastError();
-    if (err == hipSuccess) err = finish_split(p, fa, !cs.exact, s);
+    if (err == hipSuccess && !sep_head) err = finish_split(p, fa, !cs.exact, s);
+    if (err == hipSuccess && sep_head) {
+        FwdArgs fs = fa;  // the contraction's planes, in units of I_S
+        fs.n_split = sp.split;
+        fs.split_part = reinterpret_cast<float*>(ws + sp.off_planes);
+        fs.out_scale = (float)cs.i_s;
+        err = finish_sep(fs, fa, sep_head, !cs.exact, s);
+    }
     prof_stop(s, prof);
     if (err != hipSuccess) return hip_fail(err, "forward launch");
     if (stats) {
@@ -4487,8 +4555,11 @@ int run_backward(const CallSetup& cs, const float* x, const float* vth_pos, cons
     }
     if (!grad_out) return fail(ISA_EKV_EINVAL, "grad_out is null");
     const BwdPlan p = plan_backward(M, K, O, cs.exact ? 0 : cs.n_entries, need_x, need_w, glue != nullptr);
-    if (!workspace || workspace_bytes < p.bytes)
-        return fail(ISA_EKV_EINVAL, "backward workspace too small (%zu < %zu bytes)", workspace_bytes, p.bytes);
+    SepPlan sp{};
+    sp.bytes = p.bytes;
+    if (cs.exact && K > 0) sp = plan_sep(M, K, O, true, need_x, need_w, p.bytes);
+    if (!workspace || workspace_bytes < sp.bytes)
+        return fail(ISA_EKV_EINVAL, "backward workspace too small (%zu < %zu bytes)", workspace_bytes, sp.bytes);
     char* ws = static_cast<char*>(workspace);
     CallTimer call_timer(s, 3);
     float* col_part = reinterpret_cast<float*>(ws + p.off_glue);
@@ -4516,10 +4587,22 @@ int run_backward(const CallSetup& cs, const float* x, const float* vth_pos, cons
     }
     // the prep, and with the layer glue its gradient pass (G_eff for the main kernel)
     const PrepArgs pa = make_prep(cs, x, vth_pos, vth_neg, M, K, O, p.Kp, p.Op, v_sat, 4, ws, p.off_xrec, p.off_wsT,
-                                  p.off_xrec_alt, p.off_wsT_alt, p.off_part, glue);
-    const int64_t glue_blocks = glue ? (int64_t)kGlueBlocks * (p.Op / 256) : 0;
-    hipLaunchKernelGGL(bwd_prep_kernel, dim3((unsigned)(kPrepBlocksX + kPrepBlocksW + glue_blocks)), dim3(256), 0, s,
-                       pa, ga);
+                            p.off_xrec_alt, p.off_wsT_alt, p.off_part, glue);
+    const SepHead* sep_head = nullptr;
+    if (sp.max_terms > 0) {
+        SepArgs a = make_sep(cs, x, vth_pos, vth_neg, M, K, O, v_sat, glue);
+        a.g = grad_out;
+        a.ldg = O;
+        a.need_x = need_x;
+        a.need_w = need_w;
+        err = sep_backward(sp, a, pa, ws, s);
+        if (err != hipSuccess) return hip_fail(err, "backward contraction launch");
+        sep_head = reinterpret_cast<const SepHead*>(ws + sp.off_head);
+    } else {
+        const int64_t glue_blocks = glue ? (int64_t)kGlueBlocks * (p.Op / 256) : 0;
+        hipLaunchKernelGGL(bwd_prep_kernel, dim3((unsigned)(kPrepBlocksX + kPrepBlocksW + glue_blocks)), dim3(256), 0, s,
+                           pa, ga);
+    }
     err = hipGetLastError();
     if (err != hipSuccess) return hip_fail(err, "backward prep launch");
     const float* g = grad_out;
@@ -4556,6 +4639,7 @@ int run_backward(const CallSetup& cs, const float* x, const float* vth_pos, cons
     ba.m_chunk = p.m_chunk;
     ba.n_items = p.n_items;
     ba.dv_group = p.dv_group ? 1 : 0;
+    ba.skip = sep_head;
     float scale = 1.0f;
     if (cs.exact) {
         ba.k2 = cs.k2;
@@ -4669,11 +4753,24 @@ int run_backward(const CallSetup& cs, const float* x, const float* vth_pos, cons
     }
     const bool glue_after = gg && gg->in_affine;  // needs aff_part from the dX blocks
     const int first_blocks = dx_blocks + dv_blocks + (glue_after ? 0 : gl_blocks);
-    if (first_blocks > 0)
+    if (first_blocks > 0 && !sep_head)
         hipLaunchKernelGGL(grad_reduce_kernel, dim3((unsigned)first_blocks), dim3(256), 0, s, dxa, dx_blocks, dva,
                            dv_blocks, gra);
     if (need_glue && glue_after)
         hipLaunchKernelGGL(glue_reduce_kernel, dim3((unsigned)gl_blocks), dim3(256), 0, s, gra);
+    if (sep_head) {
+        DxReduceArgs dxs = dxa;  // the contraction's planes, in units of I_S
+        dxs.part = reinterpret_cast<const float*>(ws + sp.off_planes);
+        dxs.n_planes = sp.split_dx;
+        dxs.scale = (float)cs.i_s;
+        DvReduceArgs dvs = dva;
+        dvs.part = reinterpret_cast<const float*>(ws + sp.off_planes_dv);
+        dvs.n_split = sp.split_dv;
+        dvs.scale = (float)cs.i_s;
+        dvs.mode_word = nullptr;
+        hipLaunchKernelGGL(sep_reduce_bwd_kernel, dim3((unsigned)(dx_blocks + dv_blocks)), dim3(256), 0, s, dxs, dxa,
+                           dx_blocks, dvs, dva, dv_blocks, sep_head);
+    }
     err = hipGetLastError();
     if (err != hipSuccess) return hip_fail(err, "gradient reduction launch");
     return 0;
@@ -5143,7 +5240,7 @@ int isa_ekv_backward(const float* x, const float* vth_pos, const float* vth_neg,
 
 size_t isa_ekv_exact_forward_workspace(int64_t M, int64_t K, int64_t O) {
     if (M < 0 || K < 0 || O < 0) return 0;
-    return plan_forward(M, K, O, true).bytes;
+    return plan_sep(M, K, O, false, false, false, plan_forward(M, K, O, true).bytes).bytes;
 }
 
 int isa_ekv_exact_forward(const float* x, const float* vth_pos, const float* vth_neg, int64_t M, int64_t K,
@@ -5160,7 +5257,9 @@ int isa_ekv_exact_forward(const float* x, const float* vth_pos, const float* vth
 
 size_t isa_ekv_exact_backward_workspace(int64_t M, int64_t K, int64_t O, int need_grad_x, int need_grad_w) {
     if (M < 0 || K < 0 || O < 0) return 0;
-    return plan_backward(M, K, O, 0, need_grad_x != 0, need_grad_w != 0).bytes;
+    return plan_sep(M, K, O, true, need_grad_x != 0, need_grad_w != 0,
+                    plan_backward(M, K, O, 0, need_grad_x != 0, need_grad_w != 0).bytes)
+        .bytes;
 }
 
 int isa_ekv_exact_backward(const float* x, const float* vth_pos, const float* vth_neg, const float* grad_out,
