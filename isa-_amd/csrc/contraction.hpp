@@ -27,6 +27,19 @@
 // by the per-cell kernels, 0.30 ms here; backward 8.17 and 0.74 ms; error against float64 of
 // the forward 2.8e-6 and 2.6e-7, of dX 2.3e-6 and 3.4e-7, of dVth 3.5e-7 and 2.7e-7 (2-norm).
 //
+// Tables. A lookup is the line between two entries, L(c) = F(c) + S(c) a (1 - a) / 2 with F the
+// smooth function through the entries, S its second difference and a the coordinate's fraction
+// (the next term is smaller by the relative change from entry to entry, 1.5% at 4096 entries).
+// With a (1 - a) = 1/6 - sum_q cos(2 pi q a) / (pi q)^2 and c = xs - ws,
+//     L(xs - ws) = (F + S / 12)(xs - ws)
+//                  - sum_q S(xs - ws) (cos 2 pi q xs cos 2 pi q ws + sin 2 pi q xs sin 2 pi q ws) / (2 pi^2 q^2):
+// the first part is smooth and expands as above, the others are 1e-5 of it and take R / 4 terms
+// of S per cosine and sine in plain f16. Two harmonics (none from about 14000 entries on) keep
+// the remainder below the per-cell kernels' own rounding of coordinates and of the records'
+// intercepts: 4096 entries, initial thresholds, 2-norm against float64 lookups, forward 9.8e-6
+// by the lookups. Sums of T's differences give back the entries exactly. A table that
+// is not smooth (bf16 entries) runs the per-cell kernels.
+//
 // R is chosen per call on the device from the thresholds' spread (sep_terms); a call whose
 // operands do not suit (non-finite values, x near -V_sat or spread over more than the table
 // holds, thresholds spread too far) runs the per-cell kernels, which return at once otherwise.
@@ -36,11 +49,13 @@ typedef _Float16 sep_h2 __attribute__((ext_vector_type(2)));
 typedef float sep_f16 __attribute__((ext_vector_type(16)));
 typedef unsigned sep_u4 __attribute__((ext_vector_type(4)));
 
-constexpr int kSepStatBlocks = 256;     // blocks of each statistics pass (partials each)
+constexpr int kSepStatX = 1024, kSepStatW = 256;  // blocks of the ranges of x and of the thresholds
+constexpr int kSepStatG = 512;          // blocks of the largest |G| of each row
 constexpr int kSepColChunks = 64;       // row chunks of a column pass, at most
 constexpr int kSepGridMax = 16384;      // x-table points, at most
 constexpr double kSepStep = 0.0148;     // x-table step in units of 2 n U_T
 constexpr int kSepMaxTerms = 64;
+constexpr int kSepLutMin = 2900, kSepLutMax = 65536;  // table entries: the kinks small enough, a thread per partial
 constexpr float kSepQScale = 256.0f;    // of the threshold-side operand (values in [-2, 2])
 
 // Widest threshold spread, in units of 2 n U_T, that R = 8, 16, 32, 64 terms take: there the
@@ -50,16 +65,26 @@ __host__ __device__ inline int sep_terms(float spread_u) {
     return spread_u <= 1.12f ? 8 : spread_u <= 4.4f ? 16 : spread_u <= 11.0f ? 32 : spread_u <= 24.0f ? 64 : 0;
 }
 
+// Table calls: the per-cell kernels' own rounding (2e-6) allows a little more at 16 terms, and
+// 32 terms would cost what the lookups do.
+__host__ __device__ inline int sep_terms_lut(float spread_u) { return spread_u <= 1.12f ? 8 : spread_u <= 5.0f ? 16 : 0; }
+
 // What the passes of a call share, in its workspace.
 struct SepHead {
     int terms;    // 0: the per-cell kernels run
+    unsigned gmax;  // backward: bits of the largest |G|: not finite: the per-cell kernels run
+    int rough;    // the series does not converge as its terms assume: the per-cell kernels run
+    int harmonics;  // 1: the kinks' two harmonics are summed
     int n_grid;
+    float xlo, xhi, wlo, whi;
+    float lut_min, lut_scale;  // table coordinate (v - lut_min) * lut_scale
     float x0, step, inv_step; // table point i stands for x0 + i * step; step a power of two, x0 a multiple of it
     double wc, inv_wh, wh;   // t = (w - wc) * inv_wh
 };
 
-__device__ inline bool sep_gate(const SepHead* head, bool want) {
-    return head == nullptr || (head->terms != 0) == want;
+__device__ bool sep_takes(const SepHead* head) {
+    return head != nullptr && __builtin_amdgcn_readfirstlane(head->terms != 0 && head->rough == 0 &&
+                                                             head->gmax < 0x7f800000u) != 0;
 }
 
 struct SepArgs {
@@ -74,11 +99,17 @@ struct SepArgs {
     double a, v_d;           // 1 / (2 n U_T), V_D
     double v_sat;
     int max_terms;
+    // table (lut_n > 0): records {A, dT} or {A_I, dI, A_D, dD}
+    const float* lut;
+    int lut_n;
+    double lut_min, lut_scale;
+    double2* lut_val;        // [lut_n]: smooth part, second difference
+    float2* lut_info;        // per 256 entries {largest relative growth from entry to entry, 1 where they do not suit}
+    float* tabE;             // second difference's coefficients, -r e_i / (2 pi^2): [n_grid][R / 4]
     // workspace
     SepHead* head;
-    float2* xpart;           // [kSepStatBlocks]
-    float2* wpart;           // [kSepStatBlocks]
-    unsigned* gpart;         // [kSepStatBlocks]
+    float2* xpart;           // [kSepStatX]
+    float2* wpart;           // [kSepStatW]
     float2* xrow;            // forward: [M] row ranges of x
     float2* xcol;            // backward: [kSepColChunks][K]
     unsigned* grow;          // backward: [M] largest |G| of a row (bits)
@@ -89,6 +120,10 @@ struct SepArgs {
     _Float16* wop;           // forward [O][Kd], backward [K R][Od]
     _Float16* gop;           // backward [M][Od]
     _Float16* gopT;          // backward [O][Md]
+    _Float16* xoph;          // backward, harmonics: [K ng 8][Md] single f16, 64 a slab
+    _Float16* woph;          // backward, harmonics: [K ng 8][Od]
+    _Float16* goph;          // backward, harmonics: [M][Od]
+    _Float16* gophT;         // backward, harmonics: [O][Md]
     float* xscale;           // forward [M], backward [K]: inverse scale of xop's rows
     float* gscale;           // backward [M]
     float* gscaleT;          // backward [O]
@@ -105,6 +140,12 @@ __device__ inline float sep_input(const SepArgs& a, float x, float s, float b) {
 // terms of four inputs a slab (K padded to fours), tokens and outputs of the backward.
 __host__ __device__ inline int64_t sep_slabs_kj(int64_t K, int terms) { return (K + 3) / 4 * (terms / 8); }
 __host__ __device__ inline int64_t sep_slabs(int64_t n) { return (n + 31) / 32; }
+// Harmonics: an input has terms / 8 groups of eight values, slabs of 64 single f16. At 8 terms
+// one group, of each harmonic its two cosines and two sines; at 16 a group per harmonic, of four
+// cosines and four sines.
+__host__ __device__ inline int sep_groups(int terms, int harmonics) { return harmonics * (terms / 8); }
+__host__ __device__ inline int64_t sep_slabs_harm(int64_t K, int groups) { return (K + 7) / 8 * groups; }
+__host__ __device__ inline int64_t sep_slabs64(int64_t n) { return (n + 63) / 64; }
 
 // ----------------------------------------------------------------------------------
 // Statistics: ranges of x (per row forward, per column backward), of the thresholds, and the
@@ -125,19 +166,82 @@ __device__ inline void sep_wave_minmax(float& lo, float& hi) {
     }
 }
 
+// Block b of the table's 256-entry ranges: its entries from the records' differences (each block
+// sums those before its range itself), as the smooth part F + S / 12 and S, and whether they
+// suit: fourth differences within 3e-6 of the entries (what the cubic interpolation and the two
+// terms of the lookup's line leave out), and for the backward a slope table that is the current
+// table's slope (dX takes the currents from it; within 2e-5 of the difference).
+__device__ inline void sep_lut_block(const SepArgs& a, int b) {
+    constexpr int kHalo = 2, kSpan = 256 + 2 * kHalo;
+    __shared__ double s_t[kSpan];
+    __shared__ double s_sum[4];
+    __shared__ float s_growth[4];
+    __shared__ int s_bad;
+    const int t = threadIdx.x, n = a.lut_n;
+    const bool bwd = a.tab2 != nullptr;
+    const int rec = bwd ? 4 : 2, val = bwd ? 2 : 0;  // the slope table backward, the currents forward
+    const float* r0 = a.lut + (size_t)kPad * rec;
+    const int base = b * 256, first = max(base - kHalo, 0), count = min(n - first, kSpan);
+    if (t == 0) s_bad = 0;
+    double sum = 0.0;
+    for (int j = t; j < first; j += 256) sum += (double)r0[(size_t)j * rec + val + 1];
+    for (int d = 32; d > 0; d >>= 1) sum += __shfl_xor(sum, d);
+    if ((t & 63) == 0) s_sum[t >> 6] = sum;
+    for (int i = t; i < kSpan; i += 256)  // element i + 1 gets entry i's difference
+        if (i + 1 < kSpan) s_t[i + 1] = i + 1 < count ? (double)r0[(size_t)(first + i) * rec + val + 1] : 0.0;
+    __syncthreads();
+    if (t == 0) s_t[0] = (double)a.lut[val] + ((s_sum[0] + s_sum[1]) + (s_sum[2] + s_sum[3]));  // entry 0, padded
+    __syncthreads();
+    for (int d = 1; d < kSpan; d <<= 1) {
+        const double u = t >= d ? s_t[t - d] : 0.0;
+        const double v = t < kSpan - 256 && t + 256 >= d ? s_t[t + 256 - d] : 0.0;
+        __syncthreads();
+        s_t[t] += u;
+        if (t < kSpan - 256) s_t[t + 256] += v;
+        __syncthreads();
+    }
+    const int j = base + t, i = j - first;
+    float growth = 0.0f;
+    bool bad = false;
+    double second = 0.0;
+    if (j >= 1 && j + 1 < n) second = s_t[i - 1] - 2.0 * s_t[i] + s_t[i + 1];
+    if (j >= kHalo && j + kHalo < n) {
+        const double m2 = s_t[i - 2], m1 = s_t[i - 1], v = s_t[i], p1 = s_t[i + 1], p2 = s_t[i + 2];
+        const double fourth = fabs((m2 + p2) - 4.0 * (m1 + p1) + 6.0 * v);
+        if (!(fourth <= 3e-6 * fabs(v) + 1e-42)) bad = true;
+        if (v > 1e-30) growth = (float)((p1 - v) / v);
+        if (bwd) {  // the current's difference against the slope's integral (error of fourth order)
+            const double di = (double)r0[(size_t)j * 4 + 1];
+            const double want = (0.5 * (v + p1) - ((p2 - p1) - (v - m1)) / 24.0) / a.lut_scale;
+            const double cur = fabs((double)r0[(size_t)j * 4] + (double)(j + kPad) * di);
+            if (!(fabs(di - want) <= 2e-5 * fabs(want) + 4e-7 * cur + 1e-42)) bad = true;
+        }
+    }
+    if (j < n) a.lut_val[j] = make_double2(s_t[i] + second / 12.0, second);
+    if (bad) atomicOr(&s_bad, 1);
+    for (int d = 32; d > 0; d >>= 1) growth = fmaxf(growth, __shfl_xor(growth, d));
+    if ((t & 63) == 0) s_growth[t >> 6] = growth;
+    __syncthreads();
+    if (t == 0)
+        a.lut_info[b] = make_float2(fmaxf(fmaxf(s_growth[0], s_growth[1]), fmaxf(s_growth[2], s_growth[3])), (float)s_bad);
+}
+
 __device__ inline unsigned sep_bits(float v) { return __float_as_uint(v) & 0x7fffffffu; }
 
-// Blocks of 16 waves: kSepStatBlocks of x, kSepStatBlocks of the thresholds, then (g)
-// kSepStatBlocks of G's rows and kSepColChunks / 4 x ceil(O / 256) of its columns, and (xcol)
-// kSepColChunks / 4 x ceil(K / 256) of x's columns. Four loads in flight per thread.
-__global__ __launch_bounds__(1024) void sep_stat_kernel(SepArgs a) {
+// Blocks: kSepStatX of x, kSepStatW of the thresholds, (xcol) kSepColChunks x ceil(K / 256) of
+// x's columns, ceil(lut_n / 256) of the table, then the layer glue's gradient blocks (glue.geff).
+__global__ __launch_bounds__(256) void sep_stat_kernel(SepArgs a, GlueGradArgs glue) {
     int b = blockIdx.x;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const float as = a.in_affine ? a.in_affine[0] : 1.0f, ab = a.in_affine ? a.in_affine[1] : 0.0f;
-    if (b < kSepStatBlocks) {
+    if (b == 0 && t == 0) {
+        a.head->gmax = 0;
+        a.head->rough = 0;
+    }
+    if (b < kSepStatX) {
         float lo = INFINITY, hi = -INFINITY;
         if (a.xrow) {  // a wave per row
-            for (int64_t m = (int64_t)b * 16 + wave; m < a.M; m += (int64_t)kSepStatBlocks * 16) {
+            for (int64_t m = (int64_t)b * 4 + wave; m < a.M; m += (int64_t)kSepStatX * 4) {
                 float l = INFINITY, h = -INFINITY;
                 const float* row = a.x + m * a.K;
                 for (int64_t k = lane; k < a.K; k += 256) {
@@ -153,8 +257,8 @@ __global__ __launch_bounds__(1024) void sep_stat_kernel(SepArgs a) {
                 hi = fmaxf(hi, h);
             }
         } else {
-            const int64_t n = a.M * a.K, stride = (int64_t)kSepStatBlocks * 1024;
-            for (int64_t e = (int64_t)b * 1024 + t; e < n; e += 4 * stride) {
+            const int64_t n = a.M * a.K, stride = (int64_t)kSepStatX * 256;
+            for (int64_t e = (int64_t)b * 256 + t; e < n; e += 4 * stride) {
                 float v[4];
 #pragma unroll
                 for (int q = 0; q < 4; ++q) v[q] = a.x[e + q * stride < n ? e + q * stride : e];
@@ -165,23 +269,54 @@ __global__ __launch_bounds__(1024) void sep_stat_kernel(SepArgs a) {
         block_minmax(lo, hi, &a.xpart[b]);
         return;
     }
-    b -= kSepStatBlocks;
-    if (b < kSepStatBlocks) {
+    b -= kSepStatX;
+    if (b < kSepStatW) {
         float lo = INFINITY, hi = -INFINITY;
-        const int64_t n = a.O * a.K, stride = (int64_t)kSepStatBlocks * 1024;
-        for (int64_t e = (int64_t)b * 1024 + t; e < n; e += 2 * stride) {
-            const int64_t f = e + stride < n ? e + stride : e;
-            const float v[4] = {a.wp[e], a.wn[e], a.wp[f], a.wn[f]};
+        const int64_t n = a.O * a.K, stride = (int64_t)kSepStatW * 256;
+        for (int64_t e = (int64_t)b * 256 + t; e < n; e += 4 * stride) {
+            float v[8];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) sep_minmax(v[q], lo, hi);
+            for (int q = 0; q < 4; ++q) {
+                const int64_t f = e + q * stride < n ? e + q * stride : e;
+                v[2 * q] = a.wp[f];
+                v[2 * q + 1] = a.wn[f];
+            }
+#pragma unroll
+            for (int q = 0; q < 8; ++q) sep_minmax(v[q], lo, hi);
         }
         block_minmax(lo, hi, &a.wpart[b]);
         return;
     }
-    b -= kSepStatBlocks;
-    if (b < kSepStatBlocks) {
+    b -= kSepStatW;
+    const int lut_blocks = (a.lut_n + 255) / 256;
+    if (b < lut_blocks) {
+        sep_lut_block(a, b);
+        return;
+    }
+    b -= lut_blocks;
+    const int xcols = a.xcol ? kSepColChunks * (int)((a.K + 255) / 256) : 0;
+    if (b < xcols) {
+        const int64_t rows = (a.M + kSepColChunks - 1) / kSepColChunks;
+        const int chunk = b % kSepColChunks;
+        const int64_t col = (int64_t)(b / kSepColChunks) * 256 + t;
+        const int64_t m0 = chunk * rows, m1 = m0 + rows < a.M ? m0 + rows : a.M;
+        if (col >= a.K) return;
+        float lo = INFINITY, hi = -INFINITY;
+#pragma unroll 8
+        for (int64_t m = m0; m < m1; ++m) sep_minmax(sep_input(a, a.x[m * a.K + col], as, ab), lo, hi);
+        a.xcol[(int64_t)chunk * a.K + col] = make_float2(lo, hi);
+        return;
+    }
+    b -= xcols;
+    glue_grad_block(glue, b % kGlueBlocks, b / kGlueBlocks, (int)(glue.Op / 256));
+}
+
+// The largest |G| of a row or column (blocks of the table kernel's launch).
+__device__ inline void sep_grad_block(const SepArgs& a, int b) {
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    if (b < kSepStatG) {
         unsigned all = 0;
-        for (int64_t m = (int64_t)b * 16 + wave; m < a.M; m += (int64_t)kSepStatBlocks * 16) {
+        for (int64_t m = (int64_t)b * 4 + wave; m < a.M; m += (int64_t)kSepStatG * 4) {
             unsigned h = 0;
             const float* row = a.g + m * a.ldg;
             for (int64_t o = lane; o < a.O; o += 256) {
@@ -194,35 +329,24 @@ __global__ __launch_bounds__(1024) void sep_stat_kernel(SepArgs a) {
             if (lane == 0) a.grow[m] = h;
             all = max(all, h);
         }
-        __shared__ unsigned s_all;
+        __shared__ unsigned s_all;  // one atomic per block: they all meet at one address
         if (t == 0) s_all = 0;
         __syncthreads();
         if (lane == 0) atomicMax(&s_all, all);
         __syncthreads();
-        if (t == 0) a.gpart[b] = s_all;
+        if (t == 0) atomicMax(&a.head->gmax, s_all);
         return;
     }
-    b -= kSepStatBlocks;
-    const int gcols = a.need_w ? kSepColChunks / 4 * (int)((a.O + 255) / 256) : 0;
+    b -= kSepStatG;
     const int64_t rows = (a.M + kSepColChunks - 1) / kSepColChunks;
-    const bool of_g = b < gcols;
-    if (!of_g) b -= gcols;
-    const int chunk = b % (kSepColChunks / 4) * 4 + (t >> 8);
-    const int64_t col = (int64_t)(b / (kSepColChunks / 4)) * 256 + (t & 255);
+    const int chunk = b % kSepColChunks;
+    const int64_t col = (int64_t)(b / kSepColChunks) * 256 + t;
     const int64_t m0 = chunk * rows, m1 = m0 + rows < a.M ? m0 + rows : a.M;
-    if (of_g) {
-        if (col >= a.O) return;
-        unsigned h = 0;
+    if (col >= a.O) return;
+    unsigned h = 0;
 #pragma unroll 8
-        for (int64_t m = m0; m < m1; ++m) h = max(h, sep_bits(a.g[m * a.ldg + col]));
-        a.gcol[(int64_t)chunk * a.O + col] = h;
-    } else {
-        if (col >= a.K) return;
-        float lo = INFINITY, hi = -INFINITY;
-#pragma unroll 8
-        for (int64_t m = m0; m < m1; ++m) sep_minmax(sep_input(a, a.x[m * a.K + col], as, ab), lo, hi);
-        a.xcol[(int64_t)chunk * a.K + col] = make_float2(lo, hi);
-    }
+    for (int64_t m = m0; m < m1; ++m) h = max(h, sep_bits(a.g[m * a.ldg + col]));
+    a.gcol[(int64_t)chunk * a.O + col] = h;
 }
 
 // ----------------------------------------------------------------------------------
@@ -240,75 +364,175 @@ __device__ inline double sep_slope(double v, double a, double v_d) {  // f'(v) o
     return 2.0 * a * (s1 * g1 - s2 * g2);
 }
 
+// The lookup's smooth part (cubic) or its second difference (linear) at coordinate c, which
+// lies two entries or more inside the table.
+__device__ inline double sep_lut_smooth(const double2* val, int n, double c) {
+    int i = (int)c;
+    i = i < 1 ? 1 : i > n - 3 ? n - 3 : i;
+    const double f = c - i, g = 1.0 - f;
+    return -f * g * (1.0 + g) / 6.0 * val[i - 1].x + g * (1.0 + f) * (1.0 + g) * 0.5 * val[i].x +
+           f * (1.0 + f) * (1.0 + g) * 0.5 * val[i + 1].x - f * g * (1.0 + f) / 6.0 * val[i + 2].x;
+}
+
+__device__ inline double sep_lut_second(const double2* val, int n, double c) {
+    int i = (int)c;
+    i = i < 1 ? 1 : i > n - 3 ? n - 3 : i;
+    return val[i].y + (c - i) * (val[i + 1].y - val[i].y);
+}
+
+constexpr int kSepTableBlocks = 256;
+
+// Blocks: kSepTableBlocks of the tables, then (g) kSepStatG of G's rows and kSepColChunks x
+// ceil(O / 256) of its columns.
 __global__ __launch_bounds__(256) void sep_table_kernel(SepArgs a) {
-    __shared__ float2 s_x, s_w;
-    __shared__ unsigned s_g;
+    __shared__ float2 s_x, s_w, s_info;
     __shared__ SepHead s_head;
-    __shared__ double s_cos[4 * kSepMaxTerms], s_val[256], s_d[256];
+    __shared__ double s_cos[4 * kSepMaxTerms], s_val[256], s_sec[256], s_d[256];
     const int t = threadIdx.x;
-    block_minmax(a.xpart[t].x, a.xpart[t].y, &s_x);
-    __syncthreads();
-    block_minmax(a.wpart[t].x, a.wpart[t].y, &s_w);
-    if (t == 0) s_g = 0;
-    __syncthreads();
-    if (a.g) atomicMax(&s_g, a.gpart[t]);
-    __syncthreads();
+    const bool lut = a.lut_n > 0;
+    {
+        float lo = INFINITY, hi = -INFINITY;
+#pragma unroll
+        for (int q = 0; q < kSepStatX / 256; ++q) {
+            const float2 v = a.xpart[t + q * 256];
+            lo = fminf(lo, v.x);
+            hi = fmaxf(hi, v.y);
+        }
+        const float2 w = a.wpart[t];
+        static_assert(kSepStatW == 256 && kSepLutMax <= 256 * 256, "a thread per partial");
+        const float2 info = t * 256 < a.lut_n ? a.lut_info[t] : make_float2(0.0f, 0.0f);
+        block_minmax(lo, hi, &s_x);
+        __syncthreads();
+        block_minmax(w.x, w.y, &s_w);
+        __syncthreads();
+        block_minmax(-info.y, info.x, &s_info);  // (-1 where some do not suit, growth)
+        __syncthreads();
+    }
     if (t == 0) {
         SepHead h{};
         const float xlo = s_x.x, xhi = s_x.y, wlo = s_w.x, whi = s_w.y;
-        const double step = exp2(floor(log2(kSepStep / a.a)));
+        // a: the current's e-folds per volt of overdrive are 2 a at most
+        const double growth = lut ? (double)s_info.y : 0.0;
+        const double ua = lut ? 0.5 * growth * a.lut_scale : a.a;
+        const double step = exp2(floor(log2(kSepStep / ua)));
         const double rlo = 1.0 + (double)xlo / a.v_sat, rhi = 1.0 + (double)xhi / a.v_sat;
         const double first = floor((double)xlo / step) - 1.0;
         const double points = floor((double)xhi / step) - first + 3.0;
-        const bool finite = xlo > -1e30f && xhi < 1e30f && wlo > -1e30f && whi < 1e30f && s_g < 0x7f800000u;
-        const float spread = (float)(((double)whi - (double)wlo) * a.a);
-        const int terms = sep_terms(spread);
-        // |u| far below the exponent range of fp64, r and the table over x well behaved
-        if (finite && terms > 0 && terms <= a.max_terms && rlo > 0.1 && rhi > 0.1 && points <= (double)kSepGridMax &&
-            fmax(fabs((double)xlo), fabs((double)xhi)) < step * (1 << 23) &&
-            fmax(fabs((double)xlo), fabs((double)xhi)) * a.a < 300.0 &&
-            fmax(fabs((double)wlo), fabs((double)whi)) * a.a < 300.0) {
+        const bool finite = xlo > -1e30f && xhi < 1e30f && wlo > -1e30f && whi < 1e30f;
+        const float spread = (float)(((double)whi - (double)wlo) * ua);
+        const int terms = lut ? sep_terms_lut(spread) : sep_terms(spread);
+        bool ok = finite && terms > 0 && terms <= a.max_terms && rlo > 0.1 && rhi > 0.1 &&
+                  points <= (double)kSepGridMax && fmax(fabs((double)xlo), fabs((double)xhi)) < step * (1 << 23);
+        if (lut) {  // every lookup inside the table, the x table's margin included
+            h.harmonics = growth > 0.009 ? 1 : 0;
+            const double margin = 4.0 * step * a.lut_scale + 4.0;
+            ok = ok && s_info.x == 0.0f && growth > 1e-6 && growth < 0.045 &&
+                 ((double)xlo - (double)whi - a.lut_min) * a.lut_scale >= margin &&
+                 ((double)xhi - (double)wlo - a.lut_min) * a.lut_scale <= (double)(a.lut_n - 1) - margin;
+            h.lut_min = (float)a.lut_min;
+            h.lut_scale = (float)a.lut_scale;
+        } else {  // |u| far below the exponent range of fp64
+            ok = ok && fmax(fabs((double)xlo), fabs((double)xhi)) * ua < 300.0 &&
+                 fmax(fabs((double)wlo), fabs((double)whi)) * ua < 300.0;
+        }
+        if (ok) {
             h.terms = terms;
             h.n_grid = (int)points;
             h.x0 = (float)(first * step);
             h.step = (float)step;
             h.inv_step = (float)(1.0 / step);
             h.wc = 0.5 * ((double)wlo + (double)whi);
-            h.wh = fmax(0.5 * ((double)whi - (double)wlo), 1e-3 / a.a);
+            h.wh = fmax(0.5 * ((double)whi - (double)wlo), 1e-3 / ua);
             h.inv_wh = 1.0 / h.wh;
         }
+        h.xlo = xlo;
+        h.xhi = xhi;
+        h.wlo = wlo;
+        h.whi = whi;
         s_head = h;
-        if (blockIdx.x == 0) *a.head = h;
+        if (blockIdx.x == 0) {  // all but gmax and rough, which other blocks add to
+            SepHead* g = a.head;
+            g->terms = h.terms;
+            g->harmonics = h.harmonics;
+            g->n_grid = h.n_grid;
+            g->xlo = xlo;
+            g->xhi = xhi;
+            g->wlo = wlo;
+            g->whi = whi;
+            g->lut_min = h.lut_min;
+            g->lut_scale = h.lut_scale;
+            g->x0 = h.x0;
+            g->step = h.step;
+            g->inv_step = h.inv_step;
+            g->wc = h.wc;
+            g->inv_wh = h.inv_wh;
+            g->wh = h.wh;
+        }
     }
     __syncthreads();
     const SepHead h = s_head;
     const int R = h.terms;
     if (R == 0) return;
+    if (blockIdx.x >= kSepTableBlocks) {
+        sep_grad_block(a, blockIdx.x - kSepTableBlocks);
+        return;
+    }
     for (int q = t; q < 4 * R; q += 256) s_cos[q] = cospi((double)q / (2.0 * R));
     // a block takes 256 / R points at a time: a thread per (point, Chebyshev point), then per
     // (point, j)
     const int per = 256 / R, pl = t / R, n = t - pl * R;
-    for (int i0 = blockIdx.x * per; i0 < h.n_grid; i0 += gridDim.x * per) {
+    for (int i0 = blockIdx.x * per; i0 < h.n_grid; i0 += kSepTableBlocks * per) {
         const double x = (double)h.x0 + (double)(i0 + pl) * (double)h.step;
         const double r = 1.0 / (1.0 + x / a.v_sat);
         __syncthreads();
-        s_val[t] = sep_slope(x - (h.wc + h.wh * s_cos[2 * n + 1]), a.a, a.v_d);
+        const double v = x - (h.wc + h.wh * s_cos[2 * n + 1]);
+        if (lut) {
+            const double c = (v - a.lut_min) * a.lut_scale;
+            s_val[t] = sep_lut_smooth(a.lut_val, a.lut_n, c);
+            s_sec[t] = h.harmonics > 0 ? sep_lut_second(a.lut_val, a.lut_n, c) : 0.0;
+        } else {
+            s_val[t] = sep_slope(v, a.a, a.v_d);
+        }
         __syncthreads();
+        // the slope's d_n; the forward's tables hold currents: their coefficient n + 1 (of the
+        // polynomial of degree R - 1, so that the last is zero)
+        const int j = n + 1;
+        const bool direct = lut && !a.tab2;
+        const int jd = direct ? j : n;
         double d = 0.0;
-        for (int q = 0; q < R; ++q) d += s_val[pl * R + q] * s_cos[(n * (2 * q + 1)) % (4 * R)];
+        for (int q = 0; q < R; ++q) d += s_val[pl * R + q] * s_cos[(jd * (2 * q + 1)) % (4 * R)];
         d *= 2.0 / R;
+        if (direct && j == R) d = 0.0;
         s_d[t] = d;
+        double e2 = 0.0;
+        if (h.harmonics > 0 && n < R / 4) {
+            for (int q = 0; q < R; ++q) e2 += s_sec[pl * R + q] * s_cos[(n * (2 * q + 1)) % (4 * R)];
+            e2 *= (n == 0 ? 1.0 : 2.0) / R;
+        }
         __syncthreads();
         if (i0 + pl < h.n_grid) {
-            const int j = n + 1;  // c_j from d_(j-1) = d and d_(j+1)
-            const double d_next = j < R ? s_d[t + 1] : 0.0, d_after = j + 1 < R ? s_d[t + 2] : 0.0;
-            const double c = -h.wh / (2.0 * j) * (d - d_after);
             const size_t e = (size_t)(i0 + pl) * R + n;
-            if (a.tab2) {
-                a.tab[e] = (float)((n == 0 ? 0.5 * d : d) * r);
-                a.tab2[e] = (float)(r * (d_next - r / a.v_sat * c));
-            } else {
-                a.tab[e] = (float)(c * r);
+            if (direct) {
+                a.tab[e] = (float)(d * r);
+            } else {  // c_j from d_(j-1) = d and d_(j+1)
+                const double d_next = j < R ? s_d[t + 1] : 0.0, d_after = j + 1 < R ? s_d[t + 2] : 0.0;
+                const double c = -h.wh / (2.0 * j) * (d - d_after);
+                if (a.tab2) {
+                    a.tab[e] = (float)((n == 0 ? 0.5 * d : d) * r);
+                    a.tab2[e] = (float)(r * (d_next - r / a.v_sat * c));
+                } else {
+                    a.tab[e] = (float)(c * r);
+                }
+            }
+            if (h.harmonics > 0 && n < R / 4)
+                a.tabE[(size_t)(i0 + pl) * (R / 4) + n] = (float)(-r * e2 * 0.050660591821168886);  // 1 / (2 pi^2)
+            // the last coefficients of a table that grows otherwise than its steepest part says
+            if (lut && n == 0) {
+                const int last = direct ? R - 2 : R - 1;  // of degree R - 1
+                double big = 0.0;
+                for (int q = direct ? 0 : 1; q < R; ++q) big = fmax(big, fabs(s_d[t + q]));
+                const double mean = direct ? 0.0 : fabs(0.5 * s_d[t]);
+                if (!(fabs(s_d[t + last]) <= 2e-5 * big + 2e-6 * mean + 1e-35)) atomicOr(&a.head->rough, 1);
             }
         }
     }
@@ -421,17 +645,112 @@ struct SepChebPair {
     }
 };
 
+// cos and sin of 2 pi q theta, q = 1, 2 (theta in revolutions).
+__device__ inline void sep_trig(float theta, float* c, float* sn) {
+    const float f = theta - floorf(theta);
+    c[0] = __builtin_amdgcn_cosf(f);
+    sn[0] = __builtin_amdgcn_sinf(f);
+    c[1] = 2.0f * c[0] * c[0] - 1.0f;
+    sn[1] = 2.0f * sn[0] * c[0];
+}
+
+__device__ inline sep_h8 sep_pack8(const float v[8]) {
+    sep_h8 h;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) h[q] = (_Float16)v[q];
+    return h;
+}
+
+// Group blk of an input's harmonic values on the token side: the second difference's
+// coefficients e times cosine and sine.
+__device__ inline void sep_harm_x(float v[8], const float e[4], int terms, int blk, const float c[2], const float sn[2],
+                                  float scale) {
+    if (terms == 8) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            v[i] = e[i] * (c[0] * scale);
+            v[2 + i] = e[i] * (sn[0] * scale);
+            v[4 + i] = e[i] * (c[1] * 0.25f * scale);
+            v[6 + i] = e[i] * (sn[1] * 0.25f * scale);
+        }
+    } else {
+        const float f = blk ? 0.25f * scale : scale, fc = (blk ? c[1] : c[0]) * f, fs = (blk ? sn[1] : sn[0]) * f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            v[i] = e[i] * fc;
+            v[4 + i] = e[i] * fs;
+        }
+    }
+}
+
+// Likewise on the threshold side: T_i(t+) cos - T_i(t-) cos, ...
+__device__ inline void sep_harm_w(float v[8], const float tp[4], const float tn[4], int terms, int blk, const float cp[2],
+                                  const float sp[2], const float cn[2], const float sn[2], float scale) {
+    if (terms == 8) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            v[i] = (tp[i] * cp[0] - tn[i] * cn[0]) * scale;
+            v[2 + i] = (tp[i] * sp[0] - tn[i] * sn[0]) * scale;
+            v[4 + i] = (tp[i] * cp[1] - tn[i] * cn[1]) * scale;
+            v[6 + i] = (tp[i] * sp[1] - tn[i] * sn[1]) * scale;
+        }
+    } else {
+        const float c0 = blk ? cp[1] : cp[0], s0 = blk ? sp[1] : sp[0], c1 = blk ? cn[1] : cn[0], s1 = blk ? sn[1] : sn[0];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            v[i] = (tp[i] * c0 - tn[i] * c1) * scale;
+            v[4 + i] = (tp[i] * s0 - tn[i] * s1) * scale;
+        }
+    }
+}
+
+__device__ inline void sep_cheb4(float t, float v[4]) {  // T_0 .. T_3
+    v[0] = 1.0f;
+    v[1] = t;
+    v[2] = 2.0f * t * t - 1.0f;
+    v[3] = 2.0f * t * v[2] - t;
+}
+
+// The nearest table point's R / 4 second-difference coefficients (they change by 1.5% from
+// point to point, and are 1e-5 of the result).
+__device__ inline void sep_second(const SepHead& h, const float* tabE, const SepAt& at, float e[4]) {
+    const size_t i = (size_t)(at.i + (at.w[2] > at.w[1] ? 2 : 1));
+    if (h.terms == 8) {
+        const float2 v = *reinterpret_cast<const float2*>(tabE + i * 2);
+        e[0] = v.x; e[1] = v.y; e[2] = e[3] = 0.0f;
+    } else {
+        const float4 v = *reinterpret_cast<const float4*>(tabE + i * 4);
+        e[0] = v.x; e[1] = v.y; e[2] = v.z; e[3] = v.w;
+    }
+}
+
+// The per-cell range partials of a call that the contraction takes (the passes that record the
+// table mode read them).
+__device__ inline void sep_write_partials(const SepHead& h, const PrepArgs& p) {
+    for (int i = threadIdx.x; i < kPrepBlocksX + kPrepBlocksW; i += blockDim.x) {
+        float2 v = make_float2(INFINITY, -INFINITY);
+        if (i == 0) v = make_float2(fmaf(h.xlo - p.xoff, p.scale, p.xadd), fmaf(h.xhi - p.xoff, p.scale, p.xadd));
+        if (i == kPrepBlocksX) v = make_float2(h.wlo * p.scale, h.whi * p.scale);
+        p.partials[i] = v;
+    }
+    if (p.stat_bits && threadIdx.x == 0) *p.stat_bits = 0u;
+}
+
 // Where the per-cell kernels take the call: their prep, in the same launch.
 __global__ __launch_bounds__(256) void sep_expand_fwd_kernel(SepArgs a, PrepArgs prep) {
-    const SepHead h = *a.head;
-    const int R = h.terms;
-    if (R == 0) {
+    if (!sep_takes(a.head)) {
         if (blockIdx.x < kPrepBlocksX + kPrepBlocksW) prep_block(prep, blockIdx.x);
         return;
     }
+    const SepHead h = *a.head;
+    const int R = h.terms;
+    if (blockIdx.x == 0) sep_write_partials(h, prep);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t slabs = sep_slabs_kj(a.K, R);
-    const int64_t kc = (a.K + 3) / 4 * 4;  // inputs with their padding
+    const int groups = sep_groups(R, h.harmonics);
+    const int64_t stride = (slabs + sep_slabs_harm(a.K, groups)) * 64;  // of a row, in f16
+    const int64_t kc = (a.K + 3) / 4 * 4, k8 = (a.K + 7) / 8 * 8;  // inputs with their padding
+    const int64_t kw = groups > 0 ? k8 : kc;
     const int64_t row_waves = (int64_t)gridDim.x * 4;
     const float as = a.in_affine ? a.in_affine[0] : 1.0f, ab = a.in_affine ? a.in_affine[1] : 0.0f;
     float v[8];
@@ -440,33 +759,54 @@ __global__ __launch_bounds__(256) void sep_expand_fwd_kernel(SepArgs a, PrepArgs
             float inv;
             const float scale = sep_scale_of(sep_bound(h, a.tab, 0, a.xrow[row], (float)a.v_sat), &inv);
             if (lane == 0) a.xscale[row] = inv / kSepQScale;
-            _Float16* dst = a.xop + row * slabs * 64;
-            for (int64_t k = lane; k < kc; k += 64) {
-                if (k < a.K) {
-                    const SepAt at = sep_at(h, sep_input(a, a.x[row * a.K + k], as, ab));
+            _Float16* dst = a.xop + row * stride;
+            for (int64_t k = lane; k < kw; k += 64) {
+                const bool real = k < a.K;
+                const float x = sep_input(a, a.x[row * a.K + (real ? k : a.K - 1)], as, ab);
+                const float sc = real ? scale : 0.0f;
+                const SepAt at = sep_at(h, x);
+                if (k < kc) {
                     for (int j = 0; j < R; j += 8) {
                         const float4 lo = sep_eval4(a.tab, R, at, j), hi = sep_eval4(a.tab, R, at, j + 4);
-                        v[0] = lo.x * scale; v[1] = lo.y * scale; v[2] = lo.z * scale; v[3] = lo.w * scale;
-                        v[4] = hi.x * scale; v[5] = hi.y * scale; v[6] = hi.z * scale; v[7] = hi.w * scale;
+                        v[0] = lo.x * sc; v[1] = lo.y * sc; v[2] = lo.z * sc; v[3] = lo.w * sc;
+                        v[4] = hi.x * sc; v[5] = hi.y * sc; v[6] = hi.z * sc; v[7] = hi.w * sc;
                         sep_store8(dst, kc * j + k * 8, v);
                     }
-                } else {
-#pragma unroll
-                    for (int q = 0; q < 8; ++q) v[q] = 0.0f;
-                    for (int j = 0; j < R; j += 8) sep_store8(dst, kc * j + k * 8, v);
+                }
+                if (groups > 0) {
+                    float e[4], c[2], sn[2];
+                    sep_second(h, a.tabE, at, e);
+                    sep_trig((x - h.lut_min) * h.lut_scale, c, sn);
+                    for (int blk = 0; blk < groups; ++blk) {
+                        sep_harm_x(v, e, R, blk, c, sn, sc);
+                        *reinterpret_cast<sep_h8*>(dst + slabs * 64 + (blk * k8 + k) * 8) = sep_pack8(v);
+                    }
                 }
             }
         } else {
             const int64_t o = row - a.M;
-            _Float16* dst = a.wop + o * slabs * 64;
-            for (int64_t k = lane; k < kc; k += 64) {
+            _Float16* dst = a.wop + o * stride;
+            for (int64_t k = lane; k < kw; k += 64) {
                 const bool real = k < a.K;
                 const double tp = real ? ((double)a.wp[o * a.K + k] - h.wc) * h.inv_wh : 0.0;
                 const double tn = real ? ((double)a.wn[o * a.K + k] - h.wc) * h.inv_wh : 0.0;
-                SepChebPair c(tp, tn);
-                for (int j = 0; j < R; j += 8) {
-                    c.next8(v, kSepQScale);
-                    sep_store8(dst, kc * j + k * 8, v);
+                if (k < kc) {
+                    SepChebPair c(tp, tn);
+                    for (int j = 0; j < R; j += 8) {
+                        c.next8(v, kSepQScale);
+                        sep_store8(dst, kc * j + k * 8, v);
+                    }
+                }
+                if (groups > 0) {
+                    float p[4], n[4], cp[2], sp[2], cn[2], sn[2];
+                    sep_cheb4((float)tp, p);
+                    sep_cheb4((float)tn, n);
+                    sep_trig((float)((h.wc + h.wh * tp) * h.lut_scale), cp, sp);
+                    sep_trig((float)((h.wc + h.wh * tn) * h.lut_scale), cn, sn);
+                    for (int blk = 0; blk < groups; ++blk) {
+                        sep_harm_w(v, p, n, R, blk, cp, sp, cn, sn, kSepQScale);
+                        *reinterpret_cast<sep_h8*>(dst + slabs * 64 + (blk * k8 + k) * 8) = sep_pack8(v);
+                    }
                 }
             }
         }
@@ -480,13 +820,23 @@ __global__ __launch_bounds__(256) void sep_expand_fwd_kernel(SepArgs a, PrepArgs
 // along the inner index. HBM-bound.
 // ----------------------------------------------------------------------------------
 
+__device__ inline void sep_store2h(_Float16* row, int64_t e, float v0, float v1) {  // single f16
+    sep_h2 h;
+    h.x = (_Float16)v0;
+    h.y = (_Float16)v1;
+    *reinterpret_cast<sep_h2*>(row + e) = h;
+}
+
 __global__ __launch_bounds__(256) void sep_expand_bwd_kernel(SepArgs a, int x_blocks, int w_blocks, PrepArgs prep) {
-    const SepHead h = *a.head;
-    const int R = h.terms;
-    if (R == 0) {  // the per-cell kernels take the call: their prep
+    if (!sep_takes(a.head)) {  // the per-cell kernels take the call: their prep
         if (blockIdx.x < kPrepBlocksX + kPrepBlocksW) prep_block(prep, blockIdx.x);
         return;
     }
+    const SepHead h = *a.head;
+    const int R = h.terms;
+    if (blockIdx.x == 0) sep_write_partials(h, prep);
+    const int groups = sep_groups(R, h.harmonics);
+    const int64_t m64 = sep_slabs64(a.M) * 64, o64 = sep_slabs64(a.O) * 64;  // harmonics' inner lengths
     __shared__ float s_a[32][130], s_b[32][130];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int64_t m_slabs = sep_slabs(a.M), o_slabs = sep_slabs(a.O);
@@ -510,10 +860,25 @@ __global__ __launch_bounds__(256) void sep_expand_bwd_kernel(SepArgs a, int x_bl
             if (m0 == 0 && lane == 0) a.xscale[k] = inv;
             const int ml = 2 * lane;
             const int64_t m = m0 + ml;
-            if (m >= m_slabs * 32) continue;
+            if (m >= (groups > 0 ? m64 : m_slabs * 32)) continue;
             const float s0 = m < a.M ? scale : 0.0f, s1 = m + 1 < a.M ? scale : 0.0f;
             const SepAt p0 = sep_at(h, m < a.M ? s_a[kk][ml] : range.y);
             const SepAt p1 = sep_at(h, m + 1 < a.M ? s_a[kk][ml + 1] : range.y);
+            if (groups > 0) {
+                float e0[4], e1[4], c0[2], n0[2], c1[2], n1[2], u[8], v[8];
+                sep_second(h, a.tabE, p0, e0);
+                sep_second(h, a.tabE, p1, e1);
+                sep_trig((s_a[kk][ml] - h.lut_min) * h.lut_scale, c0, n0);
+                sep_trig((s_a[kk][ml + 1] - h.lut_min) * h.lut_scale, c1, n1);
+                _Float16* dst = a.xoph + k * groups * 8 * m64;
+                for (int blk = 0; blk < groups; ++blk) {
+                    sep_harm_x(u, e0, R, blk, c0, n0, s0);
+                    sep_harm_x(v, e1, R, blk, c1, n1, s1);
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) sep_store2h(dst + (blk * 8 + i) * m64, m, u[i], v[i]);
+                }
+            }
+            if (m >= m_slabs * 32) continue;
             for (int j = 0; j < R; j += 4) {
                 const float4 u = sep_eval4(a.tab, R, p0, j), v = sep_eval4(a.tab, R, p1, j);
                 _Float16* dst = a.xop + (k * R + j) * m_slabs * 64;
@@ -540,7 +905,7 @@ __global__ __launch_bounds__(256) void sep_expand_bwd_kernel(SepArgs a, int x_bl
             const int64_t k = k0 + kk;
             const int ol = 2 * lane;
             const int64_t o = o0 + ol;
-            if (o >= o_slabs * 32) continue;
+            if (o >= (groups > 0 ? o64 : o_slabs * 32)) continue;
             double t_[4];
 #pragma unroll
             for (int q = 0; q < 2; ++q) {
@@ -553,6 +918,25 @@ __global__ __launch_bounds__(256) void sep_expand_bwd_kernel(SepArgs a, int x_bl
             }
             if (!a.need_x) continue;
             const bool r0 = o < a.O, r1 = o + 1 < a.O;
+            if (groups > 0) {
+                _Float16* dst = a.woph + k * groups * 8 * o64;
+                float p0[4], n0[4], p1[4], n1[4], c0[4], d0[4], c1[4], d1[4], u[8], v[8];
+                sep_cheb4((float)t_[0], p0);
+                sep_cheb4((float)t_[1], n0);
+                sep_cheb4((float)t_[2], p1);
+                sep_cheb4((float)t_[3], n1);
+                sep_trig(s_a[kk][ol] * h.lut_scale, c0, d0);
+                sep_trig(s_b[kk][ol] * h.lut_scale, c0 + 2, d0 + 2);
+                sep_trig(s_a[kk][ol + 1] * h.lut_scale, c1, d1);
+                sep_trig(s_b[kk][ol + 1] * h.lut_scale, c1 + 2, d1 + 2);
+                for (int blk = 0; blk < groups; ++blk) {
+                    sep_harm_w(u, p0, n0, R, blk, c0, d0, c0 + 2, d0 + 2, r0 ? kSepQScale : 0.0f);
+                    sep_harm_w(v, p1, n1, R, blk, c1, d1, c1 + 2, d1 + 2, r1 ? kSepQScale : 0.0f);
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) sep_store2h(dst + (blk * 8 + i) * o64, o, u[i], v[i]);
+                }
+                if (o >= o_slabs * 32) continue;
+            }
             SepChebPair c0(r0 ? t_[0] : 0.0, r0 ? t_[1] : 0.0), c1(r1 ? t_[2] : 0.0, r1 ? t_[3] : 0.0);
             float u[8], v[8];
             for (int j = 0; j < R; j += 8) {
@@ -581,8 +965,9 @@ __global__ __launch_bounds__(256) void sep_expand_bwd_kernel(SepArgs a, int x_bl
             float inv;
             const float scale = sep_scale_of(__uint_as_float(a.grow[m]), &inv);
             if (o0 == 0 && lane == 0) a.gscale[m] = inv / kSepQScale;
-            if (o < o_slabs * 32)
-                sep_store2(a.gop + m * o_slabs * 64, o, s_a[mm][2 * lane] * scale, s_a[mm][2 * lane + 1] * scale);
+            const float g0 = s_a[mm][2 * lane] * scale, g1 = s_a[mm][2 * lane + 1] * scale;
+            if (o < o_slabs * 32) sep_store2(a.gop + m * o_slabs * 64, o, g0, g1);
+            if (groups > 0 && o < o64) sep_store2h(a.goph + m * o64, o, g0, g1);
         }
     }
     if (a.need_w) {
@@ -596,65 +981,94 @@ __global__ __launch_bounds__(256) void sep_expand_bwd_kernel(SepArgs a, int x_bl
             const float scale = sep_scale_of(__uint_as_float(big), &inv);
             if (m0 == 0 && (t & 15) == 0) a.gscaleT[o] = inv;
             const int mm = 2 * (t & 15);
-            sep_store2(a.gopT + o * m_slabs * 64, m0 + mm, s_a[mm][q] * scale, s_a[mm + 1][q] * scale);
+            const float g0 = s_a[mm][q] * scale, g1 = s_a[mm + 1][q] * scale;
+            sep_store2(a.gopT + o * m_slabs * 64, m0 + mm, g0, g1);
+            if (groups > 0) {
+                sep_store2h(a.gophT + o * m64, m0 + mm, g0, g1);
+                if (m0 + 32 >= a.M && m0 + 32 < m64) sep_store2h(a.gophT + o * m64, m0 + 32 + mm, 0.0f, 0.0f);
+            }
         }
     }
 }
 
 // ----------------------------------------------------------------------------------
-// The product of two operands of hi/lo slabs, C[i][j] = sum_e A[i][e] B[j][e]: tiles of
-// (WM MI 32) x (WN NI 32), one slab (32 inner elements, 128 bytes per row) of both operands at
-// a time in two LDS buffers. A slab's loads are issued before the arithmetic of the one
-// before it, which takes three products per pair of fragments (hi hi, hi lo, lo hi):
-// 3072 matrix-core cycles per 64 KB of operands for the 256 x 256 tile, so that one buffer
-// ahead covers the memory's latency and the operands need ~21 bytes per cycle and CU. Rows are
-// 128 bytes and their eight 16-byte parts are stored at part ^ (row / 2 % 8), so that the 16
-// rows that a quarter-wave reads lie on different banks. Rows past the operand's end read its
-// last row (their results are dropped).
+// The product of two operands of slabs, C[i][j] = sum_e A[i][e] B[j][e]: tiles of
+// (WM MI 32) x (WN NI 32), one slab (128 bytes per row) of both operands at a time in two LDS
+// buffers. A slab holds 32 inner elements as hi/lo pairs, which take three products per pair of
+// fragments (hi hi, hi lo, lo hi), or (harmonics) 64 as single f16. A slab's loads are issued
+// before the arithmetic of the one before it: 3072 matrix-core cycles per 64 KB of operands for
+// the 256 x 256 tile of pairs, so that one buffer ahead covers the memory's latency and the
+// operands need ~21 bytes per cycle and CU. Rows are 128 bytes and their eight 16-byte parts are
+// stored at part ^ (row / 2 % 8), so that the 16 rows that a quarter-wave reads lie on different
+// banks. Rows past the operand's end read its last row (their results are dropped).
 // Blocks are dealt so that each XCD works on neighbouring tiles (whose operands its L2 holds).
+//
+// A launch runs up to four products after one another in its grid (the backward's dX and dVth,
+// of pairs and of harmonics), so that one's last blocks overlap the next one's first.
 // ----------------------------------------------------------------------------------
 
-enum SepEpilogue { kSepForward, kSepDx, kSepDv };
+enum SepKind { kSepForward, kSepDx, kSepDv, kSepDxHarm, kSepDvHarm };
+
+struct SepProduct {
+    const char* a;
+    const char* b;
+    int kind;
+    int64_t a_rows, b_rows;   // A rows per eight of an input's terms (dX, dVth), else in all
+    int64_t inner;            // elements; forward: inputs
+    int n_split;
+    float* out;               // forward: planes [n_split][M][O]; dX: [n_split][M][K]; dVth: [n_split][2][Kp][Op]
+};
 
 struct SepGemm {
-    const uint4* a;
-    const uint4* b;
+    SepProduct p[4];
+    int n;
     const SepHead* head;
-    int64_t a_rows, b_rows;   // a_rows: per term where it depends on R (rows_of_terms)
-    int rows_of_terms;        // 1: the A operand has a_rows * R rows
-    int64_t inner;            // inner elements; with inner_of_terms the (k, j) index of a_rows... K inputs
-    int inner_of_terms;
-    int n_split;
-    int tiles_a, tiles_b;     // at the most terms
-    float* out;               // forward: planes [n_split][M][O]; dX: [n_split][M][K]; dVth: [n_split][2][Kp][Op]
     int64_t M, K, O, Kp, Op;
-    const float* scale_a;     // forward [M], dVth [K]
-    const float* scale_b;     // dX [M], dVth [O]
-    // dX
+    const float* xscale;      // forward [M], dVth [K]
+    const float* gscale;      // dX [M]
+    const float* gscaleT;     // dVth [O]
     const float* x;
     const float* in_affine;
     float in_lo, in_hi;
     const float* tab2;
-    // dVth
+    const float* tabE;
     const float2* tT;
 };
 
-template <int WM, int WN, int MI, int NI, SepEpilogue EPI>
+template <int WM, int WN, int MI, int NI, bool FORWARD>
 __global__ __launch_bounds__(WM * WN * 64, 2) void sep_gemm_kernel(SepGemm g) {
     constexpr int kThreads = WM * WN * 64, TM = WM * MI * 32, TN = WN * NI * 32;
     constexpr int kLoadA = TM * 8 / kThreads, kLoadB = TN * 8 / kThreads, kRowStep = kThreads / 8;
     extern __shared__ __attribute__((aligned(16))) char s_sep[];
     const SepHead* head = g.head;
+    if (!sep_takes(head)) return;
     const int R = __builtin_amdgcn_readfirstlane(head->terms);
-    if (R == 0) return;
-    const int64_t a_rows = g.rows_of_terms ? g.a_rows * R : g.a_rows;
-    const int slabs = (int)(g.inner_of_terms ? sep_slabs_kj(g.inner, R) : sep_slabs(g.inner));
-    const int ta = (int)((a_rows + TM - 1) / TM), tb = g.tiles_b;
-    // blocks run over the XCDs round robin: give XCD c the tiles [c n / 8, (c + 1) n / 8)
-    const int n = ta * tb * g.n_split;
-    int id = blockIdx.x;
-    if (id >= n) return;
-    {
+    const int groups = sep_groups(R, __builtin_amdgcn_readfirstlane(head->harmonics));
+    const int nb = R / 8;
+    // the product this block works on, its rows and slabs
+    int id = blockIdx.x, which = 0, ta = 0, tb = 0, n = 0, slabs = 0, pair_slabs = 0;
+    int64_t a_rows = 0;
+    for (;; ++which) {
+        if (which >= g.n) return;
+        const SepProduct& p = g.p[which];
+        const bool harm = p.kind >= kSepDxHarm;
+        if constexpr (FORWARD) {
+            a_rows = p.a_rows;
+            pair_slabs = (int)sep_slabs_kj(p.inner, R);
+            slabs = pair_slabs + (int)sep_slabs_harm(p.inner, groups);
+        } else {
+            a_rows = p.a_rows * 8 * (harm ? groups : nb);
+            slabs = (int)(harm ? sep_slabs64(p.inner) : sep_slabs(p.inner));
+            pair_slabs = harm ? 0 : slabs;
+        }
+        ta = (int)((a_rows + TM - 1) / TM);
+        tb = (int)((p.b_rows + TN - 1) / TN);
+        n = ta * tb * p.n_split;
+        if (id < n) break;
+        id -= n;
+    }
+    const SepProduct& p = g.p[which];
+    {   // blocks run over the XCDs round robin: give XCD c the tiles [c n / 8, (c + 1) n / 8)
         const int per = n / 8, rest = n % 8, xcd = id & 7;
         id = xcd * per + (xcd < rest ? xcd : rest) + (id >> 3);
     }
@@ -665,7 +1079,8 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void sep_gemm_kernel(SepGemm g) {
     const int height = min(4, ta - group * 4);
     const int tile_a = group * 4 + in_group % height, tile_b = in_group / height;
     const int64_t a0 = (int64_t)tile_a * TM, b0 = (int64_t)tile_b * TN;
-    const int s_begin = (int)((int64_t)slabs * split / g.n_split), s_end = (int)((int64_t)slabs * (split + 1) / g.n_split);
+    const int s_begin = (int)((int64_t)slabs * split / p.n_split);
+    const int s_end = (int)((int64_t)slabs * (split + 1) / p.n_split);
 
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int wr = wave / WN, wc = wave % WN;
@@ -679,7 +1094,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void sep_gemm_kernel(SepGemm g) {
 #pragma unroll
     for (int q = 0; q < kLoadB; ++q) {
         const int64_t row = b0 + row0 + q * kRowStep;
-        pb[q] = (unsigned)(((row < g.b_rows ? row : g.b_rows - 1) * slabs * 8 + part) * 16);
+        pb[q] = (unsigned)(((row < p.b_rows ? row : p.b_rows - 1) * slabs * 8 + part) * 16);
     }
     constexpr int kBuf = (TM + TN) * 128;
     // kRowStep rows further on the swizzle is the same: kRowStep is a multiple of 16
@@ -697,8 +1112,8 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void sep_gemm_kernel(SepGemm g) {
 #pragma unroll
             for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.0f;
 
-    const char* abase = reinterpret_cast<const char*>(g.a);
-    const char* bbase = reinterpret_cast<const char*>(g.b);
+    const char* abase = p.a;
+    const char* bbase = p.b;
     sep_u4 ra[kLoadA], rb[kLoadB];
     auto load = [&](int s) {
 #pragma unroll
@@ -713,12 +1128,21 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void sep_gemm_kernel(SepGemm g) {
 #pragma unroll
         for (int q = 0; q < kLoadB; ++q) *reinterpret_cast<sep_u4*>(base + TM * 128 + q * kRowStep * 128) = rb[q];
     };
+    auto multiply = [&](const sep_h8* u, const sep_h8* v) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NI; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(u[i], v[j], acc[i][j], 0, 0, 0);
+    };
     if (s_begin < s_end) {
         load(s_begin);
         store(0);
     }
     __syncthreads();
-    for (int s = s_begin; s < s_end; ++s) {
+    int s = s_begin;
+    const int pair_end = min(s_end, pair_slabs);
+    for (; s < pair_end; ++s) {
         const int buf = (s - s_begin) & 1;
         const bool more = s + 1 < s_end;
         if (more) load(s + 1);
@@ -737,36 +1161,43 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void sep_gemm_kernel(SepGemm g) {
                 bh[j] = *reinterpret_cast<const sep_h8*>(base + fb + j * 4096 + off);
                 bl[j] = *reinterpret_cast<const sep_h8*>(base + fb + j * 4096 + (off ^ 64));
             }
+            multiply(ah, bl);
+            multiply(al, bh);
+            multiply(ah, bh);
+        }
+        if (more) store(buf ^ 1);
+        __syncthreads();
+    }
+    for (; s < s_end; ++s) {
+        const int buf = (s - s_begin) & 1;
+        const bool more = s + 1 < s_end;
+        if (more) load(s + 1);
+        const char* base = s_sep + buf * kBuf;
 #pragma unroll
-            for (int i = 0; i < MI; ++i)
+        for (int ks = 0; ks < 4; ++ks) {
+            sep_h8 av[MI], bv[NI];
+            const int off = frag ^ (ks << 5);
 #pragma unroll
-                for (int j = 0; j < NI; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i], bl[j], acc[i][j], 0, 0, 0);
+            for (int i = 0; i < MI; ++i) av[i] = *reinterpret_cast<const sep_h8*>(base + fa + i * 4096 + off);
 #pragma unroll
-            for (int i = 0; i < MI; ++i)
-#pragma unroll
-                for (int j = 0; j < NI; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[i], bh[j], acc[i][j], 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < MI; ++i)
-#pragma unroll
-                for (int j = 0; j < NI; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i], bh[j], acc[i][j], 0, 0, 0);
+            for (int j = 0; j < NI; ++j) bv[j] = *reinterpret_cast<const sep_h8*>(base + fb + j * 4096 + off);
+            multiply(av, bv);
+            if (ks == 1) __builtin_amdgcn_sched_barrier(0);  // two steps' fragments at a time fit the registers
         }
         if (more) store(buf ^ 1);
         __syncthreads();
     }
 
     // lane (fl, fh) holds rows q % 4 + 8 (q / 4) + 4 fh of column fl of each 32 x 32 tile
-    if constexpr (EPI == kSepForward) {
-        float* out = g.out + (int64_t)split * g.M * g.O;
+    if constexpr (FORWARD) {
+        float* out = p.out + (int64_t)split * g.M * g.O;
 #pragma unroll
         for (int i = 0; i < MI; ++i) {
 #pragma unroll
             for (int q = 0; q < 16; ++q) {
                 const int64_t m = a0 + (wr * MI + i) * 32 + (q & 3) + 8 * (q >> 2) + 4 * fh;
                 if (m >= g.M) continue;
-                const float sc = g.scale_a[m];
+                const float sc = g.xscale[m];
 #pragma unroll
                 for (int j = 0; j < NI; ++j) {
                     const int64_t o = b0 + (wc * NI + j) * 32 + fl;
@@ -774,96 +1205,138 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void sep_gemm_kernel(SepGemm g) {
                 }
             }
         }
-    } else if constexpr (EPI == kSepDx) {
+    } else {
         const SepHead h = *head;
-        const float as = g.in_affine ? g.in_affine[0] : 1.0f, ab = g.in_affine ? g.in_affine[1] : 0.0f;
-        float* out = g.out + (int64_t)split * g.M * g.K;
-        const int nb = R / 8, sh = __builtin_ctz(nb);
+        const int kind = p.kind;
+        const bool harm = kind >= kSepDxHarm, dx = kind == kSepDx || kind == kSepDxHarm;
+        const int per = harm ? groups : nb, sh = __builtin_ctz(per);  // blocks of eight rows per input
+        if (dx) {
+            const float as = g.in_affine ? g.in_affine[0] : 1.0f, ab = g.in_affine ? g.in_affine[1] : 0.0f;
+            float* out = p.out + (int64_t)split * g.M * g.K;
 #pragma unroll
-        for (int j = 0; j < NI; ++j) {
-            const int64_t m = b0 + (wc * NI + j) * 32 + fl;
-            const int64_t mc = m < g.M ? m : g.M - 1;
-            const float sc = g.scale_b[mc];
-            float sum = 0.0f;
+            for (int j = 0; j < NI; ++j) {
+                const int64_t m = b0 + (wc * NI + j) * 32 + fl;
+                const int64_t mc = m < g.M ? m : g.M - 1;
+                const float sc = g.gscale[mc];
+                float sum = 0.0f;
 #pragma unroll
-            for (int i = 0; i < MI; ++i) {
+                for (int i = 0; i < MI; ++i) {
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {  // eight rows (k, 8 jb ..)
-                    const int64_t block = (a0 + (wr * MI + i) * 32) / 8 + q;
-                    const int64_t k = block >> sh;
-                    const int jb = (int)block & (nb - 1);
-                    const int64_t kc = k < g.K ? k : g.K - 1;
-                    const float xr = g.x[mc * g.K + kc];
-                    const SepAt at = sep_at(h, g.in_affine ? input_map(xr, as, ab, g.in_lo, g.in_hi) : xr);
-                    const float4 v = sep_eval4(g.tab2, R, at, jb * 8 + 4 * fh);
-                    float s = acc[i][j][4 * q] * v.x;
-                    s = fmaf(acc[i][j][4 * q + 1], v.y, s);
-                    s = fmaf(acc[i][j][4 * q + 2], v.z, s);
-                    s = fmaf(acc[i][j][4 * q + 3], v.w, s);
-                    sum += s;
-                    if (jb == nb - 1) {
-                        sum += __shfl_xor(sum, 32);
-                        if (fh == 0 && m < g.M && k < g.K) out[m * g.K + k] = sum * sc;
-                        sum = 0.0f;
+                    for (int q = 0; q < 4; ++q) {  // eight rows of input k
+                        const int64_t block = (a0 + (wr * MI + i) * 32) / 8 + q;
+                        const int64_t k = block >> sh;
+                        const int jb = (int)block & (per - 1);
+                        const int64_t kc = k < g.K ? k : g.K - 1;
+                        const float xr = g.x[mc * g.K + kc];
+                        const float x = g.in_affine ? input_map(xr, as, ab, g.in_lo, g.in_hi) : xr;
+                        const SepAt at = sep_at(h, x);
+                        float4 v;
+                        if (!harm) {
+                            v = sep_eval4(g.tab2, R, at, jb * 8 + 4 * fh);
+                        } else {
+                            // 8 terms: harmonic fh's two cosines and two sines; 16: harmonic jb's four
+                            // cosines (fh = 0) or sines
+                            const int hq = nb == 1 ? fh : jb;
+                            const float th = (x - h.lut_min) * h.lut_scale * (float)(hq + 1);
+                            const float f = th - floorf(th), w = hq ? 0.25f : 1.0f;
+                            const float c = __builtin_amdgcn_cosf(f) * w, sn = __builtin_amdgcn_sinf(f) * w;
+                            float e[4];
+                            sep_second(h, g.tabE, at, e);
+                            if (nb == 1) {
+                                v = make_float4(e[0] * c, e[1] * c, e[0] * sn, e[1] * sn);
+                            } else {
+                                const float tr = fh ? sn : c;
+                                v = make_float4(e[0] * tr, e[1] * tr, e[2] * tr, e[3] * tr);
+                            }
+                        }
+                        float s = acc[i][j][4 * q] * v.x;
+                        s = fmaf(acc[i][j][4 * q + 1], v.y, s);
+                        s = fmaf(acc[i][j][4 * q + 2], v.z, s);
+                        s = fmaf(acc[i][j][4 * q + 3], v.w, s);
+                        sum += s;
+                        if (jb == per - 1) {
+                            sum += __shfl_xor(sum, 32);
+                            if (fh == 0 && m < g.M && k < g.K) out[m * g.K + k] = sum * sc;
+                            sum = 0.0f;
+                        }
                     }
                 }
             }
-        }
-    } else {
-        float* out = g.out + (int64_t)split * 2 * g.Kp * g.Op;
-        const int nb = R / 8, sh = __builtin_ctz(nb);
+        } else {
+            float* out = p.out + (int64_t)split * 2 * g.Kp * g.Op;
 #pragma unroll
-        for (int j = 0; j < NI; ++j) {
-            const int64_t o = b0 + (wc * NI + j) * 32 + fl;
-            const int64_t oc = o < g.O ? o : g.O - 1;
-            const float sb = g.scale_b[oc];
-            float sp = 0.0f, sn = 0.0f, p0 = 0.0f, p1 = 0.0f, n0 = 0.0f, n1 = 0.0f;
-            float2 tt = make_float2(0.0f, 0.0f);
+            for (int j = 0; j < NI; ++j) {
+                const int64_t o = b0 + (wc * NI + j) * 32 + fl;
+                const int64_t oc = o < g.O ? o : g.O - 1;
+                const float sb = g.gscaleT[oc];
+                float sp = 0.0f, sn = 0.0f, p0 = 0.0f, p1 = 0.0f, n0 = 0.0f, n1 = 0.0f;
+                float2 tt = make_float2(0.0f, 0.0f);
 #pragma unroll
-            for (int i = 0; i < MI; ++i) {
+                for (int i = 0; i < MI; ++i) {
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int64_t block = (a0 + (wr * MI + i) * 32) / 8 + q;
-                    const int64_t k = block >> sh;
-                    const int jb = (int)block & (nb - 1);
-                    const int64_t kc = k < g.K ? k : g.K - 1;
-                    if (jb == 0) {
-                        tt = g.tT[kc * g.Op + oc];
-                        p0 = n0 = 1.0f;  // T_0, T_1
-                        p1 = tt.x;
-                        n1 = tt.y;
-                    }
-                    float vp[4], vn[4];  // this lane's four of the eight polynomials
+                    for (int q = 0; q < 4; ++q) {
+                        const int64_t block = (a0 + (wr * MI + i) * 32) / 8 + q;
+                        const int64_t k = block >> sh;
+                        const int jb = (int)block & (per - 1);
+                        const int64_t kc = k < g.K ? k : g.K - 1;
+                        if (jb == 0) tt = g.tT[kc * g.Op + oc];
+                        float rp = 0.0f, rn = 0.0f;
+                        if (!harm) {
+                            if (jb == 0) {  // T_0, T_1
+                                p0 = n0 = 1.0f;
+                                p1 = tt.x;
+                                n1 = tt.y;
+                            }
+                            float vp[4], vn[4];  // this lane's four of the eight polynomials
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        vp[e & 3] = e < 4 || fh ? p0 : vp[e & 3];
-                        vn[e & 3] = e < 4 || fh ? n0 : vn[e & 3];
-                        const float p2 = fmaf(2.0f * tt.x, p1, -p0), n2 = fmaf(2.0f * tt.y, n1, -n0);
-                        p0 = p1;
-                        p1 = p2;
-                        n0 = n1;
-                        n1 = n2;
-                    }
+                            for (int e = 0; e < 8; ++e) {
+                                vp[e & 3] = e < 4 || fh ? p0 : vp[e & 3];
+                                vn[e & 3] = e < 4 || fh ? n0 : vn[e & 3];
+                                const float p2 = fmaf(2.0f * tt.x, p1, -p0), n2 = fmaf(2.0f * tt.y, n1, -n0);
+                                p0 = p1;
+                                p1 = p2;
+                                n0 = n1;
+                                n1 = n2;
+                            }
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        sp = fmaf(acc[i][j][4 * q + e], vp[e], sp);
-                        sn = fmaf(acc[i][j][4 * q + e], vn[e], sn);
-                    }
-                    if (jb == nb - 1) {
-                        sp += __shfl_xor(sp, 32);
-                        sn += __shfl_xor(sn, 32);
-                        if (o < g.O && k < g.K)
-                            out[((int64_t)fh * g.Kp + k) * g.Op + o] = (fh ? sn : sp) * sb * g.scale_a[k];
-                        sp = sn = 0.0f;
+                            for (int e = 0; e < 4; ++e) {
+                                rp = fmaf(acc[i][j][4 * q + e], vp[e], rp);
+                                rn = fmaf(acc[i][j][4 * q + e], vn[e], rn);
+                            }
+                        } else {  // the rows' order as for dX
+                            const int hq = nb == 1 ? fh : jb;
+                            const float ws = h.lut_scale * (float)(hq + 1);
+                            const float tp = ((float)h.wc + (float)h.wh * tt.x) * ws, tn = ((float)h.wc + (float)h.wh * tt.y) * ws;
+                            const float fp = tp - floorf(tp), fn = tn - floorf(tn);
+                            const float cp = __builtin_amdgcn_cosf(fp), dp = __builtin_amdgcn_sinf(fp);
+                            const float cn = __builtin_amdgcn_cosf(fn), dn = __builtin_amdgcn_sinf(fn);
+                            const float a0 = acc[i][j][4 * q], a1 = acc[i][j][4 * q + 1], a2 = acc[i][j][4 * q + 2],
+                                        a3 = acc[i][j][4 * q + 3];
+                            if (nb == 1) {
+                                rp = cp * fmaf(a1, tt.x, a0) + dp * fmaf(a3, tt.x, a2);
+                                rn = cn * fmaf(a1, tt.y, a0) + dn * fmaf(a3, tt.y, a2);
+                            } else {
+                                float vp[4], vn[4];
+                                sep_cheb4(tt.x, vp);
+                                sep_cheb4(tt.y, vn);
+                                rp = (fh ? dp : cp) * fmaf(a3, vp[3], fmaf(a2, vp[2], fmaf(a1, vp[1], a0)));
+                                rn = (fh ? dn : cn) * fmaf(a3, vn[3], fmaf(a2, vn[2], fmaf(a1, vn[1], a0)));
+                            }
+                        }
+                        sp += rp;
+                        sn += rn;
+                        if (jb == per - 1) {
+                            sp += __shfl_xor(sp, 32);
+                            sn += __shfl_xor(sn, 32);
+                            if (o < g.O && k < g.K)
+                                out[((int64_t)fh * g.Kp + k) * g.Op + o] = (fh ? sn : sp) * sb * g.xscale[k];
+                            sp = sn = 0.0f;
+                        }
                     }
                 }
             }
         }
     }
-}
-
-__device__ bool sep_takes(const SepHead* head) {
-    return head != nullptr && __builtin_amdgcn_readfirstlane(head->terms) != 0;
 }
 
 // Finishes the forward (split_reduce_body) from the planes of whichever path took the call; a
@@ -877,12 +1350,21 @@ __global__ __launch_bounds__(256) void sep_reduce_fwd_kernel(FwdArgs sep, FwdArg
         split_reduce_body<VEC>(cell, clamp_out);
 }
 
-// grad_reduce_kernel's dX and dVth parts from the planes of whichever path took the call.
+// grad_reduce_kernel's work from the planes of whichever path took the call.
 __global__ __launch_bounds__(256) void sep_reduce_bwd_kernel(DxReduceArgs dx, DxReduceArgs dx_cell, int dx_blocks,
                                                              DvReduceArgs dv, DvReduceArgs dv_cell, int dv_blocks,
-                                                             const SepHead* head) {
+                                                             GlueReduceArgs gl, const SepHead* head, int harm_dx,
+                                                             int harm_dv) {
     const int b = blockIdx.x;
+    if (b >= dx_blocks + dv_blocks) {
+        glue_reduce_block(gl, b - dx_blocks - dv_blocks);
+        return;
+    }
     if (sep_takes(head)) {
+        if (head->harmonics == 0) {  // their planes, the last ones, were not written
+            dx.n_planes -= harm_dx;
+            dv.n_split -= harm_dv;
+        }
         if (b < dx_blocks)
             dx_reduce_block(dx, b, dx_blocks);
         else
@@ -912,14 +1394,19 @@ __global__ __launch_bounds__(256) void sep_reduce_bwd_kernel(DxReduceArgs dx, Dx
 #ifndef ISA_EKV_CONTRACT_MIN_CELLS
 #define ISA_EKV_CONTRACT_MIN_CELLS (1 << 25)
 #endif
+#ifndef ISA_EKV_CONTRACT_MIN_CELLS_LUT
+#define ISA_EKV_CONTRACT_MIN_CELLS_LUT (1 << 29)
+#endif
 
 struct SepPlan {
     int max_terms;  // 0: not considered
     bool big;       // 256 x 256 tiles instead of 128 x 128
-    int split, split_dx, split_dv;
+    int split, split_dx, split_dv, split_dxh, split_dvh;
+    int planes_dx, planes_dv;
     int64_t Kp, Op;
-    size_t off_head, off_part, off_row, off_col, off_grow, off_gcol, off_tab, off_tab2, off_xop, off_wop, off_gop,
-        off_gopT, off_scale, off_gscale, off_gscaleT, off_tT, off_planes, off_planes_dv, bytes;
+    size_t off_head, off_part, off_row, off_col, off_grow, off_gcol, off_tab, off_tab2, off_tabE, off_lut, off_xop, off_wop,
+        off_xoph, off_woph, off_gop, off_gopT, off_goph, off_gophT, off_scale, off_gscale, off_gscaleT, off_tT,
+        off_planes, off_planes_dv, bytes;
 };
 
 constexpr int64_t kSepOperandBytes = (int64_t)2 << 30;  // of one operand, at most (32-bit byte offsets)
@@ -948,16 +1435,23 @@ inline bool sep_big(int64_t rows_a, int64_t rows_b, int64_t slabs) {
     return ((rows_a + 255) / 256) * ((rows_b + 255) / 256) * (slabs / 16 + 1) >= 2 * kCUs && rows_a >= 192 && rows_b >= 192;
 }
 
-SepPlan plan_sep(int64_t M, int64_t K, int64_t O, bool backward, bool need_x, bool need_w, size_t base) {
+// lut_n: table entries, 0 for the formula.
+SepPlan plan_sep(int lut_n, int64_t M, int64_t K, int64_t O, bool backward, bool need_x, bool need_w, size_t base) {
     SepPlan p{};
     p.bytes = base;
     const double cells = (double)M * (double)K * (double)O;
-    if (M < 16 || O < 16 || K < 8 || cells < (double)ISA_EKV_CONTRACT_MIN_CELLS) return p;
+    if (M < 16 || O < 16 || K < 8 || (backward && !need_x && !need_w) ||
+        cells < (double)(lut_n > 0 ? (int64_t)ISA_EKV_CONTRACT_MIN_CELLS_LUT : (int64_t)ISA_EKV_CONTRACT_MIN_CELLS) ||
+        (lut_n > 0 && (lut_n < kSepLutMin || lut_n > kSepLutMax)))
+        return p;
     p.Kp = round_up(K, 8);
     p.Op = round_up(O, 256);
-    const int64_t Mr = round_up(M, 32), Or = round_up(O, 32), Kr = round_up(K, 4);
-    int terms = cells >= 1 << 30 ? 64 : cells >= 1 << 28 ? 32 : 16;
-    while (terms >= 8 && (Mr * Kr * terms * 4 >= kSepOperandBytes || Or * Kr * terms * 4 >= kSepOperandBytes)) terms /= 2;
+    const int64_t Mr = round_up(M, 64), Or = round_up(O, 64), Kr = round_up(K, 8);
+    // bytes per (row, input): R hi/lo pairs, and in the forward's rows the harmonics
+    const int harm = lut_n > 0 ? 1 : 0;
+    auto width = [&](int terms) { return (int64_t)terms * (4 + (backward ? 0 : 2 * harm)); };
+    int terms = lut_n > 0 ? 16 : cells >= 1 << 30 ? 64 : cells >= 1 << 28 ? 32 : 16;
+    while (terms >= 8 && (Mr * Kr * width(terms) >= kSepOperandBytes || Or * Kr * width(terms) >= kSepOperandBytes)) terms /= 2;
     if (terms < 8 || Mr * Or * 4 >= kSepOperandBytes) return p;
     p.max_terms = terms;
     size_t off = (size_t)round_up((int64_t)base, 256);
@@ -967,117 +1461,145 @@ SepPlan plan_sep(int64_t M, int64_t K, int64_t O, bool backward, bool need_x, bo
         return at;
     };
     p.off_head = take(sizeof(SepHead));
-    p.off_part = take(kSepStatBlocks * 24);
-    p.off_tab = take((int64_t)kSepGridMax * 8 * 4 * (terms / 8));
-    p.off_xop = take(Mr * Kr * terms * 4);
-    p.off_wop = take(Or * Kr * terms * 4);
+    p.off_part = take((kSepStatX + kSepStatW) * 8);
+    p.off_tab = take((int64_t)kSepGridMax * 4 * terms);
+    if (lut_n > 0) {
+        p.off_lut = take((int64_t)lut_n * 16 + 256 * 8);
+        p.off_tabE = take((int64_t)kSepGridMax * terms);
+    }
+    p.off_xop = take(Mr * Kr * width(terms));
+    p.off_wop = take(Or * Kr * width(terms));
     if (!backward) {
         p.off_row = take(M * 8);
         p.off_scale = take(M * 4);
-        const int64_t slabs = (K + 3) / 4;
+        const int64_t slabs = (K + 3) / 4 + (K + 7) / 8 * harm;
         p.big = sep_big(M, O, slabs);
         const int64_t tile = p.big ? 256 : 128;
         p.split = sep_splits(((M + tile - 1) / tile) * ((O + tile - 1) / tile), slabs, p.big, 8.0 * M * O);
         p.off_planes = take((int64_t)p.split * M * O * 4);
     } else {
-        p.off_tab2 = take((int64_t)kSepGridMax * 8 * 4 * (terms / 8));
+        p.off_tab2 = take((int64_t)kSepGridMax * 4 * terms);
         p.off_col = take(kSepColChunks * K * 8);
         p.off_grow = take(M * 4);
         p.off_gcol = take(kSepColChunks * O * 4);
         p.off_gop = take(Mr * Or * 4);
         p.off_gopT = take(Mr * Or * 4);
+        if (harm > 0) {
+            p.off_xoph = take(Mr * Kr * terms * 2 * harm);
+            p.off_woph = take(Or * Kr * terms * 2 * harm);
+            p.off_goph = take(Mr * Or * 2);
+            p.off_gophT = take(Mr * Or * 2);
+        }
         p.off_scale = take(K * 4);
         p.off_gscale = take(M * 4);
         p.off_gscaleT = take(O * 4);
         p.off_tT = take(K * p.Op * 8);
         p.big = sep_big(8 * K, std::min(M, O), std::min(M, O) / 32);
-        const int64_t tile = p.big ? 256 : 128, tk = (8 * K + tile - 1) / tile;
-        p.split_dx = sep_splits(tk * ((M + tile - 1) / tile), (O + 31) / 32, p.big, 8.0 * M * K);
-        p.split_dv = sep_splits(tk * ((O + tile - 1) / tile), (M + 31) / 32, p.big, 16.0 * p.Kp * p.Op);
-        if (need_x) p.off_planes = take((int64_t)p.split_dx * M * K * 4);
-        if (need_w) p.off_planes_dv = take((int64_t)p.split_dv * 2 * p.Kp * p.Op * 4);
+        const int64_t tile = p.big ? 256 : 128, tk = (8 * K + tile - 1) / tile, tkh = (8 * K * harm + tile - 1) / tile;
+        const int64_t tm = (M + tile - 1) / tile, to = (O + tile - 1) / tile;
+        p.split_dx = sep_splits(tk * tm, (O + 31) / 32, p.big, 8.0 * M * K);
+        p.split_dv = sep_splits(tk * to, (M + 31) / 32, p.big, 16.0 * p.Kp * p.Op);
+        p.split_dxh = harm > 0 ? sep_splits(tkh * tm, (O + 63) / 64, p.big, 8.0 * M * K) : 0;
+        p.split_dvh = harm > 0 ? sep_splits(tkh * to, (M + 63) / 64, p.big, 16.0 * p.Kp * p.Op) : 0;
+        p.planes_dx = p.split_dx + p.split_dxh;
+        p.planes_dv = p.split_dv + p.split_dvh;
+        if (need_x) p.off_planes = take((int64_t)p.planes_dx * M * K * 4);
+        if (need_w) p.off_planes_dv = take((int64_t)p.planes_dv * 2 * p.Kp * p.Op * 4);
     }
     p.bytes = off;
     return p;
 }
 
-template <SepEpilogue EPI>
-void launch_sep_gemm(bool big, int max_terms, SepGemm g, hipStream_t s) {
-    const int64_t tile = big ? 256 : 128;
-    const int64_t rows_a = g.rows_of_terms ? g.a_rows * max_terms : g.a_rows;
-    g.tiles_b = (int)((g.b_rows + tile - 1) / tile);
-    const dim3 grid((unsigned)((rows_a + tile - 1) / tile * g.tiles_b * g.n_split));
+template <bool FORWARD>
+void launch_sep_gemm(bool big, unsigned blocks, const SepGemm& g, hipStream_t s) {
     if (big)
-        hipLaunchKernelGGL((sep_gemm_kernel<2, 4, 4, 2, EPI>), grid, dim3(512), 131072, s, g);
+        hipLaunchKernelGGL((sep_gemm_kernel<2, 4, 4, 2, FORWARD>), dim3(blocks), dim3(512), 131072, s, g);
     else
-        hipLaunchKernelGGL((sep_gemm_kernel<2, 2, 2, 2, EPI>), grid, dim3(256), 65536, s, g);
+        hipLaunchKernelGGL((sep_gemm_kernel<2, 2, 2, 2, FORWARD>), dim3(blocks), dim3(256), 65536, s, g);
 }
 
-constexpr int kSepTableBlocks = 256;
-
-// The forward up to its planes (statistics, tables, operands, product).
-hipError_t sep_forward(const SepPlan& p, SepArgs a, const PrepArgs& prep, char* ws, hipStream_t s) {
+void sep_point(const SepPlan& p, SepArgs& a, char* ws) {
     a.head = reinterpret_cast<SepHead*>(ws + p.off_head);
     a.xpart = reinterpret_cast<float2*>(ws + p.off_part);
-    a.wpart = a.xpart + kSepStatBlocks;
-    a.xrow = reinterpret_cast<float2*>(ws + p.off_row);
+    a.wpart = a.xpart + kSepStatX;
     a.tab = reinterpret_cast<float*>(ws + p.off_tab);
+    a.tabE = reinterpret_cast<float*>(ws + p.off_tabE);
+    a.lut_info = reinterpret_cast<float2*>(ws + p.off_lut);
+    a.lut_val = reinterpret_cast<double2*>(ws + p.off_lut + 256 * 8);
     a.xop = reinterpret_cast<_Float16*>(ws + p.off_xop);
     a.wop = reinterpret_cast<_Float16*>(ws + p.off_wop);
     a.xscale = reinterpret_cast<float*>(ws + p.off_scale);
     a.max_terms = p.max_terms;
-    hipLaunchKernelGGL(sep_stat_kernel, dim3(2 * kSepStatBlocks), dim3(1024), 0, s, a);
+}
+
+// The forward's operands (and, where it does not take the call, the per-cell kernels' prep).
+hipError_t sep_forward_operands(const SepPlan& p, SepArgs a, const PrepArgs& prep, char* ws, hipStream_t s) {
+    sep_point(p, a, ws);
+    a.xrow = reinterpret_cast<float2*>(ws + p.off_row);
+    hipLaunchKernelGGL(sep_stat_kernel, dim3(kSepStatX + kSepStatW + (a.lut_n + 255) / 256), dim3(256), 0, s, a,
+                       GlueGradArgs{});
     hipLaunchKernelGGL(sep_table_kernel, dim3(kSepTableBlocks), dim3(256), 0, s, a);
     const int64_t expand = std::min<int64_t>((a.M + a.O + 3) / 4, kSepExpandBlocks);
     hipLaunchKernelGGL(sep_expand_fwd_kernel, dim3((unsigned)std::max<int64_t>(expand, kPrepBlocksX + kPrepBlocksW)),
                        dim3(256), 0, s, a, prep);
-    SepGemm g{};
-    g.a = reinterpret_cast<const uint4*>(a.xop);
-    g.b = reinterpret_cast<const uint4*>(a.wop);
-    g.head = a.head;
-    g.a_rows = a.M;
-    g.b_rows = a.O;
-    g.inner = a.K;
-    g.inner_of_terms = 1;
-    g.n_split = p.split;
-    g.out = reinterpret_cast<float*>(ws + p.off_planes);
-    g.M = a.M;
-    g.K = a.K;
-    g.O = a.O;
-    g.scale_a = a.xscale;
-    launch_sep_gemm<kSepForward>(p.big, p.max_terms, g, s);
     return hipGetLastError();
 }
 
-// The backward up to its dX and dVth planes.
-hipError_t sep_backward(const SepPlan& p, SepArgs a, const PrepArgs& prep, char* ws, hipStream_t s) {
-    a.head = reinterpret_cast<SepHead*>(ws + p.off_head);
-    a.xpart = reinterpret_cast<float2*>(ws + p.off_part);
-    a.wpart = a.xpart + kSepStatBlocks;
-    a.gpart = reinterpret_cast<unsigned*>(a.wpart + kSepStatBlocks);
-    a.xcol = reinterpret_cast<float2*>(ws + p.off_col);
+// The forward's product, into its planes.
+hipError_t sep_forward_product(const SepPlan& p, SepArgs a, char* ws, hipStream_t s) {
+    sep_point(p, a, ws);
+    SepGemm g{};
+    g.head = a.head;
+    g.M = a.M;
+    g.K = a.K;
+    g.O = a.O;
+    g.xscale = a.xscale;
+    g.n = 1;
+    g.p[0] = SepProduct{reinterpret_cast<const char*>(a.xop), reinterpret_cast<const char*>(a.wop), kSepForward, a.M, a.O,
+                        a.K, p.split, reinterpret_cast<float*>(ws + p.off_planes)};
+    const int64_t tile = p.big ? 256 : 128;
+    launch_sep_gemm<true>(p.big, (unsigned)((a.M + tile - 1) / tile * ((a.O + tile - 1) / tile) * p.split), g, s);
+    return hipGetLastError();
+}
+
+void sep_point_backward(const SepPlan& p, SepArgs& a, char* ws) {
+    sep_point(p, a, ws);
+    a.xcol = a.need_w ? reinterpret_cast<float2*>(ws + p.off_col) : nullptr;
     a.grow = reinterpret_cast<unsigned*>(ws + p.off_grow);
     a.gcol = reinterpret_cast<unsigned*>(ws + p.off_gcol);
-    a.tab = reinterpret_cast<float*>(ws + p.off_tab);
     a.tab2 = reinterpret_cast<float*>(ws + p.off_tab2);
-    a.xop = reinterpret_cast<_Float16*>(ws + p.off_xop);
-    a.wop = reinterpret_cast<_Float16*>(ws + p.off_wop);
     a.gop = reinterpret_cast<_Float16*>(ws + p.off_gop);
     a.gopT = reinterpret_cast<_Float16*>(ws + p.off_gopT);
-    a.xscale = reinterpret_cast<float*>(ws + p.off_scale);
+    a.xoph = reinterpret_cast<_Float16*>(ws + p.off_xoph);
+    a.woph = reinterpret_cast<_Float16*>(ws + p.off_woph);
+    a.goph = reinterpret_cast<_Float16*>(ws + p.off_goph);
+    a.gophT = reinterpret_cast<_Float16*>(ws + p.off_gophT);
     a.gscale = reinterpret_cast<float*>(ws + p.off_gscale);
     a.gscaleT = reinterpret_cast<float*>(ws + p.off_gscaleT);
     a.tT = reinterpret_cast<float2*>(ws + p.off_tT);
     a.Op = p.Op;
-    a.max_terms = p.max_terms;
-    const int64_t col_blocks = kSepColChunks / 4 * ((a.need_w ? (a.O + 255) / 256 : 0) + (a.K + 255) / 256);
-    hipLaunchKernelGGL(sep_stat_kernel, dim3((unsigned)(3 * kSepStatBlocks + col_blocks)), dim3(1024), 0, s, a);
-    hipLaunchKernelGGL(sep_table_kernel, dim3(kSepTableBlocks), dim3(256), 0, s, a);
+}
+
+// The backward's operands; glue: the layer glue's gradient pass, which writes a.g.
+hipError_t sep_backward_operands(const SepPlan& p, SepArgs a, const PrepArgs& prep, const GlueGradArgs* glue, char* ws,
+                                 hipStream_t s) {
+    sep_point_backward(p, a, ws);
+    const int64_t xcols = a.xcol ? kSepColChunks * ((a.K + 255) / 256) : 0;
+    const int64_t stat = kSepStatX + kSepStatW + (a.lut_n + 255) / 256 + xcols + (glue ? (int64_t)kGlueBlocks * (glue->Op / 256) : 0);
+    hipLaunchKernelGGL(sep_stat_kernel, dim3((unsigned)stat), dim3(256), 0, s, a, glue ? *glue : GlueGradArgs{});
+    const int64_t gcols = a.need_w ? kSepColChunks * ((a.O + 255) / 256) : 0;
+    hipLaunchKernelGGL(sep_table_kernel, dim3((unsigned)(kSepTableBlocks + kSepStatG + gcols)), dim3(256), 0, s, a);
     const int64_t kt = (a.K + 31) / 32, ot = (a.O + 127) / 128;
     const int64_t x_blocks = a.need_w ? kt * ((a.M + 127) / 128) : 0, w_blocks = kt * ot, g_blocks = ot * ((a.M + 31) / 32);
     const int64_t expand = x_blocks + w_blocks + g_blocks;
     hipLaunchKernelGGL(sep_expand_bwd_kernel, dim3((unsigned)std::max<int64_t>(expand, kPrepBlocksX + kPrepBlocksW)),
                        dim3(256), 0, s, a, (int)x_blocks, (int)w_blocks, prep);
+    return hipGetLastError();
+}
+
+// The backward's products, into the dX and dVth planes.
+hipError_t sep_backward_products(const SepPlan& p, SepArgs a, char* ws, hipStream_t s) {
+    sep_point_backward(p, a, ws);
     SepGemm g{};
     g.head = a.head;
     g.M = a.M;
@@ -1085,36 +1607,33 @@ hipError_t sep_backward(const SepPlan& p, SepArgs a, const PrepArgs& prep, char*
     g.O = a.O;
     g.Kp = p.Kp;
     g.Op = p.Op;
-    g.a_rows = a.K;
-    g.rows_of_terms = 1;
-    if (a.need_x) {
-        SepGemm d = g;
-        d.a = reinterpret_cast<const uint4*>(a.wop);
-        d.b = reinterpret_cast<const uint4*>(a.gop);
-        d.b_rows = a.M;
-        d.inner = a.O;
-        d.n_split = p.split_dx;
-        d.out = reinterpret_cast<float*>(ws + p.off_planes);
-        d.scale_b = a.gscale;
-        d.x = a.x;
-        d.in_affine = a.in_affine;
-        d.in_lo = a.in_lo;
-        d.in_hi = a.in_hi;
-        d.tab2 = a.tab2;
-        launch_sep_gemm<kSepDx>(p.big, p.max_terms, d, s);
-    }
-    if (a.need_w) {
-        SepGemm d = g;
-        d.a = reinterpret_cast<const uint4*>(a.xop);
-        d.b = reinterpret_cast<const uint4*>(a.gopT);
-        d.b_rows = a.O;
-        d.inner = a.M;
-        d.n_split = p.split_dv;
-        d.out = reinterpret_cast<float*>(ws + p.off_planes_dv);
-        d.scale_a = a.xscale;
-        d.scale_b = a.gscaleT;
-        d.tT = a.tT;
-        launch_sep_gemm<kSepDv>(p.big, p.max_terms, d, s);
-    }
+    g.xscale = a.xscale;
+    g.gscale = a.gscale;
+    g.gscaleT = a.gscaleT;
+    g.x = a.x;
+    g.in_affine = a.in_affine;
+    g.in_lo = a.in_lo;
+    g.in_hi = a.in_hi;
+    g.tab2 = a.tab2;
+    g.tabE = a.tabE;
+    g.tT = a.tT;
+    const int64_t tile = p.big ? 256 : 128;
+    int64_t blocks = 0;
+    auto add = [&](int kind, const _Float16* x, const _Float16* y, int64_t b_rows, int64_t inner, int split, float* out,
+                   int eights) {
+        if (split < 1) return;
+        g.p[g.n++] = SepProduct{reinterpret_cast<const char*>(x), reinterpret_cast<const char*>(y), kind, a.K, b_rows,
+                                inner, split, out};
+        blocks += (8 * a.K * eights + tile - 1) / tile * ((b_rows + tile - 1) / tile) * split;
+    };
+    float* dx = reinterpret_cast<float*>(ws + p.off_planes);
+    float* dv = reinterpret_cast<float*>(ws + p.off_planes_dv);
+    const int nb = p.max_terms / 8, nh = nb;
+    if (a.need_x) add(kSepDx, a.wop, a.gop, a.M, a.O, p.split_dx, dx, nb);
+    if (a.need_w) add(kSepDv, a.xop, a.gopT, a.O, a.M, p.split_dv, dv, nb);
+    if (a.need_x) add(kSepDxHarm, a.woph, a.goph, a.M, a.O, p.split_dxh, dx + (int64_t)p.split_dx * a.M * a.K, nh);
+    if (a.need_w)
+        add(kSepDvHarm, a.xoph, a.gophT, a.O, a.M, p.split_dvh, dv + (int64_t)p.split_dv * 2 * p.Kp * p.Op, nh);
+    launch_sep_gemm<false>(p.big, (unsigned)blocks, g, s);
     return hipGetLastError();
 }

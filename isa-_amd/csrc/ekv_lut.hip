@@ -1215,7 +1215,9 @@ __global__ __launch_bounds__(kAssignThreads) void fwd_copy_assign_kernel(float2*
                                                               const float2* __restrict__ partials, int NP,
                                                               int max_window, int* __restrict__ mode_word,
                                                               int64_t Kp, int64_t Op, int copy_offset,
-                                                              int skip_from) {
+                                                              int skip_from, const SepHead* skip) {
+    // (where the contraction takes the call, the first block alone records the mode)
+    if (blockIdx.x != 0 && sep_takes(skip)) return;
     static_assert(LANES == 32 || LANES == 16, "half-wave or quarter-wave gathers");
     constexpr int kGroups = 64 / LANES, kMask = LANES - 1;
     // skip_from > 0: a pass earlier in the call recorded a mode of its own (the ranked backward,
@@ -1224,7 +1226,7 @@ __global__ __launch_bounds__(kAssignThreads) void fwd_copy_assign_kernel(float2*
     if (skip_from > 0 && __builtin_amdgcn_readfirstlane(*mode_word) >= skip_from) return;
     const bool on = launch_copy_mode(partials, NP, max_window);
     if (blockIdx.x == 0 && threadIdx.x == 0) *mode_word = on ? 1 : 0;
-    if (!on) return;
+    if (!on || sep_takes(skip)) return;
     __shared__ float s_cnt[LANES][kAssignThreads];  // per-thread bank loads; [bin][thread]: conflict-free
     const int tid = threadIdx.x;
     const int64_t n_ot = Op / (64 * kFwdORR);
@@ -1436,12 +1438,13 @@ __global__ __launch_bounds__(kMcThreads) void fwd_multi_assign_kernel(float2* __
                                                           const float2* __restrict__ partials, int NP, int budget,
                                                           int max_copies, int* __restrict__ mode_word, int64_t Kp,
                                                           int64_t Op, int dhalf, int max_window, int wide_dhalf,
-                                                          float after_rank) {
+                                                          float after_rank, const SepHead* skip) {
+    if (blockIdx.x != 0 && sep_takes(skip)) return;
     if (after_rank > 0.0f && ranked_mode(partials, NP, after_rank, nullptr)) return;
     const MultiLayout ml =
         multi_layout(read_coord_range(partials), NP, budget, max_copies, dhalf, max_window, wide_dhalf);
     if (blockIdx.x == 0 && threadIdx.x == 0) *mode_word = multi_mode_word(ml.copies);
-    if (ml.copies == 0) return;
+    if (ml.copies == 0 || sep_takes(skip)) return;
     __shared__ float s_sw[32 * kMcProblems];       // [rank][problem]: the thresholds in order
     __shared__ unsigned s_info[32 * kMcProblems];  // [rank][problem] (multi_greedy)
     __shared__ unsigned s_pe[64 * kMcProblems];    // bit planes (multi_greedy)
@@ -1548,6 +1551,7 @@ __device__ inline void stage_table2(float2* dst, const float2* __restrict__ src,
 template <int MR, bool SPLITS, bool WIN = false>
 __global__ __launch_bounds__(2 * kFwdWaves * 64) void fwd_kernel(FwdArgs a) {
     extern __shared__ float2 s_lut_fwd[];
+    if (sep_takes(a.skip)) return;
     const BlockClock clk(a.clock_acc);
     if constexpr (!WIN) stage_table2(s_lut_fwd, a.lut, a.NP);
     // fast loop and copy mode from one read of the range partials (as coords_in_padded_range,
@@ -1608,6 +1612,7 @@ __global__ __launch_bounds__(2 * kFwdWaves * 64) void fwd_kernel(FwdArgs a) {
 // the same tiling and cells, the gathers served by the L1/L2 caches.
 template <int MR, bool SPLITS>
 __global__ __launch_bounds__(kFwdWaves * 64) void fwd_global_kernel(FwdArgs a) {
+    if (sep_takes(a.skip)) return;
     const bool fast = coords_in_padded_range(a.partials, a.NP);
     FwdTile t;
     if (!fwd_tile<SPLITS>(a, MR, t)) return;
@@ -2130,12 +2135,14 @@ __device__ inline void bwd_table_items(const BwdArgs& a, const Table t, bool fas
 template <bool NEED_X, bool NEED_W, bool SPLIT, bool LANE_RED = false, int MODE = kBwdAlone>
 __global__ __launch_bounds__(1024, kBwdWavesPerEU) void bwd_kernel(BwdArgs a) {
     static_assert(MODE != kBwdTwoCopies, "bwd_two_copies_kernel");
+    if (sep_takes(a.skip)) return;
     const BlockClock clk(a.clock_acc);
     if (bwd_table_body<NEED_X, NEED_W, SPLIT, LANE_RED, MODE>(a)) clk.stop();  // (idle launches add nothing)
 }
 
 template <bool NEED_X, bool NEED_W, bool SPLIT>
 __global__ __launch_bounds__(1024) void bwd_two_copies_kernel(BwdArgs a) {
+    if (sep_takes(a.skip)) return;
     const BlockClock clk(a.clock_acc ? a.clock_acc + 3 : nullptr);  // the two-copy kind
     if (bwd_table_body<NEED_X, NEED_W, SPLIT, true, kBwdTwoCopies>(a)) clk.stop();
 }
@@ -2204,6 +2211,7 @@ struct RankArgs {
     int Kp, Op, n_ob, NP;
     float max_spread;     // the widest threshold spread (records) the ranked launch takes
     float greedy_min;     // spreads past this are dealt by bwd_deal_kernel, the rest by rank
+    const SepHead* skip;  // the contraction's head: only the mode word is recorded where it takes the call
 };
 
 #ifndef ISA_EKV_RANK_MERGE_MAX
@@ -2232,10 +2240,11 @@ __device__ inline bool ranked_mode(const float2* __restrict__ partials, int NP, 
 // as one contiguous run (each thread's own stores would land 32 bytes apart across a wave).
 constexpr int kRankQ = 256 / kRankClasses;
 __global__ __launch_bounds__(256) void bwd_rank_kernel(RankArgs a) {
+    if (blockIdx.x != 0 && sep_takes(a.skip)) return;
     float spread = 0.0f;
     const bool on = ranked_mode(a.partials, a.NP, a.max_spread, &spread);  // block-uniform
     if (blockIdx.x == 0 && threadIdx.x == 0) *a.mode_word = on ? kModeRanked : 0;
-    if (!on || spread > a.greedy_min) return;  // (wide spreads: bwd_deal_kernel deals)
+    if (!on || spread > a.greedy_min || sep_takes(a.skip)) return;  // (wide spreads: bwd_deal_kernel deals)
     __shared__ float4 s_dealt[kRankQ * 64 * 2];  // per pair: 64 lanes x 8 slots
     const int64_t n_q = (int64_t)a.Kp * a.n_ob;
     const int64_t q0 = (int64_t)blockIdx.x * kRankQ;
@@ -2328,6 +2337,7 @@ __device__ inline void wave_lds_sync() {
 // LDS (per bank pair 16 bits: the distinct records there, 2 bits saturating at 3, and the first
 // one's id), so only the cross-lane minima leave a lane. 7 KB per problem: two blocks per CU.
 __global__ __launch_bounds__(kDealWaves * 64, 2) void bwd_deal_kernel(RankArgs a) {
+    if (sep_takes(a.skip)) return;
     float spread = 0.0f;
     if (!ranked_mode(a.partials, a.NP, a.max_spread, &spread) || !(spread > a.greedy_min)) return;
     __shared__ __align__(16) float s_key[kDealProblems][16 * 32];  // [class][branch]; then the dealt [lane][slot]
@@ -2449,6 +2459,7 @@ template <bool NEED_W>
 __global__ __launch_bounds__(kRankWaves * 64, kRankWaves * 2 / 4) void bwd_ranked_kernel(BwdArgs a, const float* __restrict__ ws_ranked,
                                                                      const uint2* __restrict__ branch) {
     if (__builtin_amdgcn_readfirstlane(*a.copy_mode) != kModeRanked) return;
+    if (sep_takes(a.skip)) return;
     const BlockClock clk(a.clock_acc ? a.clock_acc + 6 : nullptr);  // the ranked kind
     extern __shared__ float4 s_ranked[];
     char* smem = reinterpret_cast<char*>(s_ranked);
@@ -2728,6 +2739,7 @@ __device__ inline void bwd_body_half(const BwdArgs& a, const float2* tab, int it
 template <int HALF, bool NEED_X, bool NEED_W>
 __global__ __launch_bounds__(1024) void bwd_half_kernel(BwdArgs a) {
     extern __shared__ float2 s_half[];
+    if (sep_takes(a.skip)) return;
     stage_to_lds<8>(a.lut, a.NP, [&](int i, float4 rec) {
         s_half[i] = HALF == 0 ? make_float2(rec.z, rec.w) : make_float2(rec.x, rec.y);
     });
@@ -2750,6 +2762,7 @@ __global__ __launch_bounds__(1024) void bwd_half_kernel(BwdArgs a) {
 template <bool NEED_X, bool NEED_W>
 __global__ __launch_bounds__(1024, ISA_EKV_BWD_MIN_BLOCKS) void bwd_global_kernel(BwdArgs a) {
     extern __shared__ float4 s_red_global[];
+    if (sep_takes(a.skip)) return;
     constexpr bool LANE_RED = NEED_X;
     const bool fast = coords_in_padded_range(a.partials, a.NP);
     const int waves = blockDim.x >> 6;
@@ -4376,22 +4389,34 @@ SepArgs make_sep(const CallSetup& cs, const float* x, const float* wp, const flo
         a.in_lo = glue->in_lo;
         a.in_hi = glue->in_hi;
     }
-    a.a = cs.inv_2nut;
-    a.v_d = cs.v_d;
     a.v_sat = v_sat;
+    if (cs.exact) {
+        a.a = cs.inv_2nut;
+        a.v_d = cs.v_d;
+    } else {
+        a.lut = static_cast<const float*>(cs.lut);
+        a.lut_n = cs.n_entries;
+        a.lut_min = cs.delta_min;
+        a.lut_scale = cs.n_entries > 1 ? (double)(cs.n_entries - 1) / ((double)cs.delta_max - (double)cs.delta_min) : 0.0;
+    }
     return a;
 }
 
 int run_forward(const CallSetup& cs, const float* x, const float* vth_pos, const float* vth_neg, int64_t M,
                 int64_t K, int64_t O, float v_sat, float out_min, float out_max, float* out, void* workspace,
                 size_t workspace_bytes, hipStream_t s, const isa_ekv_glue* glue = nullptr,
-                float* idiff = nullptr, bool timed = true) {
+                float* idiff = nullptr, bool timed = true, bool contract = true) {
     if (M == 0 || O == 0) return 0;
     if (!out) return fail(ISA_EKV_EINVAL, "out is null");
     const FwdPlan p = plan_forward_call(cs.exact, cs.n_entries, M, K, O);
     SepPlan sp{};
     sp.bytes = p.bytes;
-    if (cs.exact) sp = plan_sep(M, K, O, false, false, false, p.bytes);
+    sp = plan_sep(cs.exact ? 0 : cs.n_entries, M, K, O, false, false, false, p.bytes);
+    // a workspace that only the per-cell kernels' plan fits runs them
+    if (!contract || (workspace_bytes < sp.bytes && workspace_bytes >= p.bytes)) {
+        sp = SepPlan{};
+        sp.bytes = p.bytes;
+    }
     if (!workspace || workspace_bytes < sp.bytes)
         return fail(ISA_EKV_EINVAL, "forward workspace too small (%zu < %zu bytes)", workspace_bytes, sp.bytes);
     char* ws = static_cast<char*>(workspace);
@@ -4402,8 +4427,9 @@ int run_forward(const CallSetup& cs, const float* x, const float* vth_pos, const
     unsigned* stat_bits = stats ? reinterpret_cast<unsigned*>(ws + p.off_stat) : nullptr;
     pa.stat_bits = stat_bits;
     const SepHead* sep_head = nullptr;
+    const SepArgs sep = make_sep(cs, x, vth_pos, vth_neg, M, K, O, v_sat, glue);
     if (sp.max_terms > 0) {  // its launches hold the prep for the case that it does not take the call
-        const hipError_t e = sep_forward(sp, make_sep(cs, x, vth_pos, vth_neg, M, K, O, v_sat, glue), pa, ws, s);
+        const hipError_t e = sep_forward_operands(sp, sep, pa, ws, s);
         if (e != hipSuccess) return hip_fail(e, "forward contraction launch");
         sep_head = reinterpret_cast<const SepHead*>(ws + sp.off_head);
     } else {
@@ -4466,7 +4492,7 @@ int run_forward(const CallSetup& cs, const float* x, const float* vth_pos, const
             hipLaunchKernelGGL(fwd_multi_assign_kernel, dim3((unsigned)((problems + kMcProblems - 1) / kMcProblems)),
                                dim3(kMcThreads), 0, s,
                                reinterpret_cast<float2*>(ws + p.off_wsT), fa.partials, fa.NP, tc.mc_budget,
-                               tc.mc_max, mode, p.Kp, p.Op, 0, fa.NP, 0, 0.0f);
+                               tc.mc_max, mode, p.Kp, p.Op, 0, fa.NP, 0, 0.0f, sep_head);
             err = hipGetLastError();
             if (err != hipSuccess) return hip_fail(err, "forward windowed-copy assignment launch");
         }
@@ -4474,7 +4500,7 @@ int run_forward(const CallSetup& cs, const float* x, const float* vth_pos, const
             hipLaunchKernelGGL(fwd_copy_assign_kernel<32>, agrid, dim3(kAssignThreads), 0, s,
                                reinterpret_cast<float2*>(ws + p.off_wsT), fa.partials, fa.NP,
                                fa.copy_window > 0 ? fa.copy_window : fa.NP, mode, p.Kp, p.Op, tc.copy_offset,
-                               tc.mc_budget > 0 ? kModeMultiMin : 0);
+                               tc.mc_budget > 0 ? kModeMultiMin : 0, sep_head);
             err = hipGetLastError();
             if (err != hipSuccess) return hip_fail(err, "forward copy assignment launch");
         }
@@ -4486,14 +4512,18 @@ int run_forward(const CallSetup& cs, const float* x, const float* vth_pos, const
     ProfiledLaunch* prof = nullptr;
     if (timed) prof_start(s, 0, &prof);
     if (timed && !cs.exact) fa.clock_acc = clock_acc(0);
+    if (sep_head) {
+        err = sep_forward_product(sp, sep, ws, s);
+        if (err != hipSuccess) return hip_fail(err, "forward contraction launch");
+    }
     launch_forward(cs.exact, gtab, p.mr, p.wpb, dim3(p.blocks), lds, s, fa);
     err = hipGetLastError();
     if (err == hipSuccess && !sep_head) err = finish_split(p, fa, !cs.exact, s);
     if (err == hipSuccess && sep_head) {
-        FwdArgs fs = fa;  // the contraction's planes, in units of I_S
+        FwdArgs fs = fa;  // the contraction's planes, the formula's in units of I_S
         fs.n_split = sp.split;
         fs.split_part = reinterpret_cast<float*>(ws + sp.off_planes);
-        fs.out_scale = (float)cs.i_s;
+        if (cs.exact) fs.out_scale = (float)cs.i_s;
         err = finish_sep(fs, fa, sep_head, !cs.exact, s);
     }
     prof_stop(s, prof);
@@ -4557,7 +4587,11 @@ int run_backward(const CallSetup& cs, const float* x, const float* vth_pos, cons
     const BwdPlan p = plan_backward(M, K, O, cs.exact ? 0 : cs.n_entries, need_x, need_w, glue != nullptr);
     SepPlan sp{};
     sp.bytes = p.bytes;
-    if (cs.exact && K > 0) sp = plan_sep(M, K, O, true, need_x, need_w, p.bytes);
+    sp = plan_sep(cs.exact ? 0 : cs.n_entries, M, K, O, true, need_x, need_w, p.bytes);
+    if (workspace_bytes < sp.bytes && workspace_bytes >= p.bytes) {  // as the forward's
+        sp = SepPlan{};
+        sp.bytes = p.bytes;
+    }
     if (!workspace || workspace_bytes < sp.bytes)
         return fail(ISA_EKV_EINVAL, "backward workspace too small (%zu < %zu bytes)", workspace_bytes, sp.bytes);
     char* ws = static_cast<char*>(workspace);
@@ -4589,13 +4623,13 @@ int run_backward(const CallSetup& cs, const float* x, const float* vth_pos, cons
     const PrepArgs pa = make_prep(cs, x, vth_pos, vth_neg, M, K, O, p.Kp, p.Op, v_sat, 4, ws, p.off_xrec, p.off_wsT,
                             p.off_xrec_alt, p.off_wsT_alt, p.off_part, glue);
     const SepHead* sep_head = nullptr;
+    SepArgs sep = make_sep(cs, x, vth_pos, vth_neg, M, K, O, v_sat, glue);
+    sep.need_x = need_x;
+    sep.need_w = need_w;
+    sep.g = glue ? ga.geff : grad_out;
+    sep.ldg = glue ? p.Op : O;
     if (sp.max_terms > 0) {
-        SepArgs a = make_sep(cs, x, vth_pos, vth_neg, M, K, O, v_sat, glue);
-        a.g = grad_out;
-        a.ldg = O;
-        a.need_x = need_x;
-        a.need_w = need_w;
-        err = sep_backward(sp, a, pa, ws, s);
+        err = sep_backward_operands(sp, sep, pa, glue ? &ga : nullptr, ws, s);
         if (err != hipSuccess) return hip_fail(err, "backward contraction launch");
         sep_head = reinterpret_cast<const SepHead*>(ws + sp.off_head);
     } else {
@@ -4661,7 +4695,7 @@ int run_backward(const CallSetup& cs, const float* x, const float* vth_pos, cons
                               reinterpret_cast<float*>(ws + p.off_rank_ws),
                               reinterpret_cast<uint2*>(ws + p.off_rank_branch), ba.partials, mode,
                               (int)p.Kp, (int)p.Op, p.n_ob, ba.NP, rank_max_spread,
-                              (float)g_rank_greedy_min.load(std::memory_order_relaxed)};
+                              (float)g_rank_greedy_min.load(std::memory_order_relaxed), sep_head};
             const int64_t threads = p.Kp * p.n_ob * kRankClasses;
             hipLaunchKernelGGL(bwd_rank_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, ra);
             // the greedy deal of spreads past greedy_min (exits at once when the rank deal
@@ -4680,18 +4714,18 @@ int run_backward(const CallSetup& cs, const float* x, const float* vth_pos, cons
             hipLaunchKernelGGL(fwd_multi_assign_kernel, dim3((unsigned)((problems + kMcProblems - 1) / kMcProblems)),
                                dim3(kMcThreads), 0, s, reinterpret_cast<float2*>(ws + p.off_wsT), ba.partials,
                                ba.NP, kBwdWinBudget, p.mc_max, mode, p.Kp, p.Op, kBwdWinDOffset, kBwdWinWindow,
-                               kBwdWinWideDOffset, p.ranked ? rank_max_spread : 0.0f);
+                               kBwdWinWideDOffset, p.ranked ? rank_max_spread : 0.0f, sep_head);
         }
         // (a pass before it recorded the ranked mode or the windowed copies: skip_from)
         const int skip_from = p.ranked ? kModeRanked : p.mc_max > 0 ? kModeMultiMin : 0;
         if (p.split)
             hipLaunchKernelGGL(fwd_copy_assign_kernel<32>, agrid, dim3(kAssignThreads), 0, s,
                                reinterpret_cast<float2*>(ws + p.off_wsT), ba.partials, ba.NP, kSplitRecords, mode,
-                               p.Kp, p.Op, kBwdCopyOffset, skip_from);
+                               p.Kp, p.Op, kBwdCopyOffset, skip_from, sep_head);
         else
             hipLaunchKernelGGL(fwd_copy_assign_kernel<16>, agrid, dim3(kAssignThreads), 0, s,
                                reinterpret_cast<float2*>(ws + p.off_wsT), ba.partials, ba.NP, kSplitRecords, mode,
-                               p.Kp, p.Op, kBwdCopyOffsetI, skip_from);
+                               p.Kp, p.Op, kBwdCopyOffsetI, skip_from, sep_head);
         ba.copy_mode = mode;
         err = hipGetLastError();
         if (err != hipSuccess) return hip_fail(err, "backward copy assignment launch");
@@ -4699,6 +4733,10 @@ int run_backward(const CallSetup& cs, const float* x, const float* vth_pos, cons
     ProfiledLaunch* prof;
     prof_start(s, 1, &prof);
     if (!cs.exact) ba.clock_acc = clock_acc(1);
+    if (sep_head) {
+        err = sep_backward_products(sp, sep, ws, s);
+        if (err != hipSuccess) return hip_fail(err, "backward contraction launch");
+    }
     if (p.halves)
         launch_backward_halves(need_x, need_w, grid, block, p.lds_bytes, s, ba);
     else if (copies) {
@@ -4756,21 +4794,20 @@ int run_backward(const CallSetup& cs, const float* x, const float* vth_pos, cons
     if (first_blocks > 0 && !sep_head)
         hipLaunchKernelGGL(grad_reduce_kernel, dim3((unsigned)first_blocks), dim3(256), 0, s, dxa, dx_blocks, dva,
                            dv_blocks, gra);
-    if (need_glue && glue_after)
-        hipLaunchKernelGGL(glue_reduce_kernel, dim3((unsigned)gl_blocks), dim3(256), 0, s, gra);
     if (sep_head) {
-        DxReduceArgs dxs = dxa;  // the contraction's planes, in units of I_S
+        DxReduceArgs dxs = dxa;  // the contraction's planes, the formula's in units of I_S
         dxs.part = reinterpret_cast<const float*>(ws + sp.off_planes);
-        dxs.n_planes = sp.split_dx;
-        dxs.scale = (float)cs.i_s;
+        dxs.n_planes = sp.planes_dx;
         DvReduceArgs dvs = dva;
         dvs.part = reinterpret_cast<const float*>(ws + sp.off_planes_dv);
-        dvs.n_split = sp.split_dv;
-        dvs.scale = (float)cs.i_s;
+        dvs.n_split = sp.planes_dv;
+        dxs.scale = dvs.scale = cs.exact ? (float)cs.i_s : 1.0f;
         dvs.mode_word = nullptr;
-        hipLaunchKernelGGL(sep_reduce_bwd_kernel, dim3((unsigned)(dx_blocks + dv_blocks)), dim3(256), 0, s, dxs, dxa,
-                           dx_blocks, dvs, dva, dv_blocks, sep_head);
+        hipLaunchKernelGGL(sep_reduce_bwd_kernel, dim3((unsigned)first_blocks), dim3(256), 0, s, dxs, dxa, dx_blocks, dvs,
+                           dva, dv_blocks, gra, sep_head, sp.split_dxh, sp.split_dvh);
     }
+    if (need_glue && glue_after)
+        hipLaunchKernelGGL(glue_reduce_kernel, dim3((unsigned)gl_blocks), dim3(256), 0, s, gra);
     err = hipGetLastError();
     if (err != hipSuccess) return hip_fail(err, "gradient reduction launch");
     return 0;
@@ -5178,8 +5215,10 @@ int isa_ekv_profile_end(double* ms, int* launches) {
 
 size_t isa_ekv_forward_workspace(int64_t M, int64_t K, int64_t O) {
     if (M < 0 || K < 0 || O < 0) return 0;
-    // the table size is not an argument: cover both block shapes run_forward may plan
-    return std::max(plan_forward(M, K, O, false).bytes, plan_forward(M, K, O, false, true, 2 * kFwdWaves).bytes);
+    // the table size is not an argument: cover both block shapes run_forward may plan, and the
+    // contraction's plan of the largest table it takes
+    const size_t cell = std::max(plan_forward(M, K, O, false).bytes, plan_forward(M, K, O, false, true, 2 * kFwdWaves).bytes);
+    return plan_sep(kSepLutMax, M, K, O, false, false, false, cell).bytes;
 }
 
 int isa_ekv_forward(const float* x, const float* vth_pos, const float* vth_neg, const void* lut_fwd, int64_t M,
@@ -5215,13 +5254,15 @@ int isa_ekv_forward_noalloc(const float* x, const float* vth_pos, const float* v
     if (src) return src;
     return run_forward(lut_setup(lut_fwd, n_entries, delta_min, delta_max), x, vth_pos, vth_neg, M, K, O, v_sat,
                        out_min, out_max, out, ws, kScratchBytes, static_cast<hipStream_t>(stream), nullptr, nullptr,
-                       false);
+                       false, false);
 }
 
 size_t isa_ekv_backward_workspace(int64_t M, int64_t K, int64_t O, int n_entries, int need_grad_x,
                                   int need_grad_w) {
     if (M < 0 || K < 0 || O < 0 || n_entries < 1) return 0;
-    return plan_backward(M, K, O, n_entries, need_grad_x != 0, need_grad_w != 0).bytes;
+    return plan_sep(n_entries, M, K, O, true, need_grad_x != 0, need_grad_w != 0,
+                    plan_backward(M, K, O, n_entries, need_grad_x != 0, need_grad_w != 0).bytes)
+        .bytes;
 }
 
 int isa_ekv_backward(const float* x, const float* vth_pos, const float* vth_neg, const float* grad_out,
@@ -5240,7 +5281,7 @@ int isa_ekv_backward(const float* x, const float* vth_pos, const float* vth_neg,
 
 size_t isa_ekv_exact_forward_workspace(int64_t M, int64_t K, int64_t O) {
     if (M < 0 || K < 0 || O < 0) return 0;
-    return plan_sep(M, K, O, false, false, false, plan_forward(M, K, O, true).bytes).bytes;
+    return plan_sep(0, M, K, O, false, false, false, plan_forward(M, K, O, true).bytes).bytes;
 }
 
 int isa_ekv_exact_forward(const float* x, const float* vth_pos, const float* vth_neg, int64_t M, int64_t K,
@@ -5257,7 +5298,7 @@ int isa_ekv_exact_forward(const float* x, const float* vth_pos, const float* vth
 
 size_t isa_ekv_exact_backward_workspace(int64_t M, int64_t K, int64_t O, int need_grad_x, int need_grad_w) {
     if (M < 0 || K < 0 || O < 0) return 0;
-    return plan_sep(M, K, O, true, need_grad_x != 0, need_grad_w != 0,
+    return plan_sep(0, M, K, O, true, need_grad_x != 0, need_grad_w != 0,
                     plan_backward(M, K, O, 0, need_grad_x != 0, need_grad_w != 0).bytes)
         .bytes;
 }
@@ -5282,7 +5323,9 @@ size_t isa_ekv_layer_forward_workspace(int64_t M, int64_t K, int64_t O) {
 size_t isa_ekv_layer_backward_workspace(int64_t M, int64_t K, int64_t O, int n_entries, int need_grad_x,
                                         int need_grad_w) {
     if (M < 0 || K < 0 || O < 0 || n_entries < 1) return 0;
-    return plan_backward(M, K, O, n_entries, need_grad_x != 0, need_grad_w != 0, true).bytes;
+    return plan_sep(n_entries, M, K, O, true, need_grad_x != 0, need_grad_w != 0,
+                    plan_backward(M, K, O, n_entries, need_grad_x != 0, need_grad_w != 0, true).bytes)
+        .bytes;
 }
 
 int isa_ekv_layer_forward(const float* x, const float* vth_pos, const float* vth_neg, const void* lut_fwd, int64_t M,
@@ -5382,7 +5425,7 @@ int isa_ekv_plan_info(int which, int64_t M, int64_t K, int64_t O, int n_entries,
     } else if (which == ISA_EKV_PLAN_BACKWARD || which == ISA_EKV_PLAN_LAYER_BACKWARD) {
         const bool nx = need_grad_x != 0, nw = need_grad_w != 0;
         const BwdPlan p = plan_backward(M, K, O, n_entries, nx, nw, which == ISA_EKV_PLAN_LAYER_BACKWARD);
-        v[0] = (int64_t)p.bytes;
+        v[0] = (int64_t)plan_sep(n_entries, M, K, O, true, nx, nw, p.bytes).bytes;
         v[1] = bwd_may_use_copies(p, false, nx) ? (int64_t)p.off_mode : -1;
         v[2] = p.n_split;
         v[3] = p.Kp / p.n_kb;
