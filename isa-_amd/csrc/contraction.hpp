@@ -17,8 +17,11 @@
 //
 // Precision. Operands are kept to 22 bits as the sum of two f16 (hi + lo, scaled by a power of
 // two per row so that the row's largest value is near 2^12), and every product is formed as
-// hi hi + hi lo + lo hi in fp32 accumulators; the differences T_j(t+) - T_j(t-) are formed in
-// fp64 before they are rounded, so that a cell no longer loses the bits in which its two
+// hi hi + hi lo + lo hi in fp32 accumulators. The upper half of the terms is below 1e-3 of the
+// lower half (their coefficients fall like rho^-j; for the slope's own sum, dVth, 4e-3) and is
+// kept as single f16, 1e-7 of the result: 2 R products per cell instead of 3 R. (The formula's
+// dVth keeps all its terms as pairs: its error before was 3.5e-7.) The differences
+// T_j(t+) - T_j(t-) are formed in fp64 before they are rounded, so that a cell no longer loses the bits in which its two
 // branches agree. c_j, d_j and g_j come from tables over x built per call in fp64 (cubic
 // interpolation, step at most kSepStep of 2 n U_T: 2e-8 relative; the step is a power of two,
 // so that a position within a step is exact in fp32).
@@ -45,6 +48,7 @@
 // holds, thresholds spread too far) runs the per-cell kernels, which return at once otherwise.
 
 typedef _Float16 sep_h8 __attribute__((ext_vector_type(8)));
+typedef _Float16 sep_h4 __attribute__((ext_vector_type(4)));
 typedef _Float16 sep_h2 __attribute__((ext_vector_type(2)));
 typedef float sep_f16 __attribute__((ext_vector_type(16)));
 typedef unsigned sep_u4 __attribute__((ext_vector_type(4)));
@@ -116,14 +120,16 @@ struct SepArgs {
     unsigned* gcol;          // backward: [kSepColChunks][O]
     float* tab;              // forward c_j r (j = 1..R), backward d_j r (j = 0..R-1): [n_grid][R]
     float* tab2;             // backward g_j (j = 1..R)
-    _Float16* xop;           // forward [M][Kd], backward [K R][Md]: hi/lo pairs, 32 + 32
-    _Float16* wop;           // forward [O][Kd], backward [K R][Od]
-    _Float16* gop;           // backward [M][Od]
-    _Float16* gopT;          // backward [O][Md]
-    _Float16* xoph;          // backward, harmonics: [K ng 8][Md] single f16, 64 a slab
-    _Float16* woph;          // backward, harmonics: [K ng 8][Od]
-    _Float16* goph;          // backward, harmonics: [M][Od]
-    _Float16* gophT;         // backward, harmonics: [O][Md]
+    _Float16* xop;           // forward [M][Kd], backward (pairs, lower terms) [rows][Md]
+    _Float16* wop;           // forward [O][Kd], backward [rows][Od]
+    _Float16* xops;          // backward, upper terms, singles: [rows][Md]
+    _Float16* wops;          // [rows][Od]
+    _Float16* xoph;          // backward, harmonics, singles: [rows][Md]
+    _Float16* woph;          // [rows][Od]
+    _Float16* gop;           // backward, pairs: [M][Od]
+    _Float16* gopT;          // [O][Md]
+    _Float16* goph;          // backward, singles: [M][Od]
+    _Float16* gophT;         // [O][Md]
     float* xscale;           // forward [M], backward [K]: inverse scale of xop's rows
     float* gscale;           // backward [M]
     float* gscaleT;          // backward [O]
@@ -136,16 +142,26 @@ __device__ inline float sep_input(const SepArgs& a, float x, float s, float b) {
     return a.in_affine ? input_map(x, s, b, a.in_lo, a.in_hi) : x;
 }
 
-// Inner lengths in f16 pairs' slabs of 32: the forward's (j / 8, k, j % 8) index, each eight
-// terms of four inputs a slab (K padded to fours), tokens and outputs of the backward.
-__host__ __device__ inline int64_t sep_slabs_kj(int64_t K, int terms) { return (K + 3) / 4 * (terms / 8); }
+// Layouts. An operand's row is a run of slabs of 128 bytes: 32 inner elements as pairs (their hi
+// halves, then their lo halves) or 64 single f16.
+// Forward, a row's inner elements: the lower terms as pairs, ordered (j / 4, k, j % 4), the
+// upper ones as singles likewise, then (tables) the harmonics as singles; inputs padded to 16.
+// Backward, tokens or outputs inside, rows in blocks of eight: four terms of an even input and of
+// the odd one after it, so that a lane of the matrix cores' result holds one input's. The lower
+// terms, the upper ones and the harmonics are operands of their own.
+// Harmonics: an input has R values in blocks of four, at 8 terms of each harmonic its two cosines
+// and two sines, at 16 the first one's four cosines, its four sines, then the second one's.
+__host__ __device__ inline int64_t sep_inputs(int64_t K) { return (K + 15) / 16 * 16; }
+__host__ __device__ inline int64_t sep_slabs_pairs(int64_t K, int terms) { return sep_inputs(K) * (terms / 2) / 32; }
+__host__ __device__ inline int64_t sep_slabs_singles(int64_t K, int terms, int harmonics) {
+    return sep_inputs(K) * (terms / 2 + harmonics * terms) / 64;
+}
 __host__ __device__ inline int64_t sep_slabs(int64_t n) { return (n + 31) / 32; }
-// Harmonics: an input has terms / 8 groups of eight values, slabs of 64 single f16. At 8 terms
-// one group, of each harmonic its two cosines and two sines; at 16 a group per harmonic, of four
-// cosines and four sines.
-__host__ __device__ inline int sep_groups(int terms, int harmonics) { return harmonics * (terms / 8); }
-__host__ __device__ inline int64_t sep_slabs_harm(int64_t K, int groups) { return (K + 7) / 8 * groups; }
 __host__ __device__ inline int64_t sep_slabs64(int64_t n) { return (n + 63) / 64; }
+// Row of input k's value v (of its `per`) among the backward's rows.
+__host__ __device__ inline int64_t sep_row(int64_t k, int per, int v) {
+    return ((k >> 1) * (per / 4) + (v >> 2)) * 8 + (k & 1) * 4 + (v & 3);
+}
 
 // ----------------------------------------------------------------------------------
 // Statistics: ranges of x (per row forward, per column backward), of the thresholds, and the
@@ -607,34 +623,40 @@ __device__ inline void sep_store2(_Float16* row, int64_t e, float v0, float v1) 
 }
 
 // ----------------------------------------------------------------------------------
-// Forward operands: xop[m][(j / 8, k, j % 8)] = c_j r (a wave per row, lanes along k) and
-// wop[o][(j / 8, k, j % 8)] = T_j(t+) - T_j(t-), each (row, k) R values in 16-byte stores. HBM-bound: four
-// bytes per value written.
+// Forward operands: xop[m] = c_j r (a wave per row, lanes along k) and wop[o] = T_j(t+) - T_j(t-),
+// each (row, k) four values in 8-byte stores that neighbouring lanes continue. HBM-bound.
 // ----------------------------------------------------------------------------------
 
 constexpr int kSepExpandBlocks = 2048;
 
-__device__ inline void sep_store8(_Float16* row, int64_t e, const float v[8]) {
-    sep_h8 hi, lo;
+__device__ inline void sep_store4(_Float16* row, int64_t e, const float v[4]) {  // pairs
+    sep_h4 hi, lo;
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
+    for (int q = 0; q < 4; ++q) {
         _Float16 h, l;
         sep_split(v[q], h, l);
         hi[q] = h;
         lo[q] = l;
     }
     _Float16* p = row + (e >> 5) * 64 + (e & 31);
-    *reinterpret_cast<sep_h8*>(p) = hi;
-    *reinterpret_cast<sep_h8*>(p + 32) = lo;
+    *reinterpret_cast<sep_h4*>(p) = hi;
+    *reinterpret_cast<sep_h4*>(p + 32) = lo;
 }
 
-// Walks T_1, T_2, ... of both branches and hands out blocks of eight differences.
+__device__ inline void sep_store4h(_Float16* row, int64_t e, const float v[4]) {  // singles
+    sep_h4 h;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) h[q] = (_Float16)v[q];
+    *reinterpret_cast<sep_h4*>(row + e) = h;
+}
+
+// Walks T_1, T_2, ... of both branches and hands out blocks of four differences.
 struct SepChebPair {
     double p0 = 1.0, p1, n0 = 1.0, n1, tp, tn;
     __device__ SepChebPair(double a, double b) : p1(a), n1(b), tp(2.0 * a), tn(2.0 * b) {}
-    __device__ void next8(float* v, float scale) {  // T_j(t+) - T_j(t-) of the next eight j
+    __device__ void next4(float* v, float scale) {  // T_j(t+) - T_j(t-) of the next four j
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
+        for (int q = 0; q < 4; ++q) {
             v[q] = (float)(p1 - n1) * scale;
             const double p2 = tp * p1 - p0, n2 = tn * n1 - n0;
             p0 = p1;
@@ -654,53 +676,40 @@ __device__ inline void sep_trig(float theta, float* c, float* sn) {
     sn[1] = 2.0f * sn[0] * c[0];
 }
 
-__device__ inline sep_h8 sep_pack8(const float v[8]) {
-    sep_h8 h;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) h[q] = (_Float16)v[q];
-    return h;
-}
-
-// Group blk of an input's harmonic values on the token side: the second difference's
+// Block blk of an input's harmonic values on the token side: the second difference's
 // coefficients e times cosine and sine.
-__device__ inline void sep_harm_x(float v[8], const float e[4], int terms, int blk, const float c[2], const float sn[2],
+__device__ inline void sep_harm_x(float v[4], const float e[4], int terms, int blk, const float c[2], const float sn[2],
                                   float scale) {
+    const float ca = c[0], cb = c[1], sa = sn[0], sb = sn[1];
     if (terms == 8) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            v[i] = e[i] * (c[0] * scale);
-            v[2 + i] = e[i] * (sn[0] * scale);
-            v[4 + i] = e[i] * (c[1] * 0.25f * scale);
-            v[6 + i] = e[i] * (sn[1] * 0.25f * scale);
-        }
+        const float f = blk ? 0.25f * scale : scale, fc = (blk ? cb : ca) * f, fs = (blk ? sb : sa) * f;
+        v[0] = e[0] * fc;
+        v[1] = e[1] * fc;
+        v[2] = e[0] * fs;
+        v[3] = e[1] * fs;
     } else {
-        const float f = blk ? 0.25f * scale : scale, fc = (blk ? c[1] : c[0]) * f, fs = (blk ? sn[1] : sn[0]) * f;
+        const float t = blk & 1 ? (blk & 2 ? sb : sa) : (blk & 2 ? cb : ca);
+        const float f = t * (blk & 2 ? 0.25f * scale : scale);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            v[i] = e[i] * fc;
-            v[4 + i] = e[i] * fs;
-        }
+        for (int i = 0; i < 4; ++i) v[i] = e[i] * f;
     }
 }
 
 // Likewise on the threshold side: T_i(t+) cos - T_i(t-) cos, ...
-__device__ inline void sep_harm_w(float v[8], const float tp[4], const float tn[4], int terms, int blk, const float cp[2],
+__device__ inline void sep_harm_w(float v[4], const float tp[4], const float tn[4], int terms, int blk, const float cp[2],
                                   const float sp[2], const float cn[2], const float sn[2], float scale) {
+    const float cpa = cp[0], cpb = cp[1], spa = sp[0], spb = sp[1], cna = cn[0], cnb = cn[1], sna = sn[0], snb = sn[1];
     if (terms == 8) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            v[i] = (tp[i] * cp[0] - tn[i] * cn[0]) * scale;
-            v[2 + i] = (tp[i] * sp[0] - tn[i] * sn[0]) * scale;
-            v[4 + i] = (tp[i] * cp[1] - tn[i] * cn[1]) * scale;
-            v[6 + i] = (tp[i] * sp[1] - tn[i] * sn[1]) * scale;
-        }
+        const float c0 = blk ? cpb : cpa, s0 = blk ? spb : spa, c1 = blk ? cnb : cna, s1 = blk ? snb : sna;
+        v[0] = (c0 - c1) * scale;
+        v[1] = (tp[1] * c0 - tn[1] * c1) * scale;
+        v[2] = (s0 - s1) * scale;
+        v[3] = (tp[1] * s0 - tn[1] * s1) * scale;
     } else {
-        const float c0 = blk ? cp[1] : cp[0], s0 = blk ? sp[1] : sp[0], c1 = blk ? cn[1] : cn[0], s1 = blk ? sn[1] : sn[0];
+        const float f0 = blk & 1 ? (blk & 2 ? spb : spa) : (blk & 2 ? cpb : cpa);
+        const float f1 = blk & 1 ? (blk & 2 ? snb : sna) : (blk & 2 ? cnb : cna);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            v[i] = (tp[i] * c0 - tn[i] * c1) * scale;
-            v[4 + i] = (tp[i] * s0 - tn[i] * s1) * scale;
-        }
+        for (int i = 0; i < 4; ++i) v[i] = (tp[i] * f0 - tn[i] * f1) * scale;
     }
 }
 
@@ -746,66 +755,65 @@ __global__ __launch_bounds__(256) void sep_expand_fwd_kernel(SepArgs a, PrepArgs
     const int R = h.terms;
     if (blockIdx.x == 0) sep_write_partials(h, prep);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t slabs = sep_slabs_kj(a.K, R);
-    const int groups = sep_groups(R, h.harmonics);
-    const int64_t stride = (slabs + sep_slabs_harm(a.K, groups)) * 64;  // of a row, in f16
-    const int64_t kc = (a.K + 3) / 4 * 4, k8 = (a.K + 7) / 8 * 8;  // inputs with their padding
-    const int64_t kw = groups > 0 ? k8 : kc;
+    const int64_t kc = sep_inputs(a.K), pairs = sep_slabs_pairs(a.K, R) * 64;
+    const int64_t stride = pairs + sep_slabs_singles(a.K, R, h.harmonics) * 64;  // of a row, in f16
+    const int64_t harm = pairs + kc * (R / 2);
     const int64_t row_waves = (int64_t)gridDim.x * 4;
     const float as = a.in_affine ? a.in_affine[0] : 1.0f, ab = a.in_affine ? a.in_affine[1] : 0.0f;
-    float v[8];
+    float v[4];
     for (int64_t row = (int64_t)blockIdx.x * 4 + wave; row < a.M + a.O; row += row_waves) {
         if (row < a.M) {
             float inv;
             const float scale = sep_scale_of(sep_bound(h, a.tab, 0, a.xrow[row], (float)a.v_sat), &inv);
             if (lane == 0) a.xscale[row] = inv / kSepQScale;
             _Float16* dst = a.xop + row * stride;
-            for (int64_t k = lane; k < kw; k += 64) {
+            for (int64_t k = lane; k < kc; k += 64) {
                 const bool real = k < a.K;
                 const float x = sep_input(a, a.x[row * a.K + (real ? k : a.K - 1)], as, ab);
                 const float sc = real ? scale : 0.0f;
                 const SepAt at = sep_at(h, x);
-                if (k < kc) {
-                    for (int j = 0; j < R; j += 8) {
-                        const float4 lo = sep_eval4(a.tab, R, at, j), hi = sep_eval4(a.tab, R, at, j + 4);
-                        v[0] = lo.x * sc; v[1] = lo.y * sc; v[2] = lo.z * sc; v[3] = lo.w * sc;
-                        v[4] = hi.x * sc; v[5] = hi.y * sc; v[6] = hi.z * sc; v[7] = hi.w * sc;
-                        sep_store8(dst, kc * j + k * 8, v);
-                    }
+                for (int j = 0; j < R; j += 4) {
+                    const float4 c = sep_eval4(a.tab, R, at, j);
+                    v[0] = c.x * sc; v[1] = c.y * sc; v[2] = c.z * sc; v[3] = c.w * sc;
+                    if (j < R / 2)
+                        sep_store4(dst, j * kc + k * 4, v);
+                    else
+                        sep_store4h(dst + pairs, (j - R / 2) * kc + k * 4, v);
                 }
-                if (groups > 0) {
+                if (h.harmonics > 0) {
                     float e[4], c[2], sn[2];
                     sep_second(h, a.tabE, at, e);
                     sep_trig((x - h.lut_min) * h.lut_scale, c, sn);
-                    for (int blk = 0; blk < groups; ++blk) {
+                    for (int blk = 0; blk < R / 4; ++blk) {
                         sep_harm_x(v, e, R, blk, c, sn, sc);
-                        *reinterpret_cast<sep_h8*>(dst + slabs * 64 + (blk * k8 + k) * 8) = sep_pack8(v);
+                        sep_store4h(dst + harm, blk * 4 * kc + k * 4, v);
                     }
                 }
             }
         } else {
             const int64_t o = row - a.M;
             _Float16* dst = a.wop + o * stride;
-            for (int64_t k = lane; k < kw; k += 64) {
+            for (int64_t k = lane; k < kc; k += 64) {
                 const bool real = k < a.K;
                 const double tp = real ? ((double)a.wp[o * a.K + k] - h.wc) * h.inv_wh : 0.0;
                 const double tn = real ? ((double)a.wn[o * a.K + k] - h.wc) * h.inv_wh : 0.0;
-                if (k < kc) {
-                    SepChebPair c(tp, tn);
-                    for (int j = 0; j < R; j += 8) {
-                        c.next8(v, kSepQScale);
-                        sep_store8(dst, kc * j + k * 8, v);
-                    }
+                SepChebPair c(tp, tn);
+                for (int j = 0; j < R; j += 4) {
+                    c.next4(v, kSepQScale);
+                    if (j < R / 2)
+                        sep_store4(dst, j * kc + k * 4, v);
+                    else
+                        sep_store4h(dst + pairs, (j - R / 2) * kc + k * 4, v);
                 }
-                if (groups > 0) {
+                if (h.harmonics > 0) {
                     float p[4], n[4], cp[2], sp[2], cn[2], sn[2];
                     sep_cheb4((float)tp, p);
                     sep_cheb4((float)tn, n);
                     sep_trig((float)((h.wc + h.wh * tp) * h.lut_scale), cp, sp);
                     sep_trig((float)((h.wc + h.wh * tn) * h.lut_scale), cn, sn);
-                    for (int blk = 0; blk < groups; ++blk) {
+                    for (int blk = 0; blk < R / 4; ++blk) {
                         sep_harm_w(v, p, n, R, blk, cp, sp, cn, sn, kSepQScale);
-                        *reinterpret_cast<sep_h8*>(dst + slabs * 64 + (blk * k8 + k) * 8) = sep_pack8(v);
+                        sep_store4h(dst + harm, blk * 4 * kc + k * 4, v);
                     }
                 }
             }
@@ -814,7 +822,7 @@ __global__ __launch_bounds__(256) void sep_expand_fwd_kernel(SepArgs a, PrepArgs
 }
 
 // ----------------------------------------------------------------------------------
-// Backward operands, inner index contiguous: xop[(k, j)][m] = d_j r, wop[(k, j)][o] = T_j(t+) -
+// Backward operands, tokens or outputs inside: xop[(k, j)][m] = d_j r, wop[(k, j)][o] = T_j(t+) -
 // T_j(t-) with tT[k][o] = {t+, t-}, gop[m][o] and gopT[o][m]. Tiles of 32 inputs (or rows of G)
 // by 128 inner elements go through LDS, so that reads run along the tensors' rows and writes
 // along the inner index. HBM-bound.
@@ -835,8 +843,8 @@ __global__ __launch_bounds__(256) void sep_expand_bwd_kernel(SepArgs a, int x_bl
     const SepHead h = *a.head;
     const int R = h.terms;
     if (blockIdx.x == 0) sep_write_partials(h, prep);
-    const int groups = sep_groups(R, h.harmonics);
-    const int64_t m64 = sep_slabs64(a.M) * 64, o64 = sep_slabs64(a.O) * 64;  // harmonics' inner lengths
+    const int64_t m64 = sep_slabs64(a.M) * 64, o64 = sep_slabs64(a.O) * 64;  // the singles' inner lengths
+    const int xpairs = a.lut_n > 0 ? R / 2 : R;  // terms of xop as pairs
     __shared__ float s_a[32][130], s_b[32][130];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int64_t m_slabs = sep_slabs(a.M), o_slabs = sep_slabs(a.O);
@@ -860,32 +868,35 @@ __global__ __launch_bounds__(256) void sep_expand_bwd_kernel(SepArgs a, int x_bl
             if (m0 == 0 && lane == 0) a.xscale[k] = inv;
             const int ml = 2 * lane;
             const int64_t m = m0 + ml;
-            if (m >= (groups > 0 ? m64 : m_slabs * 32)) continue;
+            if (m >= m64) continue;
+            const bool pair = m < m_slabs * 32;
             const float s0 = m < a.M ? scale : 0.0f, s1 = m + 1 < a.M ? scale : 0.0f;
-            const SepAt p0 = sep_at(h, m < a.M ? s_a[kk][ml] : range.y);
-            const SepAt p1 = sep_at(h, m + 1 < a.M ? s_a[kk][ml + 1] : range.y);
-            if (groups > 0) {
-                float e0[4], e1[4], c0[2], n0[2], c1[2], n1[2], u[8], v[8];
+            const float x0 = m < a.M ? s_a[kk][ml] : range.y, x1 = m + 1 < a.M ? s_a[kk][ml + 1] : range.y;
+            const SepAt p0 = sep_at(h, x0), p1 = sep_at(h, x1);
+            for (int j = 0; j < R; j += 4) {
+                const float4 u = sep_eval4(a.tab, R, p0, j), v = sep_eval4(a.tab, R, p1, j);
+                const float u4[4] = {u.x * s0, u.y * s0, u.z * s0, u.w * s0}, v4[4] = {v.x * s1, v.y * s1, v.z * s1, v.w * s1};
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    if (j < xpairs) {
+                        if (pair) sep_store2(a.xop + sep_row(k, xpairs, j + q) * m_slabs * 64, m, u4[q], v4[q]);
+                    } else {
+                        sep_store2h(a.xops + sep_row(k, R / 2, j + q - R / 2) * m64, m, u4[q], v4[q]);
+                    }
+                }
+            }
+            if (h.harmonics > 0) {
+                float e0[4], e1[4], c0[2], n0[2], c1[2], n1[2], u[4], v[4];
                 sep_second(h, a.tabE, p0, e0);
                 sep_second(h, a.tabE, p1, e1);
-                sep_trig((s_a[kk][ml] - h.lut_min) * h.lut_scale, c0, n0);
-                sep_trig((s_a[kk][ml + 1] - h.lut_min) * h.lut_scale, c1, n1);
-                _Float16* dst = a.xoph + k * groups * 8 * m64;
-                for (int blk = 0; blk < groups; ++blk) {
+                sep_trig((x0 - h.lut_min) * h.lut_scale, c0, n0);
+                sep_trig((x1 - h.lut_min) * h.lut_scale, c1, n1);
+                for (int blk = 0; blk < R / 4; ++blk) {
                     sep_harm_x(u, e0, R, blk, c0, n0, s0);
                     sep_harm_x(v, e1, R, blk, c1, n1, s1);
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) sep_store2h(dst + (blk * 8 + i) * m64, m, u[i], v[i]);
+                    for (int q = 0; q < 4; ++q) sep_store2h(a.xoph + sep_row(k, R, blk * 4 + q) * m64, m, u[q], v[q]);
                 }
-            }
-            if (m >= m_slabs * 32) continue;
-            for (int j = 0; j < R; j += 4) {
-                const float4 u = sep_eval4(a.tab, R, p0, j), v = sep_eval4(a.tab, R, p1, j);
-                _Float16* dst = a.xop + (k * R + j) * m_slabs * 64;
-                sep_store2(dst, m, u.x * s0, v.x * s1);
-                sep_store2(dst + m_slabs * 64, m, u.y * s0, v.y * s1);
-                sep_store2(dst + 2 * m_slabs * 64, m, u.z * s0, v.z * s1);
-                sep_store2(dst + 3 * m_slabs * 64, m, u.w * s0, v.w * s1);
             }
         }
         return;
@@ -905,7 +916,8 @@ __global__ __launch_bounds__(256) void sep_expand_bwd_kernel(SepArgs a, int x_bl
             const int64_t k = k0 + kk;
             const int ol = 2 * lane;
             const int64_t o = o0 + ol;
-            if (o >= (groups > 0 ? o64 : o_slabs * 32)) continue;
+            if (o >= o64) continue;
+            const bool pair = o < o_slabs * 32;
             double t_[4];
 #pragma unroll
             for (int q = 0; q < 2; ++q) {
@@ -917,34 +929,37 @@ __global__ __launch_bounds__(256) void sep_expand_bwd_kernel(SepArgs a, int x_bl
                     make_float4((float)t_[0], (float)t_[1], (float)t_[2], (float)t_[3]);
             }
             if (!a.need_x) continue;
-            const bool r0 = o < a.O, r1 = o + 1 < a.O;
-            if (groups > 0) {
-                _Float16* dst = a.woph + k * groups * 8 * o64;
-                float p0[4], n0[4], p1[4], n1[4], c0[4], d0[4], c1[4], d1[4], u[8], v[8];
+            // padded outputs: both branches at the centre, so that their differences vanish
+            SepChebPair c0(t_[0], t_[1]), c1(t_[2], t_[3]);
+            float u[4], v[4];
+            for (int j = 0; j < R; j += 4) {
+                c0.next4(u, kSepQScale);
+                c1.next4(v, kSepQScale);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    if (j < R / 2) {
+                        if (pair) sep_store2(a.wop + sep_row(k, R / 2, j + q) * o_slabs * 64, o, u[q], v[q]);
+                    } else {
+                        sep_store2h(a.wops + sep_row(k, R / 2, j + q - R / 2) * o64, o, u[q], v[q]);
+                    }
+                }
+            }
+            if (h.harmonics > 0) {
+                float p0[4], n0[4], p1[4], n1[4], e0[4], d0[4], e1[4], d1[4];
                 sep_cheb4((float)t_[0], p0);
                 sep_cheb4((float)t_[1], n0);
                 sep_cheb4((float)t_[2], p1);
                 sep_cheb4((float)t_[3], n1);
-                sep_trig(s_a[kk][ol] * h.lut_scale, c0, d0);
-                sep_trig(s_b[kk][ol] * h.lut_scale, c0 + 2, d0 + 2);
-                sep_trig(s_a[kk][ol + 1] * h.lut_scale, c1, d1);
-                sep_trig(s_b[kk][ol + 1] * h.lut_scale, c1 + 2, d1 + 2);
-                for (int blk = 0; blk < groups; ++blk) {
-                    sep_harm_w(u, p0, n0, R, blk, c0, d0, c0 + 2, d0 + 2, r0 ? kSepQScale : 0.0f);
-                    sep_harm_w(v, p1, n1, R, blk, c1, d1, c1 + 2, d1 + 2, r1 ? kSepQScale : 0.0f);
+                sep_trig(s_a[kk][ol] * h.lut_scale, e0, d0);
+                sep_trig(s_b[kk][ol] * h.lut_scale, e0 + 2, d0 + 2);
+                sep_trig(s_a[kk][ol + 1] * h.lut_scale, e1, d1);
+                sep_trig(s_b[kk][ol + 1] * h.lut_scale, e1 + 2, d1 + 2);
+                for (int blk = 0; blk < R / 4; ++blk) {
+                    sep_harm_w(u, p0, n0, R, blk, e0, d0, e0 + 2, d0 + 2, kSepQScale);
+                    sep_harm_w(v, p1, n1, R, blk, e1, d1, e1 + 2, d1 + 2, kSepQScale);
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) sep_store2h(dst + (blk * 8 + i) * o64, o, u[i], v[i]);
+                    for (int q = 0; q < 4; ++q) sep_store2h(a.woph + sep_row(k, R, blk * 4 + q) * o64, o, u[q], v[q]);
                 }
-                if (o >= o_slabs * 32) continue;
-            }
-            SepChebPair c0(r0 ? t_[0] : 0.0, r0 ? t_[1] : 0.0), c1(r1 ? t_[2] : 0.0, r1 ? t_[3] : 0.0);
-            float u[8], v[8];
-            for (int j = 0; j < R; j += 8) {
-                c0.next8(u, kSepQScale);
-                c1.next8(v, kSepQScale);
-                _Float16* dst = a.wop + (k * R + j) * o_slabs * 64;
-#pragma unroll
-                for (int q = 0; q < 8; ++q) sep_store2(dst + q * o_slabs * 64, o, u[q], v[q]);
             }
         }
         return;
@@ -967,7 +982,7 @@ __global__ __launch_bounds__(256) void sep_expand_bwd_kernel(SepArgs a, int x_bl
             if (o0 == 0 && lane == 0) a.gscale[m] = inv / kSepQScale;
             const float g0 = s_a[mm][2 * lane] * scale, g1 = s_a[mm][2 * lane + 1] * scale;
             if (o < o_slabs * 32) sep_store2(a.gop + m * o_slabs * 64, o, g0, g1);
-            if (groups > 0 && o < o64) sep_store2h(a.goph + m * o64, o, g0, g1);
+            if (o < o64) sep_store2h(a.goph + m * o64, o, g0, g1);
         }
     }
     if (a.need_w) {
@@ -983,10 +998,8 @@ __global__ __launch_bounds__(256) void sep_expand_bwd_kernel(SepArgs a, int x_bl
             const int mm = 2 * (t & 15);
             const float g0 = s_a[mm][q] * scale, g1 = s_a[mm + 1][q] * scale;
             sep_store2(a.gopT + o * m_slabs * 64, m0 + mm, g0, g1);
-            if (groups > 0) {
-                sep_store2h(a.gophT + o * m64, m0 + mm, g0, g1);
-                if (m0 + 32 >= a.M && m0 + 32 < m64) sep_store2h(a.gophT + o * m64, m0 + 32 + mm, 0.0f, 0.0f);
-            }
+            sep_store2h(a.gophT + o * m64, m0 + mm, g0, g1);
+            if (m0 + 32 >= a.M && m0 + 32 < m64) sep_store2h(a.gophT + o * m64, m0 + 32 + mm, 0.0f, 0.0f);
         }
     }
 }
@@ -1003,24 +1016,24 @@ __global__ __launch_bounds__(256) void sep_expand_bwd_kernel(SepArgs a, int x_bl
 // banks. Rows past the operand's end read its last row (their results are dropped).
 // Blocks are dealt so that each XCD works on neighbouring tiles (whose operands its L2 holds).
 //
-// A launch runs up to four products after one another in its grid (the backward's dX and dVth,
-// of pairs and of harmonics), so that one's last blocks overlap the next one's first.
+// A launch runs up to six products after one another in its grid (the backward's dX and dVth, of
+// the lower terms, the upper ones and the harmonics), so that one's last blocks overlap the next one's first.
 // ----------------------------------------------------------------------------------
 
-enum SepKind { kSepForward, kSepDx, kSepDv, kSepDxHarm, kSepDvHarm };
+enum SepKind { kSepForward, kSepDx, kSepDv, kSepDxUpper, kSepDvUpper, kSepDxHarm, kSepDvHarm };
 
 struct SepProduct {
     const char* a;
     const char* b;
     int kind;
-    int64_t a_rows, b_rows;   // A rows per eight of an input's terms (dX, dVth), else in all
+    int64_t a_rows, b_rows;   // dX, dVth: inputs in the place of A's rows
     int64_t inner;            // elements; forward: inputs
     int n_split;
     float* out;               // forward: planes [n_split][M][O]; dX: [n_split][M][K]; dVth: [n_split][2][Kp][Op]
 };
 
 struct SepGemm {
-    SepProduct p[4];
+    SepProduct p[6];
     int n;
     const SepHead* head;
     int64_t M, K, O, Kp, Op;
@@ -1033,6 +1046,7 @@ struct SepGemm {
     const float* tab2;
     const float* tabE;
     const float2* tT;
+    int dv_all;               // the dVth product of pairs holds every term
 };
 
 template <int WM, int WN, int MI, int NI, bool FORWARD>
@@ -1043,23 +1057,23 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void sep_gemm_kernel(SepGemm g) {
     const SepHead* head = g.head;
     if (!sep_takes(head)) return;
     const int R = __builtin_amdgcn_readfirstlane(head->terms);
-    const int groups = sep_groups(R, __builtin_amdgcn_readfirstlane(head->harmonics));
-    const int nb = R / 8;
-    // the product this block works on, its rows and slabs
-    int id = blockIdx.x, which = 0, ta = 0, tb = 0, n = 0, slabs = 0, pair_slabs = 0;
+    const int harmonics = __builtin_amdgcn_readfirstlane(head->harmonics);
+    // the product this block works on, its rows and slabs, and the blocks of four values per input
+    int id = blockIdx.x, which = 0, ta = 0, tb = 0, n = 0, slabs = 0, pair_slabs = 0, per = 0;
     int64_t a_rows = 0;
     for (;; ++which) {
         if (which >= g.n) return;
         const SepProduct& p = g.p[which];
-        const bool harm = p.kind >= kSepDxHarm;
         if constexpr (FORWARD) {
             a_rows = p.a_rows;
-            pair_slabs = (int)sep_slabs_kj(p.inner, R);
-            slabs = pair_slabs + (int)sep_slabs_harm(p.inner, groups);
+            pair_slabs = (int)sep_slabs_pairs(p.inner, R);
+            slabs = pair_slabs + (int)sep_slabs_singles(p.inner, R, harmonics);
         } else {
-            a_rows = p.a_rows * 8 * (harm ? groups : nb);
-            slabs = (int)(harm ? sep_slabs64(p.inner) : sep_slabs(p.inner));
-            pair_slabs = harm ? 0 : slabs;
+            const bool pairs = p.kind == kSepDx || p.kind == kSepDv;
+            per = p.kind >= kSepDxHarm ? harmonics * R / 4 : p.kind == kSepDv && g.dv_all ? R / 4 : R / 8;
+            a_rows = (p.a_rows + 1) / 2 * 8 * per;
+            slabs = (int)(pairs ? sep_slabs(p.inner) : sep_slabs64(p.inner));
+            pair_slabs = pairs ? slabs : 0;
         }
         ta = (int)((a_rows + TM - 1) / TM);
         tb = (int)((p.b_rows + TN - 1) / TN);
@@ -1084,7 +1098,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void sep_gemm_kernel(SepGemm g) {
 
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int wr = wave / WN, wc = wave % WN;
-    const int part = t & 7, row0 = t >> 3;
+    const int row0 = t >> 3, part = (t & 7) ^ ((row0 >> 1) & 7);
     unsigned pa[kLoadA], pb[kLoadB];  // byte offsets (an operand holds less than 4 GiB)
 #pragma unroll
     for (int q = 0; q < kLoadA; ++q) {
@@ -1099,7 +1113,6 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void sep_gemm_kernel(SepGemm g) {
     constexpr int kBuf = (TM + TN) * 128;
     // kRowStep rows further on the swizzle is the same: kRowStep is a multiple of 16
     static_assert(kRowStep % 16 == 0, "");
-    const int st_off = row0 * 128 + ((part ^ ((row0 >> 1) & 7)) << 4);
     const int fl = lane & 31, fh = lane >> 5;
     const int frag = fl * 128 + ((fh ^ ((fl >> 1) & 7)) << 4);
     const int fa = wr * MI * 32 * 128, fb = TM * 128 + wc * NI * 32 * 128;
@@ -1114,19 +1127,18 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void sep_gemm_kernel(SepGemm g) {
 
     const char* abase = p.a;
     const char* bbase = p.b;
-    sep_u4 ra[kLoadA], rb[kLoadB];
-    auto load = [&](int s) {
+    // a wave's loads of a slab: eight rows of 128 bytes each, straight into LDS (lane i to byte
+    // 16 i of the kilobyte): the lane that fills part p of a row reads part p ^ (row / 2 % 8)
+    auto copy = [&](int s, int buf) {
+        char* dst = s_sep + buf * kBuf + wave * 1024;
 #pragma unroll
-        for (int q = 0; q < kLoadA; ++q) ra[q] = *reinterpret_cast<const sep_u4*>(abase + (pa[q] + (unsigned)s * 128u));
+        for (int q = 0; q < kLoadA; ++q)
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(abase + (pa[q] + (unsigned)s * 128u)),
+                                             (__attribute__((address_space(3))) void*)(dst + q * kThreads * 16), 16, 0, 0);
 #pragma unroll
-        for (int q = 0; q < kLoadB; ++q) rb[q] = *reinterpret_cast<const sep_u4*>(bbase + (pb[q] + (unsigned)s * 128u));
-    };
-    auto store = [&](int buf) {
-        char* base = s_sep + buf * kBuf + st_off;
-#pragma unroll
-        for (int q = 0; q < kLoadA; ++q) *reinterpret_cast<sep_u4*>(base + q * kRowStep * 128) = ra[q];
-#pragma unroll
-        for (int q = 0; q < kLoadB; ++q) *reinterpret_cast<sep_u4*>(base + TM * 128 + q * kRowStep * 128) = rb[q];
+        for (int q = 0; q < kLoadB; ++q)
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(bbase + (pb[q] + (unsigned)s * 128u)),
+                                             (__attribute__((address_space(3))) void*)(dst + TM * 128 + q * kThreads * 16), 16, 0, 0);
     };
     auto multiply = [&](const sep_h8* u, const sep_h8* v) {
 #pragma unroll
@@ -1135,57 +1147,50 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void sep_gemm_kernel(SepGemm g) {
             for (int j = 0; j < NI; ++j)
                 acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(u[i], v[j], acc[i][j], 0, 0, 0);
     };
-    if (s_begin < s_end) {
-        load(s_begin);
-        store(0);
-    }
-    __syncthreads();
+    if (s_begin < s_end) copy(s_begin, 0);
     int s = s_begin;
     const int pair_end = min(s_end, pair_slabs);
     for (; s < pair_end; ++s) {
         const int buf = (s - s_begin) & 1;
-        const bool more = s + 1 < s_end;
-        if (more) load(s + 1);
+        __syncthreads();  // this slab has landed, and the other buffer's has been read
         const char* base = s_sep + buf * kBuf;
+        sep_h8 ah[2][MI], al[2][MI], bh[2][NI], bl[2][NI];
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
-            sep_h8 ah[MI], al[MI], bh[NI], bl[NI];
             const int off = frag ^ (ks << 5);  // parts ks * 2 + fh (hi), + 4 (lo)
 #pragma unroll
-            for (int i = 0; i < MI; ++i) {
-                ah[i] = *reinterpret_cast<const sep_h8*>(base + fa + i * 4096 + off);
-                al[i] = *reinterpret_cast<const sep_h8*>(base + fa + i * 4096 + (off ^ 64));
-            }
+            for (int j = 0; j < NI; ++j) bh[ks][j] = *reinterpret_cast<const sep_h8*>(base + fb + j * 4096 + off);
 #pragma unroll
-            for (int j = 0; j < NI; ++j) {
-                bh[j] = *reinterpret_cast<const sep_h8*>(base + fb + j * 4096 + off);
-                bl[j] = *reinterpret_cast<const sep_h8*>(base + fb + j * 4096 + (off ^ 64));
-            }
-            multiply(ah, bl);
-            multiply(al, bh);
-            multiply(ah, bh);
+            for (int i = 0; i < MI; ++i) ah[ks][i] = *reinterpret_cast<const sep_h8*>(base + fa + i * 4096 + off);
+#pragma unroll
+            for (int j = 0; j < NI; ++j) bl[ks][j] = *reinterpret_cast<const sep_h8*>(base + fb + j * 4096 + (off ^ 64));
+#pragma unroll
+            for (int i = 0; i < MI; ++i) al[ks][i] = *reinterpret_cast<const sep_h8*>(base + fa + i * 4096 + (off ^ 64));
         }
-        if (more) store(buf ^ 1);
-        __syncthreads();
+        if (s + 1 < s_end) copy(s + 1, buf ^ 1);
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            multiply(ah[ks], bh[ks]);
+            multiply(ah[ks], bl[ks]);
+            multiply(al[ks], bh[ks]);
+        }
     }
     for (; s < s_end; ++s) {
         const int buf = (s - s_begin) & 1;
-        const bool more = s + 1 < s_end;
-        if (more) load(s + 1);
+        __syncthreads();
         const char* base = s_sep + buf * kBuf;
+        sep_h8 av[4][MI], bv[4][NI];
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
-            sep_h8 av[MI], bv[NI];
             const int off = frag ^ (ks << 5);
 #pragma unroll
-            for (int i = 0; i < MI; ++i) av[i] = *reinterpret_cast<const sep_h8*>(base + fa + i * 4096 + off);
+            for (int i = 0; i < MI; ++i) av[ks][i] = *reinterpret_cast<const sep_h8*>(base + fa + i * 4096 + off);
 #pragma unroll
-            for (int j = 0; j < NI; ++j) bv[j] = *reinterpret_cast<const sep_h8*>(base + fb + j * 4096 + off);
-            multiply(av, bv);
-            if (ks == 1) __builtin_amdgcn_sched_barrier(0);  // two steps' fragments at a time fit the registers
+            for (int j = 0; j < NI; ++j) bv[ks][j] = *reinterpret_cast<const sep_h8*>(base + fb + j * 4096 + off);
         }
-        if (more) store(buf ^ 1);
-        __syncthreads();
+        if (s + 1 < s_end) copy(s + 1, buf ^ 1);
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) multiply(av[ks], bv[ks]);
     }
 
     // lane (fl, fh) holds rows q % 4 + 8 (q / 4) + 4 fh of column fl of each 32 x 32 tile
@@ -1208,9 +1213,10 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void sep_gemm_kernel(SepGemm g) {
     } else {
         const SepHead h = *head;
         const int kind = p.kind;
-        const bool harm = kind >= kSepDxHarm, dx = kind == kSepDx || kind == kSepDxHarm;
-        const int per = harm ? groups : nb, sh = __builtin_ctz(per);  // blocks of eight rows per input
-        if (dx) {
+        const bool harm = kind >= kSepDxHarm, upper = kind == kSepDxUpper || kind == kSepDvUpper;
+        const int sh = __builtin_ctz(per), j_first = upper ? R / 2 : 0;
+        const bool eight = R == 8;
+        if (kind == kSepDx || kind == kSepDxUpper || kind == kSepDxHarm) {
             const float as = g.in_affine ? g.in_affine[0] : 1.0f, ab = g.in_affine ? g.in_affine[1] : 0.0f;
             float* out = p.out + (int64_t)split * g.M * g.K;
 #pragma unroll
@@ -1222,41 +1228,36 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void sep_gemm_kernel(SepGemm g) {
 #pragma unroll
                 for (int i = 0; i < MI; ++i) {
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) {  // eight rows of input k
+                    for (int q = 0; q < 4; ++q) {  // block jb of inputs k (fh = 0) and k + 1
                         const int64_t block = (a0 + (wr * MI + i) * 32) / 8 + q;
-                        const int64_t k = block >> sh;
+                        const int64_t k = (block >> sh) * 2 + fh;
                         const int jb = (int)block & (per - 1);
-                        const int64_t kc = k < g.K ? k : g.K - 1;
-                        const float xr = g.x[mc * g.K + kc];
+                        const float xr = g.x[mc * g.K + (k < g.K ? k : g.K - 1)];
                         const float x = g.in_affine ? input_map(xr, as, ab, g.in_lo, g.in_hi) : xr;
                         const SepAt at = sep_at(h, x);
                         float4 v;
                         if (!harm) {
-                            v = sep_eval4(g.tab2, R, at, jb * 8 + 4 * fh);
+                            v = sep_eval4(g.tab2, R, at, j_first + 4 * jb);
                         } else {
-                            // 8 terms: harmonic fh's two cosines and two sines; 16: harmonic jb's four
-                            // cosines (fh = 0) or sines
-                            const int hq = nb == 1 ? fh : jb;
-                            const float th = (x - h.lut_min) * h.lut_scale * (float)(hq + 1);
-                            const float f = th - floorf(th), w = hq ? 0.25f : 1.0f;
+                            const bool second = eight ? jb & 1 : jb & 2;
+                            const float th = (x - h.lut_min) * h.lut_scale * (second ? 2.0f : 1.0f);
+                            const float f = th - floorf(th), w = second ? 0.25f : 1.0f;
                             const float c = __builtin_amdgcn_cosf(f) * w, sn = __builtin_amdgcn_sinf(f) * w;
                             float e[4];
                             sep_second(h, g.tabE, at, e);
-                            if (nb == 1) {
+                            if (eight) {
                                 v = make_float4(e[0] * c, e[1] * c, e[0] * sn, e[1] * sn);
                             } else {
-                                const float tr = fh ? sn : c;
+                                const float tr = jb & 1 ? sn : c;
                                 v = make_float4(e[0] * tr, e[1] * tr, e[2] * tr, e[3] * tr);
                             }
                         }
-                        float s = acc[i][j][4 * q] * v.x;
-                        s = fmaf(acc[i][j][4 * q + 1], v.y, s);
-                        s = fmaf(acc[i][j][4 * q + 2], v.z, s);
-                        s = fmaf(acc[i][j][4 * q + 3], v.w, s);
-                        sum += s;
+                        sum = fmaf(acc[i][j][4 * q], v.x, sum);
+                        sum = fmaf(acc[i][j][4 * q + 1], v.y, sum);
+                        sum = fmaf(acc[i][j][4 * q + 2], v.z, sum);
+                        sum = fmaf(acc[i][j][4 * q + 3], v.w, sum);
                         if (jb == per - 1) {
-                            sum += __shfl_xor(sum, 32);
-                            if (fh == 0 && m < g.M && k < g.K) out[m * g.K + k] = sum * sc;
+                            if (m < g.M && k < g.K) out[m * g.K + k] = sum * sc;
                             sum = 0.0f;
                         }
                     }
@@ -1276,60 +1277,65 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void sep_gemm_kernel(SepGemm g) {
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
                         const int64_t block = (a0 + (wr * MI + i) * 32) / 8 + q;
-                        const int64_t k = block >> sh;
+                        const int64_t k = (block >> sh) * 2 + fh;
                         const int jb = (int)block & (per - 1);
-                        const int64_t kc = k < g.K ? k : g.K - 1;
-                        if (jb == 0) tt = g.tT[kc * g.Op + oc];
+                        if (jb == 0) tt = g.tT[(k < g.K ? k : g.K - 1) * g.Op + oc];
+                        const float a0_ = acc[i][j][4 * q], a1_ = acc[i][j][4 * q + 1], a2_ = acc[i][j][4 * q + 2],
+                                    a3_ = acc[i][j][4 * q + 3];
                         float rp = 0.0f, rn = 0.0f;
                         if (!harm) {
-                            if (jb == 0) {  // T_0, T_1
-                                p0 = n0 = 1.0f;
-                                p1 = tt.x;
-                                n1 = tt.y;
+                            if (jb == 0) {
+                                if (!upper) {  // T_0, T_1
+                                    p0 = n0 = 1.0f;
+                                    p1 = tt.x;
+                                    n1 = tt.y;
+                                } else {  // T_(R/2), T_(R/2 + 1) = cos(j acos t): 1e-5, of terms below 4e-3
+                                    const float u = acosf(fminf(fmaxf(tt.x, -1.0f), 1.0f)) * 0.15915494f;
+                                    const float w = acosf(fminf(fmaxf(tt.y, -1.0f), 1.0f)) * 0.15915494f;
+                                    const float jf = (float)j_first;
+                                    auto cosj = [](float r) { return __builtin_amdgcn_cosf(r - floorf(r)); };
+                                    p0 = cosj(u * jf);
+                                    p1 = cosj(u * (jf + 1.0f));
+                                    n0 = cosj(w * jf);
+                                    n1 = cosj(w * (jf + 1.0f));
+                                }
                             }
-                            float vp[4], vn[4];  // this lane's four of the eight polynomials
 #pragma unroll
-                            for (int e = 0; e < 8; ++e) {
-                                vp[e & 3] = e < 4 || fh ? p0 : vp[e & 3];
-                                vn[e & 3] = e < 4 || fh ? n0 : vn[e & 3];
+                            for (int e = 0; e < 4; ++e) {
+                                rp = fmaf(acc[i][j][4 * q + e], p0, rp);
+                                rn = fmaf(acc[i][j][4 * q + e], n0, rn);
                                 const float p2 = fmaf(2.0f * tt.x, p1, -p0), n2 = fmaf(2.0f * tt.y, n1, -n0);
                                 p0 = p1;
                                 p1 = p2;
                                 n0 = n1;
                                 n1 = n2;
                             }
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) {
-                                rp = fmaf(acc[i][j][4 * q + e], vp[e], rp);
-                                rn = fmaf(acc[i][j][4 * q + e], vn[e], rn);
-                            }
-                        } else {  // the rows' order as for dX
-                            const int hq = nb == 1 ? fh : jb;
-                            const float ws = h.lut_scale * (float)(hq + 1);
+                        } else {
+                            const bool second = eight ? jb & 1 : jb & 2;
+                            const float ws = h.lut_scale * (second ? 2.0f : 1.0f);
                             const float tp = ((float)h.wc + (float)h.wh * tt.x) * ws, tn = ((float)h.wc + (float)h.wh * tt.y) * ws;
                             const float fp = tp - floorf(tp), fn = tn - floorf(tn);
                             const float cp = __builtin_amdgcn_cosf(fp), dp = __builtin_amdgcn_sinf(fp);
                             const float cn = __builtin_amdgcn_cosf(fn), dn = __builtin_amdgcn_sinf(fn);
-                            const float a0 = acc[i][j][4 * q], a1 = acc[i][j][4 * q + 1], a2 = acc[i][j][4 * q + 2],
-                                        a3 = acc[i][j][4 * q + 3];
-                            if (nb == 1) {
-                                rp = cp * fmaf(a1, tt.x, a0) + dp * fmaf(a3, tt.x, a2);
-                                rn = cn * fmaf(a1, tt.y, a0) + dn * fmaf(a3, tt.y, a2);
+                            if (eight) {
+                                rp = cp * fmaf(a1_, tt.x, a0_) + dp * fmaf(a3_, tt.x, a2_);
+                                rn = cn * fmaf(a1_, tt.y, a0_) + dn * fmaf(a3_, tt.y, a2_);
                             } else {
                                 float vp[4], vn[4];
                                 sep_cheb4(tt.x, vp);
                                 sep_cheb4(tt.y, vn);
-                                rp = (fh ? dp : cp) * fmaf(a3, vp[3], fmaf(a2, vp[2], fmaf(a1, vp[1], a0)));
-                                rn = (fh ? dn : cn) * fmaf(a3, vn[3], fmaf(a2, vn[2], fmaf(a1, vn[1], a0)));
+                                rp = (jb & 1 ? dp : cp) * fmaf(a3_, vp[3], fmaf(a2_, vp[2], fmaf(a1_, vp[1], a0_)));
+                                rn = (jb & 1 ? dn : cn) * fmaf(a3_, vn[3], fmaf(a2_, vn[2], fmaf(a1_, vn[1], a0_)));
                             }
                         }
                         sp += rp;
                         sn += rn;
                         if (jb == per - 1) {
-                            sp += __shfl_xor(sp, 32);
-                            sn += __shfl_xor(sn, 32);
-                            if (o < g.O && k < g.K)
-                                out[((int64_t)fh * g.Kp + k) * g.Op + o] = (fh ? sn : sp) * sb * g.xscale[k];
+                            if (o < g.O && k < g.K) {
+                                const float sc = sb * g.xscale[k];
+                                out[k * g.Op + o] = sp * sc;
+                                out[(g.Kp + k) * g.Op + o] = sn * sc;
+                            }
                             sp = sn = 0.0f;
                         }
                     }
@@ -1401,11 +1407,11 @@ __global__ __launch_bounds__(256) void sep_reduce_bwd_kernel(DxReduceArgs dx, Dx
 struct SepPlan {
     int max_terms;  // 0: not considered
     bool big;       // 256 x 256 tiles instead of 128 x 128
-    int split, split_dx, split_dv, split_dxh, split_dvh;
+    int split, split_dx, split_dv, split_dxs, split_dvs, split_dxh, split_dvh;
     int planes_dx, planes_dv;
     int64_t Kp, Op;
     size_t off_head, off_part, off_row, off_col, off_grow, off_gcol, off_tab, off_tab2, off_tabE, off_lut, off_xop, off_wop,
-        off_xoph, off_woph, off_gop, off_gopT, off_goph, off_gophT, off_scale, off_gscale, off_gscaleT, off_tT,
+        off_xops, off_wops, off_xoph, off_woph, off_gop, off_gopT, off_goph, off_gophT, off_scale, off_gscale, off_gscaleT, off_tT,
         off_planes, off_planes_dv, bytes;
 };
 
@@ -1446,10 +1452,11 @@ SepPlan plan_sep(int lut_n, int64_t M, int64_t K, int64_t O, bool backward, bool
         return p;
     p.Kp = round_up(K, 8);
     p.Op = round_up(O, 256);
-    const int64_t Mr = round_up(M, 64), Or = round_up(O, 64), Kr = round_up(K, 8);
-    // bytes per (row, input): R hi/lo pairs, and in the forward's rows the harmonics
+    const int64_t Mr = round_up(M, 64), Or = round_up(O, 64), Kr = sep_inputs(K);
     const int harm = lut_n > 0 ? 1 : 0;
-    auto width = [&](int terms) { return (int64_t)terms * (4 + (backward ? 0 : 2 * harm)); };
+    // bytes per (row, input), forward: R / 2 pairs, R / 2 singles and the harmonics; an operand's
+    // size backward: at most R pairs
+    auto width = [&](int terms) { return (int64_t)terms * (backward ? 4 : 3 + 2 * harm); };
     int terms = lut_n > 0 ? 16 : cells >= 1 << 30 ? 64 : cells >= 1 << 28 ? 32 : 16;
     while (terms >= 8 && (Mr * Kr * width(terms) >= kSepOperandBytes || Or * Kr * width(terms) >= kSepOperandBytes)) terms /= 2;
     if (terms < 8 || Mr * Or * 4 >= kSepOperandBytes) return p;
@@ -1467,12 +1474,12 @@ SepPlan plan_sep(int lut_n, int64_t M, int64_t K, int64_t O, bool backward, bool
         p.off_lut = take((int64_t)lut_n * 16 + 256 * 8);
         p.off_tabE = take((int64_t)kSepGridMax * terms);
     }
-    p.off_xop = take(Mr * Kr * width(terms));
-    p.off_wop = take(Or * Kr * width(terms));
     if (!backward) {
+        p.off_xop = take(Mr * Kr * width(terms));
+        p.off_wop = take(Or * Kr * width(terms));
         p.off_row = take(M * 8);
         p.off_scale = take(M * 4);
-        const int64_t slabs = (K + 3) / 4 + (K + 7) / 8 * harm;
+        const int64_t slabs = sep_slabs_pairs(K, 8) + sep_slabs_singles(K, 8, harm);
         p.big = sep_big(M, O, slabs);
         const int64_t tile = p.big ? 256 : 128;
         p.split = sep_splits(((M + tile - 1) / tile) * ((O + tile - 1) / tile), slabs, p.big, 8.0 * M * O);
@@ -1484,25 +1491,33 @@ SepPlan plan_sep(int lut_n, int64_t M, int64_t K, int64_t O, bool backward, bool
         p.off_gcol = take(kSepColChunks * O * 4);
         p.off_gop = take(Mr * Or * 4);
         p.off_gopT = take(Mr * Or * 4);
-        if (harm > 0) {
-            p.off_xoph = take(Mr * Kr * terms * 2 * harm);
-            p.off_woph = take(Or * Kr * terms * 2 * harm);
-            p.off_goph = take(Mr * Or * 2);
-            p.off_gophT = take(Mr * Or * 2);
+        p.off_goph = take(Mr * Or * 2);
+        p.off_gophT = take(Mr * Or * 2);
+        if (need_w) p.off_xop = take(Mr * Kr * terms * (harm ? 2 : 4));
+        if (need_w && harm) p.off_xops = take(Mr * Kr * terms);
+        if (need_w && harm) p.off_xoph = take(Mr * Kr * terms * 2);
+        if (need_x) {
+            p.off_wop = take(Or * Kr * terms * 2);
+            p.off_wops = take(Or * Kr * terms);
+            if (harm) p.off_woph = take(Or * Kr * terms * 2);
         }
         p.off_scale = take(K * 4);
         p.off_gscale = take(M * 4);
         p.off_gscaleT = take(O * 4);
         p.off_tT = take(K * p.Op * 8);
         p.big = sep_big(8 * K, std::min(M, O), std::min(M, O) / 32);
-        const int64_t tile = p.big ? 256 : 128, tk = (8 * K + tile - 1) / tile, tkh = (8 * K * harm + tile - 1) / tile;
+        // at 8 terms: 4 rows per input of lower and of upper terms (8 of the formula's dVth), 8 of harmonics
+        const int64_t tile = p.big ? 256 : 128, t4 = (4 * K + tile - 1) / tile, t8 = (8 * K + tile - 1) / tile;
         const int64_t tm = (M + tile - 1) / tile, to = (O + tile - 1) / tile;
-        p.split_dx = sep_splits(tk * tm, (O + 31) / 32, p.big, 8.0 * M * K);
-        p.split_dv = sep_splits(tk * to, (M + 31) / 32, p.big, 16.0 * p.Kp * p.Op);
-        p.split_dxh = harm > 0 ? sep_splits(tkh * tm, (O + 63) / 64, p.big, 8.0 * M * K) : 0;
-        p.split_dvh = harm > 0 ? sep_splits(tkh * to, (M + 63) / 64, p.big, 16.0 * p.Kp * p.Op) : 0;
-        p.planes_dx = p.split_dx + p.split_dxh;
-        p.planes_dv = p.split_dv + p.split_dvh;
+        const double dx_bytes = 8.0 * M * K, dv_bytes = 16.0 * p.Kp * p.Op;
+        p.split_dx = sep_splits(t4 * tm, (O + 31) / 32, p.big, dx_bytes);
+        p.split_dxs = sep_splits(t4 * tm, (O + 63) / 64, p.big, dx_bytes);
+        p.split_dv = sep_splits((harm ? t4 : t8) * to, (M + 31) / 32, p.big, dv_bytes);
+        p.split_dvs = harm ? sep_splits(t4 * to, (M + 63) / 64, p.big, dv_bytes) : 0;
+        p.split_dxh = harm ? sep_splits(t8 * tm, (O + 63) / 64, p.big, dx_bytes) : 0;
+        p.split_dvh = harm ? sep_splits(t8 * to, (M + 63) / 64, p.big, dv_bytes) : 0;
+        p.planes_dx = p.split_dx + p.split_dxs + p.split_dxh;
+        p.planes_dv = p.split_dv + p.split_dvs + p.split_dvh;
         if (need_x) p.off_planes = take((int64_t)p.planes_dx * M * K * 4);
         if (need_w) p.off_planes_dv = take((int64_t)p.planes_dv * 2 * p.Kp * p.Op * 4);
     }
@@ -1570,6 +1585,8 @@ void sep_point_backward(const SepPlan& p, SepArgs& a, char* ws) {
     a.tab2 = reinterpret_cast<float*>(ws + p.off_tab2);
     a.gop = reinterpret_cast<_Float16*>(ws + p.off_gop);
     a.gopT = reinterpret_cast<_Float16*>(ws + p.off_gopT);
+    a.xops = reinterpret_cast<_Float16*>(ws + p.off_xops);
+    a.wops = reinterpret_cast<_Float16*>(ws + p.off_wops);
     a.xoph = reinterpret_cast<_Float16*>(ws + p.off_xoph);
     a.woph = reinterpret_cast<_Float16*>(ws + p.off_woph);
     a.goph = reinterpret_cast<_Float16*>(ws + p.off_goph);
@@ -1617,23 +1634,27 @@ hipError_t sep_backward_products(const SepPlan& p, SepArgs a, char* ws, hipStrea
     g.tab2 = a.tab2;
     g.tabE = a.tabE;
     g.tT = a.tT;
+    g.dv_all = a.lut_n > 0 ? 0 : 1;
     const int64_t tile = p.big ? 256 : 128;
     int64_t blocks = 0;
-    auto add = [&](int kind, const _Float16* x, const _Float16* y, int64_t b_rows, int64_t inner, int split, float* out,
-                   int eights) {
+    auto add = [&](int kind, const _Float16* x, const _Float16* y, int64_t b_rows, int64_t inner, int split, float*& out,
+                   int64_t plane, int rows) {  // rows: of an input, at most
         if (split < 1) return;
         g.p[g.n++] = SepProduct{reinterpret_cast<const char*>(x), reinterpret_cast<const char*>(y), kind, a.K, b_rows,
                                 inner, split, out};
-        blocks += (8 * a.K * eights + tile - 1) / tile * ((b_rows + tile - 1) / tile) * split;
+        out += split * plane;
+        blocks += ((a.K + 1) / 2 * 2 * rows + tile - 1) / tile * ((b_rows + tile - 1) / tile) * split;
     };
     float* dx = reinterpret_cast<float*>(ws + p.off_planes);
     float* dv = reinterpret_cast<float*>(ws + p.off_planes_dv);
-    const int nb = p.max_terms / 8, nh = nb;
-    if (a.need_x) add(kSepDx, a.wop, a.gop, a.M, a.O, p.split_dx, dx, nb);
-    if (a.need_w) add(kSepDv, a.xop, a.gopT, a.O, a.M, p.split_dv, dv, nb);
-    if (a.need_x) add(kSepDxHarm, a.woph, a.goph, a.M, a.O, p.split_dxh, dx + (int64_t)p.split_dx * a.M * a.K, nh);
-    if (a.need_w)
-        add(kSepDvHarm, a.xoph, a.gophT, a.O, a.M, p.split_dvh, dv + (int64_t)p.split_dv * 2 * p.Kp * p.Op, nh);
+    const int64_t px = a.M * a.K, pv = 2 * p.Kp * p.Op;
+    const int R = p.max_terms;
+    if (a.need_x) add(kSepDx, a.wop, a.gop, a.M, a.O, p.split_dx, dx, px, R / 2);
+    if (a.need_w) add(kSepDv, a.xop, a.gopT, a.O, a.M, p.split_dv, dv, pv, g.dv_all ? R : R / 2);
+    if (a.need_x) add(kSepDxUpper, a.wops, a.goph, a.M, a.O, p.split_dxs, dx, px, R / 2);
+    if (a.need_w) add(kSepDvUpper, a.xops, a.gophT, a.O, a.M, p.split_dvs, dv, pv, R / 2);
+    if (a.need_x) add(kSepDxHarm, a.woph, a.goph, a.M, a.O, p.split_dxh, dx, px, R);
+    if (a.need_w) add(kSepDvHarm, a.xoph, a.gophT, a.O, a.M, p.split_dvh, dv, pv, R);
     launch_sep_gemm<false>(p.big, (unsigned)blocks, g, s);
     return hipGetLastError();
 }
