@@ -1505,7 +1505,9 @@ SepPlan plan_sep(int lut_n, int64_t M, int64_t K, int64_t O, bool backward, bool
         p.off_gscale = take(M * 4);
         p.off_gscaleT = take(O * 4);
         p.off_tT = take(K * p.Op * 8);
-        p.big = sep_big(8 * K, std::min(M, O), std::min(M, O) / 32);
+        // (a wave sums all of an input's values of a product: 64 terms of the formula's dVth take the
+        // 128 rows that a wave of the large tile has)
+        p.big = sep_big(8 * K, std::min(M, O), std::min(M, O) / 32) || terms == 64;
         // at 8 terms: 4 rows per input of lower and of upper terms (8 of the formula's dVth), 8 of harmonics
         const int64_t tile = p.big ? 256 : 128, t4 = (4 * K + tile - 1) / tile, t8 = (8 * K + tile - 1) / tile;
         const int64_t tm = (M + tile - 1) / tile, to = (O + tile - 1) / tile;
