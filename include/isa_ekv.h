@@ -78,7 +78,10 @@ int isa_ekv_lut_build(const double params[4], double delta_min, double delta_max
 int isa_ekv_lut_pack(const void* table_i, const void* table_ddelta, int n_entries, int src_dtype, int layout,
                      void* dst, void* stream);
 
-/* Workspace bytes for isa_ekv_forward at this shape. */
+/* Workspace bytes for isa_ekv_forward at this shape. Large calls hold the operands of their
+ * products on the matrix cores too; a workspace that holds the per-cell kernels' plan
+ * (isa_ekv_plan_info slot [0]) but not those is accepted and runs the per-cell kernels. The
+ * exact-formula calls' workspaces are accepted likewise. */
 size_t isa_ekv_forward_workspace(int64_t M, int64_t K, int64_t O);
 
 /* out[m,o] = clamp(sum_k (L(x-vth_pos) - L(x-vth_neg)) / (1 + x/v_sat), out_min, out_max)
@@ -93,12 +96,14 @@ int isa_ekv_forward(const float* x, const float* vth_pos, const float* vth_neg, 
 
 /* isa_ekv_forward without a workspace argument, for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that forbid it). No
- * counterpart in the reference. Same arguments, results and errors as isa_ekv_forward, bitwise
- * equal outputs; the call allocates nothing (no hipMalloc/hipFree, no allocating library
- * routine, no profiling events). Its scratch is a file-scope device array of
- * ISA_EKV_NOALLOC_MAX_BYTES that each device the library runs on holds until the process
- * ends; shapes whose forward needs more (isa_ekv_plan_info slot [0]) are rejected with
- * ISA_EKV_EINVAL before anything is enqueued. All calls on one device share that array:
+ * counterpart in the reference. Same arguments, results and errors as isa_ekv_forward; the
+ * call allocates nothing (no hipMalloc/hipFree, no allocating library routine, no profiling
+ * events). It runs the per-cell kernels: where isa_ekv_forward, given the workspace that its
+ * query asks for, runs a large call on the matrix cores, the outputs agree to the two paths'
+ * rounding, and bitwise with isa_ekv_forward given slot [0] bytes. Its scratch is a file-scope
+ * device array of ISA_EKV_NOALLOC_MAX_BYTES that each device the library runs on holds until
+ * the process ends; shapes whose forward needs more (isa_ekv_plan_info slot [0]) are rejected
+ * with ISA_EKV_EINVAL before anything is enqueued. All calls on one device share that array:
  * calls that overlap on a device (different streams, or threads without ordering) race. */
 #define ISA_EKV_NOALLOC_MAX_BYTES ((size_t)128 << 20)
 int isa_ekv_forward_noalloc(const float* x, const float* vth_pos, const float* vth_neg, const void* lut_fwd,
@@ -290,11 +295,12 @@ int isa_ekv_profile_clock(double* out);
  * which: ISA_EKV_PLAN_FORWARD (isa_ekv_forward, isa_ekv_layer_forward), ISA_EKV_PLAN_BACKWARD
  * (isa_ekv_backward), ISA_EKV_PLAN_LAYER_BACKWARD (isa_ekv_layer_backward). Writes
  * min(n_info, ISA_EKV_PLAN_INFO_LEN) values (later slots get 0):
- *   [0] workspace bytes
+ *   [0] workspace bytes (forward: of the per-cell kernels' plan, which the query's may exceed)
  *   [1] byte offset in the workspace of the table-copy mode word (int32: after the call, 1 when
  *       the main kernel ran with the second, bank-rotated table copy, 0 when with one copy,
  *       2 when the backward ran ranked: see ISA_EKV_OPT_RANKED, 3 to 32 when the main kernel
- *       held that many windowed copies and 33 when it held two: see ISA_EKV_OPT_WINDOW_COPIES),
+ *       held that many windowed copies and 33 when it held two: see ISA_EKV_OPT_WINDOW_COPIES;
+ *       the mode that they would have run in where the call ran on the matrix cores),
  *       or -1 when the call cannot
  *       use a second copy (the word is then not written)
  *   [2] forward: K ranges summed separately (1: no split); backward: token splits

@@ -77,7 +77,8 @@ __host__ __device__ inline int sep_terms_lut(float spread_u) { return spread_u <
 struct SepHead {
     int terms;    // 0: the per-cell kernels run
     unsigned gmax;  // backward: bits of the largest |G|: not finite: the per-cell kernels run
-    int rough;    // the series does not converge as its terms assume: the per-cell kernels run
+    int rough;    // 1: the series does not converge as its terms assume, 2: a sample of the thresholds or of
+                  // the table ruled the contraction out (then the other fields are not set): the per-cell kernels run
     int harmonics;  // 1: the kinks' two harmonics are summed
     int n_grid;
     float xlo, xhi, wlo, whi;
@@ -244,15 +245,61 @@ __device__ inline void sep_lut_block(const SepArgs& a, int b) {
 
 __device__ inline unsigned sep_bits(float v) { return __float_as_uint(v) & 0x7fffffffu; }
 
+// Whether a sample of the operands already rules the contraction out: 128 thresholds spread wider
+// than its terms reach, or 16 places of the table not smooth (entries rounded to bf16). Wave-uniform
+// and the same in every wave of the launch. What the sample passes the full statistics judge; what
+// it fails they would refuse too (a sample's spread, growth and roughness are at most the whole's).
+// Four neighbours at each of 16 places: every wave of the launch reads them, and 64 places cost
+// the launch 6 us of L2 requests.
+__device__ inline bool sep_sample_refuses(const SepArgs& a) {
+    const int lane = threadIdx.x & 63, place = lane >> 2, off = lane & 3;
+    const uint64_t n = (uint64_t)(a.O * a.K);
+    float lo = INFINITY, hi = -INFINITY;
+    // scattered, so that they are not a few inputs' (n >= 128)
+    const uint64_t f = (((((uint64_t)place * 0x9e3779b97f4a7c15u) >> 32) * (n - 3)) >> 32) + off;
+    const float wp = a.wp[f], wn = a.wn[f];
+    double ua = a.a;
+    bool bad = false;
+    if (a.lut_n > 0) {
+        const bool bwd = a.tab2 != nullptr;  // entries {A, dT}, backward the slope table's
+        const int i = 2 + (int)((int64_t)place * (a.lut_n - 6) / 16);
+        const float2 r = *reinterpret_cast<const float2*>(a.lut + (size_t)(kPad + i - 2 + off) * (bwd ? 4 : 2) + (bwd ? 2 : 0));
+        const double d0 = __shfl(r.y, place * 4), d1 = __shfl(r.y, place * 4 + 1), d2 = __shfl(r.y, place * 4 + 2),
+                     d3 = __shfl(r.y, place * 4 + 3);
+        const double v = (double)__shfl(r.x, place * 4 + 2) + (double)(i + kPad) * d2;  // entry i, to 1e-5
+        bad = !(fabs((d3 - d0) - 3.0 * (d2 - d1)) <= 4e-6 * fabs(v) + 2e-42);
+        float growth = v > 1e-30 ? (float)(d2 / v) : 0.0f;
+        for (int d = 32; d > 0; d >>= 1) growth = fmaxf(growth, __shfl_xor(growth, d));
+        ua = 0.5 * 0.999 * (double)growth * a.lut_scale;
+    }
+    sep_minmax(wp, lo, hi);
+    sep_minmax(wn, lo, hi);
+    sep_wave_minmax(lo, hi);
+    const float spread = (float)(((double)hi - (double)lo) * ua);
+    const int terms = a.lut_n > 0 ? sep_terms_lut(spread) : sep_terms(spread);
+    return __builtin_amdgcn_readfirstlane((int)(__any(bad) || terms == 0 || terms > a.max_terms)) != 0;
+}
+
 // Blocks: kSepStatX of x, kSepStatW of the thresholds, (xcol) kSepColChunks x ceil(K / 256) of
 // x's columns, ceil(lut_n / 256) of the table, then the layer glue's gradient blocks (glue.geff).
-__global__ __launch_bounds__(256) void sep_stat_kernel(SepArgs a, GlueGradArgs glue) {
+__global__ __launch_bounds__(256) void sep_stat_kernel(SepArgs a, PrepArgs prep, GlueGradArgs glue) {
     int b = blockIdx.x;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const float as = a.in_affine ? a.in_affine[0] : 1.0f, ab = a.in_affine ? a.in_affine[1] : 0.0f;
-    if (b == 0 && t == 0) {
-        a.head->gmax = 0;
-        a.head->rough = 0;
+    const int lut_blocks = (a.lut_n + 255) / 256;
+    const int xcols = a.xcol ? kSepColChunks * (int)((a.K + 255) / 256) : 0;
+    if (b < kSepStatX + kSepStatW + lut_blocks + xcols) {
+        const bool refuses = sep_sample_refuses(a);
+        if (b == 0 && t == 0) {
+            a.head->gmax = 0;
+            a.head->rough = refuses ? 2 : 0;
+            a.head->terms = 0;
+        }
+        if (refuses) {  // the per-cell kernels' prep at once, beside the glue's gradient
+            static_assert(kSepStatX + kSepStatW == kPrepBlocksX + kPrepBlocksW, "the prep's blocks");
+            if (b < kPrepBlocksX + kPrepBlocksW) prep_block(prep, b);
+            return;
+        }
     }
     if (b < kSepStatX) {
         float lo = INFINITY, hi = -INFINITY;
@@ -304,13 +351,11 @@ __global__ __launch_bounds__(256) void sep_stat_kernel(SepArgs a, GlueGradArgs g
         return;
     }
     b -= kSepStatW;
-    const int lut_blocks = (a.lut_n + 255) / 256;
     if (b < lut_blocks) {
         sep_lut_block(a, b);
         return;
     }
     b -= lut_blocks;
-    const int xcols = a.xcol ? kSepColChunks * (int)((a.K + 255) / 256) : 0;
     if (b < xcols) {
         const int64_t rows = (a.M + kSepColChunks - 1) / kSepColChunks;
         const int chunk = b % kSepColChunks;
@@ -406,6 +451,8 @@ __global__ __launch_bounds__(256) void sep_table_kernel(SepArgs a) {
     __shared__ double s_cos[4 * kSepMaxTerms], s_val[256], s_sec[256], s_d[256];
     const int t = threadIdx.x;
     const bool lut = a.lut_n > 0;
+    // (other blocks of this launch set rough to 1, never to 2)
+    if (__builtin_amdgcn_readfirstlane(a.head->rough) == 2) return;
     {
         float lo = INFINITY, hi = -INFINITY;
 #pragma unroll
@@ -745,10 +792,11 @@ __device__ inline void sep_write_partials(const SepHead& h, const PrepArgs& p) {
     if (p.stat_bits && threadIdx.x == 0) *p.stat_bits = 0u;
 }
 
-// Where the per-cell kernels take the call: their prep, in the same launch.
+// Where the per-cell kernels take the call: their prep, in the same launch (unless the statistics'
+// launch has run it).
 __global__ __launch_bounds__(256) void sep_expand_fwd_kernel(SepArgs a, PrepArgs prep) {
     if (!sep_takes(a.head)) {
-        if (blockIdx.x < kPrepBlocksX + kPrepBlocksW) prep_block(prep, blockIdx.x);
+        if (blockIdx.x < kPrepBlocksX + kPrepBlocksW && a.head->rough != 2) prep_block(prep, blockIdx.x);
         return;
     }
     const SepHead h = *a.head;
@@ -837,7 +885,7 @@ __device__ inline void sep_store2h(_Float16* row, int64_t e, float v0, float v1)
 
 __global__ __launch_bounds__(256) void sep_expand_bwd_kernel(SepArgs a, int x_blocks, int w_blocks, PrepArgs prep) {
     if (!sep_takes(a.head)) {  // the per-cell kernels take the call: their prep
-        if (blockIdx.x < kPrepBlocksX + kPrepBlocksW) prep_block(prep, blockIdx.x);
+        if (blockIdx.x < kPrepBlocksX + kPrepBlocksW && a.head->rough != 2) prep_block(prep, blockIdx.x);
         return;
     }
     const SepHead h = *a.head;
@@ -1395,8 +1443,10 @@ __global__ __launch_bounds__(256) void sep_reduce_bwd_kernel(DxReduceArgs dx, Dx
 // 51 / 90, at 128 43 / 87 against 50 / 84; 16 terms at 256 66 / 104 against 60 / 103, at 512
 // 97 / 165 against 64 / 114; 32 terms 768 x 3072 at 128 (2^28.2) 317 / 625 against 281 / 436,
 // at 64 225 / 359 against 261 / 347; 64 terms at 512 (2^30.2) 1120 / 2202 against 798 / 1435,
-// at 256 592 / 1216 against 570 / 936. A call that turns out not to suit pays the statistics
-// and the launches that return: 13-20 us.
+// at 256 592 / 1216 against 570 / 936. A call that turns out not to suit pays the launches
+// that return, 14 us where the sample refuses it (sep_sample_refuses), and the statistics, 11 us,
+// where only they do. (768 -> 3072 -> 768, 2048 tokens, thresholds over 5 V, forward and backward:
+// 9.15 ms without the contraction, 9.13 here, with the assignment passes in one launch.)
 #ifndef ISA_EKV_CONTRACT_MIN_CELLS
 #define ISA_EKV_CONTRACT_MIN_CELLS (1 << 25)
 #endif
@@ -1554,7 +1604,7 @@ hipError_t sep_forward_operands(const SepPlan& p, SepArgs a, const PrepArgs& pre
     sep_point(p, a, ws);
     a.xrow = reinterpret_cast<float2*>(ws + p.off_row);
     hipLaunchKernelGGL(sep_stat_kernel, dim3(kSepStatX + kSepStatW + (a.lut_n + 255) / 256), dim3(256), 0, s, a,
-                       GlueGradArgs{});
+                       prep, GlueGradArgs{});
     hipLaunchKernelGGL(sep_table_kernel, dim3(kSepTableBlocks), dim3(256), 0, s, a);
     const int64_t expand = std::min<int64_t>((a.M + a.O + 3) / 4, kSepExpandBlocks);
     hipLaunchKernelGGL(sep_expand_fwd_kernel, dim3((unsigned)std::max<int64_t>(expand, kPrepBlocksX + kPrepBlocksW)),
@@ -1605,7 +1655,8 @@ hipError_t sep_backward_operands(const SepPlan& p, SepArgs a, const PrepArgs& pr
     sep_point_backward(p, a, ws);
     const int64_t xcols = a.xcol ? kSepColChunks * ((a.K + 255) / 256) : 0;
     const int64_t stat = kSepStatX + kSepStatW + (a.lut_n + 255) / 256 + xcols + (glue ? (int64_t)kGlueBlocks * (glue->Op / 256) : 0);
-    hipLaunchKernelGGL(sep_stat_kernel, dim3((unsigned)stat), dim3(256), 0, s, a, glue ? *glue : GlueGradArgs{});
+    hipLaunchKernelGGL(sep_stat_kernel, dim3((unsigned)stat), dim3(256), 0, s, a, prep,
+                       glue ? *glue : GlueGradArgs{});
     const int64_t gcols = a.need_w ? kSepColChunks * ((a.O + 255) / 256) : 0;
     hipLaunchKernelGGL(sep_table_kernel, dim3((unsigned)(kSepTableBlocks + kSepStatG + gcols)), dim3(256), 0, s, a);
     const int64_t kt = (a.K + 31) / 32, ot = (a.O + 127) / 128;

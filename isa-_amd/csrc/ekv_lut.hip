@@ -153,7 +153,7 @@ std::atomic<int64_t> g_window_copies{32};
 
 // Planning options ISA_EKV_OPT_RANK_MAX_SPREAD / ISA_EKV_OPT_RANK_GREEDY_MIN: the widest threshold
 // spread (table records) the ranked backward takes, and the spread past which its branches are
-// dealt by the greedy bank-aware deal (bwd_deal_kernel) instead of by rank (bwd_rank_kernel).
+// dealt by the greedy bank-aware deal (bwd_deal_kernel) instead of by rank (rank_deal_block).
 std::atomic<int64_t> g_rank_max_spread{ISA_EKV_RANK_MAX_SPREAD};
 std::atomic<int64_t> g_rank_greedy_min{ISA_EKV_RANK_GREEDY_MIN};
 
@@ -537,7 +537,7 @@ __device__ inline void prep_block(const PrepArgs& a, int b) {
     const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8
     // all of a tile's loads are in flight together, and while the tile before it is stored: waited
     // for one by one they were the pass's time (768 x 3072 and 2048 tokens, 5 tiles a block: the
-    // forward's prep 37-42 us, now 20-26; a call of one token 23 us for both layers, now 11)
+    // forward's prep 37-42 us, now 20-26; one token through both layers 201 us, now 180)
     float2 next[8];
     auto load = [&](int64_t t) {
         const int64_t ot = t % n_ot, kt = t / n_ot;
@@ -669,7 +669,7 @@ __device__ inline bool coords_in_padded_range(const float2* __restrict__ partial
 // thresholds, and once the thresholds spread over more than ~100 records, lanes of a
 // half-wave often hit one LDS bank pair with different records. A second copy of the table
 // 16 bank pairs away (the copy starts T1 records after the first, T1 % 32 == 16) lets each
-// (input, output) threshold pick the copy whose bank is less loaded (fwd_copy_assign_kernel;
+// (input, output) threshold pick the copy whose bank is less loaded (copy_assign_block;
 // the choice folds into the threshold coordinate, c' = c + T1, and copy 1 stores
 // A' = A - T1 dT so that fma(c', dT, A') = fma(c, dT, A)). With narrow thresholds (the
 // initial ones span ~69 records) the lanes share records often enough that splitting them
@@ -1193,7 +1193,8 @@ __device__ inline bool fwd_tile(const FwdArgs& a, int MR, FwdTile& t) {
 // bank pair (floor coordinate, and its neighbour for the tokens whose fraction crosses the
 // threshold's) has the smaller expected load so far. Copy-1 thresholds are stored as
 // ws - T1 (so c' = xs - ws' = c + T1). Changes no record unless the launch is in copy mode.
-constexpr int kAssignThreads = 128;
+constexpr int kAssignThreads = 256;  // of every assignment pass (assign_kernel)
+constexpr int kAssignLdsFloats = 8192;  // LDS of an assignment block, shared by the passes' bodies
 
 // Records [lo, lo + n) of the padded table hold every record the clamp-free loop reads, with
 // two records of margin each side (the second copy's coordinates c + T1 round separately).
@@ -1217,39 +1218,28 @@ __device__ inline bool launch_copy_mode(const float2* __restrict__ partials, int
 }
 
 // Mode word values: 0 one table copy, 1 the second copy, kModeRanked the ranked backward (whose
-// branch-deal pass runs before the copy assignment and records its decision first), and
-// C >= kModeMultiMin: C bank-rotated copies of the coordinate window (fwd_multi_assign_kernel,
-// which also runs before the two-copy assignment), recorded as kModeWindowed2 for C = 2.
+// branch deal goes before the copy assignments), and C >= kModeMultiMin: C bank-rotated copies of
+// the coordinate window (multi_assign_block, which goes before the two-copy assignment), recorded
+// as kModeWindowed2 for C = 2.
 constexpr int kModeRanked = 2;
 constexpr int kModeMultiMin = 3;
 constexpr int kMultiMax = 32;
 constexpr int kModeWindowed2 = kMultiMax + 1;
 
+// Block b of the two-copy assignment.
 // LANES = 32: 8-byte records, gathered by half-waves over 32 bank pairs; LANES = 16: 16-byte
 // records, gathered by quarter-waves over 16 bank quads. Copy 1 sits LANES / 2 bins away.
-// Every wave decides the launch's copy mode from the range partials (launch_copy_mode);
-// block 0 records it in the mode word for the launches that follow.
 template <int LANES>
-__global__ __launch_bounds__(kAssignThreads) void fwd_copy_assign_kernel(float2* __restrict__ wsT,
-                                                              const float2* __restrict__ partials, int NP,
-                                                              int max_window, int* __restrict__ mode_word,
-                                                              int64_t Kp, int64_t Op, int copy_offset,
-                                                              int skip_from, const SepHead* skip) {
-    // (where the contraction takes the call, the first block alone records the mode)
-    if (blockIdx.x != 0 && sep_takes(skip)) return;
+__device__ __forceinline__ void copy_assign_block(float2* __restrict__ wsT, int64_t Kp, int64_t Op, int copy_offset, int b,
+                                         float* s_raw) {
     static_assert(LANES == 32 || LANES == 16, "half-wave or quarter-wave gathers");
+    static_assert(LANES * kAssignThreads <= kAssignLdsFloats, "the bank loads' LDS");
     constexpr int kGroups = 64 / LANES, kMask = LANES - 1;
-    // skip_from > 0: a pass earlier in the call recorded a mode of its own (the ranked backward,
-    // skip_from = kModeRanked; the forward's windowed copies, skip_from = kModeMultiMin), which
-    // this call keeps (this pass writes only 0 or 1, so every block reads the same decision)
-    if (skip_from > 0 && __builtin_amdgcn_readfirstlane(*mode_word) >= skip_from) return;
-    const bool on = launch_copy_mode(partials, NP, max_window);
-    if (blockIdx.x == 0 && threadIdx.x == 0) *mode_word = on ? 1 : 0;
-    if (!on || sep_takes(skip)) return;
-    __shared__ float s_cnt[LANES][kAssignThreads];  // per-thread bank loads; [bin][thread]: conflict-free
+    // per-thread bank loads; [bin][thread]: conflict-free
+    float(*s_cnt)[kAssignThreads] = reinterpret_cast<float(*)[kAssignThreads]>(s_raw);
     const int tid = threadIdx.x;
     const int64_t n_ot = Op / (64 * kFwdORR);
-    const int64_t p = (int64_t)blockIdx.x * blockDim.x + tid;
+    const int64_t p = (int64_t)b * kAssignThreads + tid;
     if (p >= Kp * n_ot * kFwdORR * 2 * kGroups) return;
     const int sign = (int)(p & 1), group = (int)((p >> 1) % kGroups);
     const int64_t rest0 = (p >> 1) / kGroups;
@@ -1354,7 +1344,7 @@ __device__ inline bool ranked_mode(const float2* __restrict__ partials, int NP, 
                                    float* spread);
 
 // Copy choice for the windowed copies. A problem is the 32 thresholds one half-wave gather
-// reads (as in fwd_copy_assign_kernel<32>: input k, sign, output slot j, half of an output
+// reads (as in copy_assign_block<32>: input k, sign, output slot j, half of an output
 // block); kMcGroup threads share it, each pricing C / kMcGroup of the copies. The thresholds
 // are taken in increasing order, so that lanes reading one record for a token follow each
 // other. At kMultiSamples token-coordinate fractions f_q = (q + 1/2) / kMultiSamples, a
@@ -1378,7 +1368,7 @@ constexpr int kMcThreads = kMcProblems * kMcGroup;
 // samples reading the record below (bits 5-12), the samples whose record differs from the
 // previous threshold's (bits 13-20) and its lane (bits 21-25).
 template <int kPer>  // copies priced by this thread: c = sub + kMcGroup * i < copies, i < kPer
-__device__ inline void multi_greedy(const float* s_sw, const unsigned* s_info, unsigned* s_pe, int prob, int sub,
+__device__ __forceinline__ void multi_greedy(const float* s_sw, const unsigned* s_info, unsigned* s_pe, int prob, int sub,
                                     bool active, float* w0, int64_t lane_stride, int copies, int stride) {
     static_assert(kPer >= 1 && kPer * kMcGroup <= kMultiMax && kMcGroup == 4 && kMultiSamples == 8,
                   "copies per thread; quads; a byte of samples");
@@ -1449,30 +1439,19 @@ __device__ inline unsigned multi_lo_mask(float w, float fl) {
     return (1u << nlo) - 1u;
 }
 
-// Block 0 records the launch's mode in the mode word: the number of copies, or 0 (the two-copy
-// pass that follows then decides between one and two copies).
-// (The backward's two-copy launch takes the same pass with dhalf > 0; after_rank > 0: the
-// ranked backward's spread limit, and when its mode applies it keeps the word its pass wrote.)
-__global__ __launch_bounds__(kMcThreads) void fwd_multi_assign_kernel(float2* __restrict__ wsT,
-                                                          const float2* __restrict__ partials, int NP, int budget,
-                                                          int max_copies, int* __restrict__ mode_word, int64_t Kp,
-                                                          int64_t Op, int dhalf, int max_window, int wide_dhalf,
-                                                          float after_rank, const SepHead* skip) {
-    if (blockIdx.x != 0 && sep_takes(skip)) return;
-    if (after_rank > 0.0f && ranked_mode(partials, NP, after_rank, nullptr)) return;
-    const MultiLayout ml =
-        multi_layout(read_coord_range(partials), NP, budget, max_copies, dhalf, max_window, wide_dhalf);
-    if (blockIdx.x == 0 && threadIdx.x == 0) *mode_word = multi_mode_word(ml.copies);
-    if (ml.copies == 0 || sep_takes(skip)) return;
-    __shared__ float s_sw[32 * kMcProblems];       // [rank][problem]: the thresholds in order
-    __shared__ unsigned s_info[32 * kMcProblems];  // [rank][problem] (multi_greedy)
-    __shared__ unsigned s_pe[64 * kMcProblems];    // bit planes (multi_greedy)
+// Block b of the windowed copies' assignment, with layout ml.
+__device__ __forceinline__ void multi_assign_block(float2* __restrict__ wsT, int64_t Kp, int64_t Op, const MultiLayout& ml,
+                                          int b, float* s_raw) {
+    static_assert(kMcThreads == kAssignThreads && 128 * kMcProblems <= kAssignLdsFloats, "the pass's block and LDS");
+    float* s_sw = s_raw;                                                        // [rank][problem]: the thresholds in order
+    unsigned* s_info = reinterpret_cast<unsigned*>(s_raw) + 32 * kMcProblems;  // [rank][problem] (multi_greedy)
+    unsigned* s_pe = s_info + 32 * kMcProblems;                                // bit planes (multi_greedy)
     const int tid = threadIdx.x;
     for (int i = tid; i < 64 * kMcProblems; i += kMcThreads) s_pe[i] = 0u;
     const int prob = tid / kMcGroup, sub = tid % kMcGroup;
     constexpr int kGroups = 2;
     const int64_t n_ot = Op / (64 * kFwdORR);
-    const int64_t p = (int64_t)blockIdx.x * kMcProblems + prob;
+    const int64_t p = (int64_t)b * kMcProblems + prob;
     const bool active = p < Kp * n_ot * kFwdORR * 2 * kGroups;
     const int sign = (int)(p & 1), group = (int)((p >> 1) % kGroups);
     const int64_t rest0 = (p >> 1) / kGroups;
@@ -2013,7 +1992,7 @@ constexpr int kBwdCopyOffsetI = kSplitRecords + 8;
 constexpr size_t kBwdTwoCopiesLds = (size_t)(kBwdCopyOffset + 2 * kSplitRecords) * 8;
 constexpr size_t kBwdTwoCopiesLdsI = (size_t)(kBwdCopyOffsetI + kSplitRecords) * 16;
 // Windowed copies in the two-copy launch (split tables; mode word C >= kModeMultiMin, chosen
-// by fwd_multi_assign_kernel with dhalf = kBwdWinDOffset): copy c holds the coordinate
+// by multi_assign_block with dhalf = kBwdWinDOffset): copy c holds the coordinate
 // window's I records from LDS record T_c and their D records kBwdWinDOffset further (a
 // multiple of 32 that is not one of 64, so the two reads stay two ds_read_b64 through the
 // immediate offset), for windows of at most kBwdWinWindow records, in the whole LDS of the
@@ -2226,11 +2205,10 @@ struct RankArgs {
     float* ws_ranked;     // [Kp][n_ob][64 lanes][8 slots] threshold coordinate of each slot's branch
     uint2* branch;        // [Kp][n_ob][64 lanes]: slot s in byte s: t (output c + kRankClasses t) | sign << 4
     const float2* partials;
-    int* mode_word;
     int Kp, Op, n_ob, NP;
     float max_spread;     // the widest threshold spread (records) the ranked launch takes
     float greedy_min;     // spreads past this are dealt by bwd_deal_kernel, the rest by rank
-    const SepHead* skip;  // the contraction's head: only the mode word is recorded where it takes the call
+    const SepHead* skip;  // the contraction's head: nothing is dealt where it takes the call
 };
 
 #ifndef ISA_EKV_RANK_MERGE_MAX
@@ -2254,19 +2232,15 @@ __device__ inline bool ranked_mode(const float2* __restrict__ partials, int NP, 
 // The branch deal, one thread per (input, output block, residue class): ranks by (coordinate,
 // branch index), so ties keep a fixed order, and rank r goes to half-wave h = r / (B / 2)
 // (B branches per class), lane c + kRankClasses (r' mod L) + 32 h and slot r' / L, where
-// r' = r mod (B / 2) and L = the class's lanes per half-wave. Block 0 records the mode word.
+// r' = r mod (B / 2) and L = the class's lanes per half-wave.
 // A block deals kRankQ (input, output block) pairs and writes their dealt thresholds from LDS
 // as one contiguous run (each thread's own stores would land 32 bytes apart across a wave).
 constexpr int kRankQ = 256 / kRankClasses;
-__global__ __launch_bounds__(256) void bwd_rank_kernel(RankArgs a) {
-    if (blockIdx.x != 0 && sep_takes(a.skip)) return;
-    float spread = 0.0f;
-    const bool on = ranked_mode(a.partials, a.NP, a.max_spread, &spread);  // block-uniform
-    if (blockIdx.x == 0 && threadIdx.x == 0) *a.mode_word = on ? kModeRanked : 0;
-    if (!on || spread > a.greedy_min || sep_takes(a.skip)) return;  // (wide spreads: bwd_deal_kernel deals)
-    __shared__ float4 s_dealt[kRankQ * 64 * 2];  // per pair: 64 lanes x 8 slots
+__device__ __forceinline__ void rank_deal_block(const RankArgs& a, int b, float* s_raw) {
+    static_assert(kRankQ * 64 * 8 <= kAssignLdsFloats && kAssignThreads == 256, "the deal's LDS and block");
+    float4* s_dealt = reinterpret_cast<float4*>(s_raw);  // per pair: 64 lanes x 8 slots
     const int64_t n_q = (int64_t)a.Kp * a.n_ob;
-    const int64_t q0 = (int64_t)blockIdx.x * kRankQ;
+    const int64_t q0 = (int64_t)b * kRankQ;
     const int tq = threadIdx.x / kRankClasses, c = threadIdx.x % kRankClasses;
     const int64_t q = q0 + tq;  // k * n_ob + ob
     if (q < n_q) {
@@ -2312,6 +2286,57 @@ __global__ __launch_bounds__(256) void bwd_rank_kernel(RankArgs a) {
     const int n = (int)min<int64_t>(kRankQ, n_q - q0) * 64 * 2;
     float4* out = reinterpret_cast<float4*>(a.ws_ranked + q0 * 64 * 8);
     for (int i = threadIdx.x; i < n; i += 256) out[i] = s_dealt[i];
+}
+
+// ----------------------------------------------------------------------------------
+// The assignment passes of a table call in one launch: the ranked deal's blocks (RANK), then the
+// windowed copies', then the two copies'. Every wave decides the call's mode from the range
+// partials (ranked, else windowed copies, else two copies, else one), the blocks of the other
+// passes return, and block 0 records it in the mode word for the launches that follow. The passes
+// exclude each other, so that one launch of their blocks costs what the one that applies does;
+// as launches of their own the others cost ~4.5 us each to find out that they do not apply.
+// Where the contraction takes the call, the first block alone records the mode.
+// ----------------------------------------------------------------------------------
+struct AssignArgs {
+    float2* wsT;
+    const float2* partials;
+    int* mode_word;
+    int64_t Kp, Op;
+    int NP;
+    int mc_budget, mc_max, dhalf, max_window, wide_dhalf;  // windowed copies (mc_budget > 0), as multi_layout takes them
+    int copy_offset, copy_window;                          // two copies (copy_offset > 0)
+    int rank_blocks, multi_blocks, copy_blocks;
+    const SepHead* skip;
+};
+
+template <int LANES, bool RANK>
+__global__ __launch_bounds__(kAssignThreads) void assign_kernel(AssignArgs a, RankArgs ra) {
+    __shared__ __align__(16) float s_raw[kAssignLdsFloats];
+    if (blockIdx.x != 0 && sep_takes(a.skip)) return;
+    float spread = 0.0f;
+    const bool ranked = RANK && ranked_mode(a.partials, a.NP, ra.max_spread, &spread);
+    MultiLayout ml{};
+    if (!ranked && a.mc_budget > 0)
+        ml = multi_layout(read_coord_range(a.partials), a.NP, a.mc_budget, a.mc_max, a.dhalf, a.max_window,
+                          a.wide_dhalf);
+    const bool windowed = ml.copies > 0;
+    const bool two = !ranked && !windowed && a.copy_offset > 0 && launch_copy_mode(a.partials, a.NP, a.copy_window);
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+        *a.mode_word = ranked ? kModeRanked : windowed ? multi_mode_word(ml.copies) : two ? 1 : 0;
+    if (sep_takes(a.skip)) return;
+    int b = blockIdx.x;
+    if constexpr (RANK) {
+        if (b < a.rank_blocks) {  // (wide spreads: bwd_deal_kernel deals)
+            if (ranked && !(spread > ra.greedy_min)) rank_deal_block(ra, b, s_raw);
+            return;
+        }
+        b -= a.rank_blocks;
+    }
+    if (b < a.multi_blocks) {
+        if (windowed) multi_assign_block(a.wsT, a.Kp, a.Op, ml, b, s_raw);
+        return;
+    }
+    if (two) copy_assign_block<LANES>(a.wsT, a.Kp, a.Op, a.copy_offset, b - a.multi_blocks, s_raw);
 }
 
 // ----------------------------------------------------------------------------------
@@ -4421,6 +4446,29 @@ SepArgs make_sep(const CallSetup& cs, const float* x, const float* wp, const flo
     return a;
 }
 
+// The assignment passes' launch (rank nullable: no ranked deal); orr: the launch's outputs a lane.
+hipError_t launch_assign(AssignArgs& a, int lanes, const RankArgs* rank, int orr, hipStream_t s) {
+    const int64_t problems = a.Kp * (a.Op / (64 * orr)) * orr * 2 * (64 / lanes);
+    const int64_t halves = a.Kp * (a.Op / (64 * orr)) * orr * 4;  // the windowed copies' problems: half-waves
+    if (rank) a.rank_blocks = (int)(((int64_t)rank->Kp * rank->n_ob * kRankClasses + 255) / 256);
+    if (a.mc_budget > 0) a.multi_blocks = (int)((halves + kMcProblems - 1) / kMcProblems);
+    if (a.copy_offset > 0) a.copy_blocks = (int)((problems + kAssignThreads - 1) / kAssignThreads);
+    const dim3 grid((unsigned)(a.rank_blocks + a.multi_blocks + a.copy_blocks)), block(kAssignThreads);
+    const RankArgs ra = rank ? *rank : RankArgs{};
+    if (lanes == 32) {
+        if (rank)
+            hipLaunchKernelGGL((assign_kernel<32, true>), grid, block, 0, s, a, ra);
+        else
+            hipLaunchKernelGGL((assign_kernel<32, false>), grid, block, 0, s, a, ra);
+    } else {
+        if (rank)
+            hipLaunchKernelGGL((assign_kernel<16, true>), grid, block, 0, s, a, ra);
+        else
+            hipLaunchKernelGGL((assign_kernel<16, false>), grid, block, 0, s, a, ra);
+    }
+    return hipGetLastError();
+}
+
 int run_forward(const CallSetup& cs, const float* x, const float* vth_pos, const float* vth_neg, int64_t M,
                 int64_t K, int64_t O, float v_sat, float out_min, float out_max, float* out, void* workspace,
                 size_t workspace_bytes, hipStream_t s, const isa_ekv_glue* glue = nullptr,
@@ -4504,23 +4552,11 @@ int run_forward(const CallSetup& cs, const float* x, const float* vth_pos, const
         fa.copy_window = tc.copy_window;
         fa.mc_budget = tc.mc_budget;
         fa.mc_max = tc.mc_max;
-        int* mode = reinterpret_cast<int*>(ws + p.off_mode);
-        const int64_t problems = p.Kp * (p.Op / (64 * kFwdORR)) * kFwdORR * 4;
-        const dim3 agrid((unsigned)((problems + kAssignThreads - 1) / kAssignThreads));
-        if (tc.mc_budget > 0) {
-            hipLaunchKernelGGL(fwd_multi_assign_kernel, dim3((unsigned)((problems + kMcProblems - 1) / kMcProblems)),
-                               dim3(kMcThreads), 0, s,
-                               reinterpret_cast<float2*>(ws + p.off_wsT), fa.partials, fa.NP, tc.mc_budget,
-                               tc.mc_max, mode, p.Kp, p.Op, 0, fa.NP, 0, 0.0f, sep_head);
-            err = hipGetLastError();
-            if (err != hipSuccess) return hip_fail(err, "forward windowed-copy assignment launch");
-        }
-        if (tc.copy_offset > 0) {
-            hipLaunchKernelGGL(fwd_copy_assign_kernel<32>, agrid, dim3(kAssignThreads), 0, s,
-                               reinterpret_cast<float2*>(ws + p.off_wsT), fa.partials, fa.NP,
-                               fa.copy_window > 0 ? fa.copy_window : fa.NP, mode, p.Kp, p.Op, tc.copy_offset,
-                               tc.mc_budget > 0 ? kModeMultiMin : 0, sep_head);
-            err = hipGetLastError();
+        AssignArgs aa{reinterpret_cast<float2*>(ws + p.off_wsT), fa.partials,
+                      reinterpret_cast<int*>(ws + p.off_mode), p.Kp, p.Op, fa.NP, tc.mc_budget, tc.mc_max, 0,
+                      fa.NP, 0, tc.copy_offset, fa.copy_window > 0 ? fa.copy_window : fa.NP, 0, 0, 0, sep_head};
+        if (tc.mc_budget > 0 || tc.copy_offset > 0) {
+            err = launch_assign(aa, 32, nullptr, kFwdORR, s);
             if (err != hipSuccess) return hip_fail(err, "forward copy assignment launch");
         }
     }
@@ -4709,42 +4745,29 @@ int run_backward(const CallSetup& cs, const float* x, const float* vth_pos, cons
     const float rank_max_spread = (float)g_rank_max_spread.load(std::memory_order_relaxed);
     if (copies) {
         int* mode = reinterpret_cast<int*>(ws + p.off_mode);
-        if (p.ranked) {  // the branch deal first: it records the ranked mode when that launch works
-            const RankArgs ra{reinterpret_cast<const float2*>(ws + p.off_wsT),
-                              reinterpret_cast<float*>(ws + p.off_rank_ws),
-                              reinterpret_cast<uint2*>(ws + p.off_rank_branch), ba.partials, mode,
-                              (int)p.Kp, (int)p.Op, p.n_ob, ba.NP, rank_max_spread,
-                              (float)g_rank_greedy_min.load(std::memory_order_relaxed), sep_head};
-            const int64_t threads = p.Kp * p.n_ob * kRankClasses;
-            hipLaunchKernelGGL(bwd_rank_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, ra);
-            // the greedy deal of spreads past greedy_min (exits at once when the rank deal
-            // applies); not launched when no spread the ranked mode takes can exceed greedy_min
-            const int64_t problems_q = p.Kp * p.n_ob;
-            if (ra.greedy_min < ra.max_spread)
-                hipLaunchKernelGGL(bwd_deal_kernel, dim3((unsigned)((problems_q + kDealProblems - 1) / kDealProblems)),
-                                   dim3(kDealWaves * 64), 0, s, ra);
+        const RankArgs ra{reinterpret_cast<const float2*>(ws + p.off_wsT),
+                          reinterpret_cast<float*>(ws + p.off_rank_ws),
+                          reinterpret_cast<uint2*>(ws + p.off_rank_branch), ba.partials,
+                          (int)p.Kp, (int)p.Op, p.n_ob, ba.NP, rank_max_spread,
+                          (float)g_rank_greedy_min.load(std::memory_order_relaxed), sep_head};
+        AssignArgs aa{reinterpret_cast<float2*>(ws + p.off_wsT), ba.partials, mode, p.Kp, p.Op, ba.NP, 0, 0, 0, 0, 0,
+                      p.split ? kBwdCopyOffset : kBwdCopyOffsetI, kSplitRecords, 0, 0, 0, sep_head};
+        if (p.mc_max > 0) {  // the windowed copies of the two-copy launch, unless ranked
+            ba.mc_budget = aa.mc_budget = kBwdWinBudget;
+            ba.mc_max = aa.mc_max = p.mc_max;
+            aa.dhalf = kBwdWinDOffset;
+            aa.max_window = kBwdWinWindow;
+            aa.wide_dhalf = kBwdWinWideDOffset;
         }
         // split tables: 8-byte records (half-wave banks); interleaved: 16-byte (quarter-wave)
-        const int64_t problems = p.Kp * (p.Op / (64 * kBwdORR)) * kBwdORR * (p.split ? 4 : 8);
-        const dim3 agrid((unsigned)((problems + kAssignThreads - 1) / kAssignThreads));
-        if (p.mc_max > 0) {  // then the windowed copies of the two-copy launch, unless ranked
-            ba.mc_budget = kBwdWinBudget;
-            ba.mc_max = p.mc_max;
-            hipLaunchKernelGGL(fwd_multi_assign_kernel, dim3((unsigned)((problems + kMcProblems - 1) / kMcProblems)),
-                               dim3(kMcThreads), 0, s, reinterpret_cast<float2*>(ws + p.off_wsT), ba.partials,
-                               ba.NP, kBwdWinBudget, p.mc_max, mode, p.Kp, p.Op, kBwdWinDOffset, kBwdWinWindow,
-                               kBwdWinWideDOffset, p.ranked ? rank_max_spread : 0.0f, sep_head);
-        }
-        // (a pass before it recorded the ranked mode or the windowed copies: skip_from)
-        const int skip_from = p.ranked ? kModeRanked : p.mc_max > 0 ? kModeMultiMin : 0;
-        if (p.split)
-            hipLaunchKernelGGL(fwd_copy_assign_kernel<32>, agrid, dim3(kAssignThreads), 0, s,
-                               reinterpret_cast<float2*>(ws + p.off_wsT), ba.partials, ba.NP, kSplitRecords, mode,
-                               p.Kp, p.Op, kBwdCopyOffset, skip_from, sep_head);
-        else
-            hipLaunchKernelGGL(fwd_copy_assign_kernel<16>, agrid, dim3(kAssignThreads), 0, s,
-                               reinterpret_cast<float2*>(ws + p.off_wsT), ba.partials, ba.NP, kSplitRecords, mode,
-                               p.Kp, p.Op, kBwdCopyOffsetI, skip_from, sep_head);
+        err = launch_assign(aa, p.split ? 32 : 16, p.ranked ? &ra : nullptr, kBwdORR, s);
+        if (err != hipSuccess) return hip_fail(err, "backward copy assignment launch");
+        // the greedy deal of spreads past greedy_min (exits at once when the rank deal
+        // applies); not launched when no spread the ranked mode takes can exceed greedy_min
+        if (p.ranked && ra.greedy_min < ra.max_spread)
+            hipLaunchKernelGGL(bwd_deal_kernel,
+                               dim3((unsigned)((p.Kp * p.n_ob + kDealProblems - 1) / kDealProblems)),
+                               dim3(kDealWaves * 64), 0, s, ra);
         ba.copy_mode = mode;
         err = hipGetLastError();
         if (err != hipSuccess) return hip_fail(err, "backward copy assignment launch");

@@ -137,7 +137,8 @@ def rank_xcd_order(value: Optional[bool] = None) -> bool:
 def copy_mode(workspace: torch.Tensor, plan: dict) -> Optional[int]:
     """After a call that used `workspace` (and synchronised), which table mode its main kernel
     ran in: 1 the second table copy, 0 one copy, 2 the ranked backward, 3 to 32 the forward's
-    windowed copies (their number); None when the plan has no second copy."""
+    windowed copies (their number); None when the plan has no second copy. A call that ran as
+    products on the matrix cores records the mode the table kernels would have run in."""
     off = plan["mode_offset"]
     if off < 0:
         return None
