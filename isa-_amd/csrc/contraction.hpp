@@ -37,11 +37,18 @@
 //     L(xs - ws) = (F + S / 12)(xs - ws)
 //                  - sum_q S(xs - ws) (cos 2 pi q xs cos 2 pi q ws + sin 2 pi q xs sin 2 pi q ws) / (2 pi^2 q^2):
 // the first part is smooth and expands as above, the others are 1e-5 of it and take R / 4 terms
-// of S per cosine and sine in plain f16. Two harmonics (none from about 14000 entries on) keep
-// the remainder below the per-cell kernels' own rounding of coordinates and of the records'
-// intercepts: 4096 entries, initial thresholds, 2-norm against float64 lookups, forward 9.8e-6
-// by the lookups. Sums of T's differences give back the entries exactly. A table that
-// is not smooth (bf16 entries) runs the per-cell kernels.
+// of S per cosine and sine in plain f16. One harmonic keeps the forward's and dVth's remainder
+// below the per-cell kernels' own rounding of coordinates and of the records' intercepts up to
+// growths of 3.3% from entry to entry (about 3900 entries), and dX's, which they round less, up to
+// 2.2% (about 6000); coarser tables take two, finer ones than about 14000 entries none. 2-norm
+// against float64 lookups, initial thresholds, per-cell kernels against this: 4096 entries forward
+// 9.8e-6 and 3.8e-6, dX 5.4e-6 and 3.2e-6, dVth 1.1e-6 and 8.1e-7; 5500 entries 9.1e-6 and 2.1e-6,
+// 5.2e-6 and 1.7e-6, 1.2e-6 and 4.8e-7; 8192 entries 7.8e-6 and 9.9e-7, 5.6e-6 and 1.5e-6, 1.3e-6
+// and 2.9e-7 (over 0.5 and 1 V also smaller, closest for
+// dVth over 1 V at 4096 entries, 1.7e-6 and 1.6e-6). With two harmonics throughout 768 -> 3072
+// at 8192 tokens took 1.06 ms forward and 2.47 backward, with one 0.92 and 2.35. Sums of T's
+// differences give back the entries exactly. A table that is not smooth (bf16 entries) runs the
+// per-cell kernels.
 //
 // R is chosen per call on the device from the thresholds' spread (sep_terms); a call whose
 // operands do not suit (non-finite values, x near -V_sat or spread over more than the table
@@ -79,7 +86,7 @@ struct SepHead {
     unsigned gmax;  // backward: bits of the largest |G|: not finite: the per-cell kernels run
     int rough;    // 1: the series does not converge as its terms assume, 2: a sample of the thresholds or of
                   // the table ruled the contraction out (then the other fields are not set): the per-cell kernels run
-    int harmonics;  // 1: the kinks' two harmonics are summed
+    int harmonics, harmonics_dx;  // of the table's kinks that are summed (0 to 2): forward and dVth, dX
     int n_grid;
     float xlo, xhi, wlo, whi;
     float lut_min, lut_scale;  // table coordinate (v - lut_min) * lut_scale
@@ -155,7 +162,7 @@ __device__ inline float sep_input(const SepArgs& a, float x, float s, float b) {
 __host__ __device__ inline int64_t sep_inputs(int64_t K) { return (K + 15) / 16 * 16; }
 __host__ __device__ inline int64_t sep_slabs_pairs(int64_t K, int terms) { return sep_inputs(K) * (terms / 2) / 32; }
 __host__ __device__ inline int64_t sep_slabs_singles(int64_t K, int terms, int harmonics) {
-    return sep_inputs(K) * (terms / 2 + harmonics * terms) / 64;
+    return sep_inputs(K) * (terms / 2 + harmonics * terms / 2) / 64;
 }
 __host__ __device__ inline int64_t sep_slabs(int64_t n) { return (n + 31) / 32; }
 __host__ __device__ inline int64_t sep_slabs64(int64_t n) { return (n + 63) / 64; }
@@ -487,7 +494,8 @@ __global__ __launch_bounds__(256) void sep_table_kernel(SepArgs a) {
         bool ok = finite && terms > 0 && terms <= a.max_terms && rlo > 0.1 && rhi > 0.1 &&
                   points <= (double)kSepGridMax && fmax(fabs((double)xlo), fabs((double)xhi)) < step * (1 << 23);
         if (lut) {  // every lookup inside the table, the x table's margin included
-            h.harmonics = growth > 0.009 ? 1 : 0;
+            h.harmonics = growth > 0.033 ? 2 : growth > 0.009 ? 1 : 0;
+            h.harmonics_dx = growth > 0.022 ? 2 : h.harmonics;
             const double margin = 4.0 * step * a.lut_scale + 4.0;
             ok = ok && s_info.x == 0.0f && growth > 1e-6 && growth < 0.045 &&
                  ((double)xlo - (double)whi - a.lut_min) * a.lut_scale >= margin &&
@@ -517,6 +525,7 @@ __global__ __launch_bounds__(256) void sep_table_kernel(SepArgs a) {
             SepHead* g = a.head;
             g->terms = h.terms;
             g->harmonics = h.harmonics;
+            g->harmonics_dx = h.harmonics_dx;
             g->n_grid = h.n_grid;
             g->xlo = xlo;
             g->xhi = xhi;
@@ -832,7 +841,7 @@ __global__ __launch_bounds__(256) void sep_expand_fwd_kernel(SepArgs a, PrepArgs
                     float e[4], c[2], sn[2];
                     sep_second(h, a.tabE, at, e);
                     sep_trig((x - h.lut_min) * h.lut_scale, c, sn);
-                    for (int blk = 0; blk < R / 4; ++blk) {
+                    for (int blk = 0; blk < h.harmonics * R / 8; ++blk) {
                         sep_harm_x(v, e, R, blk, c, sn, sc);
                         sep_store4h(dst + harm, blk * 4 * kc + k * 4, v);
                     }
@@ -859,7 +868,7 @@ __global__ __launch_bounds__(256) void sep_expand_fwd_kernel(SepArgs a, PrepArgs
                     sep_cheb4((float)tn, n);
                     sep_trig((float)((h.wc + h.wh * tp) * h.lut_scale), cp, sp);
                     sep_trig((float)((h.wc + h.wh * tn) * h.lut_scale), cn, sn);
-                    for (int blk = 0; blk < R / 4; ++blk) {
+                    for (int blk = 0; blk < h.harmonics * R / 8; ++blk) {
                         sep_harm_w(v, p, n, R, blk, cp, sp, cn, sn, kSepQScale);
                         sep_store4h(dst + harm, blk * 4 * kc + k * 4, v);
                     }
@@ -939,11 +948,11 @@ __global__ __launch_bounds__(256) void sep_expand_bwd_kernel(SepArgs a, int x_bl
                 sep_second(h, a.tabE, p1, e1);
                 sep_trig((x0 - h.lut_min) * h.lut_scale, c0, n0);
                 sep_trig((x1 - h.lut_min) * h.lut_scale, c1, n1);
-                for (int blk = 0; blk < R / 4; ++blk) {
+                for (int blk = 0; blk < h.harmonics * R / 8; ++blk) {
                     sep_harm_x(u, e0, R, blk, c0, n0, s0);
                     sep_harm_x(v, e1, R, blk, c1, n1, s1);
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) sep_store2h(a.xoph + sep_row(k, R, blk * 4 + q) * m64, m, u[q], v[q]);
+                    for (int q = 0; q < 4; ++q) sep_store2h(a.xoph + sep_row(k, h.harmonics * R / 2, blk * 4 + q) * m64, m, u[q], v[q]);
                 }
             }
         }
@@ -992,7 +1001,7 @@ __global__ __launch_bounds__(256) void sep_expand_bwd_kernel(SepArgs a, int x_bl
                     }
                 }
             }
-            if (h.harmonics > 0) {
+            if (h.harmonics_dx > 0) {
                 float p0[4], n0[4], p1[4], n1[4], e0[4], d0[4], e1[4], d1[4];
                 sep_cheb4((float)t_[0], p0);
                 sep_cheb4((float)t_[1], n0);
@@ -1002,11 +1011,11 @@ __global__ __launch_bounds__(256) void sep_expand_bwd_kernel(SepArgs a, int x_bl
                 sep_trig(s_b[kk][ol] * h.lut_scale, e0 + 2, d0 + 2);
                 sep_trig(s_a[kk][ol + 1] * h.lut_scale, e1, d1);
                 sep_trig(s_b[kk][ol + 1] * h.lut_scale, e1 + 2, d1 + 2);
-                for (int blk = 0; blk < R / 4; ++blk) {
+                for (int blk = 0; blk < h.harmonics_dx * R / 8; ++blk) {
                     sep_harm_w(u, p0, n0, R, blk, e0, d0, e0 + 2, d0 + 2, kSepQScale);
                     sep_harm_w(v, p1, n1, R, blk, e1, d1, e1 + 2, d1 + 2, kSepQScale);
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) sep_store2h(a.woph + sep_row(k, R, blk * 4 + q) * o64, o, u[q], v[q]);
+                    for (int q = 0; q < 4; ++q) sep_store2h(a.woph + sep_row(k, h.harmonics_dx * R / 2, blk * 4 + q) * o64, o, u[q], v[q]);
                 }
             }
         }
@@ -1106,6 +1115,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void sep_gemm_kernel(SepGemm g) {
     if (!sep_takes(head)) return;
     const int R = __builtin_amdgcn_readfirstlane(head->terms);
     const int harmonics = __builtin_amdgcn_readfirstlane(head->harmonics);
+    const int harmonics_dx = FORWARD ? 0 : __builtin_amdgcn_readfirstlane(head->harmonics_dx);
     // the product this block works on, its rows and slabs, and the blocks of four values per input
     int id = blockIdx.x, which = 0, ta = 0, tb = 0, n = 0, slabs = 0, pair_slabs = 0, per = 0;
     int64_t a_rows = 0;
@@ -1118,7 +1128,10 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void sep_gemm_kernel(SepGemm g) {
             slabs = pair_slabs + (int)sep_slabs_singles(p.inner, R, harmonics);
         } else {
             const bool pairs = p.kind == kSepDx || p.kind == kSepDv;
-            per = p.kind >= kSepDxHarm ? harmonics * R / 4 : p.kind == kSepDv && g.dv_all ? R / 4 : R / 8;
+            per = p.kind == kSepDxHarm             ? harmonics_dx * R / 8
+                  : p.kind == kSepDvHarm           ? harmonics * R / 8
+                  : p.kind == kSepDv && g.dv_all ? R / 4
+                                                   : R / 8;
             a_rows = (p.a_rows + 1) / 2 * 8 * per;
             slabs = (int)(pairs ? sep_slabs(p.inner) : sep_slabs64(p.inner));
             pair_slabs = pairs ? slabs : 0;
@@ -1450,6 +1463,12 @@ __global__ __launch_bounds__(256) void sep_reduce_bwd_kernel(DxReduceArgs dx, Dx
 #ifndef ISA_EKV_CONTRACT_MIN_CELLS
 #define ISA_EKV_CONTRACT_MIN_CELLS (1 << 25)
 #endif
+// Table calls, from 2^29 cells. Measured (us, forward / backward, per-cell kernels against the
+// contraction, 4096 entries): 384 x 1536 at 2^29 cells 224 / 329 against 98 / 200 at the initial
+// thresholds, 219 / 414 against 142 / 296 over 1 V (16 terms), and 237 / 462 against 246 / 472
+// over 5 V (refused); at 2^28 135 / 190 against 82 / 150, 137 / 240 against 112 / 217, and 150 /
+// 245 against 162 / 255: there a refused call would pay 4 to 8%. 768 x 3072 at 2^29 267 / 356
+// against 111 / 261, over 1 V 275 / 449 against 169 / 404.
 #ifndef ISA_EKV_CONTRACT_MIN_CELLS_LUT
 #define ISA_EKV_CONTRACT_MIN_CELLS_LUT (1 << 29)
 #endif
@@ -1558,7 +1577,8 @@ SepPlan plan_sep(int lut_n, int64_t M, int64_t K, int64_t O, bool backward, bool
         // (a wave sums all of an input's values of a product: 64 terms of the formula's dVth take the
         // 128 rows that a wave of the large tile has)
         p.big = sep_big(8 * K, std::min(M, O), std::min(M, O) / 32) || terms == 64;
-        // at 8 terms: 4 rows per input of lower and of upper terms (8 of the formula's dVth), 8 of harmonics
+        // at 8 terms: 4 rows per input of lower and of upper terms (8 of the formula's dVth), 4 of a harmonic
+        // (dX has two below ~6000 entries)
         const int64_t tile = p.big ? 256 : 128, t4 = (4 * K + tile - 1) / tile, t8 = (8 * K + tile - 1) / tile;
         const int64_t tm = (M + tile - 1) / tile, to = (O + tile - 1) / tile;
         const double dx_bytes = 8.0 * M * K, dv_bytes = 16.0 * p.Kp * p.Op;
@@ -1566,8 +1586,8 @@ SepPlan plan_sep(int lut_n, int64_t M, int64_t K, int64_t O, bool backward, bool
         p.split_dxs = sep_splits(t4 * tm, (O + 63) / 64, p.big, dx_bytes);
         p.split_dv = sep_splits((harm ? t4 : t8) * to, (M + 31) / 32, p.big, dv_bytes);
         p.split_dvs = harm ? sep_splits(t4 * to, (M + 63) / 64, p.big, dv_bytes) : 0;
-        p.split_dxh = harm ? sep_splits(t8 * tm, (O + 63) / 64, p.big, dx_bytes) : 0;
-        p.split_dvh = harm ? sep_splits(t8 * to, (M + 63) / 64, p.big, dv_bytes) : 0;
+        p.split_dxh = harm ? sep_splits((lut_n < 6000 ? t8 : t4) * tm, (O + 63) / 64, p.big, dx_bytes) : 0;
+        p.split_dvh = harm ? sep_splits(t4 * to, (M + 63) / 64, p.big, dv_bytes) : 0;
         p.planes_dx = p.split_dx + p.split_dxs + p.split_dxh;
         p.planes_dv = p.split_dv + p.split_dvs + p.split_dvh;
         if (need_x) p.off_planes = take((int64_t)p.planes_dx * M * K * 4);
