@@ -65,19 +65,21 @@ constexpr int kSepStatG = 512;          // blocks of the largest |G| of each row
 constexpr int kSepColChunks = 64;       // row chunks of a column pass, at most
 constexpr int kSepGridMax = 16384;      // x-table points, at most
 constexpr double kSepStep = 0.0148;     // x-table step in units of 2 n U_T
-constexpr int kSepMaxTerms = 64;
+constexpr int kSepMaxTerms = 16;
 constexpr int kSepLutMin = 2900, kSepLutMax = 65536;  // table entries: the kinks small enough, a thread per partial
 constexpr float kSepQScale = 256.0f;    // of the threshold-side operand (values in [-2, 2])
 
-// Widest threshold spread, in units of 2 n U_T, that R = 8, 16, 32, 64 terms take: there the
-// truncation is 1e-7 of the gradients (the forward's is ten times smaller), below the fp32
-// sums' own rounding (float64 evaluation of the truncated series against the formula).
-__host__ __device__ inline int sep_terms(float spread_u) {
-    return spread_u <= 1.12f ? 8 : spread_u <= 4.4f ? 16 : spread_u <= 11.0f ? 32 : spread_u <= 24.0f ? 64 : 0;
-}
+// Widest threshold spread, in units of 2 n U_T, that R = 8 and 16 terms take: there the
+// truncation is 1e-7 of the gradients (the forward's is ten times smaller). More would converge
+// (16 terms to 4.4), but as the spread grows the per-cell kernels lose fewer bits to the branches'
+// difference while the sums here have more terms: 2-norm against float64, 768 x 768 at 1900
+// tokens, per-cell kernels against this, forward and dVth: 0.2142 V 2.8e-6 and 2.1e-7, 3.6e-7 and
+// 2.5e-7; 0.3 V (1.4 units) 8.2e-7 and 3.7e-7, 3.0e-7 and 3.0e-7; 0.9 V 4.2e-7 and 4.2e-7, 3.1e-7
+// and 3.3e-7. The formula goes over to the per-cell kernels where dVth's errors meet.
+__host__ __device__ inline int sep_terms(float spread_u) { return spread_u <= 1.12f ? 8 : spread_u <= 1.45f ? 16 : 0; }
 
-// Table calls: the per-cell kernels' own rounding (2e-6) allows a little more at 16 terms, and
-// 32 terms would cost what the lookups do.
+// Table calls: the lookups round more (over 1 V, 4.7 units, forward 2.7e-6 and 1.8e-6, dVth 1.7e-6
+// and 1.6e-6 at 4096 entries), and 32 terms would cost what the lookups do.
 __host__ __device__ inline int sep_terms_lut(float spread_u) { return spread_u <= 1.12f ? 8 : spread_u <= 5.0f ? 16 : 0; }
 
 // What the passes of a call share, in its workspace.
@@ -1448,29 +1450,23 @@ __global__ __launch_bounds__(256) void sep_reduce_bwd_kernel(DxReduceArgs dx, Dx
 // Host side: plans and launches.
 // ----------------------------------------------------------------------------------
 
-// Exact-formula calls of fewer cells M K O run the per-cell kernels; larger ones consider 16 terms
-// at most, 32 from 2^28 cells and 64 from 2^30. The operands' passes cost R bytes x 4 per input
-// of x and of the thresholds whatever the other side's length is, so many terms need a long
-// other side. Measured (one box, forward and backward, us, per-cell kernels against the
-// contraction, K x O at M tokens): 8 terms 192 x 768 at 256 (2^25.2 cells) 66 / 104 against
-// 51 / 90, at 128 43 / 87 against 50 / 84; 16 terms at 256 66 / 104 against 60 / 103, at 512
-// 97 / 165 against 64 / 114; 32 terms 768 x 3072 at 128 (2^28.2) 317 / 625 against 281 / 436,
-// at 64 225 / 359 against 261 / 347; 64 terms at 512 (2^30.2) 1120 / 2202 against 798 / 1435,
-// at 256 592 / 1216 against 570 / 936. A call that turns out not to suit pays the launches
-// that return, 14 us where the sample refuses it (sep_sample_refuses), and the statistics, 11 us,
-// where only they do. (768 -> 3072 -> 768, 2048 tokens, thresholds over 5 V, forward and backward:
-// 9.15 ms without the contraction, 9.13 here, with the assignment passes in one launch.)
+// Calls of fewer cells M K O run the per-cell kernels. A call that the contraction refuses pays for
+// the launches that return, 14 us where the sample refuses it (sep_sample_refuses; 5 us less for
+// tables, whose assignment passes are one launch), and the statistics, 11 us, where only they do:
+// the lines lie where that is 1% of the call. Measured (us, forward and backward, without the
+// contraction against refused): formula, 192 x 768 over 2 V at 2^27.2 cells 444 against 458, at
+// 2^28 over 4 V 804 against 820; tables over 5 V at 2^29 614 against 626, 768 -> 3072 -> 768 at
+// 2048 tokens (two calls of 2^32.2) 9125 against 9135. Taken calls gain from far smaller sizes on:
+// formula, 192 x 768 at 2^25.2 164 against 153, at 2^27.2 444 against 156.
 #ifndef ISA_EKV_CONTRACT_MIN_CELLS
-#define ISA_EKV_CONTRACT_MIN_CELLS (1 << 25)
+#define ISA_EKV_CONTRACT_MIN_CELLS (1 << 29)
 #endif
-// Table calls, from 2^29 cells. Measured (us, forward / backward, per-cell kernels against the
-// contraction, 4096 entries): 384 x 1536 at 2^29 cells 224 / 329 against 98 / 200 at the initial
-// thresholds, 219 / 414 against 142 / 296 over 1 V (16 terms), and 237 / 462 against 246 / 472
-// over 5 V (refused); at 2^28 135 / 190 against 82 / 150, 137 / 240 against 112 / 217, and 150 /
-// 245 against 162 / 255: there a refused call would pay 4 to 8%. 768 x 3072 at 2^29 267 / 356
-// against 111 / 261, over 1 V 275 / 449 against 169 / 404.
+// Table calls (us, forward / backward, per-cell kernels against the contraction, 4096 entries):
+// 384 x 1536 at 2^30 cells 334 / 557 against 137 / 261 at the initial thresholds, 344 / 740 against
+// 222 / 398 over 1 V (16 terms), 399 / 783 against 410 / 791 over 5 V (refused); at 2^29 224 / 329
+// against 98 / 200, 219 / 414 against 142 / 296, and 237 / 462 against 246 / 472.
 #ifndef ISA_EKV_CONTRACT_MIN_CELLS_LUT
-#define ISA_EKV_CONTRACT_MIN_CELLS_LUT (1 << 29)
+#define ISA_EKV_CONTRACT_MIN_CELLS_LUT (1 << 30)
 #endif
 
 struct SepPlan {
@@ -1526,7 +1522,7 @@ SepPlan plan_sep(int lut_n, int64_t M, int64_t K, int64_t O, bool backward, bool
     // bytes per (row, input), forward: R / 2 pairs, R / 2 singles and the harmonics; an operand's
     // size backward: at most R pairs
     auto width = [&](int terms) { return (int64_t)terms * (backward ? 4 : 3 + 2 * harm); };
-    int terms = lut_n > 0 ? 16 : cells >= 1 << 30 ? 64 : cells >= 1 << 28 ? 32 : 16;
+    int terms = kSepMaxTerms;
     while (terms >= 8 && (Mr * Kr * width(terms) >= kSepOperandBytes || Or * Kr * width(terms) >= kSepOperandBytes)) terms /= 2;
     if (terms < 8 || Mr * Or * 4 >= kSepOperandBytes) return p;
     p.max_terms = terms;
@@ -1574,9 +1570,7 @@ SepPlan plan_sep(int lut_n, int64_t M, int64_t K, int64_t O, bool backward, bool
         p.off_gscale = take(M * 4);
         p.off_gscaleT = take(O * 4);
         p.off_tT = take(K * p.Op * 8);
-        // (a wave sums all of an input's values of a product: 64 terms of the formula's dVth take the
-        // 128 rows that a wave of the large tile has)
-        p.big = sep_big(8 * K, std::min(M, O), std::min(M, O) / 32) || terms == 64;
+        p.big = sep_big(8 * K, std::min(M, O), std::min(M, O) / 32);
         // at 8 terms: 4 rows per input of lower and of upper terms (8 of the formula's dVth), 4 of a harmonic
         // (dX has two below ~6000 entries)
         const int64_t tile = p.big ? 256 : 128, t4 = (4 * K + tile - 1) / tile, t8 = (8 * K + tile - 1) / tile;

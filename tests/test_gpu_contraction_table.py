@@ -92,25 +92,25 @@ def _errors(got, ref):
     return [float((a.double() - r).norm() / r.norm()) for a, r in zip(got, ref)]
 
 
-# (M, K, O, entries, threshold spread): 2^29 cells and just above; 8 terms up to 0.24 V, 16 to
+# (M, K, O, entries, threshold spread): 2^30 cells and just above; 8 terms up to 0.24 V, 16 to
 # 1.07 V; two harmonics (3400 entries; dX also at 4096 and 5500), one, none (16384); remainders of
 # the 128 and 256 tiles, of the slabs, of the inputs' fours and of the table's 256-entry ranges; odd
 # and even inputs; few tokens, few outputs, few inputs
 CASES = [
-    (1024, 384, 1536, 4096, 0.2142),
-    (1111, 389, 1533, 4096, 0.2142),
-    (257, 1031, 2051, 3400, 0.2142),
-    (1027, 513, 1031, 3400, 0.8),
-    (1029, 515, 1031, 5500, 0.2142),
-    (1024, 511, 1037, 8192, 0.2142),
-    (16, 5800, 5801, 4096, 0.2142),
-    (9001, 9, 6650, 4099, 0.2142),
-    (5801, 5799, 17, 4096, 0.2142),
-    (999, 515, 1100, 4096, 1.0),
-    (1030, 513, 1027, 8192, 0.8),
-    (770, 769, 1025, 13000, 0.2142),
-    (769, 770, 1029, 16384, 1.0),
-    (1025, 512, 1026, 16384, 0.2142),
+    (2048, 384, 1536, 4096, 0.2142),
+    (2111, 389, 1533, 4096, 0.2142),
+    (515, 1031, 2051, 3400, 0.2142),
+    (2051, 513, 1031, 3400, 0.8),
+    (2053, 515, 1031, 5500, 0.2142),
+    (2048, 511, 1037, 8192, 0.2142),
+    (16, 8200, 8201, 4096, 0.2142),
+    (18001, 9, 6650, 4099, 0.2142),
+    (11001, 5799, 17, 4096, 0.2142),
+    (1999, 515, 1100, 4096, 1.0),
+    (2060, 513, 1027, 8192, 0.8),
+    (1370, 769, 1025, 13000, 0.2142),
+    (1369, 770, 1029, 16384, 1.0),
+    (2050, 512, 1026, 16384, 0.2142),
 ]
 
 
@@ -130,7 +130,7 @@ def test_contraction_matches_lookups(cuda_device, M, K, O, entries, spread):
 def test_table_contraction_takes_the_call(cuda_device):
     """A workspace of the per-cell plan runs the per-cell kernels: other roundings, the same result."""
     cfg = flash_cfg(4096)
-    x, wp, wn, g = _inputs(1024, 384, 1536, 0.2142, seed=1)
+    x, wp, wn, g = _inputs(2048, 384, 1536, 0.2142, seed=1)
     out, *grads = _run(x, wp, wn, g, cfg)
     cell = _per_cell(x, wp, wn, g, cfg)
     assert not torch.equal(out, cell)
@@ -145,7 +145,7 @@ def test_table_calls_that_do_not_suit(cuda_device, what):
     spread too far (a sample shows it, or, "outlier", one threshold that no sample holds), tables
     that are not smooth or too coarse, lookups past a table end, non-finite operands."""
     cfg = flash_cfg(2048 if what == "coarse" else 4096, **({"LUT_DTYPE": "bfloat16"} if what == "bf16" else {}))
-    x, wp, wn, g = _inputs(1024, 384, 1536, 5.0 if what == "spread" else 0.2142, seed=7)
+    x, wp, wn, g = _inputs(2048, 384, 1536, 5.0 if what == "spread" else 0.2142, seed=7)
     if what == "low":
         x[5, 7] = -7.9
     elif what == "high":
@@ -160,11 +160,11 @@ def test_table_calls_that_do_not_suit(cuda_device, what):
     cell = _per_cell(x, wp, wn, g, cfg)
     if what == "nan":
         assert torch.equal(torch.nan_to_num(out, 7.0), torch.nan_to_num(cell, 7.0)) and not torch.isfinite(gx[5, 7])
-        keep = torch.arange(1024, device="cuda") != 5
+        keep = torch.arange(2048, device="cuda") != 5
         assert torch.isfinite(out[keep]).all() and torch.isfinite(gx[keep]).all()
         return
     if what == "inf":
-        keep = torch.arange(1024, device="cuda") != 9
+        keep = torch.arange(2048, device="cuda") != 9
         assert torch.isfinite(gx[keep]).all() and not torch.isfinite(gx[9]).any()
         assert torch.isfinite(gp[4]).all() and not torch.isfinite(gp[3]).any()
         return
@@ -178,7 +178,7 @@ def test_table_contraction_with_glue(cuda_device):
     from isa.kernels.transformer_ffn import ops
 
     cfg = flash_cfg(4096)
-    M, K, O = 1025, 385, 1537
+    M, K, O = 2049, 385, 1537
     x, wp, wn, g = _inputs(M, K, O, 0.2142, seed=3, x_lo=-0.7, x_hi=1.0)
     fwd, bwd, n, lo, hi = _tables(cfg)
     aff = torch.tensor([2.0, 1.5], device="cuda")
@@ -200,7 +200,7 @@ def test_table_contraction_replays_from_a_graph(cuda_device):
     """A captured forward and backward, replayed with operands that change the number of terms and
     the path between the replays, equals the eager calls bitwise."""
     cfg = flash_cfg(4096)
-    static = _inputs(1024, 384, 1536, 0.2142, seed=9)
+    static = _inputs(2048, 384, 1536, 0.2142, seed=9)
     _tables(cfg)
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
@@ -215,7 +215,7 @@ def test_table_contraction_replays_from_a_graph(cuda_device):
         out = ops.lut_forward(*static[:3], fwd, n, lo, hi, V_SAT, -1e30, 1e30)
         grads = ops.lut_backward(*static, bwd, n, lo, hi, V_SAT, True, True)
     for spread in (0.2142, 0.8, 5.0, 0.2142):
-        for s, t in zip(static, _inputs(1024, 384, 1536, spread, seed=int(spread * 100))):
+        for s, t in zip(static, _inputs(2048, 384, 1536, spread, seed=int(spread * 100))):
             s.copy_(t)
         graph.replay()
         torch.cuda.synchronize()
