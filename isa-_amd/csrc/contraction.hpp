@@ -12,23 +12,25 @@
 //     dX[m, k]     = sum_j g_j(x[m, k]) H_j[m, k],  H_j = sum_o G[m, o] (T_j(t+) - T_j(t-))[o, k]
 //     dVth+-[o, k] = -+ sum_j T_j(t+-[o, k]) S_j,   S_j = sum_m G[m, o] (d_j r)[m, k]
 // with f' = sum_j d_j T_j and g_j = r (d_j - (r / V_sat) c_j): j = 0 cancels in the difference
-// of the branches. R terms cost R products per cell and direction where the cell itself costs
-// 32 (forward) or 52 (backward) VALU instructions, four or eight of them transcendental.
+// of the branches.
 //
-// Precision. Operands are kept to 22 bits as the sum of two f16 (hi + lo, scaled by a power of
-// two per row so that the row's largest value is near 2^12), and every product is formed as
-// hi hi + hi lo + lo hi in fp32 accumulators. The upper half of the terms is below 1e-3 of the
-// lower half (their coefficients fall like rho^-j; for the slope's own sum, dVth, 4e-3) and is
-// kept as single f16, 1e-7 of the result: 2 R products per cell instead of 3 R. (The formula's
-// dVth keeps all its terms as pairs: its error before was 3.5e-7.) The differences
-// T_j(t+) - T_j(t-) are formed in fp64 before they are rounded, so that a cell no longer loses the bits in which its two
-// branches agree. c_j, d_j and g_j come from tables over x built per call in fp64 (cubic
-// interpolation, step at most kSepStep of 2 n U_T: 2e-8 relative; the step is a power of two,
-// so that a position within a step is exact in fp32).
+// Precision. The coefficients grow by 2^50 and more from the lowest inputs to the highest ones, and which of them
+// count is G's and the thresholds' affair: the highest tokens may carry no gradient, the highest inputs may
+// have equal thresholds. So operands are kept to a relative precision, with fp32's exponents: as a sum of
+// bf16, three for the first terms (24 bits; six products a pair of operands: all but those below 2^-24),
+// two for the next (16 bits, three products), one for the last, whose coefficients are below 9e-2 and 4e-5
+// of the first one's. At 8 terms 2, 4 and 2 (dVth, whose first term has no counterpart in a difference, 4, 2
+// and 2): 26 (32) products per cell where the cell itself costs 32 (forward) or 52 (backward) VALU
+// instructions, four or eight of them transcendental; at 16 terms 52 (64). Only powers of two common to a
+// whole operand are taken out. The differences T_j(t+) - T_j(t-) are formed in fp64 before they are
+// rounded, so that a cell does not lose the bits in which its two branches agree; equal thresholds give zero.
+// c_j, d_j and g_j come from tables over x built per call in fp64 (cubic interpolation, step at most
+// kSepStep of 2 n U_T: 2e-8 relative; the step is a power of two, so that a position within a step is exact
+// in fp32). Emulated in float64, rows at one input: 2.6e-7 of the output's own scale forward, 3e-7 dVth.
 //
-// Measured (GPT-L layer 768 x 3072 at 2048 tokens, initial thresholds, R = 8): forward 4.30 ms
-// by the per-cell kernels, 0.30 ms here; backward 8.17 and 0.74 ms; error against float64 of
-// the forward 2.8e-6 and 2.6e-7, of dX 2.3e-6 and 3.4e-7, of dVth 3.5e-7 and 2.7e-7 (2-norm).
+// Measured (formula, 768 x 3072 at 2048 tokens, initial thresholds, R = 8): forward 4.29 ms by the per-cell
+// kernels, 0.32 ms here; backward 8.17 and 0.85 ms. (Operands as two f16, scaled by row, took 0.22 and
+// 0.52 ms, and lost everything 2^-36 below a row's largest value.)
 //
 // Tables. A lookup is the line between two entries, L(c) = F(c) + S(c) a (1 - a) / 2 with F the
 // smooth function through the entries, S its second difference and a the coordinate's fraction
@@ -36,17 +38,17 @@
 // With a (1 - a) = 1/6 - sum_q cos(2 pi q a) / (pi q)^2 and c = xs - ws,
 //     L(xs - ws) = (F + S / 12)(xs - ws)
 //                  - sum_q S(xs - ws) (cos 2 pi q xs cos 2 pi q ws + sin 2 pi q xs sin 2 pi q ws) / (2 pi^2 q^2):
-// the first part is smooth and expands as above, the others are 1e-5 of it and take R / 4 terms
-// of S per cosine and sine in plain f16. One harmonic keeps the forward's and dVth's remainder
-// below the per-cell kernels' own rounding of coordinates and of the records' intercepts up to
-// growths of 3.3% from entry to entry (about 3900 entries), and dX's, which they round less, up to
-// 2.2% (about 6000); coarser tables take two, finer ones than about 14000 entries none. 2-norm
-// against float64 lookups, initial thresholds, per-cell kernels against this: 4096 entries forward
-// 9.8e-6 and 3.8e-6, dX 5.4e-6 and 3.2e-6, dVth 1.1e-6 and 8.1e-7; 5500 entries 9.1e-6 and 2.1e-6,
-// 5.2e-6 and 1.7e-6, 1.2e-6 and 4.8e-7; 8192 entries 7.8e-6 and 9.9e-7, 5.6e-6 and 1.5e-6, 1.3e-6
-// and 2.9e-7 (over 0.5 and 1 V also smaller, closest for
-// dVth over 1 V at 4096 entries, 1.7e-6 and 1.6e-6). With two harmonics throughout 768 -> 3072
-// at 8192 tokens took 1.06 ms forward and 2.47 backward, with one 0.92 and 2.35. Sums of T's
+// the first part is smooth and expands as above, the others are 1e-4 of it. S falls with the threshold as the
+// current does where the transistor is in weak inversion (there the kinks count most), more slowly or not at
+// all above: it is a combination of two exponentials in t, fitted per point of the x table (what they leave
+// is 2e-6 of a current's difference, 5e-6 of a slope's). So a harmonic is four values per input, one bf16
+// each. As many harmonics are summed as leave less than the per-cell kernels round, row by row: four at 4096
+// entries, two at 8192, one at 16384. Errors of a row's own scale, all inputs of it at one voltage, the largest
+// over -1 to 3.8 V, per-cell kernels against this: 4096 entries forward 6.9e-6 and 3.6e-6, dX 1.5e-5 and
+// 1.2e-5, dVth 5.0e-6 and 2.1e-6; 8192 entries 6.9e-6 and 2.1e-6, 1.9e-5 and 7.4e-6, 5.1e-6 and 1.3e-6; over
+// 1.06 V at 8192 entries 4.5e-6 and 1.2e-6, 4.7e-6 and 1.7e-6, 5.0e-6 and 1.2e-6. 768 x 3072 at 8192 tokens,
+// forward / backward, per-cell kernels against this: 4096 entries 4.35 / 8.65 ms and 1.68 / 4.05, 8192 entries
+// 4.69 / 9.32 and 1.37 / 3.47; over 1 V the forward at 4096 entries 4.58 and 2.60. Sums of T's
 // differences give back the entries exactly. A table that is not smooth (bf16 entries) runs the
 // per-cell kernels.
 //
@@ -54,33 +56,32 @@
 // operands do not suit (non-finite values, x near -V_sat or spread over more than the table
 // holds, thresholds spread too far) runs the per-cell kernels, which return at once otherwise.
 
-typedef _Float16 sep_h8 __attribute__((ext_vector_type(8)));
-typedef _Float16 sep_h4 __attribute__((ext_vector_type(4)));
-typedef _Float16 sep_h2 __attribute__((ext_vector_type(2)));
+typedef __bf16 sep_b8 __attribute__((ext_vector_type(8)));
+typedef __bf16 sep_b4 __attribute__((ext_vector_type(4)));
+typedef __bf16 sep_b2 __attribute__((ext_vector_type(2)));
 typedef float sep_f16 __attribute__((ext_vector_type(16)));
-typedef unsigned sep_u4 __attribute__((ext_vector_type(4)));
 
 constexpr int kSepStatX = 1024, kSepStatW = 256;  // blocks of the ranges of x and of the thresholds
-constexpr int kSepStatG = 512;          // blocks of the largest |G| of each row
-constexpr int kSepColChunks = 64;       // row chunks of a column pass, at most
+constexpr int kSepStatG = 512;          // blocks of the largest |G|
 constexpr int kSepGridMax = 16384;      // x-table points, at most
 constexpr double kSepStep = 0.0148;     // x-table step in units of 2 n U_T
 constexpr int kSepMaxTerms = 16;
-constexpr int kSepLutMin = 2900, kSepLutMax = 65536;  // table entries: the kinks small enough, a thread per partial
-constexpr float kSepQScale = 256.0f;    // of the threshold-side operand (values in [-2, 2])
+constexpr int kSepLutMin = 3600, kSepLutMax = 65536;  // table entries: the kinks small enough, a thread per partial
+constexpr int kSepMaxHarmonics = 4;
 
 // Widest threshold spread, in units of 2 n U_T, that R = 8 and 16 terms take: there the
-// truncation is 1e-7 of the gradients (the forward's is ten times smaller). More would converge
+// truncation is 2e-7 of the gradients (the forward's is ten times smaller). More would converge
 // (16 terms to 4.4), but as the spread grows the per-cell kernels lose fewer bits to the branches'
-// difference while the sums here have more terms: 2-norm against float64, 768 x 768 at 1900
-// tokens, per-cell kernels against this, forward and dVth: 0.2142 V 2.8e-6 and 2.1e-7, 3.6e-7 and
-// 2.5e-7; 0.3 V (1.4 units) 8.2e-7 and 3.7e-7, 3.0e-7 and 3.0e-7; 0.9 V 4.2e-7 and 4.2e-7, 3.1e-7
-// and 3.3e-7. The formula goes over to the per-cell kernels where dVth's errors meet.
+// difference while the sums here have more terms. Own scales, tokens of all magnitudes, 192 x 768 at 3700
+// tokens: 0.2142 V forward 2.7e-7, dX 4.3e-7, dVth 2.1e-7; 0.3 V 1.9e-7, 2.0e-7, 1.8e-7.
 __host__ __device__ inline int sep_terms(float spread_u) { return spread_u <= 1.12f ? 8 : spread_u <= 1.45f ? 16 : 0; }
 
-// Table calls: the lookups round more (over 1 V, 4.7 units, forward 2.7e-6 and 1.8e-6, dVth 1.7e-6
-// and 1.6e-6 at 4096 entries), and 32 terms would cost what the lookups do.
-__host__ __device__ inline int sep_terms_lut(float spread_u) { return spread_u <= 1.12f ? 8 : spread_u <= 5.0f ? 16 : 0; }
+// Table calls. Two functions a harmonic fit the currents' second differences to 2e-6 of a lookup's
+// difference over spreads up to 5 units, the slopes' to 5e-6 up to 1.45 units and, as growth^2, to what
+// the per-cell kernels round (2.5e-6) over wider ones where entries grow by at most 2.06%.
+__host__ __device__ inline int sep_terms_lut(float spread_u, float growth, bool backward) {
+    return spread_u <= 1.12f ? 8 : spread_u <= (backward && growth > 0.0206f ? 1.45f : 5.0f) ? 16 : 0;
+}
 
 // What the passes of a call share, in its workspace.
 struct SepHead {
@@ -88,12 +89,14 @@ struct SepHead {
     unsigned gmax;  // backward: bits of the largest |G|: not finite: the per-cell kernels run
     int rough;    // 1: the series does not converge as its terms assume, 2: a sample of the thresholds or of
                   // the table ruled the contraction out (then the other fields are not set): the per-cell kernels run
-    int harmonics, harmonics_dx;  // of the table's kinks that are summed (0 to 2): forward and dVth, dX
+    int harmonics;  // of the table's kinks that are summed: 0, 1, 2 or 4
     int n_grid;
     float xlo, xhi, wlo, whi;
     float lut_min, lut_scale;  // table coordinate (v - lut_min) * lut_scale
     float x0, step, inv_step; // table point i stands for x0 + i * step; step a power of two, x0 a multiple of it
     double wc, inv_wh, wh;   // t = (w - wc) * inv_wh
+    float gw, gu;             // second differences are combinations of exp(gw t) and exp(gu t)
+    float scale, inv_scale;   // of the x tables, a power of two: the largest current is near 2^60
 };
 
 __device__ bool sep_takes(const SepHead* head) {
@@ -118,31 +121,23 @@ struct SepArgs {
     int lut_n;
     double lut_min, lut_scale;
     double2* lut_val;        // [lut_n]: smooth part, second difference
-    float2* lut_info;        // per 256 entries {largest relative growth from entry to entry, 1 where they do not suit}
-    float* tabE;             // second difference's coefficients, -r e_i / (2 pi^2): [n_grid][R / 4]
+    float4* lut_info;        // per 256 entries {largest relative growth from entry to entry, 1 where they do not suit, largest |entry|, 0}
+    float* tabE;             // second difference's coefficients, -r e_i / (2 pi^2), scaled: [n_grid][2]
     // workspace
     SepHead* head;
     float2* xpart;           // [kSepStatX]
     float2* wpart;           // [kSepStatW]
-    float2* xrow;            // forward: [M] row ranges of x
-    float2* xcol;            // backward: [kSepColChunks][K]
-    unsigned* grow;          // backward: [M] largest |G| of a row (bits)
-    unsigned* gcol;          // backward: [kSepColChunks][O]
-    float* tab;              // forward c_j r (j = 1..R), backward d_j r (j = 0..R-1): [n_grid][R]
+    float* tab;              // forward c_j r (j = 1..R), backward d_j r (j = 0..R-1), scaled: [n_grid][R]
     float* tab2;             // backward g_j (j = 1..R)
-    _Float16* xop;           // forward [M][Kd], backward (pairs, lower terms) [rows][Md]
-    _Float16* wop;           // forward [O][Kd], backward [rows][Od]
-    _Float16* xops;          // backward, upper terms, singles: [rows][Md]
-    _Float16* wops;          // [rows][Od]
-    _Float16* xoph;          // backward, harmonics, singles: [rows][Md]
-    _Float16* woph;          // [rows][Od]
-    _Float16* gop;           // backward, pairs: [M][Od]
-    _Float16* gopT;          // [O][Md]
-    _Float16* goph;          // backward, singles: [M][Od]
-    _Float16* gophT;         // [O][Md]
-    float* xscale;           // forward [M], backward [K]: inverse scale of xop's rows
-    float* gscale;           // backward [M]
-    float* gscaleT;          // backward [O]
+    char* xop;               // forward [M] rows
+    char* wop;               // forward [O] rows
+    // backward, by parts {singles, pairs, triples} and the harmonics: rows of inputs and terms
+    char* xcls[4];           // over the tokens
+    char* wcls[4];           // over the outputs
+    char* gop;               // triples: [M] rows over the outputs
+    char* gops;              // singles
+    char* gopT;              // triples: [O] rows over the tokens
+    char* gopTs;             // singles
     float2* tT;              // backward [K][Op]: {t+, t-}
     int64_t Op;
     int need_x, need_w;
@@ -152,31 +147,52 @@ __device__ inline float sep_input(const SepArgs& a, float x, float s, float b) {
     return a.in_affine ? input_map(x, s, b, a.in_lo, a.in_hi) : x;
 }
 
-// Layouts. An operand's row is a run of slabs of 128 bytes: 32 inner elements as pairs (their hi
-// halves, then their lo halves) or 64 single f16.
-// Forward, a row's inner elements: the lower terms as pairs, ordered (j / 4, k, j % 4), the
-// upper ones as singles likewise, then (tables) the harmonics as singles; inputs padded to 16.
-// Backward, tokens or outputs inside, rows in blocks of eight: four terms of an even input and of
-// the odd one after it, so that a lane of the matrix cores' result holds one input's. The lower
-// terms, the upper ones and the harmonics are operands of their own.
-// Harmonics: an input has R values in blocks of four, at 8 terms of each harmonic its two cosines
-// and two sines, at 16 the first one's four cosines, its four sines, then the second one's.
-__host__ __device__ inline int64_t sep_inputs(int64_t K) { return (K + 15) / 16 * 16; }
-__host__ __device__ inline int64_t sep_slabs_pairs(int64_t K, int terms) { return sep_inputs(K) * (terms / 2) / 32; }
-__host__ __device__ inline int64_t sep_slabs_singles(int64_t K, int terms, int harmonics) {
-    return sep_inputs(K) * (terms / 2 + harmonics * terms / 2) / 64;
+// Layouts. An operand's values are kept as one, two or three bf16 (the value, what rounding it left,
+// what rounding that left), in runs of 16 inner elements: all first parts, then the second parts, then
+// the third ones, 32 bytes each. The matrix kernel reads an operand's row in slabs of up to 128 bytes:
+// 64 singles, 32 pairs, 16 triples.
+// Forward, a row's inner elements: the singles (the last terms, then the harmonics), the pairs and the
+// triples (the first terms): the small terms are summed first. Inputs are padded to 32. Terms are
+// ordered (term / 4, input, term % 4), where a class has two (input, term).
+// Backward, tokens or outputs inside, padded to 64, an operand per class; rows in blocks of eight: four
+// terms of an even input and of the odd one after it, or where a class has two terms those of two inputs
+// and of the next two, so that a lane of the matrix cores' result holds whole inputs.
+// Harmonics: an input has four values for each, two coefficients times its cosine, two times its sine.
+struct SepClasses {
+    int n3, n2, n1;  // terms kept as triples, pairs and singles, in this order
+    __host__ __device__ constexpr int first(int parts) const { return parts == 3 ? 0 : parts == 2 ? n3 : n3 + n2; }
+    __host__ __device__ constexpr int count(int parts) const { return parts == 3 ? n3 : parts == 2 ? n2 : n1; }
+};
+// The forward's and dX's terms, and dVth's (whose first one, j = 0, has no counterpart in a difference).
+__host__ __device__ constexpr SepClasses sep_classes(int terms, bool dv) {
+    return terms == 8 ? (dv ? SepClasses{4, 2, 2} : SepClasses{2, 4, 2}) : (dv ? SepClasses{8, 4, 4} : SepClasses{4, 8, 4});
 }
-__host__ __device__ inline int64_t sep_slabs(int64_t n) { return (n + 31) / 32; }
-__host__ __device__ inline int64_t sep_slabs64(int64_t n) { return (n + 63) / 64; }
-// Row of input k's value v (of its `per`) among the backward's rows.
-__host__ __device__ inline int64_t sep_row(int64_t k, int per, int v) {
-    return ((k >> 1) * (per / 4) + (v >> 2)) * 8 + (k & 1) * 4 + (v & 3);
+__host__ __device__ inline int64_t sep_inputs(int64_t K) { return (K + 31) / 32 * 32; }
+__host__ __device__ inline int64_t sep_inner(int64_t n) { return (n + 63) / 64 * 64; }
+// Byte offsets of the parts of a forward row, and its bytes.
+struct SepRow {
+    int64_t harm, pairs, triples, bytes;
+    __host__ __device__ SepRow(int64_t K, int terms, int harmonics) {
+        const SepClasses c = sep_classes(terms, false);
+        const int64_t kc = sep_inputs(K);
+        harm = kc * c.n1 * 2;
+        pairs = harm + kc * harmonics * 8;
+        triples = pairs + kc * c.n2 * 4;
+        bytes = triples + kc * c.n3 * 6;
+    }
+};
+// Row of input k's value v of its `count` among a backward class's rows; the rows that hold K inputs.
+__host__ __device__ inline int64_t sep_row(int64_t k, int count, int v) {
+    return count == 2 ? (k >> 2) * 8 + (k & 3) * 2 + v
+                      : ((k >> 1) * (count / 4) + (v >> 2)) * 8 + (k & 1) * 4 + (v & 3);
+}
+__host__ __device__ inline int64_t sep_rows(int64_t K, int count) {
+    return count == 2 ? (K + 3) / 4 * 8 : (K + 1) / 2 * 2 * count;
 }
 
 // ----------------------------------------------------------------------------------
-// Statistics: ranges of x (per row forward, per column backward), of the thresholds, and the
-// largest |G| of each row and column. NaN makes a range infinite and a maximum non-finite.
-// HBM-bound: x, the thresholds and G are read once (G and, with both gradients, twice).
+// Statistics: ranges of x and of the thresholds, and the largest |G|. NaN makes a range infinite
+// and a maximum non-finite. HBM-bound: x, the thresholds and G are read once.
 // ----------------------------------------------------------------------------------
 
 __device__ inline void sep_minmax(float v, float& lo, float& hi) {
@@ -201,7 +217,7 @@ __device__ inline void sep_lut_block(const SepArgs& a, int b) {
     constexpr int kHalo = 2, kSpan = 256 + 2 * kHalo;
     __shared__ double s_t[kSpan];
     __shared__ double s_sum[4];
-    __shared__ float s_growth[4];
+    __shared__ float s_growth[4], s_big[4];
     __shared__ int s_bad;
     const int t = threadIdx.x, n = a.lut_n;
     const bool bwd = a.tab2 != nullptr;
@@ -245,11 +261,19 @@ __device__ inline void sep_lut_block(const SepArgs& a, int b) {
     }
     if (j < n) a.lut_val[j] = make_double2(s_t[i] + second / 12.0, second);
     if (bad) atomicOr(&s_bad, 1);
-    for (int d = 32; d > 0; d >>= 1) growth = fmaxf(growth, __shfl_xor(growth, d));
-    if ((t & 63) == 0) s_growth[t >> 6] = growth;
+    float big = j < n ? fabsf((float)s_t[i]) : 0.0f;
+    for (int d = 32; d > 0; d >>= 1) {
+        growth = fmaxf(growth, __shfl_xor(growth, d));
+        big = fmaxf(big, __shfl_xor(big, d));
+    }
+    if ((t & 63) == 0) {
+        s_growth[t >> 6] = growth;
+        s_big[t >> 6] = big;
+    }
     __syncthreads();
     if (t == 0)
-        a.lut_info[b] = make_float2(fmaxf(fmaxf(s_growth[0], s_growth[1]), fmaxf(s_growth[2], s_growth[3])), (float)s_bad);
+        a.lut_info[b] = make_float4(fmaxf(fmaxf(s_growth[0], s_growth[1]), fmaxf(s_growth[2], s_growth[3])), (float)s_bad,
+                                    fmaxf(fmaxf(s_big[0], s_big[1]), fmaxf(s_big[2], s_big[3])), 0.0f);
 }
 
 __device__ inline unsigned sep_bits(float v) { return __float_as_uint(v) & 0x7fffffffu; }
@@ -268,6 +292,7 @@ __device__ inline bool sep_sample_refuses(const SepArgs& a) {
     const uint64_t f = (((((uint64_t)place * 0x9e3779b97f4a7c15u) >> 32) * (n - 3)) >> 32) + off;
     const float wp = a.wp[f], wn = a.wn[f];
     double ua = a.a;
+    float growth_all = 0.0f;
     bool bad = false;
     if (a.lut_n > 0) {
         const bool bwd = a.tab2 != nullptr;  // entries {A, dT}, backward the slope table's
@@ -279,25 +304,25 @@ __device__ inline bool sep_sample_refuses(const SepArgs& a) {
         bad = !(fabs((d3 - d0) - 3.0 * (d2 - d1)) <= 4e-6 * fabs(v) + 2e-42);
         float growth = v > 1e-30 ? (float)(d2 / v) : 0.0f;
         for (int d = 32; d > 0; d >>= 1) growth = fmaxf(growth, __shfl_xor(growth, d));
-        ua = 0.5 * 0.999 * (double)growth * a.lut_scale;
+        growth_all = 0.999f * growth;
+        ua = 0.5 * (double)growth_all * a.lut_scale;
     }
     sep_minmax(wp, lo, hi);
     sep_minmax(wn, lo, hi);
     sep_wave_minmax(lo, hi);
     const float spread = (float)(((double)hi - (double)lo) * ua);
-    const int terms = a.lut_n > 0 ? sep_terms_lut(spread) : sep_terms(spread);
+    const int terms = a.lut_n > 0 ? sep_terms_lut(spread, growth_all, a.tab2 != nullptr) : sep_terms(spread);
     return __builtin_amdgcn_readfirstlane((int)(__any(bad) || terms == 0 || terms > a.max_terms)) != 0;
 }
 
-// Blocks: kSepStatX of x, kSepStatW of the thresholds, (xcol) kSepColChunks x ceil(K / 256) of
-// x's columns, ceil(lut_n / 256) of the table, then the layer glue's gradient blocks (glue.geff).
+// Blocks: kSepStatX of x, kSepStatW of the thresholds, ceil(lut_n / 256) of the table, then the
+// layer glue's gradient blocks (glue.geff).
 __global__ __launch_bounds__(256) void sep_stat_kernel(SepArgs a, PrepArgs prep, GlueGradArgs glue) {
     int b = blockIdx.x;
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int t = threadIdx.x;
     const float as = a.in_affine ? a.in_affine[0] : 1.0f, ab = a.in_affine ? a.in_affine[1] : 0.0f;
     const int lut_blocks = (a.lut_n + 255) / 256;
-    const int xcols = a.xcol ? kSepColChunks * (int)((a.K + 255) / 256) : 0;
-    if (b < kSepStatX + kSepStatW + lut_blocks + xcols) {
+    if (b < kSepStatX + kSepStatW + lut_blocks) {
         const bool refuses = sep_sample_refuses(a);
         if (b == 0 && t == 0) {
             a.head->gmax = 0;
@@ -312,31 +337,13 @@ __global__ __launch_bounds__(256) void sep_stat_kernel(SepArgs a, PrepArgs prep,
     }
     if (b < kSepStatX) {
         float lo = INFINITY, hi = -INFINITY;
-        if (a.xrow) {  // a wave per row
-            for (int64_t m = (int64_t)b * 4 + wave; m < a.M; m += (int64_t)kSepStatX * 4) {
-                float l = INFINITY, h = -INFINITY;
-                const float* row = a.x + m * a.K;
-                for (int64_t k = lane; k < a.K; k += 256) {
-                    float v[4];
+        const int64_t n = a.M * a.K, stride = (int64_t)kSepStatX * 256;
+        for (int64_t e = (int64_t)b * 256 + t; e < n; e += 4 * stride) {
+            float v[4];
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) v[q] = row[k + q * 64 < a.K ? k + q * 64 : k];
+            for (int q = 0; q < 4; ++q) v[q] = a.x[e + q * stride < n ? e + q * stride : e];
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) sep_minmax(sep_input(a, v[q], as, ab), l, h);
-                }
-                sep_wave_minmax(l, h);
-                if (lane == 0) a.xrow[m] = make_float2(l, h);
-                lo = fminf(lo, l);
-                hi = fmaxf(hi, h);
-            }
-        } else {
-            const int64_t n = a.M * a.K, stride = (int64_t)kSepStatX * 256;
-            for (int64_t e = (int64_t)b * 256 + t; e < n; e += 4 * stride) {
-                float v[4];
-#pragma unroll
-                for (int q = 0; q < 4; ++q) v[q] = a.x[e + q * stride < n ? e + q * stride : e];
-#pragma unroll
-                for (int q = 0; q < 4; ++q) sep_minmax(sep_input(a, v[q], as, ab), lo, hi);
-            }
+            for (int q = 0; q < 4; ++q) sep_minmax(sep_input(a, v[q], as, ab), lo, hi);
         }
         block_minmax(lo, hi, &a.xpart[b]);
         return;
@@ -365,58 +372,29 @@ __global__ __launch_bounds__(256) void sep_stat_kernel(SepArgs a, PrepArgs prep,
         return;
     }
     b -= lut_blocks;
-    if (b < xcols) {
-        const int64_t rows = (a.M + kSepColChunks - 1) / kSepColChunks;
-        const int chunk = b % kSepColChunks;
-        const int64_t col = (int64_t)(b / kSepColChunks) * 256 + t;
-        const int64_t m0 = chunk * rows, m1 = m0 + rows < a.M ? m0 + rows : a.M;
-        if (col >= a.K) return;
-        float lo = INFINITY, hi = -INFINITY;
-#pragma unroll 8
-        for (int64_t m = m0; m < m1; ++m) sep_minmax(sep_input(a, a.x[m * a.K + col], as, ab), lo, hi);
-        a.xcol[(int64_t)chunk * a.K + col] = make_float2(lo, hi);
-        return;
-    }
-    b -= xcols;
     glue_grad_block(glue, b % kGlueBlocks, b / kGlueBlocks, (int)(glue.Op / 256));
 }
 
-// The largest |G| of a row or column (blocks of the table kernel's launch).
+// The largest |G| (blocks of the table kernel's launch, a wave per row of G).
 __device__ inline void sep_grad_block(const SepArgs& a, int b) {
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    if (b < kSepStatG) {
-        unsigned all = 0;
-        for (int64_t m = (int64_t)b * 4 + wave; m < a.M; m += (int64_t)kSepStatG * 4) {
-            unsigned h = 0;
-            const float* row = a.g + m * a.ldg;
-            for (int64_t o = lane; o < a.O; o += 256) {
-                unsigned v[4];
+    unsigned all = 0;
+    for (int64_t m = (int64_t)b * 4 + wave; m < a.M; m += (int64_t)kSepStatG * 4) {
+        const float* row = a.g + m * a.ldg;
+        for (int64_t o = lane; o < a.O; o += 256) {
+            unsigned v[4];
 #pragma unroll
-                for (int q = 0; q < 4; ++q) v[q] = sep_bits(row[o + q * 64 < a.O ? o + q * 64 : o]);
-                h = max(h, max(max(v[0], v[1]), max(v[2], v[3])));
-            }
-            for (int d = 32; d > 0; d >>= 1) h = max(h, (unsigned)__shfl_xor((int)h, d));
-            if (lane == 0) a.grow[m] = h;
-            all = max(all, h);
+            for (int q = 0; q < 4; ++q) v[q] = sep_bits(row[o + q * 64 < a.O ? o + q * 64 : o]);
+            all = max(all, max(max(v[0], v[1]), max(v[2], v[3])));
         }
-        __shared__ unsigned s_all;  // one atomic per block: they all meet at one address
-        if (t == 0) s_all = 0;
-        __syncthreads();
-        if (lane == 0) atomicMax(&s_all, all);
-        __syncthreads();
-        if (t == 0) atomicMax(&a.head->gmax, s_all);
-        return;
     }
-    b -= kSepStatG;
-    const int64_t rows = (a.M + kSepColChunks - 1) / kSepColChunks;
-    const int chunk = b % kSepColChunks;
-    const int64_t col = (int64_t)(b / kSepColChunks) * 256 + t;
-    const int64_t m0 = chunk * rows, m1 = m0 + rows < a.M ? m0 + rows : a.M;
-    if (col >= a.O) return;
-    unsigned h = 0;
-#pragma unroll 8
-    for (int64_t m = m0; m < m1; ++m) h = max(h, sep_bits(a.g[m * a.ldg + col]));
-    a.gcol[(int64_t)chunk * a.O + col] = h;
+    for (int d = 32; d > 0; d >>= 1) all = max(all, (unsigned)__shfl_xor((int)all, d));
+    __shared__ unsigned s_all;  // one atomic per block: they all meet at one address
+    if (t == 0) s_all = 0;
+    __syncthreads();
+    if (lane == 0) atomicMax(&s_all, all);
+    __syncthreads();
+    if (t == 0) atomicMax(&a.head->gmax, s_all);
 }
 
 // ----------------------------------------------------------------------------------
@@ -452,12 +430,11 @@ __device__ inline double sep_lut_second(const double2* val, int n, double c) {
 
 constexpr int kSepTableBlocks = 256;
 
-// Blocks: kSepTableBlocks of the tables, then (g) kSepStatG of G's rows and kSepColChunks x
-// ceil(O / 256) of its columns.
+// Blocks: kSepTableBlocks of the tables, then (backward) kSepStatG of G.
 __global__ __launch_bounds__(256) void sep_table_kernel(SepArgs a) {
-    __shared__ float2 s_x, s_w, s_info;
+    __shared__ float2 s_x, s_w, s_info, s_big;
     __shared__ SepHead s_head;
-    __shared__ double s_cos[4 * kSepMaxTerms], s_val[256], s_sec[256], s_d[256];
+    __shared__ double s_cos[4 * kSepMaxTerms], s_val[256], s_sec[256], s_d[256], s_fit[4][kSepMaxTerms];
     const int t = threadIdx.x;
     const bool lut = a.lut_n > 0;
     // (other blocks of this launch set rough to 1, never to 2)
@@ -472,12 +449,14 @@ __global__ __launch_bounds__(256) void sep_table_kernel(SepArgs a) {
         }
         const float2 w = a.wpart[t];
         static_assert(kSepStatW == 256 && kSepLutMax <= 256 * 256, "a thread per partial");
-        const float2 info = t * 256 < a.lut_n ? a.lut_info[t] : make_float2(0.0f, 0.0f);
+        const float4 info = t * 256 < a.lut_n ? a.lut_info[t] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         block_minmax(lo, hi, &s_x);
         __syncthreads();
         block_minmax(w.x, w.y, &s_w);
         __syncthreads();
         block_minmax(-info.y, info.x, &s_info);  // (-1 where some do not suit, growth)
+        __syncthreads();
+        block_minmax(0.0f, info.z, &s_big);
         __syncthreads();
     }
     if (t == 0) {
@@ -492,14 +471,16 @@ __global__ __launch_bounds__(256) void sep_table_kernel(SepArgs a) {
         const double points = floor((double)xhi / step) - first + 3.0;
         const bool finite = xlo > -1e30f && xhi < 1e30f && wlo > -1e30f && whi < 1e30f;
         const float spread = (float)(((double)whi - (double)wlo) * ua);
-        const int terms = lut ? sep_terms_lut(spread) : sep_terms(spread);
+        const int terms = lut ? sep_terms_lut(spread, (float)growth, a.tab2 != nullptr) : sep_terms(spread);
         bool ok = finite && terms > 0 && terms <= a.max_terms && rlo > 0.1 && rhi > 0.1 &&
                   points <= (double)kSepGridMax && fmax(fabs((double)xlo), fabs((double)xhi)) < step * (1 << 23);
         if (lut) {  // every lookup inside the table, the x table's margin included
-            h.harmonics = growth > 0.033 ? 2 : growth > 0.009 ? 1 : 0;
-            h.harmonics_dx = growth > 0.022 ? 2 : h.harmonics;
+            // root mean square of the harmonics left out, in records: 0.0373 growth without any, 0.0103
+            // after one, 0.0050 after two, 0.0021 after four; the per-cell kernels round to about 1e-4
+            const double left = 7.7e-5;
+            h.harmonics = 0.0373 * growth <= left ? 0 : 0.0103 * growth <= left ? 1 : 0.0050 * growth <= left ? 2 : 4;
             const double margin = 4.0 * step * a.lut_scale + 4.0;
-            ok = ok && s_info.x == 0.0f && growth > 1e-6 && growth < 0.045 &&
+            ok = ok && s_info.x == 0.0f && growth > 1e-6 && 0.0021 * growth <= left &&
                  ((double)xlo - (double)whi - a.lut_min) * a.lut_scale >= margin &&
                  ((double)xhi - (double)wlo - a.lut_min) * a.lut_scale <= (double)(a.lut_n - 1) - margin;
             h.lut_min = (float)a.lut_min;
@@ -517,6 +498,14 @@ __global__ __launch_bounds__(256) void sep_table_kernel(SepArgs a) {
             h.wc = 0.5 * ((double)wlo + (double)whi);
             h.wh = fmax(0.5 * ((double)whi - (double)wlo), 1e-3 / ua);
             h.inv_wh = 1.0 / h.wh;
+            // below threshold they fall with the threshold as the current does; above it the currents' as
+            // its root, the slopes' rise. (Narrow spreads: exponents far enough apart to be told apart.)
+            h.gw = lut ? -fmaxf((float)(log1p(growth) * a.lut_scale * h.wh), 0.25f) : 0.0f;
+            h.gu = a.tab2 ? -0.5f * h.gw : 0.5f * h.gw;
+            int e = 60;
+            if (lut && s_big.y > 0.0f) e = max(-120, min(120, 60 - ilogbf(s_big.y)));
+            h.scale = ldexpf(1.0f, e);
+            h.inv_scale = ldexpf(1.0f, -e);
         }
         h.xlo = xlo;
         h.xhi = xhi;
@@ -527,7 +516,6 @@ __global__ __launch_bounds__(256) void sep_table_kernel(SepArgs a) {
             SepHead* g = a.head;
             g->terms = h.terms;
             g->harmonics = h.harmonics;
-            g->harmonics_dx = h.harmonics_dx;
             g->n_grid = h.n_grid;
             g->xlo = xlo;
             g->xhi = xhi;
@@ -541,6 +529,10 @@ __global__ __launch_bounds__(256) void sep_table_kernel(SepArgs a) {
             g->wc = h.wc;
             g->inv_wh = h.inv_wh;
             g->wh = h.wh;
+            g->gw = h.gw;
+            g->gu = h.gu;
+            g->scale = h.scale;
+            g->inv_scale = h.inv_scale;
         }
     }
     __syncthreads();
@@ -552,6 +544,25 @@ __global__ __launch_bounds__(256) void sep_table_kernel(SepArgs a) {
         return;
     }
     for (int q = t; q < 4 * R; q += 256) s_cos[q] = cospi((double)q / (2.0 * R));
+    if (h.harmonics > 0) {  // least squares over the Chebyshev points: e = s_fit[0..1] S, of s_fit[2..3]
+        __syncthreads();
+        if (t < R) {
+            s_fit[2][t] = exp((double)h.gw * s_cos[2 * t + 1]);
+            s_fit[3][t] = exp((double)h.gu * s_cos[2 * t + 1]);
+        }
+        __syncthreads();
+        if (t < R) {
+            double aa = 0.0, ab = 0.0, bb = 0.0;
+            for (int q = 0; q < R; ++q) {
+                aa += s_fit[2][q] * s_fit[2][q];
+                ab += s_fit[2][q] * s_fit[3][q];
+                bb += s_fit[3][q] * s_fit[3][q];
+            }
+            const double det = aa * bb - ab * ab;
+            s_fit[0][t] = (bb * s_fit[2][t] - ab * s_fit[3][t]) / det;
+            s_fit[1][t] = (aa * s_fit[3][t] - ab * s_fit[2][t]) / det;
+        }
+    }
     // a block takes 256 / R points at a time: a thread per (point, Chebyshev point), then per
     // (point, j)
     const int per = 256 / R, pl = t / R, n = t - pl * R;
@@ -579,34 +590,47 @@ __global__ __launch_bounds__(256) void sep_table_kernel(SepArgs a) {
         if (direct && j == R) d = 0.0;
         s_d[t] = d;
         double e2 = 0.0;
-        if (h.harmonics > 0 && n < R / 4) {
-            for (int q = 0; q < R; ++q) e2 += s_sec[pl * R + q] * s_cos[(n * (2 * q + 1)) % (4 * R)];
-            e2 *= (n == 0 ? 1.0 : 2.0) / R;
-        }
+        if (h.harmonics > 0 && n < 2)
+            for (int q = 0; q < R; ++q) e2 += s_sec[pl * R + q] * s_fit[n][q];
         __syncthreads();
         if (i0 + pl < h.n_grid) {
             const size_t e = (size_t)(i0 + pl) * R + n;
             if (direct) {
-                a.tab[e] = (float)(d * r);
+                a.tab[e] = (float)(d * r * (double)h.scale);
             } else {  // c_j from d_(j-1) = d and d_(j+1)
                 const double d_next = j < R ? s_d[t + 1] : 0.0, d_after = j + 1 < R ? s_d[t + 2] : 0.0;
                 const double c = -h.wh / (2.0 * j) * (d - d_after);
                 if (a.tab2) {
-                    a.tab[e] = (float)((n == 0 ? 0.5 * d : d) * r);
+                    a.tab[e] = (float)((n == 0 ? 0.5 * d : d) * r * (double)h.scale);
                     a.tab2[e] = (float)(r * (d_next - r / a.v_sat * c));
                 } else {
-                    a.tab[e] = (float)(c * r);
+                    a.tab[e] = (float)(c * r * (double)h.scale);
                 }
             }
-            if (h.harmonics > 0 && n < R / 4)
-                a.tabE[(size_t)(i0 + pl) * (R / 4) + n] = (float)(-r * e2 * 0.050660591821168886);  // 1 / (2 pi^2)
+            if (h.harmonics > 0 && n < 2)
+                a.tabE[(size_t)(i0 + pl) * 2 + n] = (float)(-r * e2 * 0.050660591821168886 * (double)h.scale);  // 1 / (2 pi^2)
             // the last coefficients of a table that grows otherwise than its steepest part says
             if (lut && n == 0) {
                 const int last = direct ? R - 2 : R - 1;  // of degree R - 1
                 double big = 0.0;
                 for (int q = direct ? 0 : 1; q < R; ++q) big = fmax(big, fabs(s_d[t + q]));
                 const double mean = direct ? 0.0 : fabs(0.5 * s_d[t]);
-                if (!(fabs(s_d[t + last]) <= 2e-5 * big + 2e-6 * mean + 1e-35)) atomicOr(&a.head->rough, 1);
+                if (!(fabs(s_d[t + last]) <= 1e-5 * big + 1e-6 * mean + 1e-35)) atomicOr(&a.head->rough, 1);
+            }
+            // or second differences that the two functions do not fit
+            if (h.harmonics > 0 && n == 2) {
+                double big = 0.0, e0 = 0.0, e1 = 0.0, left = 0.0;
+                for (int q = 0; q < R; ++q) {
+                    e0 += s_sec[pl * R + q] * s_fit[0][q];
+                    e1 += s_sec[pl * R + q] * s_fit[1][q];
+                }
+                for (int q = 0; q < R; ++q) {
+                    const double u = s_sec[pl * R + q] - e0 * s_fit[2][q] - e1 * s_fit[3][q];
+                    left += u * u;
+                }
+                for (int q = direct ? 0 : 1; q < R; ++q) big = fmax(big, fabs(s_d[t - 2 + q]));
+                const double mean = direct ? 0.0 : fabs(0.5 * s_d[t - 2]);
+                if (!(0.05 * sqrt(left / R) <= 1e-5 * big + 1e-6 * mean + 1e-35)) atomicOr(&a.head->rough, 1);
             }
         }
     }
@@ -644,78 +668,54 @@ __device__ inline float4 sep_eval4(const float* tab, int R, const SepAt& at, int
     return s;
 }
 
-// The power of two that brings a largest value to [2^11, 2^12), and its inverse.
-__device__ inline float sep_scale_of(float largest, float* inverse) {
-    int e = 12;
-    if (largest > 0.0f) e = 12 - (ilogbf(largest) + 1);
-    e = e > 120 ? 120 : e < -120 ? -120 : e;
-    *inverse = ldexpf(1.0f, -e);
-    return ldexpf(1.0f, e);
+__device__ inline float2 sep_eval2(const float* tab, int R, const SepAt& at, int j) {
+    const float* p = tab + (size_t)at.i * R + j;
+    float2 s = make_float2(0.0f, 0.0f);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const float2 v = *reinterpret_cast<const float2*>(p + q * R);
+        s.x = fmaf(at.w[q], v.x, s.x);
+        s.y = fmaf(at.w[q], v.y, s.y);
+    }
+    return s;
 }
 
-// A row's largest |c_j r| or |d_j r|, from above: the first coefficient grows with x and
-// dominates the others, r falls with x.
-__device__ inline float sep_bound(const SepHead& h, const float* tab, int j, float2 range, float v_sat) {
-    const SepAt at = sep_at(h, range.y);
-    const float* p = tab + (size_t)at.i * h.terms + j;
-    float s = 0.0f;
-    for (int q = 0; q < 4; ++q) s = fmaf(at.w[q], p[q * h.terms], s);
-    return fabsf(s) * (1.0f + range.y / v_sat) / (1.0f + range.x / v_sat) * 1.001f;
-}
-
-__device__ inline void sep_split(float v, _Float16& hi, _Float16& lo) {
-    hi = (_Float16)v;
-    lo = (_Float16)(v - (float)hi);
-}
-
-// Stores a pair of neighbouring inner elements (e, e + 1; e even) of a row of hi/lo slabs.
-__device__ inline void sep_store2(_Float16* row, int64_t e, float v0, float v1) {
-    sep_h2 hi, lo;
-    _Float16 h0, l0, h1, l1;
-    sep_split(v0, h0, l0);
-    sep_split(v1, h1, l1);
-    hi.x = h0; hi.y = h1; lo.x = l0; lo.y = l1;
-    _Float16* p = row + (e >> 5) * 64 + (e & 31);
-    *reinterpret_cast<sep_h2*>(p) = hi;
-    *reinterpret_cast<sep_h2*>(p + 32) = lo;
+// Stores N neighbouring inner elements (e a multiple of N) of an operand's row as PARTS bf16 each.
+template <int N, int PARTS>
+__device__ inline void sep_put(char* row, int64_t e, const float* v) {
+    typedef __bf16 vec __attribute__((ext_vector_type(N)));
+    char* p = row + (e >> 4) * (32 * PARTS) + (e & 15) * 2;
+    float rest[N];
+#pragma unroll
+    for (int q = 0; q < N; ++q) rest[q] = v[q];
+#pragma unroll
+    for (int part = 0; part < PARTS; ++part) {
+        vec w;
+#pragma unroll
+        for (int q = 0; q < N; ++q) {
+            w[q] = (__bf16)rest[q];
+            rest[q] -= (float)w[q];
+        }
+        *reinterpret_cast<vec*>(p + 32 * part) = w;
+    }
 }
 
 // ----------------------------------------------------------------------------------
-// Forward operands: xop[m] = c_j r (a wave per row, lanes along k) and wop[o] = T_j(t+) - T_j(t-),
-// each (row, k) four values in 8-byte stores that neighbouring lanes continue. HBM-bound.
+// Forward operands: xop[m] = c_j r (a wave per row, lanes along k) and wop[o] = T_j(t+) - T_j(t-).
+// HBM-bound.
 // ----------------------------------------------------------------------------------
 
 constexpr int kSepExpandBlocks = 2048;
-
-__device__ inline void sep_store4(_Float16* row, int64_t e, const float v[4]) {  // pairs
-    sep_h4 hi, lo;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        _Float16 h, l;
-        sep_split(v[q], h, l);
-        hi[q] = h;
-        lo[q] = l;
-    }
-    _Float16* p = row + (e >> 5) * 64 + (e & 31);
-    *reinterpret_cast<sep_h4*>(p) = hi;
-    *reinterpret_cast<sep_h4*>(p + 32) = lo;
-}
-
-__device__ inline void sep_store4h(_Float16* row, int64_t e, const float v[4]) {  // singles
-    sep_h4 h;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) h[q] = (_Float16)v[q];
-    *reinterpret_cast<sep_h4*>(row + e) = h;
-}
 
 // Walks T_1, T_2, ... of both branches and hands out blocks of four differences.
 struct SepChebPair {
     double p0 = 1.0, p1, n0 = 1.0, n1, tp, tn;
     __device__ SepChebPair(double a, double b) : p1(a), n1(b), tp(2.0 * a), tn(2.0 * b) {}
-    __device__ void next4(float* v, float scale) {  // T_j(t+) - T_j(t-) of the next four j
+    __device__ void next4(float* v) {  // T_j(t+) - T_j(t-) of the next four j
+#pragma clang fp contract(off)  // the same roundings for both branches: equal thresholds give zero
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            v[q] = (float)(p1 - n1) * scale;
+            v[q] = (float)(p1 - n1);
             const double p2 = tp * p1 - p0, n2 = tn * n1 - n0;
             p0 = p1;
             p1 = p2;
@@ -725,71 +725,51 @@ struct SepChebPair {
     }
 };
 
-// cos and sin of 2 pi q theta, q = 1, 2 (theta in revolutions).
-__device__ inline void sep_trig(float theta, float* c, float* sn) {
-    const float f = theta - floorf(theta);
-    c[0] = __builtin_amdgcn_cosf(f);
-    sn[0] = __builtin_amdgcn_sinf(f);
-    c[1] = 2.0f * c[0] * c[0] - 1.0f;
-    sn[1] = 2.0f * sn[0] * c[0];
-}
-
-// Block blk of an input's harmonic values on the token side: the second difference's
-// coefficients e times cosine and sine.
-__device__ inline void sep_harm_x(float v[4], const float e[4], int terms, int blk, const float c[2], const float sn[2],
-                                  float scale) {
-    const float ca = c[0], cb = c[1], sa = sn[0], sb = sn[1];
-    if (terms == 8) {
-        const float f = blk ? 0.25f * scale : scale, fc = (blk ? cb : ca) * f, fs = (blk ? sb : sa) * f;
-        v[0] = e[0] * fc;
-        v[1] = e[1] * fc;
-        v[2] = e[0] * fs;
-        v[3] = e[1] * fs;
-    } else {
-        const float t = blk & 1 ? (blk & 2 ? sb : sa) : (blk & 2 ? cb : ca);
-        const float f = t * (blk & 2 ? 0.25f * scale : scale);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = e[i] * f;
+// cos and sin of 2 pi q theta, q = 1, 2, ... (theta in revolutions).
+struct SepTurn {
+    float c1, s1, c, s;
+    SepTurn() = default;
+    __device__ explicit SepTurn(float theta) {
+        const float f = theta - floorf(theta);
+        c = c1 = __builtin_amdgcn_cosf(f);
+        s = s1 = __builtin_amdgcn_sinf(f);
     }
-}
-
-// Likewise on the threshold side: T_i(t+) cos - T_i(t-) cos, ...
-__device__ inline void sep_harm_w(float v[4], const float tp[4], const float tn[4], int terms, int blk, const float cp[2],
-                                  const float sp[2], const float cn[2], const float sn[2], float scale) {
-    const float cpa = cp[0], cpb = cp[1], spa = sp[0], spb = sp[1], cna = cn[0], cnb = cn[1], sna = sn[0], snb = sn[1];
-    if (terms == 8) {
-        const float c0 = blk ? cpb : cpa, s0 = blk ? spb : spa, c1 = blk ? cnb : cna, s1 = blk ? snb : sna;
-        v[0] = (c0 - c1) * scale;
-        v[1] = (tp[1] * c0 - tn[1] * c1) * scale;
-        v[2] = (s0 - s1) * scale;
-        v[3] = (tp[1] * s0 - tn[1] * s1) * scale;
-    } else {
-        const float f0 = blk & 1 ? (blk & 2 ? spb : spa) : (blk & 2 ? cpb : cpa);
-        const float f1 = blk & 1 ? (blk & 2 ? snb : sna) : (blk & 2 ? cnb : cna);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = (tp[i] * f0 - tn[i] * f1) * scale;
+    __device__ void next() {
+#pragma clang fp contract(off)  // the same roundings for both branches of a pair
+        const float t = c1 * c - s1 * s;
+        s = s1 * c + c1 * s;
+        c = t;
     }
+};
+
+// 1 / q^2 of harmonic q - 1.
+__device__ inline float sep_harm_weight(int q) { return q == 0 ? 1.0f : q == 1 ? 0.25f : q == 2 ? 1.0f / 9.0f : 0.0625f; }
+
+// The nearest table point's two second-difference coefficients (they change by 1.5% from point to
+// point, and are 1e-4 of the result).
+__device__ inline float2 sep_second(const float* tabE, const SepAt& at) {
+    return reinterpret_cast<const float2*>(tabE)[at.i + (at.w[2] > at.w[1] ? 2 : 1)];
 }
 
-__device__ inline void sep_cheb4(float t, float v[4]) {  // T_0 .. T_3
-    v[0] = 1.0f;
-    v[1] = t;
-    v[2] = 2.0f * t * t - 1.0f;
-    v[3] = 2.0f * t * v[2] - t;
+// A harmonic's four values of an input on the token side (e scaled) ...
+__device__ inline void sep_harm_x(float v[4], float2 e, float c, float sn, float weight) {
+    v[0] = e.x * c * weight;
+    v[1] = e.y * c * weight;
+    v[2] = e.x * sn * weight;
+    v[3] = e.y * sn * weight;
 }
 
-// The nearest table point's R / 4 second-difference coefficients (they change by 1.5% from
-// point to point, and are 1e-5 of the result).
-__device__ inline void sep_second(const SepHead& h, const float* tabE, const SepAt& at, float e[4]) {
-    const size_t i = (size_t)(at.i + (at.w[2] > at.w[1] ? 2 : 1));
-    if (h.terms == 8) {
-        const float2 v = *reinterpret_cast<const float2*>(tabE + i * 2);
-        e[0] = v.x; e[1] = v.y; e[2] = e[3] = 0.0f;
-    } else {
-        const float4 v = *reinterpret_cast<const float4*>(tabE + i * 4);
-        e[0] = v.x; e[1] = v.y; e[2] = v.z; e[3] = v.w;
-    }
+// ... and on the threshold side, differences of the branches' (u: the two functions at t+, t-). Products
+// are rounded before they are subtracted, so that equal thresholds give zero.
+__device__ inline void sep_harm_w(float v[4], float2 up, float2 un, float cp, float sp, float cn, float sn) {
+#pragma clang fp contract(off)
+    v[0] = up.x * cp - un.x * cn;
+    v[1] = up.y * cp - un.y * cn;
+    v[2] = up.x * sp - un.x * sn;
+    v[3] = up.y * sp - un.y * sn;
 }
+
+__device__ inline float2 sep_kink_functions(const SepHead& h, float t) { return make_float2(expf(h.gw * t), expf(h.gu * t)); }
 
 // The per-cell range partials of a call that the contraction takes (the passes that record the
 // table mode read them).
@@ -803,6 +783,73 @@ __device__ inline void sep_write_partials(const SepHead& h, const PrepArgs& p) {
     if (p.stat_bits && threadIdx.x == 0) *p.stat_bits = 0u;
 }
 
+template <int R>
+__device__ inline void sep_expand_fwd(const SepArgs& a, const SepHead& h) {
+    constexpr SepClasses cls = sep_classes(R, false);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t kc = sep_inputs(a.K);
+    const SepRow at_row(a.K, R, h.harmonics);
+    const float as = a.in_affine ? a.in_affine[0] : 1.0f, ab = a.in_affine ? a.in_affine[1] : 0.0f;
+    // all terms of input k of a row, then its harmonics
+    auto terms = [&](char* row, int64_t k, const float* v) {
+        sep_put<cls.n3, 3>(row + at_row.triples, k * cls.n3, v);
+#pragma unroll
+        for (int b = 0; b < cls.n2 / 4; ++b) sep_put<4, 2>(row + at_row.pairs, (b * kc + k) * 4, v + cls.n3 + 4 * b);
+        sep_put<cls.n1, 1>(row, k * cls.n1, v + cls.n3 + cls.n2);
+    };
+    for (int64_t row = (int64_t)blockIdx.x * 4 + wave; row < a.M + a.O; row += (int64_t)gridDim.x * 4) {
+        if (row < a.M) {
+            char* dst = a.xop + row * at_row.bytes;
+            for (int64_t k = lane; k < kc; k += 64) {
+                const bool real = k < a.K;
+                const float x = sep_input(a, a.x[row * a.K + (real ? k : a.K - 1)], as, ab), one = real ? 1.0f : 0.0f;
+                const SepAt at = sep_at(h, x);
+                float v[R];
+#pragma unroll
+                for (int j = 0; j < R; j += 4) {
+                    const float4 c = sep_eval4(a.tab, R, at, j);
+                    v[j] = c.x * one; v[j + 1] = c.y * one; v[j + 2] = c.z * one; v[j + 3] = c.w * one;
+                }
+                terms(dst, k, v);
+                if (h.harmonics > 0) {
+                    const float2 e = sep_second(a.tabE, at);
+                    SepTurn turn((x - h.lut_min) * h.lut_scale);
+                    for (int q = 0; q < h.harmonics; ++q) {
+                        float u[4];
+                        sep_harm_x(u, e, turn.c, turn.s, sep_harm_weight(q) * one);
+                        sep_put<4, 1>(dst + at_row.harm, (q * kc + k) * 4, u);
+                        turn.next();
+                    }
+                }
+            }
+        } else {
+            const int64_t o = row - a.M;
+            char* dst = a.wop + o * at_row.bytes;
+            for (int64_t k = lane; k < kc; k += 64) {
+                const bool real = k < a.K;  // padded inputs: both branches at the centre
+                const double tp = real ? ((double)a.wp[o * a.K + k] - h.wc) * h.inv_wh : 0.0;
+                const double tn = real ? ((double)a.wn[o * a.K + k] - h.wc) * h.inv_wh : 0.0;
+                SepChebPair c(tp, tn);
+                float v[R];
+#pragma unroll
+                for (int j = 0; j < R; j += 4) c.next4(v + j);
+                terms(dst, k, v);
+                if (h.harmonics > 0) {
+                    const float2 fp = sep_kink_functions(h, (float)tp), fn = sep_kink_functions(h, (float)tn);
+                    SepTurn up((float)((h.wc + h.wh * tp) * h.lut_scale)), un((float)((h.wc + h.wh * tn) * h.lut_scale));
+                    for (int q = 0; q < h.harmonics; ++q) {
+                        float u[4];
+                        sep_harm_w(u, fp, fn, up.c, up.s, un.c, un.s);
+                        sep_put<4, 1>(dst + at_row.harm, (q * kc + k) * 4, u);
+                        up.next();
+                        un.next();
+                    }
+                }
+            }
+        }
+    }
+}
+
 // Where the per-cell kernels take the call: their prep, in the same launch (unless the statistics'
 // launch has run it).
 __global__ __launch_bounds__(256) void sep_expand_fwd_kernel(SepArgs a, PrepArgs prep) {
@@ -811,302 +858,292 @@ __global__ __launch_bounds__(256) void sep_expand_fwd_kernel(SepArgs a, PrepArgs
         return;
     }
     const SepHead h = *a.head;
-    const int R = h.terms;
     if (blockIdx.x == 0) sep_write_partials(h, prep);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t kc = sep_inputs(a.K), pairs = sep_slabs_pairs(a.K, R) * 64;
-    const int64_t stride = pairs + sep_slabs_singles(a.K, R, h.harmonics) * 64;  // of a row, in f16
-    const int64_t harm = pairs + kc * (R / 2);
-    const int64_t row_waves = (int64_t)gridDim.x * 4;
+    if (h.terms == 8)
+        sep_expand_fwd<8>(a, h);
+    else
+        sep_expand_fwd<16>(a, h);
+}
+
+// ----------------------------------------------------------------------------------
+// Backward operands, tokens or outputs inside: the rows (input, term) of d_j r over the tokens and of
+// T_j(t+) - T_j(t-) over the outputs, with tT[k][o] = {t+, t-}, and G in both directions, scaled by a
+// power of two to at most 1. Tiles of 32 inputs (or rows of G) by 128 inner elements go through LDS, so
+// that reads run along the tensors' rows and writes along the inner index, four elements a thread.
+// HBM-bound.
+// ----------------------------------------------------------------------------------
+
+constexpr int kSepTilePitch = 132;
+
+// Four inner elements from e on of class PARTS' rows of input k: v[term][element].
+template <int R, bool DV, int PARTS>
+__device__ inline void sep_put_rows(char* op, int64_t inner, int64_t k, int64_t e, const float (*v)[4]) {
+    constexpr SepClasses cls = sep_classes(R, DV);
+    constexpr int first = cls.first(PARTS), count = cls.count(PARTS);
+    char* row = op + sep_row(k, count, 0) * inner * (2 * PARTS);
+#pragma unroll
+    for (int i = 0; i < count; ++i)
+        sep_put<4, PARTS>(row + (sep_row(0, count, i) - sep_row(0, count, 0)) * inner * (2 * PARTS), e, v[first + i]);
+}
+
+template <int R>
+__device__ inline void sep_expand_tokens(const SepArgs& a, const SepHead& h, int b, float (*s_x)[kSepTilePitch]) {
+    const int t = threadIdx.x, n_mt = (int)((a.M + 127) / 128);
+    const int64_t inner = sep_inner(a.M), m0 = (int64_t)(b % n_mt) * 128, k0 = (int64_t)(b / n_mt) * 32;
     const float as = a.in_affine ? a.in_affine[0] : 1.0f, ab = a.in_affine ? a.in_affine[1] : 0.0f;
-    float v[4];
-    for (int64_t row = (int64_t)blockIdx.x * 4 + wave; row < a.M + a.O; row += row_waves) {
-        if (row < a.M) {
-            float inv;
-            const float scale = sep_scale_of(sep_bound(h, a.tab, 0, a.xrow[row], (float)a.v_sat), &inv);
-            if (lane == 0) a.xscale[row] = inv / kSepQScale;
-            _Float16* dst = a.xop + row * stride;
-            for (int64_t k = lane; k < kc; k += 64) {
-                const bool real = k < a.K;
-                const float x = sep_input(a, a.x[row * a.K + (real ? k : a.K - 1)], as, ab);
-                const float sc = real ? scale : 0.0f;
-                const SepAt at = sep_at(h, x);
-                for (int j = 0; j < R; j += 4) {
-                    const float4 c = sep_eval4(a.tab, R, at, j);
-                    v[0] = c.x * sc; v[1] = c.y * sc; v[2] = c.z * sc; v[3] = c.w * sc;
-                    if (j < R / 2)
-                        sep_store4(dst, j * kc + k * 4, v);
-                    else
-                        sep_store4h(dst + pairs, (j - R / 2) * kc + k * 4, v);
-                }
-                if (h.harmonics > 0) {
-                    float e[4], c[2], sn[2];
-                    sep_second(h, a.tabE, at, e);
-                    sep_trig((x - h.lut_min) * h.lut_scale, c, sn);
-                    for (int blk = 0; blk < h.harmonics * R / 8; ++blk) {
-                        sep_harm_x(v, e, R, blk, c, sn, sc);
-                        sep_store4h(dst + harm, blk * 4 * kc + k * 4, v);
-                    }
-                }
+    for (int q = t; q < 32 * 128; q += 256) {
+        const int64_t m = m0 + (q >> 5), k = k0 + (q & 31);
+        s_x[q & 31][q >> 5] = m < a.M && k < a.K ? sep_input(a, a.x[m * a.K + k], as, ab) : h.xlo;
+    }
+    __syncthreads();
+    for (int q = t; q < 32 * 32; q += 256) {
+        const int64_t k = k0 + (q >> 5), m = m0 + 4 * (q & 31);
+        if (k >= a.K || m >= inner) continue;
+        const float4 x4 = *reinterpret_cast<const float4*>(&s_x[q >> 5][4 * (q & 31)]);
+        const float x[4] = {x4.x, x4.y, x4.z, x4.w};
+        float v[R][4];
+        SepAt at[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            at[i] = sep_at(h, x[i]);
+            const float one = m + i < a.M ? 1.0f : 0.0f;
+#pragma unroll
+            for (int j = 0; j < R; j += 4) {
+                const float4 u = sep_eval4(a.tab, R, at[i], j);
+                v[j][i] = u.x * one; v[j + 1][i] = u.y * one; v[j + 2][i] = u.z * one; v[j + 3][i] = u.w * one;
             }
-        } else {
-            const int64_t o = row - a.M;
-            _Float16* dst = a.wop + o * stride;
-            for (int64_t k = lane; k < kc; k += 64) {
-                const bool real = k < a.K;
-                const double tp = real ? ((double)a.wp[o * a.K + k] - h.wc) * h.inv_wh : 0.0;
-                const double tn = real ? ((double)a.wn[o * a.K + k] - h.wc) * h.inv_wh : 0.0;
-                SepChebPair c(tp, tn);
-                for (int j = 0; j < R; j += 4) {
-                    c.next4(v, kSepQScale);
-                    if (j < R / 2)
-                        sep_store4(dst, j * kc + k * 4, v);
-                    else
-                        sep_store4h(dst + pairs, (j - R / 2) * kc + k * 4, v);
+        }
+        sep_put_rows<R, true, 3>(a.xcls[2], inner, k, m, v);
+        sep_put_rows<R, true, 2>(a.xcls[1], inner, k, m, v);
+        sep_put_rows<R, true, 1>(a.xcls[0], inner, k, m, v);
+        if (h.harmonics > 0) {
+            SepTurn turn[4];
+            float2 e[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                e[i] = sep_second(a.tabE, at[i]);
+                if (m + i >= a.M) e[i] = make_float2(0.0f, 0.0f);
+                turn[i] = SepTurn((x[i] - h.lut_min) * h.lut_scale);
+            }
+            for (int qh = 0; qh < h.harmonics; ++qh) {
+                const float weight = sep_harm_weight(qh);
+                float w[4][4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    float u[4];
+                    sep_harm_x(u, e[i], turn[i].c, turn[i].s, weight);
+                    turn[i].next();
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) w[j][i] = u[j];
                 }
-                if (h.harmonics > 0) {
-                    float p[4], n[4], cp[2], sp[2], cn[2], sn[2];
-                    sep_cheb4((float)tp, p);
-                    sep_cheb4((float)tn, n);
-                    sep_trig((float)((h.wc + h.wh * tp) * h.lut_scale), cp, sp);
-                    sep_trig((float)((h.wc + h.wh * tn) * h.lut_scale), cn, sn);
-                    for (int blk = 0; blk < h.harmonics * R / 8; ++blk) {
-                        sep_harm_w(v, p, n, R, blk, cp, sp, cn, sn, kSepQScale);
-                        sep_store4h(dst + harm, blk * 4 * kc + k * 4, v);
-                    }
-                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    sep_put<4, 1>(a.xcls[3] + sep_row(k, 4 * h.harmonics, 4 * qh + j) * inner * 2, m, w[j]);
             }
         }
     }
 }
 
-// ----------------------------------------------------------------------------------
-// Backward operands, tokens or outputs inside: xop[(k, j)][m] = d_j r, wop[(k, j)][o] = T_j(t+) -
-// T_j(t-) with tT[k][o] = {t+, t-}, gop[m][o] and gopT[o][m]. Tiles of 32 inputs (or rows of G)
-// by 128 inner elements go through LDS, so that reads run along the tensors' rows and writes
-// along the inner index. HBM-bound.
-// ----------------------------------------------------------------------------------
-
-__device__ inline void sep_store2h(_Float16* row, int64_t e, float v0, float v1) {  // single f16
-    sep_h2 h;
-    h.x = (_Float16)v0;
-    h.y = (_Float16)v1;
-    *reinterpret_cast<sep_h2*>(row + e) = h;
+template <int R>
+__device__ inline void sep_expand_thresholds(const SepArgs& a, const SepHead& h, int b, float (*s_p)[kSepTilePitch],
+                                             float (*s_n)[kSepTilePitch]) {
+    const int t = threadIdx.x, n_ot = (int)((a.O + 127) / 128);
+    const int64_t inner = sep_inner(a.O), o0 = (int64_t)(b % n_ot) * 128, k0 = (int64_t)(b / n_ot) * 32;
+    // padded outputs: both branches near the centre, so that their differences vanish
+    for (int q = t; q < 32 * 128; q += 256) {
+        const int64_t o = o0 + (q >> 5), k = k0 + (q & 31);
+        const bool real = o < a.O && k < a.K;
+        s_p[q & 31][q >> 5] = real ? a.wp[o * a.K + k] : (float)h.wc;
+        s_n[q & 31][q >> 5] = real ? a.wn[o * a.K + k] : (float)h.wc;
+    }
+    __syncthreads();
+    for (int q = t; q < 32 * 32; q += 256) {
+        const int64_t k = k0 + (q >> 5), o = o0 + 4 * (q & 31);
+        if (k >= a.K || o >= inner) continue;
+        const float* wp = &s_p[q >> 5][4 * (q & 31)];
+        const float* wn = &s_n[q >> 5][4 * (q & 31)];
+        float tp[4], tn[4], v[R][4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const double p = ((double)wp[i] - h.wc) * h.inv_wh, n = ((double)wn[i] - h.wc) * h.inv_wh;
+            tp[i] = (float)p;
+            tn[i] = (float)n;
+            SepChebPair c(p, n);
+            float u[4];
+#pragma unroll
+            for (int j = 0; j < R; j += 4) {
+                c.next4(u);
+#pragma unroll
+                for (int d = 0; d < 4; ++d) v[j + d][i] = u[d];
+            }
+        }
+        if (a.need_w) {
+            float4* dst = reinterpret_cast<float4*>(a.tT + k * a.Op + o);
+            dst[0] = make_float4(tp[0], tn[0], tp[1], tn[1]);
+            dst[1] = make_float4(tp[2], tn[2], tp[3], tn[3]);
+        }
+        if (!a.need_x) continue;
+        sep_put_rows<R, false, 3>(a.wcls[2], inner, k, o, v);
+        sep_put_rows<R, false, 2>(a.wcls[1], inner, k, o, v);
+        sep_put_rows<R, false, 1>(a.wcls[0], inner, k, o, v);
+        if (h.harmonics > 0) {
+            SepTurn up[4], un[4];
+            float2 fp[4], fn[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                fp[i] = sep_kink_functions(h, tp[i]);
+                fn[i] = sep_kink_functions(h, tn[i]);
+                up[i] = SepTurn(wp[i] * h.lut_scale);
+                un[i] = SepTurn(wn[i] * h.lut_scale);
+            }
+            for (int qh = 0; qh < h.harmonics; ++qh) {
+                float w[4][4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    float u[4];
+                    sep_harm_w(u, fp[i], fn[i], up[i].c, up[i].s, un[i].c, un[i].s);
+                    up[i].next();
+                    un[i].next();
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) w[j][i] = u[j];
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    sep_put<4, 1>(a.wcls[3] + sep_row(k, 4 * h.harmonics, 4 * qh + j) * inner * 2, o, w[j]);
+            }
+        }
+    }
 }
 
-__global__ __launch_bounds__(256) void sep_expand_bwd_kernel(SepArgs a, int x_blocks, int w_blocks, PrepArgs prep) {
+// The power of two that brings |G| to at most 1, and its inverse.
+__device__ inline float sep_grad_scale(const SepHead* head, float* inverse) {
+    const float big = __uint_as_float(head->gmax);
+    int e = big > 0.0f ? -(ilogbf(big) + 1) : 0;
+    e = e > 120 ? 120 : e < -120 ? -120 : e;
+    *inverse = ldexpf(1.0f, -e);
+    return ldexpf(1.0f, e);
+}
+
+// G: tiles of 32 rows by 128 outputs.
+__device__ inline void sep_expand_grad(const SepArgs& a, int b, float (*s_g)[kSepTilePitch]) {
+    const int t = threadIdx.x, n_ot = (int)((a.O + 127) / 128);
+    const int64_t mi = sep_inner(a.M), oi = sep_inner(a.O);
+    if (b >= n_ot * (int)(mi / 32)) return;  // blocks that only the prep needs
+    const int64_t o0 = (int64_t)(b % n_ot) * 128, m0 = (int64_t)(b / n_ot) * 32;
+    float inv;
+    const float scale = sep_grad_scale(a.head, &inv);
+    for (int q = t; q < 32 * 128; q += 256) {
+        const int64_t m = m0 + (q >> 7), o = o0 + (q & 127);
+        s_g[q >> 7][q & 127] = m < a.M && o < a.O ? a.g[m * a.ldg + o] * scale : 0.0f;
+    }
+    __syncthreads();
+    if (a.need_x) {
+        for (int q = t; q < 32 * 32; q += 256) {
+            const int64_t m = m0 + (q >> 5), o = o0 + 4 * (q & 31);
+            if (m >= a.M || o >= oi) continue;
+            const float* v = &s_g[q >> 5][4 * (q & 31)];
+            sep_put<4, 3>(a.gop + m * oi * 6, o, v);
+            sep_put<4, 1>(a.gops + m * oi * 2, o, v);
+        }
+    }
+    if (a.need_w) {
+        for (int q = t; q < 128 * 8; q += 256) {
+            const int64_t o = o0 + (q >> 3), m = m0 + 4 * (q & 7);
+            if (o >= a.O) continue;
+            float v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = s_g[4 * (q & 7) + i][q >> 3];
+            sep_put<4, 3>(a.gopT + o * mi * 6, m, v);
+            sep_put<4, 1>(a.gopTs + o * mi * 2, m, v);
+        }
+    }
+}
+
+__global__ __launch_bounds__(256, 3) void sep_expand_bwd_kernel(SepArgs a, int x_blocks, int w_blocks, PrepArgs prep) {
     if (!sep_takes(a.head)) {  // the per-cell kernels take the call: their prep
         if (blockIdx.x < kPrepBlocksX + kPrepBlocksW && a.head->rough != 2) prep_block(prep, blockIdx.x);
         return;
     }
     const SepHead h = *a.head;
-    const int R = h.terms;
     if (blockIdx.x == 0) sep_write_partials(h, prep);
-    const int64_t m64 = sep_slabs64(a.M) * 64, o64 = sep_slabs64(a.O) * 64;  // the singles' inner lengths
-    const int xpairs = a.lut_n > 0 ? R / 2 : R;  // terms of xop as pairs
-    __shared__ float s_a[32][130], s_b[32][130];
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int64_t m_slabs = sep_slabs(a.M), o_slabs = sep_slabs(a.O);
-    int b = blockIdx.x;
+    __shared__ __align__(16) float s_a[32][kSepTilePitch], s_b[32][kSepTilePitch];
+    const int b = blockIdx.x;
     if (b < x_blocks) {
-        const int n_mt = (int)((a.M + 127) / 128);
-        const int64_t m0 = (int64_t)(b % n_mt) * 128, k0 = (int64_t)(b / n_mt) * 32;
-        const float as = a.in_affine ? a.in_affine[0] : 1.0f, ab = a.in_affine ? a.in_affine[1] : 0.0f;
-        for (int q = t; q < 32 * 128; q += 256) {
-            const int64_t m = m0 + (q >> 5), k = k0 + (q & 31);
-            s_a[q & 31][q >> 5] = m < a.M && k < a.K ? sep_input(a, a.x[m * a.K + k], as, ab) : 0.0f;
-        }
-        __syncthreads();
-        for (int kk = wave; kk < 32 && k0 + kk < a.K; kk += 4) {
-            const int64_t k = k0 + kk;
-            static_assert(kSepColChunks == 64, "a lane per chunk");
-            float2 range = a.xcol[(int64_t)lane * a.K + k];
-            sep_wave_minmax(range.x, range.y);
-            float inv;
-            const float scale = sep_scale_of(2.0f * sep_bound(h, a.tab, 0, range, (float)a.v_sat), &inv);
-            if (m0 == 0 && lane == 0) a.xscale[k] = inv;
-            const int ml = 2 * lane;
-            const int64_t m = m0 + ml;
-            if (m >= m64) continue;
-            const bool pair = m < m_slabs * 32;
-            const float s0 = m < a.M ? scale : 0.0f, s1 = m + 1 < a.M ? scale : 0.0f;
-            const float x0 = m < a.M ? s_a[kk][ml] : range.y, x1 = m + 1 < a.M ? s_a[kk][ml + 1] : range.y;
-            const SepAt p0 = sep_at(h, x0), p1 = sep_at(h, x1);
-            for (int j = 0; j < R; j += 4) {
-                const float4 u = sep_eval4(a.tab, R, p0, j), v = sep_eval4(a.tab, R, p1, j);
-                const float u4[4] = {u.x * s0, u.y * s0, u.z * s0, u.w * s0}, v4[4] = {v.x * s1, v.y * s1, v.z * s1, v.w * s1};
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    if (j < xpairs) {
-                        if (pair) sep_store2(a.xop + sep_row(k, xpairs, j + q) * m_slabs * 64, m, u4[q], v4[q]);
-                    } else {
-                        sep_store2h(a.xops + sep_row(k, R / 2, j + q - R / 2) * m64, m, u4[q], v4[q]);
-                    }
-                }
-            }
-            if (h.harmonics > 0) {
-                float e0[4], e1[4], c0[2], n0[2], c1[2], n1[2], u[4], v[4];
-                sep_second(h, a.tabE, p0, e0);
-                sep_second(h, a.tabE, p1, e1);
-                sep_trig((x0 - h.lut_min) * h.lut_scale, c0, n0);
-                sep_trig((x1 - h.lut_min) * h.lut_scale, c1, n1);
-                for (int blk = 0; blk < h.harmonics * R / 8; ++blk) {
-                    sep_harm_x(u, e0, R, blk, c0, n0, s0);
-                    sep_harm_x(v, e1, R, blk, c1, n1, s1);
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) sep_store2h(a.xoph + sep_row(k, h.harmonics * R / 2, blk * 4 + q) * m64, m, u[q], v[q]);
-                }
-            }
-        }
-        return;
-    }
-    b -= x_blocks;
-    if (b < w_blocks) {
-        const int n_ot = (int)((a.O + 127) / 128);
-        const int64_t o0 = (int64_t)(b % n_ot) * 128, k0 = (int64_t)(b / n_ot) * 32;
-        for (int q = t; q < 32 * 128; q += 256) {
-            const int64_t o = o0 + (q >> 5), k = k0 + (q & 31);
-            const bool real = o < a.O && k < a.K;
-            s_a[q & 31][q >> 5] = real ? a.wp[o * a.K + k] : (float)h.wc;
-            s_b[q & 31][q >> 5] = real ? a.wn[o * a.K + k] : (float)h.wc;
-        }
-        __syncthreads();
-        for (int kk = wave; kk < 32 && k0 + kk < a.K; kk += 4) {
-            const int64_t k = k0 + kk;
-            const int ol = 2 * lane;
-            const int64_t o = o0 + ol;
-            if (o >= o64) continue;
-            const bool pair = o < o_slabs * 32;
-            double t_[4];
-#pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                t_[2 * q] = ((double)s_a[kk][ol + q] - h.wc) * h.inv_wh;
-                t_[2 * q + 1] = ((double)s_b[kk][ol + q] - h.wc) * h.inv_wh;
-            }
-            if (a.need_w) {
-                reinterpret_cast<float4*>(a.tT + k * a.Op)[o >> 1] =
-                    make_float4((float)t_[0], (float)t_[1], (float)t_[2], (float)t_[3]);
-            }
-            if (!a.need_x) continue;
-            // padded outputs: both branches at the centre, so that their differences vanish
-            SepChebPair c0(t_[0], t_[1]), c1(t_[2], t_[3]);
-            float u[4], v[4];
-            for (int j = 0; j < R; j += 4) {
-                c0.next4(u, kSepQScale);
-                c1.next4(v, kSepQScale);
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    if (j < R / 2) {
-                        if (pair) sep_store2(a.wop + sep_row(k, R / 2, j + q) * o_slabs * 64, o, u[q], v[q]);
-                    } else {
-                        sep_store2h(a.wops + sep_row(k, R / 2, j + q - R / 2) * o64, o, u[q], v[q]);
-                    }
-                }
-            }
-            if (h.harmonics_dx > 0) {
-                float p0[4], n0[4], p1[4], n1[4], e0[4], d0[4], e1[4], d1[4];
-                sep_cheb4((float)t_[0], p0);
-                sep_cheb4((float)t_[1], n0);
-                sep_cheb4((float)t_[2], p1);
-                sep_cheb4((float)t_[3], n1);
-                sep_trig(s_a[kk][ol] * h.lut_scale, e0, d0);
-                sep_trig(s_b[kk][ol] * h.lut_scale, e0 + 2, d0 + 2);
-                sep_trig(s_a[kk][ol + 1] * h.lut_scale, e1, d1);
-                sep_trig(s_b[kk][ol + 1] * h.lut_scale, e1 + 2, d1 + 2);
-                for (int blk = 0; blk < h.harmonics_dx * R / 8; ++blk) {
-                    sep_harm_w(u, p0, n0, R, blk, e0, d0, e0 + 2, d0 + 2, kSepQScale);
-                    sep_harm_w(v, p1, n1, R, blk, e1, d1, e1 + 2, d1 + 2, kSepQScale);
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) sep_store2h(a.woph + sep_row(k, h.harmonics_dx * R / 2, blk * 4 + q) * o64, o, u[q], v[q]);
-                }
-            }
-        }
-        return;
-    }
-    b -= w_blocks;
-    if (b >= (int)((a.O + 127) / 128 * ((a.M + 31) / 32))) return;  // blocks that only the prep needs
-    // G: tiles of 32 rows by 128 outputs
-    const int n_ot = (int)((a.O + 127) / 128);
-    const int64_t o0 = (int64_t)(b % n_ot) * 128, m0 = (int64_t)(b / n_ot) * 32;
-    for (int q = t; q < 32 * 128; q += 256) {
-        const int64_t m = m0 + (q >> 7), o = o0 + (q & 127);
-        s_a[q >> 7][q & 127] = m < a.M && o < a.O ? a.g[m * a.ldg + o] : 0.0f;
-    }
-    __syncthreads();
-    if (a.need_x) {
-        for (int mm = wave; mm < 32 && m0 + mm < a.M; mm += 4) {
-            const int64_t m = m0 + mm, o = o0 + 2 * lane;
-            float inv;
-            const float scale = sep_scale_of(__uint_as_float(a.grow[m]), &inv);
-            if (o0 == 0 && lane == 0) a.gscale[m] = inv / kSepQScale;
-            const float g0 = s_a[mm][2 * lane] * scale, g1 = s_a[mm][2 * lane + 1] * scale;
-            if (o < o_slabs * 32) sep_store2(a.gop + m * o_slabs * 64, o, g0, g1);
-            if (o < o64) sep_store2h(a.goph + m * o64, o, g0, g1);
-        }
-    }
-    if (a.need_w) {
-        // 16 lanes hold the 32 tokens of one output: 16 outputs at a time
-        for (int q = t >> 4; q < 128 && o0 + q < a.O; q += 16) {
-            const int64_t o = o0 + q;
-            unsigned big = 0;
-            for (int c = t & 15; c < kSepColChunks; c += 16) big = max(big, a.gcol[(int64_t)c * a.O + o]);
-            for (int d = 8; d > 0; d >>= 1) big = max(big, (unsigned)__shfl_xor((int)big, d, 16));
-            float inv;
-            const float scale = sep_scale_of(__uint_as_float(big), &inv);
-            if (m0 == 0 && (t & 15) == 0) a.gscaleT[o] = inv;
-            const int mm = 2 * (t & 15);
-            const float g0 = s_a[mm][q] * scale, g1 = s_a[mm + 1][q] * scale;
-            sep_store2(a.gopT + o * m_slabs * 64, m0 + mm, g0, g1);
-            sep_store2h(a.gophT + o * m64, m0 + mm, g0, g1);
-            if (m0 + 32 >= a.M && m0 + 32 < m64) sep_store2h(a.gophT + o * m64, m0 + 32 + mm, 0.0f, 0.0f);
-        }
+        if (h.terms == 8)
+            sep_expand_tokens<8>(a, h, b, s_a);
+        else
+            sep_expand_tokens<16>(a, h, b, s_a);
+    } else if (b < x_blocks + w_blocks) {
+        if (h.terms == 8)
+            sep_expand_thresholds<8>(a, h, b - x_blocks, s_a, s_b);
+        else
+            sep_expand_thresholds<16>(a, h, b - x_blocks, s_a, s_b);
+    } else {
+        sep_expand_grad(a, b - x_blocks - w_blocks, s_a);
     }
 }
 
 // ----------------------------------------------------------------------------------
-// The product of two operands of slabs, C[i][j] = sum_e A[i][e] B[j][e]: tiles of
-// (WM MI 32) x (WN NI 32), one slab (128 bytes per row) of both operands at a time in two LDS
-// buffers. A slab holds 32 inner elements as hi/lo pairs, which take three products per pair of
-// fragments (hi hi, hi lo, lo hi), or (harmonics) 64 as single f16. A slab's loads are issued
-// before the arithmetic of the one before it: 3072 matrix-core cycles per 64 KB of operands for
-// the 256 x 256 tile of pairs, so that one buffer ahead covers the memory's latency and the
-// operands need ~21 bytes per cycle and CU. Rows are 128 bytes and their eight 16-byte parts are
-// stored at part ^ (row / 2 % 8), so that the 16 rows that a quarter-wave reads lie on different
+// The product of two operands, C[i][j] = sum_e A[i][e] B[j][e]: tiles of (WM MI 32) x (WN NI 32), one
+// slab (up to 128 bytes per row) of both operands at a time in two LDS buffers. A slab holds 64 inner
+// elements as singles (one product per pair of fragments), 32 as pairs (three: all but the product of
+// the second parts) or 16 as triples (six). A triples' slab is summed by itself, its small products
+// first, and added to the sums so far: a sum over 8192 tokens rounds 512 times in place of 3072. A
+// slab's loads are issued before the arithmetic of the one before it: 3072 matrix-core cycles per
+// 64 KB of operands for the 256 x 256 tile, so that one buffer ahead covers the memory's latency and
+// the operands need ~21 bytes per cycle and CU. Rows are 128 bytes of LDS and their eight 16-byte parts
+// are stored at part ^ (row / 2 % 8), so that the 16 rows that a quarter-wave reads lie on different
 // banks. Rows past the operand's end read its last row (their results are dropped).
 // Blocks are dealt so that each XCD works on neighbouring tiles (whose operands its L2 holds).
 //
-// A launch runs up to six products after one another in its grid (the backward's dX and dVth, of
-// the lower terms, the upper ones and the harmonics), so that one's last blocks overlap the next one's first.
+// A launch runs up to eight products after one another in its grid (the backward's dX and dVth, each of
+// the triples, the pairs, the singles and the harmonics), so that one's last blocks overlap the next
+// one's first.
 // ----------------------------------------------------------------------------------
 
-enum SepKind { kSepForward, kSepDx, kSepDv, kSepDxUpper, kSepDvUpper, kSepDxHarm, kSepDvHarm };
+enum SepKind { kSepForward, kSepDx, kSepDv };
 
 struct SepProduct {
     const char* a;
     const char* b;
     int kind;
+    int parts;                // backward: of the terms' class; 0: the harmonics
     int64_t a_rows, b_rows;   // dX, dVth: inputs in the place of A's rows
-    int64_t inner;            // elements; forward: inputs
+    int64_t inner;            // backward: padded tokens or outputs
     int n_split;
     float* out;               // forward: planes [n_split][M][O]; dX: [n_split][M][K]; dVth: [n_split][2][Kp][Op]
 };
 
 struct SepGemm {
-    SepProduct p[6];
+    SepProduct p[8];
     int n;
     const SepHead* head;
     int64_t M, K, O, Kp, Op;
-    const float* xscale;      // forward [M], dVth [K]
-    const float* gscale;      // dX [M]
-    const float* gscaleT;     // dVth [O]
     const float* x;
     const float* in_affine;
     float in_lo, in_hi;
     const float* tab2;
     const float* tabE;
     const float2* tT;
-    int dv_all;               // the dVth product of pairs holds every term
 };
+
+// T_j(t), T_(j+1)(t) for the first term j of a class or of four in it: 0, 4, 6, 8 or 12
+// (T_(a+b) = 2 T_a T_b - T_(a-b)).
+__device__ inline float2 sep_cheb_from(int j, float t) {
+    if (j == 0) return make_float2(1.0f, t);
+    const float t2 = fmaf(2.0f * t, t, -1.0f), t3 = fmaf(2.0f * t, t2, -t);
+    const float t4 = fmaf(2.0f * t2, t2, -1.0f), t5 = fmaf(2.0f * t2, t3, -t);
+    if (j == 4) return make_float2(t4, t5);
+    if (j == 8) return make_float2(fmaf(2.0f * t4, t4, -1.0f), fmaf(2.0f * t4, t5, -t));
+    const float t6 = fmaf(2.0f * t3, t3, -1.0f), t7 = fmaf(2.0f * t3, t4, -t);
+    if (j == 6) return make_float2(t6, t7);
+    return make_float2(fmaf(2.0f * t6, t6, -1.0f), fmaf(2.0f * t6, t7, -t));  // 12
+}
+
+// Values of an input in a backward product (0: no such product).
+__host__ __device__ inline int sep_values(int kind, int parts, int terms, int harmonics) {
+    return parts == 0 ? 4 * harmonics : sep_classes(terms, kind == kSepDv).count(parts);
+}
 
 template <int WM, int WN, int MI, int NI, bool FORWARD>
 __global__ __launch_bounds__(WM * WN * 64, 2) void sep_gemm_kernel(SepGemm g) {
@@ -1117,26 +1154,30 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void sep_gemm_kernel(SepGemm g) {
     if (!sep_takes(head)) return;
     const int R = __builtin_amdgcn_readfirstlane(head->terms);
     const int harmonics = __builtin_amdgcn_readfirstlane(head->harmonics);
-    const int harmonics_dx = FORWARD ? 0 : __builtin_amdgcn_readfirstlane(head->harmonics_dx);
-    // the product this block works on, its rows and slabs, and the blocks of four values per input
-    int id = blockIdx.x, which = 0, ta = 0, tb = 0, n = 0, slabs = 0, pair_slabs = 0, per = 0;
+    // the product this block works on: its rows, their bytes, and the slabs of each kind
+    int id = blockIdx.x, which = 0, ta = 0, tb = 0, n = 0, values = 0, n1 = 0, n2 = 0, n3 = 0;
+    unsigned pitch_a = 0, pitch_b = 0, base2 = 0, base3 = 0;  // (an operand holds less than 4 GiB)
     int64_t a_rows = 0;
     for (;; ++which) {
         if (which >= g.n) return;
         const SepProduct& p = g.p[which];
         if constexpr (FORWARD) {
+            const SepRow row(g.K, R, harmonics);
             a_rows = p.a_rows;
-            pair_slabs = (int)sep_slabs_pairs(p.inner, R);
-            slabs = pair_slabs + (int)sep_slabs_singles(p.inner, R, harmonics);
+            n1 = (int)(row.pairs / 128);
+            n2 = (int)((row.triples - row.pairs) / 128);
+            n3 = (int)((row.bytes - row.triples) / 96);
+            base2 = (unsigned)row.pairs;
+            base3 = (unsigned)row.triples;
+            pitch_a = pitch_b = (unsigned)row.bytes;
         } else {
-            const bool pairs = p.kind == kSepDx || p.kind == kSepDv;
-            per = p.kind == kSepDxHarm             ? harmonics_dx * R / 8
-                  : p.kind == kSepDvHarm           ? harmonics * R / 8
-                  : p.kind == kSepDv && g.dv_all ? R / 4
-                                                   : R / 8;
-            a_rows = (p.a_rows + 1) / 2 * 8 * per;
-            slabs = (int)(pairs ? sep_slabs(p.inner) : sep_slabs64(p.inner));
-            pair_slabs = pairs ? slabs : 0;
+            values = sep_values(p.kind, p.parts, R, harmonics);
+            a_rows = sep_rows(p.a_rows, values);
+            n1 = p.parts <= 1 ? (int)(p.inner / 64) : 0;
+            n2 = p.parts == 2 ? (int)(p.inner / 32) : 0;
+            n3 = p.parts == 3 ? (int)(p.inner / 16) : 0;
+            pitch_a = (unsigned)p.inner * (p.parts == 3 ? 6 : p.parts == 2 ? 4 : 2);
+            pitch_b = (unsigned)p.inner * (p.parts >= 2 ? 6 : 2);  // G as pairs: its triples' first parts
         }
         ta = (int)((a_rows + TM - 1) / TM);
         tb = (int)((p.b_rows + TN - 1) / TN);
@@ -1156,22 +1197,27 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void sep_gemm_kernel(SepGemm g) {
     const int height = min(4, ta - group * 4);
     const int tile_a = group * 4 + in_group % height, tile_b = in_group / height;
     const int64_t a0 = (int64_t)tile_a * TM, b0 = (int64_t)tile_b * TN;
+    const int slabs = n1 + n2 + n3;
     const int s_begin = (int)((int64_t)slabs * split / p.n_split);
     const int s_end = (int)((int64_t)slabs * (split + 1) / p.n_split);
 
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wr = wave / WN, wc = wave % WN;
+    // this thread's 16 bytes of a slab's rows: where they lie in memory
     const int row0 = t >> 3, part = (t & 7) ^ ((row0 >> 1) & 7);
-    unsigned pa[kLoadA], pb[kLoadB];  // byte offsets (an operand holds less than 4 GiB)
+    const unsigned off = part * 16, off_b2 = FORWARD ? off : (part >> 2) * 96 + (part & 3) * 16;
+    const unsigned off3 = (part < 6 ? part : part - 6) * 16;  // (a slab of triples has six)
+    constexpr unsigned kStrideB2 = FORWARD ? 128 : 192;
+    unsigned pa[kLoadA], pb[kLoadB];
 #pragma unroll
     for (int q = 0; q < kLoadA; ++q) {
         const int64_t row = a0 + row0 + q * kRowStep;
-        pa[q] = (unsigned)(((row < a_rows ? row : a_rows - 1) * slabs * 8 + part) * 16);
+        pa[q] = (unsigned)(row < a_rows ? row : a_rows - 1) * pitch_a;
     }
 #pragma unroll
     for (int q = 0; q < kLoadB; ++q) {
         const int64_t row = b0 + row0 + q * kRowStep;
-        pb[q] = (unsigned)(((row < p.b_rows ? row : p.b_rows - 1) * slabs * 8 + part) * 16);
+        pb[q] = (unsigned)(row < p.b_rows ? row : p.b_rows - 1) * pitch_b;
     }
     constexpr int kBuf = (TM + TN) * 128;
     // kRowStep rows further on the swizzle is the same: kRowStep is a multiple of 16
@@ -1193,216 +1239,258 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void sep_gemm_kernel(SepGemm g) {
     // a wave's loads of a slab: eight rows of 128 bytes each, straight into LDS (lane i to byte
     // 16 i of the kilobyte): the lane that fills part p of a row reads part p ^ (row / 2 % 8)
     auto copy = [&](int s, int buf) {
+        unsigned ua, ub;
+        if (s < n1) {
+            ua = ub = (unsigned)s * 128u + off;
+        } else if (s < n1 + n2) {
+            ua = base2 + (unsigned)(s - n1) * 128u + off;
+            ub = base2 + (unsigned)(s - n1) * kStrideB2 + off_b2;
+        } else {
+            ua = ub = base3 + (unsigned)(s - n1 - n2) * 96u + off3;
+        }
         char* dst = s_sep + buf * kBuf + wave * 1024;
 #pragma unroll
         for (int q = 0; q < kLoadA; ++q)
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(abase + (pa[q] + (unsigned)s * 128u)),
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(abase + (pa[q] + ua)),
                                              (__attribute__((address_space(3))) void*)(dst + q * kThreads * 16), 16, 0, 0);
 #pragma unroll
         for (int q = 0; q < kLoadB; ++q)
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(bbase + (pb[q] + (unsigned)s * 128u)),
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(bbase + (pb[q] + ub)),
                                              (__attribute__((address_space(3))) void*)(dst + TM * 128 + q * kThreads * 16), 16, 0, 0);
     };
-    auto multiply = [&](const sep_h8* u, const sep_h8* v) {
+    auto multiply = [&](const sep_b8* u, const sep_b8* v) {
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
             for (int j = 0; j < NI; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(u[i], v[j], acc[i][j], 0, 0, 0);
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(u[i], v[j], acc[i][j], 0, 0, 0);
+    };
+    // 16-byte part `index` (even) + fh of the wave's rows
+    auto fragments = [&](const char* base, int index, sep_b8* u, sep_b8* v) {
+        const int at = frag ^ (index << 4);
+#pragma unroll
+        for (int i = 0; i < MI; ++i) u[i] = *reinterpret_cast<const sep_b8*>(base + fa + i * 4096 + at);
+#pragma unroll
+        for (int j = 0; j < NI; ++j) v[j] = *reinterpret_cast<const sep_b8*>(base + fb + j * 4096 + at);
     };
     if (s_begin < s_end) copy(s_begin, 0);
     int s = s_begin;
-    const int pair_end = min(s_end, pair_slabs);
-    for (; s < pair_end; ++s) {
+    for (const int end = min(s_end, n1); s < end; ++s) {
         const int buf = (s - s_begin) & 1;
         __syncthreads();  // this slab has landed, and the other buffer's has been read
         const char* base = s_sep + buf * kBuf;
-        sep_h8 ah[2][MI], al[2][MI], bh[2][NI], bl[2][NI];
+        sep_b8 av[4][MI], bv[4][NI];
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            const int off = frag ^ (ks << 5);  // parts ks * 2 + fh (hi), + 4 (lo)
+        for (int ks = 0; ks < 4; ++ks) fragments(base, 2 * ks, av[ks], bv[ks]);
+        if (s + 1 < s_end) copy(s + 1, buf ^ 1);
 #pragma unroll
-            for (int j = 0; j < NI; ++j) bh[ks][j] = *reinterpret_cast<const sep_h8*>(base + fb + j * 4096 + off);
+        for (int ks = 0; ks < 4; ++ks) multiply(av[ks], bv[ks]);
+    }
+    for (const int end = min(s_end, n1 + n2); s < end; ++s) {
+        const int buf = (s - s_begin) & 1;
+        __syncthreads();
+        const char* base = s_sep + buf * kBuf;
+        sep_b8 av[4][MI], bv[4][NI];  // parts 1 and 2 of the first 16 elements, then of the others
 #pragma unroll
-            for (int i = 0; i < MI; ++i) ah[ks][i] = *reinterpret_cast<const sep_h8*>(base + fa + i * 4096 + off);
-#pragma unroll
-            for (int j = 0; j < NI; ++j) bl[ks][j] = *reinterpret_cast<const sep_h8*>(base + fb + j * 4096 + (off ^ 64));
-#pragma unroll
-            for (int i = 0; i < MI; ++i) al[ks][i] = *reinterpret_cast<const sep_h8*>(base + fa + i * 4096 + (off ^ 64));
-        }
+        for (int q = 0; q < 4; ++q) fragments(base, 2 * q, av[q], bv[q]);
         if (s + 1 < s_end) copy(s + 1, buf ^ 1);
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
-            multiply(ah[ks], bh[ks]);
-            multiply(ah[ks], bl[ks]);
-            multiply(al[ks], bh[ks]);
+            multiply(av[2 * ks + 1], bv[2 * ks]);
+            multiply(av[2 * ks], bv[2 * ks + 1]);
+            multiply(av[2 * ks], bv[2 * ks]);
         }
     }
     for (; s < s_end; ++s) {
         const int buf = (s - s_begin) & 1;
         __syncthreads();
         const char* base = s_sep + buf * kBuf;
-        sep_h8 av[4][MI], bv[4][NI];
+        sep_b8 av[3][MI], bv[3][NI];
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            const int off = frag ^ (ks << 5);
-#pragma unroll
-            for (int i = 0; i < MI; ++i) av[ks][i] = *reinterpret_cast<const sep_h8*>(base + fa + i * 4096 + off);
-#pragma unroll
-            for (int j = 0; j < NI; ++j) bv[ks][j] = *reinterpret_cast<const sep_h8*>(base + fb + j * 4096 + off);
-        }
+        for (int q = 0; q < 3; ++q) fragments(base, 2 * q, av[q], bv[q]);
         if (s + 1 < s_end) copy(s + 1, buf ^ 1);
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) multiply(av[ks], bv[ks]);
+        for (int i = 0; i < MI; ++i) {
+            sep_f16 sum[NI] = {};
+            auto add = [&](int pa_, int pb_) {
+#pragma unroll
+                for (int j = 0; j < NI; ++j)
+                    sum[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[pa_][i], bv[pb_][j], sum[j], 0, 0, 0);
+            };
+            add(2, 0);
+            add(0, 2);
+            add(1, 1);
+            add(1, 0);
+            add(0, 1);
+            add(0, 0);
+#pragma unroll
+            for (int j = 0; j < NI; ++j) acc[i][j] += sum[j];
+        }
     }
 
     // lane (fl, fh) holds rows q % 4 + 8 (q / 4) + 4 fh of column fl of each 32 x 32 tile
     if constexpr (FORWARD) {
         float* out = p.out + (int64_t)split * g.M * g.O;
+        const float inv = head->inv_scale;
 #pragma unroll
         for (int i = 0; i < MI; ++i) {
 #pragma unroll
             for (int q = 0; q < 16; ++q) {
                 const int64_t m = a0 + (wr * MI + i) * 32 + (q & 3) + 8 * (q >> 2) + 4 * fh;
                 if (m >= g.M) continue;
-                const float sc = g.xscale[m];
 #pragma unroll
                 for (int j = 0; j < NI; ++j) {
                     const int64_t o = b0 + (wc * NI + j) * 32 + fl;
-                    if (o < g.O) out[m * g.O + o] = acc[i][j][q] * sc;
+                    if (o < g.O) out[m * g.O + o] = acc[i][j][q] * inv;
                 }
             }
         }
     } else {
         const SepHead h = *head;
-        const int kind = p.kind;
-        const bool harm = kind >= kSepDxHarm, upper = kind == kSepDxUpper || kind == kSepDvUpper;
-        const int sh = __builtin_ctz(per), j_first = upper ? R / 2 : 0;
-        const bool eight = R == 8;
-        if (kind == kSepDx || kind == kSepDxUpper || kind == kSepDxHarm) {
+        // two: a lane's block of four results holds two values of two inputs, otherwise four of one
+        const bool harm = p.parts == 0, two = values == 2;
+        const int per = two ? 1 : values / 4, sh = __builtin_ctz(per);
+        const int first = harm ? 0 : sep_classes(R, p.kind == kSepDv).first(p.parts);
+        float inv_g;
+        (void)sep_grad_scale(head, &inv_g);
+        // keeps the loads of the results that follow from being hoisted: the sums leave few registers
+        auto fence = [] { __builtin_amdgcn_sched_barrier(0); };
+        // block (i, q) of this wave's rows
+        auto block_of = [&](int i, int q) { return (int)(a0 / 8) + (wr * MI + i) * 4 + q; };
+        const int K = (int)g.K, M = (int)g.M, O = (int)g.O, Op = (int)g.Op;  // (an operand holds less than 4 GiB)
+        if (p.kind == kSepDx) {
             const float as = g.in_affine ? g.in_affine[0] : 1.0f, ab = g.in_affine ? g.in_affine[1] : 0.0f;
             float* out = p.out + (int64_t)split * g.M * g.K;
+            const float sc = harm ? inv_g * h.inv_scale : inv_g;
+            auto each = [&](auto values_of) {  // values_of(x, block of four in the input) -> their four factors
 #pragma unroll
-            for (int j = 0; j < NI; ++j) {
-                const int64_t m = b0 + (wc * NI + j) * 32 + fl;
-                const int64_t mc = m < g.M ? m : g.M - 1;
-                const float sc = g.gscale[mc];
-                float sum = 0.0f;
+                for (int j = 0; j < NI; ++j) {
+                    const int m = (int)b0 + (wc * NI + j) * 32 + fl;
+                    const int mc = m < M ? m : M - 1;
+                    const float* xrow = g.x + (int64_t)mc * K;
+                    float* orow = out + (int64_t)mc * K;
+                    float sum = 0.0f;
 #pragma unroll
-                for (int i = 0; i < MI; ++i) {
+                    for (int i = 0; i < MI; ++i) {
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) {  // block jb of inputs k (fh = 0) and k + 1
-                        const int64_t block = (a0 + (wr * MI + i) * 32) / 8 + q;
-                        const int64_t k = (block >> sh) * 2 + fh;
-                        const int jb = (int)block & (per - 1);
-                        const float xr = g.x[mc * g.K + (k < g.K ? k : g.K - 1)];
-                        const float x = g.in_affine ? input_map(xr, as, ab, g.in_lo, g.in_hi) : xr;
-                        const SepAt at = sep_at(h, x);
-                        float4 v;
-                        if (!harm) {
-                            v = sep_eval4(g.tab2, R, at, j_first + 4 * jb);
-                        } else {
-                            const bool second = eight ? jb & 1 : jb & 2;
-                            const float th = (x - h.lut_min) * h.lut_scale * (second ? 2.0f : 1.0f);
-                            const float f = th - floorf(th), w = second ? 0.25f : 1.0f;
-                            const float c = __builtin_amdgcn_cosf(f) * w, sn = __builtin_amdgcn_sinf(f) * w;
-                            float e[4];
-                            sep_second(h, g.tabE, at, e);
-                            if (eight) {
-                                v = make_float4(e[0] * c, e[1] * c, e[0] * sn, e[1] * sn);
-                            } else {
-                                const float tr = jb & 1 ? sn : c;
-                                v = make_float4(e[0] * tr, e[1] * tr, e[2] * tr, e[3] * tr);
+                        for (int q = 0; q < 4; ++q) {
+                            const int k = (block_of(i, q) >> sh) * 2 + fh, jb = block_of(i, q) & (per - 1);
+                            const float xr = xrow[k < K ? k : K - 1];
+                            const float4 v = values_of(g.in_affine ? input_map(xr, as, ab, g.in_lo, g.in_hi) : xr, jb);
+                            sum = fmaf(acc[i][j][4 * q], v.x, sum);
+                            sum = fmaf(acc[i][j][4 * q + 1], v.y, sum);
+                            sum = fmaf(acc[i][j][4 * q + 2], v.z, sum);
+                            sum = fmaf(acc[i][j][4 * q + 3], v.w, sum);
+                            if (jb == per - 1) {
+                                if (m < M && k < K) orow[k] = sum * sc;
+                                sum = 0.0f;
                             }
+                            fence();
                         }
-                        sum = fmaf(acc[i][j][4 * q], v.x, sum);
-                        sum = fmaf(acc[i][j][4 * q + 1], v.y, sum);
-                        sum = fmaf(acc[i][j][4 * q + 2], v.z, sum);
-                        sum = fmaf(acc[i][j][4 * q + 3], v.w, sum);
-                        if (jb == per - 1) {
-                            if (m < g.M && k < g.K) out[m * g.K + k] = sum * sc;
-                            sum = 0.0f;
+                    }
+                }
+            };
+            if (harm) {
+                each([&](float x, int jb) {
+                    const SepAt at = sep_at(h, x);
+                    const float th = (x - h.lut_min) * h.lut_scale * (float)(jb + 1);
+                    const float f = th - floorf(th), w = sep_harm_weight(jb);
+                    const float c = __builtin_amdgcn_cosf(f) * w, sn = __builtin_amdgcn_sinf(f) * w;
+                    const float2 e = sep_second(g.tabE, at);
+                    return make_float4(e.x * c, e.y * c, e.x * sn, e.y * sn);
+                });
+            } else if (!two) {
+                each([&](float x, int jb) { return sep_eval4(g.tab2, R, sep_at(h, x), first + 4 * jb); });
+            } else {
+#pragma unroll
+                for (int j = 0; j < NI; ++j) {
+                    const int m = (int)b0 + (wc * NI + j) * 32 + fl;
+                    const int mc = m < M ? m : M - 1;
+                    const float* xrow = g.x + (int64_t)mc * K;
+                    float* orow = out + (int64_t)mc * K;
+#pragma unroll
+                    for (int i = 0; i < MI; ++i) {
+#pragma unroll
+                        for (int q = 0; q < 8; ++q) {
+                            const int k = block_of(i, q >> 1) * 4 + 2 * fh + (q & 1);
+                            const float xr = xrow[k < K ? k : K - 1];
+                            const float x = g.in_affine ? input_map(xr, as, ab, g.in_lo, g.in_hi) : xr;
+                            const float2 v = sep_eval2(g.tab2, R, sep_at(h, x), first);
+                            if (m < M && k < K)
+                                orow[k] = fmaf(acc[i][j][2 * q + 1], v.y, acc[i][j][2 * q] * v.x) * sc;
+                            if (q & 1) fence();
                         }
                     }
                 }
             }
         } else {
             float* out = p.out + (int64_t)split * 2 * g.Kp * g.Op;
+            const float sc = inv_g * h.inv_scale;
+            const int64_t branch = g.Kp * Op;
+            auto store = [&](int k, int o, float vp, float vn) {
+                if (o >= O || k >= K) return;
+                float* at = out + (int64_t)k * Op + o;
+                at[0] = vp * sc;
+                at[branch] = vn * sc;
+            };
+            if (two) {
 #pragma unroll
-            for (int j = 0; j < NI; ++j) {
-                const int64_t o = b0 + (wc * NI + j) * 32 + fl;
-                const int64_t oc = o < g.O ? o : g.O - 1;
-                const float sb = g.gscaleT[oc];
-                float sp = 0.0f, sn = 0.0f, p0 = 0.0f, p1 = 0.0f, n0 = 0.0f, n1 = 0.0f;
-                float2 tt = make_float2(0.0f, 0.0f);
+                for (int j = 0; j < NI; ++j) {
+                    const int o = (int)b0 + (wc * NI + j) * 32 + fl, oc = o < O ? o : O - 1;
 #pragma unroll
-                for (int i = 0; i < MI; ++i) {
+                    for (int i = 0; i < MI; ++i) {
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const int64_t block = (a0 + (wr * MI + i) * 32) / 8 + q;
-                        const int64_t k = (block >> sh) * 2 + fh;
-                        const int jb = (int)block & (per - 1);
-                        if (jb == 0) tt = g.tT[(k < g.K ? k : g.K - 1) * g.Op + oc];
-                        const float a0_ = acc[i][j][4 * q], a1_ = acc[i][j][4 * q + 1], a2_ = acc[i][j][4 * q + 2],
-                                    a3_ = acc[i][j][4 * q + 3];
-                        float rp = 0.0f, rn = 0.0f;
-                        if (!harm) {
-                            if (jb == 0) {
-                                if (!upper) {  // T_0, T_1
-                                    p0 = n0 = 1.0f;
-                                    p1 = tt.x;
-                                    n1 = tt.y;
-                                } else {  // T_(R/2), T_(R/2 + 1) = cos(j acos t): 1e-5, of terms below 4e-3
-                                    const float u = acosf(fminf(fmaxf(tt.x, -1.0f), 1.0f)) * 0.15915494f;
-                                    const float w = acosf(fminf(fmaxf(tt.y, -1.0f), 1.0f)) * 0.15915494f;
-                                    const float jf = (float)j_first;
-                                    auto cosj = [](float r) { return __builtin_amdgcn_cosf(r - floorf(r)); };
-                                    p0 = cosj(u * jf);
-                                    p1 = cosj(u * (jf + 1.0f));
-                                    n0 = cosj(w * jf);
-                                    n1 = cosj(w * (jf + 1.0f));
-                                }
-                            }
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) {
-                                rp = fmaf(acc[i][j][4 * q + e], p0, rp);
-                                rn = fmaf(acc[i][j][4 * q + e], n0, rn);
-                                const float p2 = fmaf(2.0f * tt.x, p1, -p0), n2 = fmaf(2.0f * tt.y, n1, -n0);
-                                p0 = p1;
-                                p1 = p2;
-                                n0 = n1;
-                                n1 = n2;
-                            }
-                        } else {
-                            const bool second = eight ? jb & 1 : jb & 2;
-                            const float ws = h.lut_scale * (second ? 2.0f : 1.0f);
-                            const float tp = ((float)h.wc + (float)h.wh * tt.x) * ws, tn = ((float)h.wc + (float)h.wh * tt.y) * ws;
-                            const float fp = tp - floorf(tp), fn = tn - floorf(tn);
-                            const float cp = __builtin_amdgcn_cosf(fp), dp = __builtin_amdgcn_sinf(fp);
-                            const float cn = __builtin_amdgcn_cosf(fn), dn = __builtin_amdgcn_sinf(fn);
-                            if (eight) {
-                                rp = cp * fmaf(a1_, tt.x, a0_) + dp * fmaf(a3_, tt.x, a2_);
-                                rn = cn * fmaf(a1_, tt.y, a0_) + dn * fmaf(a3_, tt.y, a2_);
-                            } else {
-                                float vp[4], vn[4];
-                                sep_cheb4(tt.x, vp);
-                                sep_cheb4(tt.y, vn);
-                                rp = (jb & 1 ? dp : cp) * fmaf(a3_, vp[3], fmaf(a2_, vp[2], fmaf(a1_, vp[1], a0_)));
-                                rn = (jb & 1 ? dn : cn) * fmaf(a3_, vn[3], fmaf(a2_, vn[2], fmaf(a1_, vn[1], a0_)));
-                            }
-                        }
-                        sp += rp;
-                        sn += rn;
-                        if (jb == per - 1) {
-                            if (o < g.O && k < g.K) {
-                                const float sc = sb * g.xscale[k];
-                                out[k * g.Op + o] = sp * sc;
-                                out[(g.Kp + k) * g.Op + o] = sn * sc;
-                            }
-                            sp = sn = 0.0f;
+                        for (int q = 0; q < 8; ++q) {
+                            const int k = block_of(i, q >> 1) * 4 + 2 * fh + (q & 1);
+                            const float2 tt = g.tT[(int64_t)(k < K ? k : K - 1) * Op + oc];
+                            const float2 up = sep_cheb_from(first, tt.x), un = sep_cheb_from(first, tt.y);
+                            store(k, o, fmaf(acc[i][j][2 * q + 1], up.y, acc[i][j][2 * q] * up.x),
+                                  fmaf(acc[i][j][2 * q + 1], un.y, acc[i][j][2 * q] * un.x));
+                            if (q & 1) fence();
                         }
                     }
                 }
+                return;
+            }
+            // share(block of four in the input, their sums, t+ or t-) -> what they add
+            auto each = [&](auto share) {
+#pragma unroll
+                for (int j = 0; j < NI; ++j) {
+                    const int o = (int)b0 + (wc * NI + j) * 32 + fl, oc = o < O ? o : O - 1;
+                    float sp = 0.0f, sn = 0.0f;
+#pragma unroll
+                    for (int i = 0; i < MI; ++i) {
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            const int k = (block_of(i, q) >> sh) * 2 + fh, jb = block_of(i, q) & (per - 1);
+                            const float2 tt = g.tT[(int64_t)(k < K ? k : K - 1) * Op + oc];
+                            const float4 r = make_float4(acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2],
+                                                         acc[i][j][4 * q + 3]);
+                            sp += share(jb, r, tt.x);
+                            sn += share(jb, r, tt.y);
+                            if (jb == per - 1) {
+                                store(k, o, sp, sn);
+                                sp = sn = 0.0f;
+                            }
+                            if (q & 1) fence();
+                        }
+                    }
+                }
+            };
+            if (harm) {
+                each([&](int jb, float4 r, float tv) {
+                    const float th = ((float)h.wc + (float)h.wh * tv) * (h.lut_scale * (float)(jb + 1));
+                    const float f = th - floorf(th);
+                    const float2 u = sep_kink_functions(h, tv);
+                    return __builtin_amdgcn_cosf(f) * fmaf(r.y, u.y, r.x * u.x) +
+                           __builtin_amdgcn_sinf(f) * fmaf(r.w, u.y, r.z * u.x);
+                });
+            } else {
+                each([&](int jb, float4 r, float tv) {
+                    const float2 u = sep_cheb_from(first + 4 * jb, tv);
+                    const float u2 = fmaf(2.0f * tv, u.y, -u.x), u3 = fmaf(2.0f * tv, u2, -u.y);
+                    return fmaf(r.w, u3, fmaf(r.z, u2, fmaf(r.y, u.y, r.x * u.x)));
+                });
             }
         }
     }
@@ -1472,15 +1560,15 @@ __global__ __launch_bounds__(256) void sep_reduce_bwd_kernel(DxReduceArgs dx, Dx
 struct SepPlan {
     int max_terms;  // 0: not considered
     bool big;       // 256 x 256 tiles instead of 128 x 128
-    int split, split_dx, split_dv, split_dxs, split_dvs, split_dxh, split_dvh;
+    int split;                     // forward
+    int split_dx[4], split_dv[4];  // backward: of the harmonics, the singles, pairs and triples
     int planes_dx, planes_dv;
     int64_t Kp, Op;
-    size_t off_head, off_part, off_row, off_col, off_grow, off_gcol, off_tab, off_tab2, off_tabE, off_lut, off_xop, off_wop,
-        off_xops, off_wops, off_xoph, off_woph, off_gop, off_gopT, off_goph, off_gophT, off_scale, off_gscale, off_gscaleT, off_tT,
-        off_planes, off_planes_dv, bytes;
+    size_t off_head, off_part, off_tab, off_tab2, off_tabE, off_lut, off_xop, off_wop, off_xcls[4], off_wcls[4], off_gop,
+        off_gops, off_gopT, off_gopTs, off_tT, off_planes, off_planes_dv, bytes;
 };
 
-constexpr int64_t kSepOperandBytes = (int64_t)2 << 30;  // of one operand, at most (32-bit byte offsets)
+constexpr int64_t kSepOperandBytes = ((int64_t)4 << 30) - (1 << 20);  // of one operand, at most (32-bit byte offsets)
 
 // Splits of a product's inner length: the count (each at least 8 slabs) that makes the launch's
 // time least, in slabs of one tile: rounds of blocks over the CUs (one 256 x 256 block each,
@@ -1517,14 +1605,17 @@ SepPlan plan_sep(int lut_n, int64_t M, int64_t K, int64_t O, bool backward, bool
         return p;
     p.Kp = round_up(K, 8);
     p.Op = round_up(O, 256);
-    const int64_t Mr = round_up(M, 64), Or = round_up(O, 64), Kr = sep_inputs(K);
-    const int harm = lut_n > 0 ? 1 : 0;
-    // bytes per (row, input), forward: R / 2 pairs, R / 2 singles and the harmonics; an operand's
-    // size backward: at most R pairs
-    auto width = [&](int terms) { return (int64_t)terms * (backward ? 4 : 3 + 2 * harm); };
+    const int64_t Mi = sep_inner(M), Oi = sep_inner(O), Kr = sep_inputs(K);
+    const bool lut = lut_n > 0;
+    const int most = lut ? kSepMaxHarmonics : 0;  // the device takes as many harmonics as the table needs
     int terms = kSepMaxTerms;
-    while (terms >= 8 && (Mr * Kr * width(terms) >= kSepOperandBytes || Or * Kr * width(terms) >= kSepOperandBytes)) terms /= 2;
-    if (terms < 8 || Mr * Or * 4 >= kSepOperandBytes) return p;
+    auto fits = [&](int r) {  // (a backward's widest operand: dVth's triples, six bytes a value, or the harmonics)
+        const int64_t bytes = backward ? std::max(Mi, Oi) * Kr * std::max(6 * sep_classes(r, true).n3, 8 * most)
+                                       : std::max(M, O) * SepRow(K, r, most).bytes;
+        return bytes < kSepOperandBytes;
+    };
+    while (terms >= 8 && !fits(terms)) terms /= 2;
+    if (terms < 8 || Mi * Oi * 6 >= kSepOperandBytes) return p;
     p.max_terms = terms;
     size_t off = (size_t)round_up((int64_t)base, 256);
     auto take = [&](int64_t bytes) {
@@ -1535,55 +1626,54 @@ SepPlan plan_sep(int lut_n, int64_t M, int64_t K, int64_t O, bool backward, bool
     p.off_head = take(sizeof(SepHead));
     p.off_part = take((kSepStatX + kSepStatW) * 8);
     p.off_tab = take((int64_t)kSepGridMax * 4 * terms);
-    if (lut_n > 0) {
-        p.off_lut = take((int64_t)lut_n * 16 + 256 * 8);
-        p.off_tabE = take((int64_t)kSepGridMax * terms);
+    if (lut) {
+        p.off_lut = take((int64_t)lut_n * 16 + 256 * 16);
+        p.off_tabE = take((int64_t)kSepGridMax * 8);
     }
     if (!backward) {
-        p.off_xop = take(Mr * Kr * width(terms));
-        p.off_wop = take(Or * Kr * width(terms));
-        p.off_row = take(M * 8);
-        p.off_scale = take(M * 4);
-        const int64_t slabs = sep_slabs_pairs(K, 8) + sep_slabs_singles(K, 8, harm);
+        const int64_t row = std::max(SepRow(K, terms, most).bytes, SepRow(K, 8, most).bytes);
+        p.off_xop = take(M * row);
+        p.off_wop = take(O * row);
+        const int64_t slabs = SepRow(K, 8, most).bytes / 112;
         p.big = sep_big(M, O, slabs);
         const int64_t tile = p.big ? 256 : 128;
         p.split = sep_splits(((M + tile - 1) / tile) * ((O + tile - 1) / tile), slabs, p.big, 8.0 * M * O);
         p.off_planes = take((int64_t)p.split * M * O * 4);
     } else {
         p.off_tab2 = take((int64_t)kSepGridMax * 4 * terms);
-        p.off_col = take(kSepColChunks * K * 8);
-        p.off_grow = take(M * 4);
-        p.off_gcol = take(kSepColChunks * O * 4);
-        p.off_gop = take(Mr * Or * 4);
-        p.off_gopT = take(Mr * Or * 4);
-        p.off_goph = take(Mr * Or * 2);
-        p.off_gophT = take(Mr * Or * 2);
-        if (need_w) p.off_xop = take(Mr * Kr * terms * (harm ? 2 : 4));
-        if (need_w && harm) p.off_xops = take(Mr * Kr * terms);
-        if (need_w && harm) p.off_xoph = take(Mr * Kr * terms * 2);
         if (need_x) {
-            p.off_wop = take(Or * Kr * terms * 2);
-            p.off_wops = take(Or * Kr * terms);
-            if (harm) p.off_woph = take(Or * Kr * terms * 2);
+            p.off_gop = take(M * Oi * 6);
+            p.off_gops = take(M * Oi * 2);
         }
-        p.off_scale = take(K * 4);
-        p.off_gscale = take(M * 4);
-        p.off_gscaleT = take(O * 4);
+        if (need_w) {
+            p.off_gopT = take(O * Mi * 6);
+            p.off_gopTs = take(O * Mi * 2);
+        }
+        auto values = [&](int c, bool dv, int r) { return c == 0 ? 4 * most : sep_classes(r, dv).count(c); };
+        auto slabs = [&](int c, int64_t inner) { return inner / (c == 0 ? 64 : c == 3 ? 16 : 64 / c); };
+        auto tiles = [&](int c, bool dv, int64_t tile) {  // at 8 terms
+            return (sep_rows(K, values(c, dv, 8)) + tile - 1) / tile * (((dv ? O : M) + tile - 1) / tile);
+        };
+        // the work of both gradients in slabs of 256 x 256 tiles: 64 per CU take them (16384 tokens, 384 x
+        // 1536, 4096 entries: 1.93 ms against 2.16 with 128 x 128), whichever gradient the call wants, so
+        // that each has the same bits
+        int64_t work = 0;
+        for (int c = 0; c < 4; ++c) work += tiles(c, false, 256) * slabs(c, Oi) + tiles(c, true, 256) * slabs(c, Mi);
+        p.big = work >= 64 * kCUs && K >= 64 && M >= 192 && O >= 192;
+        for (int c = 0; c < 4; ++c) {  // the harmonics, singles, pairs, triples
+            const int bytes = c == 0 ? 2 : 2 * c;
+            const int vx = std::max(values(c, false, 8), values(c, false, terms));
+            const int vw = std::max(values(c, true, 8), values(c, true, terms));
+            if (vx == 0) continue;
+            if (need_w) p.off_xcls[c] = take(Kr * vw * Mi * bytes);
+            if (need_x) p.off_wcls[c] = take(Kr * vx * Oi * bytes);
+            const int64_t tile = p.big ? 256 : 128;
+            p.split_dx[c] = sep_splits(tiles(c, false, tile), slabs(c, Oi), p.big, 8.0 * M * K);
+            p.split_dv[c] = sep_splits(tiles(c, true, tile), slabs(c, Mi), p.big, 16.0 * p.Kp * p.Op);
+            p.planes_dx += p.split_dx[c];
+            p.planes_dv += p.split_dv[c];
+        }
         p.off_tT = take(K * p.Op * 8);
-        p.big = sep_big(8 * K, std::min(M, O), std::min(M, O) / 32);
-        // at 8 terms: 4 rows per input of lower and of upper terms (8 of the formula's dVth), 4 of a harmonic
-        // (dX has two below ~6000 entries)
-        const int64_t tile = p.big ? 256 : 128, t4 = (4 * K + tile - 1) / tile, t8 = (8 * K + tile - 1) / tile;
-        const int64_t tm = (M + tile - 1) / tile, to = (O + tile - 1) / tile;
-        const double dx_bytes = 8.0 * M * K, dv_bytes = 16.0 * p.Kp * p.Op;
-        p.split_dx = sep_splits(t4 * tm, (O + 31) / 32, p.big, dx_bytes);
-        p.split_dxs = sep_splits(t4 * tm, (O + 63) / 64, p.big, dx_bytes);
-        p.split_dv = sep_splits((harm ? t4 : t8) * to, (M + 31) / 32, p.big, dv_bytes);
-        p.split_dvs = harm ? sep_splits(t4 * to, (M + 63) / 64, p.big, dv_bytes) : 0;
-        p.split_dxh = harm ? sep_splits((lut_n < 6000 ? t8 : t4) * tm, (O + 63) / 64, p.big, dx_bytes) : 0;
-        p.split_dvh = harm ? sep_splits(t4 * to, (M + 63) / 64, p.big, dv_bytes) : 0;
-        p.planes_dx = p.split_dx + p.split_dxs + p.split_dxh;
-        p.planes_dv = p.split_dv + p.split_dvs + p.split_dvh;
         if (need_x) p.off_planes = take((int64_t)p.planes_dx * M * K * 4);
         if (need_w) p.off_planes_dv = take((int64_t)p.planes_dv * 2 * p.Kp * p.Op * 4);
     }
@@ -1605,18 +1695,20 @@ void sep_point(const SepPlan& p, SepArgs& a, char* ws) {
     a.wpart = a.xpart + kSepStatX;
     a.tab = reinterpret_cast<float*>(ws + p.off_tab);
     a.tabE = reinterpret_cast<float*>(ws + p.off_tabE);
-    a.lut_info = reinterpret_cast<float2*>(ws + p.off_lut);
-    a.lut_val = reinterpret_cast<double2*>(ws + p.off_lut + 256 * 8);
-    a.xop = reinterpret_cast<_Float16*>(ws + p.off_xop);
-    a.wop = reinterpret_cast<_Float16*>(ws + p.off_wop);
-    a.xscale = reinterpret_cast<float*>(ws + p.off_scale);
+    a.lut_info = reinterpret_cast<float4*>(ws + p.off_lut);
+    a.lut_val = reinterpret_cast<double2*>(ws + p.off_lut + 256 * 16);
     a.max_terms = p.max_terms;
+}
+
+void sep_point_forward(const SepPlan& p, SepArgs& a, char* ws) {
+    sep_point(p, a, ws);
+    a.xop = ws + p.off_xop;
+    a.wop = ws + p.off_wop;
 }
 
 // The forward's operands (and, where it does not take the call, the per-cell kernels' prep).
 hipError_t sep_forward_operands(const SepPlan& p, SepArgs a, const PrepArgs& prep, char* ws, hipStream_t s) {
-    sep_point(p, a, ws);
-    a.xrow = reinterpret_cast<float2*>(ws + p.off_row);
+    sep_point_forward(p, a, ws);
     hipLaunchKernelGGL(sep_stat_kernel, dim3(kSepStatX + kSepStatW + (a.lut_n + 255) / 256), dim3(256), 0, s, a,
                        prep, GlueGradArgs{});
     hipLaunchKernelGGL(sep_table_kernel, dim3(kSepTableBlocks), dim3(256), 0, s, a);
@@ -1628,16 +1720,14 @@ hipError_t sep_forward_operands(const SepPlan& p, SepArgs a, const PrepArgs& pre
 
 // The forward's product, into its planes.
 hipError_t sep_forward_product(const SepPlan& p, SepArgs a, char* ws, hipStream_t s) {
-    sep_point(p, a, ws);
+    sep_point_forward(p, a, ws);
     SepGemm g{};
     g.head = a.head;
     g.M = a.M;
     g.K = a.K;
     g.O = a.O;
-    g.xscale = a.xscale;
     g.n = 1;
-    g.p[0] = SepProduct{reinterpret_cast<const char*>(a.xop), reinterpret_cast<const char*>(a.wop), kSepForward, a.M, a.O,
-                        a.K, p.split, reinterpret_cast<float*>(ws + p.off_planes)};
+    g.p[0] = SepProduct{a.xop, a.wop, kSepForward, 0, a.M, a.O, 0, p.split, reinterpret_cast<float*>(ws + p.off_planes)};
     const int64_t tile = p.big ? 256 : 128;
     launch_sep_gemm<true>(p.big, (unsigned)((a.M + tile - 1) / tile * ((a.O + tile - 1) / tile) * p.split), g, s);
     return hipGetLastError();
@@ -1645,20 +1735,16 @@ hipError_t sep_forward_product(const SepPlan& p, SepArgs a, char* ws, hipStream_
 
 void sep_point_backward(const SepPlan& p, SepArgs& a, char* ws) {
     sep_point(p, a, ws);
-    a.xcol = a.need_w ? reinterpret_cast<float2*>(ws + p.off_col) : nullptr;
-    a.grow = reinterpret_cast<unsigned*>(ws + p.off_grow);
-    a.gcol = reinterpret_cast<unsigned*>(ws + p.off_gcol);
     a.tab2 = reinterpret_cast<float*>(ws + p.off_tab2);
-    a.gop = reinterpret_cast<_Float16*>(ws + p.off_gop);
-    a.gopT = reinterpret_cast<_Float16*>(ws + p.off_gopT);
-    a.xops = reinterpret_cast<_Float16*>(ws + p.off_xops);
-    a.wops = reinterpret_cast<_Float16*>(ws + p.off_wops);
-    a.xoph = reinterpret_cast<_Float16*>(ws + p.off_xoph);
-    a.woph = reinterpret_cast<_Float16*>(ws + p.off_woph);
-    a.goph = reinterpret_cast<_Float16*>(ws + p.off_goph);
-    a.gophT = reinterpret_cast<_Float16*>(ws + p.off_gophT);
-    a.gscale = reinterpret_cast<float*>(ws + p.off_gscale);
-    a.gscaleT = reinterpret_cast<float*>(ws + p.off_gscaleT);
+    // (harmonics last)
+    for (int c = 0; c < 4; ++c) {
+        a.xcls[(c + 3) % 4] = ws + p.off_xcls[c];
+        a.wcls[(c + 3) % 4] = ws + p.off_wcls[c];
+    }
+    a.gop = ws + p.off_gop;
+    a.gops = ws + p.off_gops;
+    a.gopT = ws + p.off_gopT;
+    a.gopTs = ws + p.off_gopTs;
     a.tT = reinterpret_cast<float2*>(ws + p.off_tT);
     a.Op = p.Op;
 }
@@ -1667,14 +1753,12 @@ void sep_point_backward(const SepPlan& p, SepArgs& a, char* ws) {
 hipError_t sep_backward_operands(const SepPlan& p, SepArgs a, const PrepArgs& prep, const GlueGradArgs* glue, char* ws,
                                  hipStream_t s) {
     sep_point_backward(p, a, ws);
-    const int64_t xcols = a.xcol ? kSepColChunks * ((a.K + 255) / 256) : 0;
-    const int64_t stat = kSepStatX + kSepStatW + (a.lut_n + 255) / 256 + xcols + (glue ? (int64_t)kGlueBlocks * (glue->Op / 256) : 0);
+    const int64_t stat = kSepStatX + kSepStatW + (a.lut_n + 255) / 256 + (glue ? (int64_t)kGlueBlocks * (glue->Op / 256) : 0);
     hipLaunchKernelGGL(sep_stat_kernel, dim3((unsigned)stat), dim3(256), 0, s, a, prep,
                        glue ? *glue : GlueGradArgs{});
-    const int64_t gcols = a.need_w ? kSepColChunks * ((a.O + 255) / 256) : 0;
-    hipLaunchKernelGGL(sep_table_kernel, dim3((unsigned)(kSepTableBlocks + kSepStatG + gcols)), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(sep_table_kernel, dim3((unsigned)(kSepTableBlocks + kSepStatG)), dim3(256), 0, s, a);
     const int64_t kt = (a.K + 31) / 32, ot = (a.O + 127) / 128;
-    const int64_t x_blocks = a.need_w ? kt * ((a.M + 127) / 128) : 0, w_blocks = kt * ot, g_blocks = ot * ((a.M + 31) / 32);
+    const int64_t x_blocks = a.need_w ? kt * ((a.M + 127) / 128) : 0, w_blocks = kt * ot, g_blocks = ot * (sep_inner(a.M) / 32);
     const int64_t expand = x_blocks + w_blocks + g_blocks;
     hipLaunchKernelGGL(sep_expand_bwd_kernel, dim3((unsigned)std::max<int64_t>(expand, kPrepBlocksX + kPrepBlocksW)),
                        dim3(256), 0, s, a, (int)x_blocks, (int)w_blocks, prep);
@@ -1691,9 +1775,6 @@ hipError_t sep_backward_products(const SepPlan& p, SepArgs a, char* ws, hipStrea
     g.O = a.O;
     g.Kp = p.Kp;
     g.Op = p.Op;
-    g.xscale = a.xscale;
-    g.gscale = a.gscale;
-    g.gscaleT = a.gscaleT;
     g.x = a.x;
     g.in_affine = a.in_affine;
     g.in_lo = a.in_lo;
@@ -1701,27 +1782,25 @@ hipError_t sep_backward_products(const SepPlan& p, SepArgs a, char* ws, hipStrea
     g.tab2 = a.tab2;
     g.tabE = a.tabE;
     g.tT = a.tT;
-    g.dv_all = a.lut_n > 0 ? 0 : 1;
     const int64_t tile = p.big ? 256 : 128;
     int64_t blocks = 0;
-    auto add = [&](int kind, const _Float16* x, const _Float16* y, int64_t b_rows, int64_t inner, int split, float*& out,
-                   int64_t plane, int rows) {  // rows: of an input, at most
-        if (split < 1) return;
-        g.p[g.n++] = SepProduct{reinterpret_cast<const char*>(x), reinterpret_cast<const char*>(y), kind, a.K, b_rows,
-                                inner, split, out};
+    auto add = [&](int kind, int parts, const char* x, const char* y, int64_t b_rows, int64_t inner, int split, float*& out,
+                   int64_t plane) {
+        g.p[g.n++] = SepProduct{x, y, kind, parts, a.K, b_rows, inner, split, out};
         out += split * plane;
-        blocks += ((a.K + 1) / 2 * 2 * rows + tile - 1) / tile * ((b_rows + tile - 1) / tile) * split;
+        int64_t rows = 0;  // at the most that the device may choose
+        for (int r = 8; r <= p.max_terms; r *= 2) rows = std::max(rows, sep_rows(a.K, sep_values(kind, parts, r, kSepMaxHarmonics)));
+        blocks += (rows + tile - 1) / tile * ((b_rows + tile - 1) / tile) * split;
     };
     float* dx = reinterpret_cast<float*>(ws + p.off_planes);
     float* dv = reinterpret_cast<float*>(ws + p.off_planes_dv);
     const int64_t px = a.M * a.K, pv = 2 * p.Kp * p.Op;
-    const int R = p.max_terms;
-    if (a.need_x) add(kSepDx, a.wop, a.gop, a.M, a.O, p.split_dx, dx, px, R / 2);
-    if (a.need_w) add(kSepDv, a.xop, a.gopT, a.O, a.M, p.split_dv, dv, pv, g.dv_all ? R : R / 2);
-    if (a.need_x) add(kSepDxUpper, a.wops, a.goph, a.M, a.O, p.split_dxs, dx, px, R / 2);
-    if (a.need_w) add(kSepDvUpper, a.xops, a.gophT, a.O, a.M, p.split_dvs, dv, pv, R / 2);
-    if (a.need_x) add(kSepDxHarm, a.woph, a.goph, a.M, a.O, p.split_dxh, dx, px, R);
-    if (a.need_w) add(kSepDvHarm, a.xoph, a.gophT, a.O, a.M, p.split_dvh, dv, pv, R);
+    for (const int c : {3, 2, 1, 0}) {  // the longest first; the harmonics' planes are the last ones
+        if (p.split_dx[c] == 0) continue;
+        const int at = (c + 3) % 4;
+        if (a.need_x) add(kSepDx, c, a.wcls[at], c >= 2 ? a.gop : a.gops, a.M, sep_inner(a.O), p.split_dx[c], dx, px);
+        if (a.need_w) add(kSepDv, c, a.xcls[at], c >= 2 ? a.gopT : a.gopTs, a.O, sep_inner(a.M), p.split_dv[c], dv, pv);
+    }
     launch_sep_gemm<false>(p.big, (unsigned)blocks, g, s);
     return hipGetLastError();
 }

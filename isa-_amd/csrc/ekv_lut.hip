@@ -4846,7 +4846,7 @@ int run_backward(const CallSetup& cs, const float* x, const float* vth_pos, cons
         dxs.scale = dvs.scale = cs.exact ? (float)cs.i_s : 1.0f;
         dvs.mode_word = nullptr;
         hipLaunchKernelGGL(sep_reduce_bwd_kernel, dim3((unsigned)first_blocks), dim3(256), 0, s, dxs, dxa, dx_blocks, dvs,
-                           dva, dv_blocks, gra, sep_head, sp.split_dxh, sp.split_dvh);
+                           dva, dv_blocks, gra, sep_head, sp.split_dx[0], sp.split_dv[0]);
     }
     if (need_glue && glue_after)
         hipLaunchKernelGGL(glue_reduce_kernel, dim3((unsigned)gl_blocks), dim3(256), 0, s, gra);
