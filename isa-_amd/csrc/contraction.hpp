@@ -121,7 +121,7 @@ struct SepArgs {
     int lut_n;
     double lut_min, lut_scale;
     double2* lut_val;        // [lut_n]: smooth part, second difference
-    float4* lut_info;        // per 256 entries {largest relative growth from entry to entry, 1 where they do not suit, largest |entry|, 0}
+    float4* lut_info;        // per 256 entries {largest relative change from entry to entry, 1 where they do not suit, largest |entry|, 0}
     float* tabE;             // second difference's coefficients, -r e_i / (2 pi^2), scaled: [n_grid][2]
     // workspace
     SepHead* head;
@@ -209,7 +209,8 @@ __device__ inline void sep_wave_minmax(float& lo, float& hi) {
 }
 
 // Block b of the table's 256-entry ranges: its entries from the records' differences (each block
-// sums those before its range itself), as the smooth part F + S / 12 and S, and whether they
+// sums those before its range itself), as the smooth part F + S / 12 and S, how fast they change (up or
+// down, or by their curvature: it sets the x table's step, the terms and the harmonics), and whether they
 // suit: fourth differences within 3e-6 of the entries (what the cubic interpolation and the two
 // terms of the lookup's line leave out), and for the backward a slope table that is the current
 // table's slope (dX takes the currents from it; within 2e-5 of the difference).
@@ -251,7 +252,9 @@ __device__ inline void sep_lut_block(const SepArgs& a, int b) {
         const double m2 = s_t[i - 2], m1 = s_t[i - 1], v = s_t[i], p1 = s_t[i + 1], p2 = s_t[i + 2];
         const double fourth = fabs((m2 + p2) - 4.0 * (m1 + p1) + 6.0 * v);
         if (!(fourth <= 3e-6 * fabs(v) + 1e-42)) bad = true;
-        if (v > 1e-30) growth = (float)((p1 - v) / v);
+        const double least = fmin(fabs(v), fabs(p1));
+        if (least > 1e-30) growth = fmaxf((float)(fabs(p1 - v) / least), sqrtf((float)(fabs(second) / fabs(v))));
+        if (v * p1 < 0.0) bad = true;
         if (bwd) {  // the current's difference against the slope's integral (error of fourth order)
             const double di = (double)r0[(size_t)j * 4 + 1];
             const double want = (0.5 * (v + p1) - ((p2 - p1) - (v - m1)) / 24.0) / a.lut_scale;
@@ -302,7 +305,7 @@ __device__ inline bool sep_sample_refuses(const SepArgs& a) {
                      d3 = __shfl(r.y, place * 4 + 3);
         const double v = (double)__shfl(r.x, place * 4 + 2) + (double)(i + kPad) * d2;  // entry i, to 1e-5
         bad = !(fabs((d3 - d0) - 3.0 * (d2 - d1)) <= 4e-6 * fabs(v) + 2e-42);
-        float growth = v > 1e-30 ? (float)(d2 / v) : 0.0f;
+        float growth = fabs(v) > 1e-30 ? (float)fabs(d2 / v) : 0.0f;  // (at most the whole table's)
         for (int d = 32; d > 0; d >>= 1) growth = fmaxf(growth, __shfl_xor(growth, d));
         growth_all = 0.999f * growth;
         ua = 0.5 * (double)growth_all * a.lut_scale;

@@ -212,10 +212,14 @@ def _shape_table(shape, n=4096, lo=-9.0, hi=4.0):
     if shape == "falling":
         s = torch.sigmoid(-v / 0.13)
         return 1e-6 * s, -1e-6 * s * (1.0 - s) / 0.13
+    if shape == "steep fall":  # rises by 0.1% from entry to entry, falls by 4%
+        s = torch.sigmoid(-(v + 0.5) / 0.08)
+        f = 1e-6 * torch.exp(0.3 * v) * s
+        return f, f * (0.3 - (1.0 - s) / 0.08)
     return 1e-6 * torch.exp(v / 0.4), 2.5e-6 * torch.exp(v / 0.4)  # "exponential"
 
 
-@pytest.mark.parametrize("shape", ["saturating", "bump", "falling", "exponential"])
+@pytest.mark.parametrize("shape", ["saturating", "bump", "falling", "steep fall", "exponential"])
 def test_tables_of_other_shapes(cuda_device, shape):
     """Packed tables may hold any curve: slopes that fall again, currents that fall, that only grow."""
     from isa.kernels.transformer_ffn import _hip, ops
@@ -223,7 +227,7 @@ def test_tables_of_other_shapes(cuda_device, shape):
     lo, hi, n = -9.0, 4.0, 4096
     ti, td = (t.float() for t in _shape_table(shape, n, lo, hi))
     packed = [ops.pack_tables(ti.cuda(), td.cuda(), layout) for layout in (_hip.LUT_FWD, _hip.LUT_BWD)]
-    x, wp, wn, g = _inputs("table", 8)
+    x, wp, wn, g = _inputs("table", 8, 0.05 if shape == "steep fall" else SPREAD)
     x = 3.3 * x  # (further up the saturating curve's differences are its entries' rounding)
     print(f"[case] {shape} table", flush=True)
     got, cells = _run("table", x, wp, wn, g, (packed, n, lo, hi, _table_cells(ti, td, lo, hi)))
