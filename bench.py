@@ -559,8 +559,8 @@ def power_phases(cfg: dict, d_model: int, d_ffn: int, tokens: int, dev, seconds:
     grad = torch.randn(tokens, d_ffn, generator=g).to(dev)
     pf = ops.plan_info("forward", tokens, d_model, d_ffn, n)
     pb = ops.plan_info("backward", tokens, d_model, d_ffn, n, True, True)
-    wsf = torch.empty(pf["workspace_bytes"], dtype=torch.uint8, device=dev)
-    wsb = torch.empty(pb["workspace_bytes"], dtype=torch.uint8, device=dev)
+    # workspaces of the per-cell kernels' plans: the phases are the table kernels'
+    wsf, wsb = (torch.empty(p["cell_bytes"], dtype=torch.uint8, device=dev) for p in (pf, pb))
     phases = {
         "table_backward": lambda: ops.lut_backward(x, vp, vn, grad, bwd_t, n, dmin, dmax, cfg["V_sat"], True, True,
                                                    workspace=wsb),

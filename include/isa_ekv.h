@@ -293,25 +293,32 @@ int isa_ekv_profile_clock(double* out);
 
 /* Plan of a LUT call at this shape (test and measurement aid, no reference counterpart).
  * which: ISA_EKV_PLAN_FORWARD (isa_ekv_forward, isa_ekv_layer_forward), ISA_EKV_PLAN_BACKWARD
- * (isa_ekv_backward), ISA_EKV_PLAN_LAYER_BACKWARD (isa_ekv_layer_backward). Writes
+ * (isa_ekv_backward), ISA_EKV_PLAN_LAYER_BACKWARD (isa_ekv_layer_backward); of the exact-formula
+ * calls, whose n_entries is not read: ISA_EKV_PLAN_EXACT_FORWARD, ISA_EKV_PLAN_EXACT_BACKWARD. Writes
  * min(n_info, ISA_EKV_PLAN_INFO_LEN) values (later slots get 0):
- *   [0] workspace bytes (forward: of the per-cell kernels' plan, which the query's may exceed)
+ *   [0] workspace bytes (table forward: [8], which the query's may exceed; the others: [9])
  *   [1] byte offset in the workspace of the table-copy mode word (int32: after the call, 1 when
  *       the main kernel ran with the second, bank-rotated table copy, 0 when with one copy,
  *       2 when the backward ran ranked: see ISA_EKV_OPT_RANKED, 3 to 32 when the main kernel
  *       held that many windowed copies and 33 when it held two: see ISA_EKV_OPT_WINDOW_COPIES;
- *       the mode that they would have run in where the call ran on the matrix cores),
- *       or -1 when the call cannot
- *       use a second copy (the word is then not written)
+ *       64 when the call ran on the matrix cores and no table kernel did), or -1 when the call
+ *       cannot use a second copy (the word is then not written)
  *   [2] forward: K ranges summed separately (1: no split); backward: token splits
  *   [3] forward: tokens per wave; backward: inputs per wave of the one-copy kernel
  *   [4] main-kernel blocks   [5] waves per block   [6] LDS bytes per block
  *   [7] backward with dVth: dVth partial planes (the token splits, or a quarter of them when
- *       the main kernel's blocks sum groups of four splits); otherwise 0 */
+ *       the main kernel's blocks sum groups of four splits); otherwise 0
+ *   [8] bytes of the per-cell kernels' plan: a workspace of this size runs them
+ *   [9] bytes with the operands of the products on the matrix cores, [8] where the call never
+ *       considers them
+ *   [10] byte offset, in a workspace of [9] bytes, of the path word (int32: after the call, 1 when it
+ *       ran on the matrix cores, 0 when the per-cell kernels did), or -1 where it never considers them */
 #define ISA_EKV_PLAN_FORWARD 0
 #define ISA_EKV_PLAN_BACKWARD 1
 #define ISA_EKV_PLAN_LAYER_BACKWARD 2
-#define ISA_EKV_PLAN_INFO_LEN 8
+#define ISA_EKV_PLAN_EXACT_FORWARD 3
+#define ISA_EKV_PLAN_EXACT_BACKWARD 4
+#define ISA_EKV_PLAN_INFO_LEN 11
 int isa_ekv_plan_info(int which, int64_t M, int64_t K, int64_t O, int n_entries, int need_grad_x, int need_grad_w,
                       int64_t* info, int n_info);
 

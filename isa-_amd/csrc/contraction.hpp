@@ -85,6 +85,7 @@ __host__ __device__ inline int sep_terms_lut(float spread_u, float growth, bool 
 
 // What the passes of a call share, in its workspace.
 struct SepHead {
+    int took;     // for the caller: 1 where the contraction took the call
     int terms;    // 0: the per-cell kernels run
     unsigned gmax;  // backward: bits of the largest |G|: not finite: the per-cell kernels run
     int rough;    // 1: the series does not converge as its terms assume, 2: a sample of the thresholds or of
@@ -774,16 +775,11 @@ __device__ inline void sep_harm_w(float v[4], float2 up, float2 un, float cp, fl
 
 __device__ inline float2 sep_kink_functions(const SepHead& h, float t) { return make_float2(expf(h.gw * t), expf(h.gu * t)); }
 
-// The per-cell range partials of a call that the contraction takes (the passes that record the
-// table mode read them).
-__device__ inline void sep_write_partials(const SepHead& h, const PrepArgs& p) {
-    for (int i = threadIdx.x; i < kPrepBlocksX + kPrepBlocksW; i += blockDim.x) {
-        float2 v = make_float2(INFINITY, -INFINITY);
-        if (i == 0) v = make_float2(fmaf(h.xlo - p.xoff, p.scale, p.xadd), fmaf(h.xhi - p.xoff, p.scale, p.xadd));
-        if (i == kPrepBlocksX) v = make_float2(h.wlo * p.scale, h.whi * p.scale);
-        p.partials[i] = v;
-    }
-    if (p.stat_bits && threadIdx.x == 0) *p.stat_bits = 0u;
+// Records who takes the call, and clears what its prep would (first block of the operands' launch).
+__device__ inline void sep_record(SepHead* head, bool took, const PrepArgs& p) {
+    if (blockIdx.x != 0 || threadIdx.x != 0) return;
+    head->took = took ? 1 : 0;
+    if (took && p.stat_bits) *p.stat_bits = 0u;
 }
 
 template <int R>
@@ -856,12 +852,13 @@ __device__ inline void sep_expand_fwd(const SepArgs& a, const SepHead& h) {
 // Where the per-cell kernels take the call: their prep, in the same launch (unless the statistics'
 // launch has run it).
 __global__ __launch_bounds__(256) void sep_expand_fwd_kernel(SepArgs a, PrepArgs prep) {
-    if (!sep_takes(a.head)) {
+    const bool takes = sep_takes(a.head);
+    sep_record(a.head, takes, prep);
+    if (!takes) {
         if (blockIdx.x < kPrepBlocksX + kPrepBlocksW && a.head->rough != 2) prep_block(prep, blockIdx.x);
         return;
     }
     const SepHead h = *a.head;
-    if (blockIdx.x == 0) sep_write_partials(h, prep);
     if (h.terms == 8)
         sep_expand_fwd<8>(a, h);
     else
@@ -1063,12 +1060,13 @@ __device__ inline void sep_expand_grad(const SepArgs& a, int b, float (*s_g)[kSe
 }
 
 __global__ __launch_bounds__(256, 3) void sep_expand_bwd_kernel(SepArgs a, int x_blocks, int w_blocks, PrepArgs prep) {
-    if (!sep_takes(a.head)) {  // the per-cell kernels take the call: their prep
+    const bool takes = sep_takes(a.head);
+    sep_record(a.head, takes, prep);
+    if (!takes) {  // the per-cell kernels take the call: their prep
         if (blockIdx.x < kPrepBlocksX + kPrepBlocksW && a.head->rough != 2) prep_block(prep, blockIdx.x);
         return;
     }
     const SepHead h = *a.head;
-    if (blockIdx.x == 0) sep_write_partials(h, prep);
     __shared__ __align__(16) float s_a[32][kSepTilePitch], s_b[32][kSepTilePitch];
     const int b = blockIdx.x;
     if (b < x_blocks) {

@@ -1225,6 +1225,7 @@ constexpr int kModeRanked = 2;
 constexpr int kModeMultiMin = 3;
 constexpr int kMultiMax = 32;
 constexpr int kModeWindowed2 = kMultiMax + 1;
+constexpr int kModeContraction = 64;  // no table kernel: the contraction took the call
 
 // Block b of the two-copy assignment.
 // LANES = 32: 8-byte records, gathered by half-waves over 32 bank pairs; LANES = 16: 16-byte
@@ -2295,7 +2296,7 @@ __device__ __forceinline__ void rank_deal_block(const RankArgs& a, int b, float*
 // passes return, and block 0 records it in the mode word for the launches that follow. The passes
 // exclude each other, so that one launch of their blocks costs what the one that applies does;
 // as launches of their own the others cost ~4.5 us each to find out that they do not apply.
-// Where the contraction takes the call, the first block alone records the mode.
+// Where the contraction takes the call, nothing is assigned and the mode says so.
 // ----------------------------------------------------------------------------------
 struct AssignArgs {
     float2* wsT;
@@ -2312,7 +2313,10 @@ struct AssignArgs {
 template <int LANES, bool RANK>
 __global__ __launch_bounds__(kAssignThreads) void assign_kernel(AssignArgs a, RankArgs ra) {
     __shared__ __align__(16) float s_raw[kAssignLdsFloats];
-    if (blockIdx.x != 0 && sep_takes(a.skip)) return;
+    if (sep_takes(a.skip)) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) *a.mode_word = kModeContraction;
+        return;
+    }
     float spread = 0.0f;
     const bool ranked = RANK && ranked_mode(a.partials, a.NP, ra.max_spread, &spread);
     MultiLayout ml{};
@@ -2323,7 +2327,6 @@ __global__ __launch_bounds__(kAssignThreads) void assign_kernel(AssignArgs a, Ra
     const bool two = !ranked && !windowed && a.copy_offset > 0 && launch_copy_mode(a.partials, a.NP, a.copy_window);
     if (blockIdx.x == 0 && threadIdx.x == 0)
         *a.mode_word = ranked ? kModeRanked : windowed ? multi_mode_word(ml.copies) : two ? 1 : 0;
-    if (sep_takes(a.skip)) return;
     int b = blockIdx.x;
     if constexpr (RANK) {
         if (b < a.rank_blocks) {  // (wide spreads: bwd_deal_kernel deals)
@@ -5450,13 +5453,19 @@ int isa_ekv_plan_info(int which, int64_t M, int64_t K, int64_t O, int n_entries,
                       int64_t* info, int n_info) {
     if (!info || n_info < 1) return fail(ISA_EKV_EINVAL, "info is null");
     if (M < 0 || K < 0 || O < 0) return fail(ISA_EKV_EINVAL, "negative shape");
-    if (n_entries < 1 || n_entries > kMaxEntriesGlobal)
+    const bool exact = which == ISA_EKV_PLAN_EXACT_FORWARD || which == ISA_EKV_PLAN_EXACT_BACKWARD;
+    if (exact)
+        n_entries = 0;
+    else if (n_entries < 1 || n_entries > kMaxEntriesGlobal)
         return fail(ISA_EKV_EINVAL, "LUT_DELTA_SIZE must be in [1, %d] (got %d)", kMaxEntriesGlobal, n_entries);
     int64_t v[ISA_EKV_PLAN_INFO_LEN];
-    if (which == ISA_EKV_PLAN_FORWARD) {
-        const FwdPlan p = plan_forward_call(false, n_entries, M, K, O);
-        const FwdTableCfg tc = fwd_table_cfg(n_entries, p.wpb, copies_pay(M, K, O));
-        v[0] = (int64_t)p.bytes;
+    SepPlan sp;
+    if (which == ISA_EKV_PLAN_FORWARD || which == ISA_EKV_PLAN_EXACT_FORWARD) {
+        const FwdPlan p = plan_forward_call(exact, n_entries, M, K, O);
+        const FwdTableCfg tc = exact ? FwdTableCfg{} : fwd_table_cfg(n_entries, p.wpb, copies_pay(M, K, O));
+        sp = plan_sep(n_entries, M, K, O, false, false, false, p.bytes);
+        v[8] = (int64_t)p.bytes;
+        v[0] = exact ? (int64_t)sp.bytes : v[8];
         v[1] = tc.copy_offset > 0 || tc.mc_budget > 0 ? (int64_t)p.off_mode : -1;
         v[2] = p.n_split;
         v[3] = p.mr;
@@ -5464,11 +5473,14 @@ int isa_ekv_plan_info(int which, int64_t M, int64_t K, int64_t O, int n_entries,
         v[5] = p.wpb;
         v[6] = (int64_t)tc.lds;
         v[7] = 0;
-    } else if (which == ISA_EKV_PLAN_BACKWARD || which == ISA_EKV_PLAN_LAYER_BACKWARD) {
+    } else if (which == ISA_EKV_PLAN_BACKWARD || which == ISA_EKV_PLAN_LAYER_BACKWARD ||
+               which == ISA_EKV_PLAN_EXACT_BACKWARD) {
         const bool nx = need_grad_x != 0, nw = need_grad_w != 0;
         const BwdPlan p = plan_backward(M, K, O, n_entries, nx, nw, which == ISA_EKV_PLAN_LAYER_BACKWARD);
-        v[0] = (int64_t)plan_sep(n_entries, M, K, O, true, nx, nw, p.bytes).bytes;
-        v[1] = bwd_may_use_copies(p, false, nx) ? (int64_t)p.off_mode : -1;
+        sp = plan_sep(n_entries, M, K, O, true, nx, nw, p.bytes);
+        v[0] = (int64_t)sp.bytes;
+        v[8] = (int64_t)p.bytes;
+        v[1] = bwd_may_use_copies(p, exact, nx) ? (int64_t)p.off_mode : -1;
         v[2] = p.n_split;
         v[3] = p.Kp / p.n_kb;
         v[4] = p.blocks;
@@ -5478,6 +5490,8 @@ int isa_ekv_plan_info(int which, int64_t M, int64_t K, int64_t O, int n_entries,
     } else {
         return fail(ISA_EKV_EINVAL, "unknown plan kind %d", which);
     }
+    v[9] = (int64_t)sp.bytes;
+    v[10] = sp.max_terms > 0 ? (int64_t)(sp.off_head + offsetof(SepHead, took)) : -1;
     for (int i = 0; i < n_info; ++i) info[i] = i < ISA_EKV_PLAN_INFO_LEN ? v[i] : 0;
     return 0;
 }

@@ -25,7 +25,9 @@ LUT_PLAIN_BF16 = 3
 PLAN_FORWARD = 0
 PLAN_BACKWARD = 1
 PLAN_LAYER_BACKWARD = 2
-PLAN_INFO_LEN = 8
+PLAN_EXACT_FORWARD = 3
+PLAN_EXACT_BACKWARD = 4
+PLAN_INFO_LEN = 11
 NOALLOC_MAX_BYTES = 128 << 20  # ISA_EKV_NOALLOC_MAX_BYTES
 OPT_COPY_MIN_CELLS = 1
 OPT_RANKED = 2

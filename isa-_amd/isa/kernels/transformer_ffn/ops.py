@@ -17,6 +17,7 @@ from isa.kernels.transformer_ffn import _hip
 
 MAX_ENTRIES_FORWARD = 16384   # forward table resident in LDS up to this size
 MAX_ENTRIES_BACKWARD = 8192   # backward table resident in LDS; the reference's shared-backward limit
+MODE_CONTRACTION = 64         # copy_mode of a call that ran on the matrix cores
 MAX_ENTRIES = 1 << 22         # larger tables up to this size are read from global memory
 
 
@@ -54,23 +55,26 @@ def _workspace(nbytes: int, device: torch.device, given: Optional[torch.Tensor] 
 
 
 _PLAN_KINDS = {"forward": _hip.PLAN_FORWARD, "backward": _hip.PLAN_BACKWARD,
-               "layer_backward": _hip.PLAN_LAYER_BACKWARD}
+               "layer_backward": _hip.PLAN_LAYER_BACKWARD, "exact_forward": _hip.PLAN_EXACT_FORWARD,
+               "exact_backward": _hip.PLAN_EXACT_BACKWARD}
 
 
 def plan_info(kind: str, M: int, K: int, O: int, n_entries: int, need_grad_x: bool = True,
               need_grad_w: bool = True) -> dict:
-    """The library's plan for a LUT call at this shape (isa_ekv_plan_info): workspace bytes,
-    the byte offset of the table-copy mode word in the workspace (-1 when the call has none),
-    K splits (forward) or token splits (backward), tokens (forward) or inputs (backward) per
-    wave, main-kernel blocks, waves per block, LDS bytes per block and (backward with dVth)
-    the dVth partial planes."""
+    """The library's plan for a call at this shape (isa_ekv_plan_info; n_entries is not read for
+    the exact formula's kinds): workspace bytes, the byte offset of the table-copy mode word in
+    the workspace (-1 when the call has none), K splits (forward) or token splits (backward), tokens (forward) or inputs (backward) per
+    wave, main-kernel blocks, waves per block, LDS bytes per block, (backward with dVth) the dVth
+    partial planes, the bytes of the per-cell kernels' plan alone (a workspace of that size runs
+    them), the bytes with the matrix cores' operands and the byte offset of their path word (-1
+    where the call never considers them)."""
     lib = _hip.load()
     info = (ctypes.c_int64 * _hip.PLAN_INFO_LEN)()
     rc = lib.isa_ekv_plan_info(_PLAN_KINDS[kind], int(M), int(K), int(O), int(n_entries), int(need_grad_x),
                                int(need_grad_w), info, _hip.PLAN_INFO_LEN)
     _hip.check(rc, "isa_ekv_plan_info")
     keys = ("workspace_bytes", "mode_offset", "splits", "per_wave", "blocks", "waves_per_block", "lds_bytes",
-            "dv_planes")
+            "dv_planes", "cell_bytes", "contraction_bytes", "path_offset")
     return dict(zip(keys, (int(v) for v in info)))
 
 
@@ -137,12 +141,21 @@ def rank_xcd_order(value: Optional[bool] = None) -> bool:
 def copy_mode(workspace: torch.Tensor, plan: dict) -> Optional[int]:
     """After a call that used `workspace` (and synchronised), which table mode its main kernel
     ran in: 1 the second table copy, 0 one copy, 2 the ranked backward, 3 to 32 the forward's
-    windowed copies (their number); None when the plan has no second copy. A call that ran as
-    products on the matrix cores records the mode the table kernels would have run in."""
+    windowed copies (their number), 64 (MODE_CONTRACTION) when no table kernel ran because the
+    call was products on the matrix cores; None when the plan has no second copy."""
     off = plan["mode_offset"]
     if off < 0:
         return None
     return int(workspace[off:off + 4].view(torch.int32).item())
+
+
+def took_contraction(workspace: torch.Tensor, plan: dict) -> bool:
+    """After a call that used `workspace` (and synchronised), whether it ran as products on the
+    matrix cores; False where the per-cell kernels ran."""
+    off = plan["path_offset"]
+    if off < 0 or workspace.numel() < plan["contraction_bytes"]:
+        return False
+    return bool(workspace[off:off + 4].view(torch.int32).item())
 
 
 def build_plain_tables(params: Tuple[float, float, float, float], delta_min: float, delta_max: float,
@@ -283,8 +296,9 @@ def _exact_params(params) -> ctypes.Array:
 
 
 def exact_forward(x: torch.Tensor, wpos: torch.Tensor, wneg: torch.Tensor,
-                  params: Tuple[float, float, float, float], v_sat: float) -> torch.Tensor:
-    """Idiff[M, O] fp32 by the exact EKV formula (no clamp)."""
+                  params: Tuple[float, float, float, float], v_sat: float,
+                  workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """Idiff[M, O] fp32 by the exact EKV formula (no clamp). workspace: optional caller buffer."""
     lib = _hip.load()
     M, K, O = _check_operands(x, wpos, wneg)
     dev = x.device
@@ -292,7 +306,7 @@ def exact_forward(x: torch.Tensor, wpos: torch.Tensor, wneg: torch.Tensor,
     if M == 0 or O == 0:
         return out
     x32, wp32, wn32 = as_kernel_f32(x), as_kernel_f32(wpos), as_kernel_f32(wneg)
-    ws = _workspace(lib.isa_ekv_exact_forward_workspace(M, K, O), dev)
+    ws = _workspace(lib.isa_ekv_exact_forward_workspace(M, K, O), dev, workspace)
     with _hip.on_device(dev):
         rc = lib.isa_ekv_exact_forward(_ptr(x32), _ptr(wp32), _ptr(wn32), M, K, O, _exact_params(params),
                                        float(v_sat), out.data_ptr(), ws.data_ptr(), ws.numel(),
@@ -302,8 +316,10 @@ def exact_forward(x: torch.Tensor, wpos: torch.Tensor, wneg: torch.Tensor,
 
 
 def exact_backward(x: torch.Tensor, wpos: torch.Tensor, wneg: torch.Tensor, grad_out: torch.Tensor,
-                   params: Tuple[float, float, float, float], v_sat: float, need_grad_x: bool, need_grad_w: bool):
-    """(dX | None, dVth+ | None, dVth- | None) of sum(grad_out * Idiff), exact formula, fp32."""
+                   params: Tuple[float, float, float, float], v_sat: float, need_grad_x: bool, need_grad_w: bool,
+                   workspace: Optional[torch.Tensor] = None):
+    """(dX | None, dVth+ | None, dVth- | None) of sum(grad_out * Idiff), exact formula, fp32. workspace:
+    optional caller buffer."""
     lib = _hip.load()
     M, K, O = _check_operands(x, wpos, wneg)
     _require_cuda(grad_out, "grad_out")
@@ -316,7 +332,8 @@ def exact_backward(x: torch.Tensor, wpos: torch.Tensor, wneg: torch.Tensor, grad
     if not (need_grad_x or need_grad_w):
         return gx, gp, gn
     x32, wp32, wn32, g32 = (as_kernel_f32(t) for t in (x, wpos, wneg, grad_out))
-    ws = _workspace(lib.isa_ekv_exact_backward_workspace(M, K, O, int(need_grad_x), int(need_grad_w)), dev)
+    ws = _workspace(lib.isa_ekv_exact_backward_workspace(M, K, O, int(need_grad_x), int(need_grad_w)), dev,
+                    workspace)
     with _hip.on_device(dev):
         rc = lib.isa_ekv_exact_backward(_ptr(x32), _ptr(wp32), _ptr(wn32), _ptr(g32), M, K, O,
                                         _exact_params(params), float(v_sat), _ptr(gx), _ptr(gp), _ptr(gn),

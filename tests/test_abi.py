@@ -275,6 +275,30 @@ def test_plan_info_reports_the_call_plans():
     assert lib.isa_ekv_plan_info(0, 1, 1, 1, 0, 1, 1, info, 7) == -1 and "LUT_DELTA_SIZE" in _err(lib)
 
 
+def test_plan_info_reports_the_matrix_cores_operands():
+    """Slots 8 to 10: the per-cell plan's bytes, the bytes with the contraction's operands and the path
+    word, where a call considers it: from 2^29 cells (formula) and 2^30 (tables of 3600 to 65536
+    entries)."""
+    from isa.kernels.transformer_ffn import ops
+
+    lib = _hip.load()
+    for kind, n in (("forward", 4096), ("backward", 4096), ("layer_backward", 8192), ("exact_forward", 0),
+                    ("exact_backward", 0)):
+        big, small = ops.plan_info(kind, 8192, 768, 3072, n), ops.plan_info(kind, 200, 768, 3072, n)
+        assert big["cell_bytes"] < big["contraction_bytes"], kind
+        assert big["cell_bytes"] <= big["path_offset"] <= big["contraction_bytes"] - 4
+        assert small["cell_bytes"] == small["contraction_bytes"] and small["path_offset"] == -1, kind
+    for n in (3599, 65537):
+        assert ops.plan_info("forward", 8192, 768, 3072, n)["path_offset"] == -1
+    assert ops.plan_info("exact_forward", 8192, 768, 3072, 0)["contraction_bytes"] == \
+        lib.isa_ekv_exact_forward_workspace(8192, 768, 3072)
+    assert ops.plan_info("exact_backward", 8192, 768, 3072, 0, True, False)["contraction_bytes"] == \
+        lib.isa_ekv_exact_backward_workspace(8192, 768, 3072, 1, 0)
+    # the forward's query covers every table
+    assert ops.plan_info("forward", 8192, 768, 3072, 65536)["contraction_bytes"] <= \
+        lib.isa_ekv_forward_workspace(8192, 768, 3072)
+
+
 def test_small_calls_plan_one_table_copy_and_one_round():
     """Calls below ISA_EKV_OPT_COPY_MIN_CELLS (default 2^28 cells) plan no second table copy;
     isa_ekv_set_option moves the threshold. Small plans keep to one round of blocks."""

@@ -16,7 +16,9 @@ ekv_lut_triton.py:52-61 and ekv_cuda.cu:224-250, :324-339):
 The glue (TIA gain and clamp, ADC affine, input mapping) is checked elementwise from the
 GPU's own idiff, and the glue parameters' gradients against float64 sums of GPU
 intermediates. The spy also reads each launch's table-copy mode word, so the regime the
-bench runs is the regime tested. A second identical step must be bitwise equal.
+bench runs is the regime tested: at these sizes and initial thresholds the matrix cores take the
+calls (fp32 tables). The per-cell kernels, which serve wider thresholds, are tested at the same
+shapes through workspaces of their plan. A second identical step must be bitwise equal.
 
 Gates (norm-wise, against the fp32-table oracle): forward <= 1e-4, dX and dVth+- <= 1e-3.
 """
@@ -40,9 +42,9 @@ SUM_TOL = 1e-4  # glue-parameter gradients: fp32 fixed-order sums vs float64
 class LayerSpy:
     """Wraps ops.lut_layer_forward / lut_layer_backward (the calls FusedCIMLayerFn makes) to keep
     every call's inputs and results, run each with a workspace whose table-copy mode word is
-    read back afterwards."""
+    read back afterwards; cells: a workspace that only the per-cell kernels' plan fits."""
 
-    def __init__(self, monkeypatch):
+    def __init__(self, monkeypatch, cells):
         from isa.kernels.transformer_ffn import _hip, ops
 
         self.fwd, self.bwd = [], []
@@ -53,7 +55,7 @@ class LayerSpy:
             M, K = x.shape
             O = wpos.shape[0]
             plan = ops.plan_info("forward", M, K, O, n_entries)
-            nbytes = max(plan["workspace_bytes"], lib.isa_ekv_layer_forward_workspace(M, K, O))
+            nbytes = plan["cell_bytes"] if cells else lib.isa_ekv_layer_forward_workspace(M, K, O)
             ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
             out, idiff = orig_f(x, wpos, wneg, fwd_records, n_entries, *a, workspace=ws, **k)
             self.fwd.append(dict(x=x, out=out, idiff=idiff, ws=ws, plan=plan))
@@ -64,7 +66,7 @@ class LayerSpy:
             O = wpos.shape[0]
             need_x = bool(k.get("need_grad_x")) or (bool(k.get("need_in_affine")) and k.get("in_affine") is not None)
             plan = ops.plan_info("layer_backward", M, K, O, n_entries, need_x, bool(k.get("need_grad_w")))
-            ws = torch.empty(plan["workspace_bytes"], dtype=torch.uint8, device=x.device)
+            ws = torch.empty(plan["cell_bytes" if cells else "workspace_bytes"], dtype=torch.uint8, device=x.device)
             res = orig_b(x, wpos, wneg, grad_out, idiff, bwd_records, n_entries, *a, workspace=ws, **k)
             self.bwd.append(dict(grad_out=grad_out, res=res, ws=ws, plan=plan))
             return res
@@ -156,6 +158,7 @@ def _inputs(B, T, D, seed):
 # the forward's windowed table copies: their number depends on the coordinate window the
 # inputs reach (3 up to ISA_EKV_OPT_WINDOW_COPIES, default 32)
 WINDOWED = range(3, 33)
+MODE_CONTRACTION = 64  # no table kernel: products on the matrix cores
 
 
 def _modes_match(got, want):
@@ -163,7 +166,8 @@ def _modes_match(got, want):
     return len(got) == len(want) and all(g in w if isinstance(w, range) else g == w for g, w in zip(got, want))
 
 
-def run_physical_ffn(monkeypatch, dev, D, F, B, T, size, expect_modes, n_rows=48, n_cols=24, seed=0, **cfg_over):
+def run_physical_ffn(monkeypatch, dev, D, F, B, T, size, expect_modes, cells, n_rows=48, n_cols=24, seed=0,
+                     **cfg_over):
     from isa.device_models.config import make_flash_transistor_ekv_config
     from isa.operators.cim import PhysicalFFN
 
@@ -174,7 +178,9 @@ def run_physical_ffn(monkeypatch, dev, D, F, B, T, size, expect_modes, n_rows=48
     ffn = PhysicalFFN(D, F, cfg).to(dev)
     x = _inputs(B, T, D, seed + 1).to(dev)
     g = torch.randn(B, T, D, generator=torch.Generator().manual_seed(seed + 2)).to(dev)
-    spy = LayerSpy(monkeypatch)
+    spy = LayerSpy(monkeypatch, cells)
+    if not cells and "LUT_DTYPE" not in cfg_over:  # (bf16 entries are not smooth: the per-cell kernels)
+        expect_modes = ([MODE_CONTRACTION] * 2,) * 2
     out, xx = _step(ffn, x, g)
     fmodes, bmodes = spy.modes()
     print(f"[case] PhysicalFFN {D}->{F}->{D} x[{B},{T},{D}] LUT {size} {cfg.get('LUT_DTYPE', 'float32')}: "
@@ -246,27 +252,31 @@ def run_physical_ffn(monkeypatch, dev, D, F, B, T, size, expect_modes, n_rows=48
     assert len(first) == len(again) and all(torch.equal(p, q) for p, q in zip(first, again))
 
 
-def test_config1_vitm_physical_ffn_4096(cuda_device, monkeypatch):
-    """configs[1] with the 4096-entry table: the initial thresholds span ~67 records; fc1's
+@pytest.mark.parametrize("cells", [False, True])
+def test_config1_vitm_physical_ffn_4096(cuda_device, monkeypatch, cells):
+    """configs[1] with the 4096-entry table. The per-cell kernels: the initial thresholds span ~67 records; fc1's
     mapped inputs reach a coordinate window of ~1400 records (as many windowed forward copies
     as fit its LDS, about seven), fc2's TIA outputs a narrow one (the cap, 32); the backward runs
     ranked."""
-    run_physical_ffn(monkeypatch, cuda_device, 256, 1024, 128, 65, 4096, ([WINDOWED, 32], [2, 2]))
+    run_physical_ffn(monkeypatch, cuda_device, 256, 1024, 128, 65, 4096, ([WINDOWED, 32], [2, 2]), cells)
 
 
-def test_config1_vitm_physical_ffn_8192(cuda_device, monkeypatch):
-    """configs[1] with the vision default of 8192 entries: the initial thresholds span ~135
+@pytest.mark.parametrize("cells", [False, True])
+def test_config1_vitm_physical_ffn_8192(cuda_device, monkeypatch, cells):
+    """configs[1] with the vision default of 8192 entries. The per-cell kernels: the initial thresholds span ~135
     records and both layers' inputs reach a coordinate window that fits (fc1's mapped inputs in
     [0, 4] V, fc2's TIA outputs within a fraction of a volt of zero): fc1's forward holds three
     bank-rotated copies of its ~2800-record window (what fits its 80 KB), fc2's as many of its
     narrow one as fit (about two dozen: twice the records per volt of the 4096-entry table),
     and every backward runs ranked."""
-    run_physical_ffn(monkeypatch, cuda_device, 256, 1024, 128, 65, 8192, ([WINDOWED, range(16, 33)], [2, 2]))
+    run_physical_ffn(monkeypatch, cuda_device, 256, 1024, 128, 65, 8192, ([WINDOWED, range(16, 33)], [2, 2]), cells)
 
 
-def test_config3_headline_physical_ffn(cuda_device, monkeypatch):
-    """configs[3], the headline Physical GPT-L FFN at full size, exactly as bench.py runs it."""
-    run_physical_ffn(monkeypatch, cuda_device, 768, 3072, 8, 1024, 4096, ([WINDOWED, 32], [2, 2]))
+@pytest.mark.parametrize("cells", [False, True])
+def test_config3_headline_physical_ffn(cuda_device, monkeypatch, cells):
+    """configs[3], the headline Physical GPT-L FFN at full size, exactly as bench.py runs it, and by the
+    per-cell kernels."""
+    run_physical_ffn(monkeypatch, cuda_device, 768, 3072, 8, 1024, 4096, ([WINDOWED, 32], [2, 2]), cells)
 
 
 def test_config3_headline_physical_ffn_bf16_tables(cuda_device, monkeypatch):
@@ -274,11 +284,12 @@ def test_config3_headline_physical_ffn_bf16_tables(cuda_device, monkeypatch):
     checked against the oracle fed the same bytes. fc2's inputs are the TIA outputs of the
     initial model, within a fraction of a volt of zero, where the reference's fp32 table
     construction and an fp64-accurate one differ most after the bf16 cast."""
-    run_physical_ffn(monkeypatch, cuda_device, 768, 3072, 8, 1024, 4096, ([WINDOWED, 32], [2, 2]),
+    run_physical_ffn(monkeypatch, cuda_device, 768, 3072, 8, 1024, 4096, ([WINDOWED, 32], [2, 2]), False,
                      LUT_DTYPE="bfloat16")
 
 
-def test_config2_gptm_hybrid_ffn(cuda_device, monkeypatch):
+@pytest.mark.parametrize("cells", [False, True])
+def test_config2_gptm_hybrid_ffn(cuda_device, monkeypatch, cells):
     """configs[2] Hybrid GPT-M: the fused CIM up-projection (input mapping, TIA gain, clamp)
     and the digital nn.Linear down-projection on rocBLAS/hipBLASLt."""
     from isa.device_models.config import make_flash_transistor_ekv_config
@@ -292,12 +303,13 @@ def test_config2_gptm_hybrid_ffn(cuda_device, monkeypatch):
     ffn = HybridFFN(D, F, cfg).to(dev)
     x = _inputs(B, T, D, 4).to(dev)
     g = torch.randn(B, T, D, generator=torch.Generator().manual_seed(5)).to(dev)
-    spy = LayerSpy(monkeypatch)
+    spy = LayerSpy(monkeypatch, cells)
     out, xx = _step(ffn, x, g)
     fmodes, bmodes = spy.modes()
     print(f"[case] HybridFFN {D}->{F} + Linear x[{B},{T},{D}]: copy modes fwd {fmodes} bwd {bmodes}")
     assert len(spy.fwd) == 1 and len(spy.bwd) == 1
-    assert _modes_match(fmodes, [WINDOWED]) and bmodes == [2], (fmodes, bmodes)
+    want = ([WINDOWED], [2]) if cells else ([MODE_CONTRACTION], [MODE_CONTRACTION])
+    assert _modes_match(fmodes, want[0]) and bmodes == want[1], (fmodes, bmodes)
 
     M = B * T
     rng = np.random.default_rng(6)

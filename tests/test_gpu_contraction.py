@@ -2,10 +2,10 @@
 the formula and its analytic gradients in float64 (oracle/exact.py, evaluated on the device in
 chunks of rows).
 
-Tolerance: the operands carry 2^-22 of each value and the truncated series 1e-7; a sum of n
-products taken 16 at a time in fp32 adds up to about sqrt(3 n / 16) * 2^-24 of its largest
-partial sum (three products per pair of operands). At the largest sums here (n = 8 terms x 5800
-inputs) that is 5.6e-6 of the output's scale, norm-wise; the per-cell kernels' own gate is 1e-4.
+Tolerance: the operands carry 2^-24 of each value, pairs, singles and the truncated series 3e-7; a
+sum over n inner elements is taken in slabs of 16, added in fp32 to about sqrt(n / 32) * 2^-24 of its
+largest partial sum: 1.7e-6 at the largest sums here (n = 2 terms x 5800 inputs), norm-wise. The
+per-cell kernels' own gate is 1e-4; which of the two ran is asserted in every test.
 """
 
 from __future__ import annotations
@@ -18,7 +18,7 @@ from tests.helpers import flash_cfg
 
 pytestmark = pytest.mark.gpu
 
-TOL = 6e-6
+TOL = 2e-6
 PARAMS = (4.1360, 0.0259, 7.5875e-7, 0.1)
 V_SAT = 8.2624
 
@@ -47,12 +47,18 @@ def _reference(x, wp, wn, g):
     return torch.cat(out), torch.cat(dx), dp, dn
 
 
-def _run(x, wp, wn, g, need_x=True, need_w=True):
+def _run(x, wp, wn, g, need_x=True, need_w=True, took=None):
+    """took: whether the contraction has to have taken both calls, or to have refused them."""
     from isa.kernels.transformer_ffn import ops
 
-    out = ops.exact_forward(x, wp, wn, PARAMS, V_SAT)
-    res = (out, *ops.exact_backward(x, wp, wn, g, PARAMS, V_SAT, need_x, need_w))
+    (M, K), O = x.shape, wp.shape[0]
+    plans = [ops.plan_info(k, M, K, O, 0, need_x, need_w) for k in ("exact_forward", "exact_backward")]
+    ws = [torch.empty(p["contraction_bytes"], dtype=torch.uint8, device=x.device) for p in plans]
+    out = ops.exact_forward(x, wp, wn, PARAMS, V_SAT, workspace=ws[0])
+    res = (out, *ops.exact_backward(x, wp, wn, g, PARAMS, V_SAT, need_x, need_w, workspace=ws[1]))
     torch.cuda.synchronize()
+    if took is not None:
+        assert [ops.took_contraction(w, p) for w, p in zip(ws, plans)] == [took, took]
     return res
 
 
@@ -81,10 +87,10 @@ CASES = [
 def test_contraction_matches_formula(cuda_device, M, K, O, spread):
     print(f"[case] contraction M={M} K={K} O={O} spread={spread}", flush=True)
     x, wp, wn, g = _inputs(M, K, O, spread, seed=M + K, x_lo=-3.0)
-    got = _run(x, wp, wn, g)
+    got = _run(x, wp, wn, g, took=spread <= 0.31)
     e = _errors(got, _reference(x, wp, wn, g))
-    print(["%.2e" % v for v in e])
-    assert max(e) <= TOL, e
+    print(["%.2e" % v for v in e], flush=True)
+    assert max(e) <= (TOL if spread <= 0.31 else 6e-6), e
     for a, b in zip(got, _run(x, wp, wn, g)):
         assert torch.equal(a, b)
 
@@ -94,21 +100,21 @@ def test_contraction_rows_keep_their_precision(cuda_device):
     so are its gradients; each is compared against its own scale."""
     x, wp, wn, g = _inputs(3700, 192, 768, 0.2142, seed=3)
     x[::2] = x[::2] * 0.1 - 1.5
-    got, ref = _run(x, wp, wn, g), _reference(x, wp, wn, g)
-    for a, r in zip(got[:2], ref[:2]):
+    got, ref = _run(x, wp, wn, g, took=True), _reference(x, wp, wn, g)
+    for a, r in zip(got[:2], ref[:2]):  # (dVth, a sum over the tokens: test_gpu_contraction_scales.py)
         e = (a.double() - r).abs().amax(1) / r.abs().amax(1)
         assert float(e.max()) <= TOL, float(e.max())
 
 
 def test_contraction_invariants(cuda_device):
     x, wp, wn, g = _inputs(3700, 192, 768, 0.2142, seed=5)
-    out, gx, gp, gn = _run(x, wp, wp, g)
+    out, gx, gp, gn = _run(x, wp, wp, g, took=True)
     assert float(out.abs().max()) == 0.0 and float(gx.abs().max()) == 0.0 and torch.equal(gp, -gn)
     # swapped thresholds negate every operand; the matrix cores' sums of 16 products do not
     # round symmetrically about zero, so the outputs agree to the sums' rounding
     a, b = _run(x, wp, wn, g)[0], -_run(x, wn, wp, g)[0]
     assert float((a - b).abs().max() / a.abs().max()) <= TOL
-    full, only_x, only_w = _run(x, wp, wn, g), _run(x, wp, wn, g, True, False), _run(x, wp, wn, g, False, True)
+    full, only_x, only_w = (_run(x, wp, wn, g, *need, took=True) for need in ((True, True), (True, False), (False, True)))
     assert torch.equal(full[1], only_x[1]) and torch.equal(full[2], only_w[2]) and torch.equal(full[3], only_w[3])
 
 
@@ -128,8 +134,8 @@ def test_calls_that_do_not_suit(cuda_device, what):
         bad = 5
     elif what == "inf":
         g[9, 3] = float("inf")
-    out, gx, gp, gn = _run(x, wp, wn, g)
-    if what == "inf":
+    out, gx, gp, gn = _run(x, wp, wn, g, took=None if what == "inf" else False)
+    if what == "inf":  # (G's: the forward is taken)
         assert torch.isfinite(out).all() and not torch.isfinite(gx[9]).any()
         keep = torch.arange(3700, device="cuda") != 9
         assert torch.isfinite(gx[keep]).all()

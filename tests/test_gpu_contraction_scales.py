@@ -83,17 +83,25 @@ def _tables(cfg):
     return packed, n, lo, hi, _table_cells(ti, td, lo, hi)
 
 
-def _run(kind, x, wp, wn, g, tables=None):
+def _run(kind, x, wp, wn, g, tables=None, took=(True, True)):
+    """took: whether the contraction has to take the forward and the backward (None: either)."""
     from isa.kernels.transformer_ffn import ops
 
+    (M, K), O = x.shape, wp.shape[0]
+    n = 0 if kind == "formula" else (tables[1] if tables else 4096)
+    plans = [ops.plan_info(k if n else "exact_" + k, M, K, O, n) for k in ("forward", "backward")]
+    ws = [torch.empty(p["contraction_bytes"], dtype=torch.uint8, device=x.device) for p in plans]
     if kind == "formula":
-        res = (ops.exact_forward(x, wp, wn, PARAMS, V_SAT), *ops.exact_backward(x, wp, wn, g, PARAMS, V_SAT, True, True))
+        res = (ops.exact_forward(x, wp, wn, PARAMS, V_SAT, workspace=ws[0]),
+               *ops.exact_backward(x, wp, wn, g, PARAMS, V_SAT, True, True, workspace=ws[1]))
         cells = _formula_cells
     else:
         (fwd, bwd), n, lo, hi, cells = tables or _tables(flash_cfg(4096))
-        res = (ops.lut_forward(x, wp, wn, fwd, n, lo, hi, V_SAT, -1e30, 1e30),
-               *ops.lut_backward(x, wp, wn, g, bwd, n, lo, hi, V_SAT, True, True))
+        res = (ops.lut_forward(x, wp, wn, fwd, n, lo, hi, V_SAT, -1e30, 1e30, workspace=ws[0]),
+               *ops.lut_backward(x, wp, wn, g, bwd, n, lo, hi, V_SAT, True, True, workspace=ws[1]))
     torch.cuda.synchronize()
+    if took is not None:
+        assert [ops.took_contraction(w, p) for w, p in zip(ws, plans)] == list(took)
     return res, cells
 
 
@@ -192,7 +200,8 @@ def test_tokens_of_all_magnitudes(cuda_device, kind, entries, spread):
     x = x * 0.3 + (6.0 * torch.rand(M, 1, generator=gen) - 2.0).cuda()
     g = g * torch.exp(-27.6 * torch.rand(M, 1, generator=gen)).cuda()
     print(f"[case] {kind} {entries} over {spread} V, tokens of all magnitudes", flush=True)
-    got, cells = _run(kind, x, wp, wn, g, _tables(flash_cfg(entries)) if entries else None)
+    got, cells = _run(kind, x, wp, wn, g, _tables(flash_cfg(entries)) if entries else None,
+                      (True, spread <= 0.31 or entries >= 6000))
     ref, scale = _reference(x, wp, wn, g, cells)
     _check("out by token", got[0], ref[0], scale[0], 1, TOL[kind])
     _check("dX by token", got[1], ref[1], scale[1], 1, TOL[kind])
@@ -230,7 +239,7 @@ def test_tables_of_other_shapes(cuda_device, shape):
     x, wp, wn, g = _inputs("table", 8, 0.05 if shape == "steep fall" else SPREAD)
     x = 3.3 * x  # (further up the saturating curve's differences are its entries' rounding)
     print(f"[case] {shape} table", flush=True)
-    got, cells = _run("table", x, wp, wn, g, (packed, n, lo, hi, _table_cells(ti, td, lo, hi)))
+    got, cells = _run("table", x, wp, wn, g, (packed, n, lo, hi, _table_cells(ti, td, lo, hi)), None)
     ref, scale = _reference(x, wp, wn, g, cells)
     # the table's own fp32 entries round to 6e-8 of the current, the branches' differences are down to
     # 1e-3 of it where a curve is flat

@@ -18,10 +18,11 @@ from tests.helpers import errs, flash_cfg, make_inputs
 pytestmark = pytest.mark.gpu
 
 
-def _run(x, vp, vn, g, cfg, dev, modes=None):
-    """Forward and backward through the C ABI; modes (a dict) receives the table mode each main
-    kernel ran in (1 two copies, 0 one copy, 2 the ranked backward, None no second copy in the
-    plan)."""
+def _run(x, vp, vn, g, cfg, dev, modes=None, cells=True):
+    """Forward and backward through the C ABI, by the per-cell kernels (a workspace of their plan) or,
+    cells False, with the workspace in which the matrix cores may take the calls; modes (a dict)
+    receives the table mode each main kernel ran in (1 two copies, 0 one copy, 2 the ranked
+    backward, 64 the matrix cores, None no second copy in the plan)."""
     from isa.approximations.delta_lut import get_packed_tables, lut_range
     from isa.kernels.transformer_ffn import ops
 
@@ -30,8 +31,8 @@ def _run(x, vp, vn, g, cfg, dev, modes=None):
     M, K = x.shape
     O = vp.shape[0]
     pf, pb = ops.plan_info("forward", M, K, O, n), ops.plan_info("backward", M, K, O, n)
-    wsf = torch.empty(pf["workspace_bytes"], dtype=torch.uint8, device=dev)
-    wsb = torch.empty(pb["workspace_bytes"], dtype=torch.uint8, device=dev)
+    size = "cell_bytes" if cells else "contraction_bytes"
+    wsf, wsb = (torch.empty(p[size], dtype=torch.uint8, device=dev) for p in (pf, pb))
     out = ops.lut_forward(x, vp, vn, fwd, n, dmin, dmax, cfg["V_sat"], -4.0, 4.0, workspace=wsf)
     gx, gp, gn = ops.lut_backward(x, vp, vn, g, bwd, n, dmin, dmax, cfg["V_sat"], True, True, workspace=wsb)
     torch.cuda.synchronize()
@@ -55,6 +56,26 @@ def _check_samples(x, vp, vn, g, res, cfg, rng, n_rows=48, n_cols=24):
     print({k: f"{v[0]:.2e}/{v[1]:.2e}" for k, v in e.items()})
     assert e["fwd"][0] <= 1e-4
     assert max(e["dX"][0], e["dVth+"][0], e["dVth-"][0]) <= 1e-3
+
+
+def test_headline_ffn_layers_on_the_matrix_cores(cuda_device):
+    """What the headline runs at its initial thresholds, both layers, forward and backward."""
+    from isa.kernels.transformer_ffn import ops
+
+    print("[case] headline fc1, fc2 on the matrix cores, M=8192", flush=True)
+    cfg = flash_cfg(4096)
+    rng = np.random.default_rng(0)
+    x, vp, vn, g = (t.to(cuda_device) for t in make_inputs(8192, 768, 3072, seed=0))
+    for _ in range(2):
+        modes = {}
+        res = _run(x, vp, vn, g, cfg, cuda_device, modes, cells=False)
+        assert modes["fwd"] == modes["bwd"] == ops.MODE_CONTRACTION, modes
+        _check_samples(x, vp, vn, g, res, cfg, rng)
+        for a, b in zip(res, _run(x, vp, vn, g, cfg, cuda_device, cells=False)):
+            assert torch.equal(a, b)
+        x = (res[0] * 1e5).clamp(-4.0, 4.0).contiguous()  # fc2's inputs
+        _, vp, vn, _ = (t.to(cuda_device) for t in make_inputs(1, 3072, 768, seed=1))
+        g = torch.randn(8192, 768, generator=torch.Generator().manual_seed(2)).to(cuda_device)
 
 
 def test_headline_ffn_layers(cuda_device):
