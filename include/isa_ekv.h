@@ -78,11 +78,16 @@ int isa_ekv_lut_build(const double params[4], double delta_min, double delta_max
 int isa_ekv_lut_pack(const void* table_i, const void* table_ddelta, int n_entries, int src_dtype, int layout,
                      void* dst, void* stream);
 
-/* Workspace bytes for isa_ekv_forward at this shape. Large calls hold the operands of their
- * products on the matrix cores too; a workspace that holds the per-cell kernels' plan
- * (isa_ekv_plan_info slot [0]) but not those is accepted and runs the per-cell kernels. The
- * exact-formula calls' workspaces are accepted likewise. */
+/* Workspace bytes for isa_ekv_forward at this shape, whatever the table. Large calls hold the
+ * operands of their products on the matrix cores too, up to 96 bytes for each of the (M + O) K
+ * elements of x and of a threshold (backward 104, and 16 for each of G's): 1.1 GB for 8192 x 768 ->
+ * 3072, 3.2 GB for 3072 -> 768. A workspace that holds the per-cell kernels' plan
+ * (isa_ekv_plan_info slot [8]) but not those is accepted and runs the per-cell kernels; so are the
+ * backward's and the exact-formula calls' workspaces. */
 size_t isa_ekv_forward_workspace(int64_t M, int64_t K, int64_t O);
+
+/* The same for a table of n_entries (fewer bytes where no product on the matrix cores takes it). */
+size_t isa_ekv_forward_table_workspace(int64_t M, int64_t K, int64_t O, int n_entries);
 
 /* out[m,o] = clamp(sum_k (L(x-vth_pos) - L(x-vth_neg)) / (1 + x/v_sat), out_min, out_max)
  * with L the linear interpolation of table_i (lut_fwd = ISA_EKV_LUT_FWD layout).

@@ -77,11 +77,12 @@ constexpr int kSepMaxHarmonics = 4;
 __host__ __device__ inline int sep_terms(float spread_u) { return spread_u <= 1.12f ? 8 : spread_u <= 1.45f ? 16 : 0; }
 
 // Table calls. Two functions a harmonic fit the currents' second differences to 2e-6 of a lookup's
-// difference over spreads up to 5 units, the slopes' to 5e-6 up to 1.45 units and, as growth^2, to what
+// difference over spreads up to 5 units, the slopes' to 5e-6 up to 1.12 units and, as growth^2, to what
 // the per-cell kernels round (2.5e-6) over wider ones where entries grow by at most 2.06%.
 __host__ __device__ inline int sep_terms_lut(float spread_u, float growth, bool backward) {
-    return spread_u <= 1.12f ? 8 : spread_u <= (backward && growth > 0.0206f ? 1.45f : 5.0f) ? 16 : 0;
+    return spread_u <= 1.12f ? 8 : spread_u <= 5.0f && !(backward && growth > 0.0206f) ? 16 : 0;
 }
+constexpr int kSepLutWideMin = 6000;  // entries that grow by 2.06% over the transistor's 13 V: operands for 16 terms
 
 // What the passes of a call share, in its workspace.
 struct SepHead {
@@ -1570,6 +1571,10 @@ struct SepPlan {
 };
 
 constexpr int64_t kSepOperandBytes = ((int64_t)4 << 30) - (1 << 20);  // of one operand, at most (32-bit byte offsets)
+// Of a call's operands and planes, at most (3% of the card). With 4096 entries a GPT-L layer's 768 -> 3072
+// stays below both limits up to 87300 tokens forward and 69800 backward, 3072 -> 768 up to 21800 and 29500;
+// larger calls run the per-cell kernels.
+constexpr size_t kSepPlanBytes = (size_t)8 << 30;
 
 // Splits of a product's inner length: the count (each at least 8 slabs) that makes the launch's
 // time least, in slabs of one tile: rounds of blocks over the CUs (one 256 x 256 block each,
@@ -1595,28 +1600,21 @@ inline bool sep_big(int64_t rows_a, int64_t rows_b, int64_t slabs) {
     return ((rows_a + 255) / 256) * ((rows_b + 255) / 256) * (slabs / 16 + 1) >= 2 * kCUs && rows_a >= 192 && rows_b >= 192;
 }
 
-// lut_n: table entries, 0 for the formula.
-SepPlan plan_sep(int lut_n, int64_t M, int64_t K, int64_t O, bool backward, bool need_x, bool need_w, size_t base) {
+// The plan for up to `terms` terms; max_terms 0 where an operand would be too large.
+SepPlan plan_sep_terms(int lut_n, int64_t M, int64_t K, int64_t O, bool backward, bool need_x, bool need_w, size_t base,
+                       int terms) {
     SepPlan p{};
     p.bytes = base;
-    const double cells = (double)M * (double)K * (double)O;
-    if (M < 16 || O < 16 || K < 8 || (backward && !need_x && !need_w) ||
-        cells < (double)(lut_n > 0 ? (int64_t)ISA_EKV_CONTRACT_MIN_CELLS_LUT : (int64_t)ISA_EKV_CONTRACT_MIN_CELLS) ||
-        (lut_n > 0 && (lut_n < kSepLutMin || lut_n > kSepLutMax)))
-        return p;
     p.Kp = round_up(K, 8);
     p.Op = round_up(O, 256);
     const int64_t Mi = sep_inner(M), Oi = sep_inner(O), Kr = sep_inputs(K);
     const bool lut = lut_n > 0;
     const int most = lut ? kSepMaxHarmonics : 0;  // the device takes as many harmonics as the table needs
-    int terms = kSepMaxTerms;
-    auto fits = [&](int r) {  // (a backward's widest operand: dVth's triples, six bytes a value, or the harmonics)
-        const int64_t bytes = backward ? std::max(Mi, Oi) * Kr * std::max(6 * sep_classes(r, true).n3, 8 * most)
-                                       : std::max(M, O) * SepRow(K, r, most).bytes;
-        return bytes < kSepOperandBytes;
-    };
-    while (terms >= 8 && !fits(terms)) terms /= 2;
-    if (terms < 8 || Mi * Oi * 6 >= kSepOperandBytes) return p;
+    // (a backward's widest operand: dVth's triples, six bytes a value, or the harmonics; or G's triples)
+    const int64_t widest = backward ? std::max(std::max(Mi, Oi) * Kr * std::max(6 * sep_classes(terms, true).n3, 8 * most),
+                                               Mi * Oi * 6)
+                                    : std::max(M, O) * SepRow(K, terms, most).bytes;
+    if (widest >= kSepOperandBytes) return p;
     p.max_terms = terms;
     size_t off = (size_t)round_up((int64_t)base, 256);
     auto take = [&](int64_t bytes) {
@@ -1680,6 +1678,22 @@ SepPlan plan_sep(int lut_n, int64_t M, int64_t K, int64_t O, bool backward, bool
     }
     p.bytes = off;
     return p;
+}
+
+// lut_n: table entries, 0 for the formula.
+SepPlan plan_sep(int lut_n, int64_t M, int64_t K, int64_t O, bool backward, bool need_x, bool need_w, size_t base) {
+    SepPlan none{};
+    none.bytes = base;
+    const double cells = (double)M * (double)K * (double)O;
+    if (M < 16 || O < 16 || K < 8 || (backward && !need_x && !need_w) ||
+        cells < (double)(lut_n > 0 ? (int64_t)ISA_EKV_CONTRACT_MIN_CELLS_LUT : (int64_t)ISA_EKV_CONTRACT_MIN_CELLS) ||
+        (lut_n > 0 && (lut_n < kSepLutMin || lut_n > kSepLutMax)))
+        return none;
+    for (int terms = backward && lut_n > 0 && lut_n < kSepLutWideMin ? 8 : kSepMaxTerms; terms >= 8; terms /= 2) {
+        const SepPlan p = plan_sep_terms(lut_n, M, K, O, backward, need_x, need_w, base, terms);
+        if (p.max_terms > 0 && p.bytes - base < kSepPlanBytes) return p;
+    }
+    return none;
 }
 
 template <bool FORWARD>

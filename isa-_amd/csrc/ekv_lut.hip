@@ -5266,6 +5266,11 @@ size_t isa_ekv_forward_workspace(int64_t M, int64_t K, int64_t O) {
     return plan_sep(kSepLutMax, M, K, O, false, false, false, cell).bytes;
 }
 
+size_t isa_ekv_forward_table_workspace(int64_t M, int64_t K, int64_t O, int n_entries) {
+    if (M < 0 || K < 0 || O < 0 || n_entries < 1) return 0;
+    return plan_sep(n_entries, M, K, O, false, false, false, plan_forward_call(false, n_entries, M, K, O).bytes).bytes;
+}
+
 int isa_ekv_forward(const float* x, const float* vth_pos, const float* vth_neg, const void* lut_fwd, int64_t M,
                     int64_t K, int64_t O, int n_entries, float delta_min, float delta_max, float v_sat,
                     float out_min, float out_max, float* out, void* workspace, size_t workspace_bytes,

@@ -44,6 +44,7 @@ EXPORTS = (
     "isa_ekv_lut_build",
     "isa_ekv_lut_pack",
     "isa_ekv_forward_workspace",
+    "isa_ekv_forward_table_workspace",
     "isa_ekv_forward",
     "isa_ekv_forward_noalloc",
     "isa_ekv_backward_workspace",
@@ -152,6 +153,8 @@ def _declare(lib) -> None:
     lib.isa_ekv_lut_pack.restype = ci
     lib.isa_ekv_forward_workspace.argtypes = [i64, i64, i64]
     lib.isa_ekv_forward_workspace.restype = sz
+    lib.isa_ekv_forward_table_workspace.argtypes = [i64, i64, i64, ci]
+    lib.isa_ekv_forward_table_workspace.restype = sz
     lib.isa_ekv_forward.argtypes = [vp, vp, vp, vp, i64, i64, i64, ci, f32, f32, f32, f32, f32, vp, vp, sz, vp]
     lib.isa_ekv_forward.restype = ci
     lib.isa_ekv_forward_noalloc.argtypes = [vp, vp, vp, vp, i64, i64, i64, ci, f32, f32, f32, f32, f32, vp, vp]

@@ -40,12 +40,20 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
 
-def _workspace(nbytes: int, device: torch.device, given: Optional[torch.Tensor] = None) -> torch.Tensor:
+def _workspace(nbytes: int, device: torch.device, given: Optional[torch.Tensor] = None,
+               plan: Optional[tuple] = None) -> torch.Tensor:
     """The call's workspace: `given` (a caller's uint8 device buffer, checked) or a new one of
-    `nbytes` (the workspace query's bound). A given buffer's size is checked by the library
-    against the call's own plan (plan_info's workspace_bytes), which the bound may exceed."""
+    `nbytes` (the workspace query's bound), or where the device has no room for the matrix cores'
+    operands in it, of the per-cell kernels' plan (`plan`: plan_info's arguments). A given buffer's
+    size is checked by the library against the call's own plan."""
     if given is None:
-        return torch.empty(max(int(nbytes), 16), dtype=torch.uint8, device=device)
+        try:
+            return torch.empty(max(int(nbytes), 16), dtype=torch.uint8, device=device)
+        except torch.OutOfMemoryError:
+            cells = plan_info(*plan)["cell_bytes"] if plan else nbytes
+            if cells >= nbytes:
+                raise
+            return torch.empty(max(int(cells), 16), dtype=torch.uint8, device=device)
     _require_cuda(given, "workspace")
     if given.dtype != torch.uint8 or not given.is_contiguous() or given.device != device:
         raise RuntimeError(f"workspace must be a contiguous uint8 tensor on {device}")
@@ -214,7 +222,7 @@ def lut_forward(x: torch.Tensor, wpos: torch.Tensor, wneg: torch.Tensor, fwd_rec
                 n_entries: int, delta_min: float, delta_max: float, v_sat: float,
                 out_min: float, out_max: float, workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Idiff[M, O] fp32 (clamped to [out_min, out_max]). workspace: optional caller buffer
-    (uint8, at least isa_ekv_forward_workspace bytes)."""
+    (uint8, at least plan_info's cell_bytes)."""
     lib = _hip.load()
     M, K, O = _check_operands(x, wpos, wneg)
     if n_entries > MAX_ENTRIES:
@@ -224,8 +232,8 @@ def lut_forward(x: torch.Tensor, wpos: torch.Tensor, wneg: torch.Tensor, fwd_rec
     if M == 0 or O == 0:
         return out
     x32, wp32, wn32 = as_kernel_f32(x), as_kernel_f32(wpos), as_kernel_f32(wneg)
-    ws_bytes = lib.isa_ekv_forward_workspace(M, K, O)
-    ws = _workspace(ws_bytes, dev, workspace)
+    ws_bytes = lib.isa_ekv_forward_table_workspace(M, K, O, int(n_entries))
+    ws = _workspace(ws_bytes, dev, workspace, ("forward", M, K, O, n_entries))
     with _hip.on_device(dev):
         rc = lib.isa_ekv_forward(_ptr(x32), _ptr(wp32), _ptr(wn32), fwd_records.data_ptr(), M, K, O,
                                  int(n_entries), float(delta_min), float(delta_max), float(v_sat),
@@ -280,7 +288,7 @@ def lut_backward(x: torch.Tensor, wpos: torch.Tensor, wneg: torch.Tensor, grad_o
         return gx, gp, gn
     x32, wp32, wn32, g32 = (as_kernel_f32(t) for t in (x, wpos, wneg, grad_out))
     ws_bytes = lib.isa_ekv_backward_workspace(M, K, O, int(n_entries), int(need_grad_x), int(need_grad_w))
-    ws = _workspace(ws_bytes, dev, workspace)
+    ws = _workspace(ws_bytes, dev, workspace, ("backward", M, K, O, n_entries, need_grad_x, need_grad_w))
     with _hip.on_device(dev):
         rc = lib.isa_ekv_backward(_ptr(x32), _ptr(wp32), _ptr(wn32), _ptr(g32), bwd_records.data_ptr(), M, K, O,
                                   int(n_entries), float(delta_min), float(delta_max), float(v_sat),
@@ -306,7 +314,7 @@ def exact_forward(x: torch.Tensor, wpos: torch.Tensor, wneg: torch.Tensor,
     if M == 0 or O == 0:
         return out
     x32, wp32, wn32 = as_kernel_f32(x), as_kernel_f32(wpos), as_kernel_f32(wneg)
-    ws = _workspace(lib.isa_ekv_exact_forward_workspace(M, K, O), dev, workspace)
+    ws = _workspace(lib.isa_ekv_exact_forward_workspace(M, K, O), dev, workspace, ("exact_forward", M, K, O, 0))
     with _hip.on_device(dev):
         rc = lib.isa_ekv_exact_forward(_ptr(x32), _ptr(wp32), _ptr(wn32), M, K, O, _exact_params(params),
                                        float(v_sat), out.data_ptr(), ws.data_ptr(), ws.numel(),
@@ -333,7 +341,7 @@ def exact_backward(x: torch.Tensor, wpos: torch.Tensor, wneg: torch.Tensor, grad
         return gx, gp, gn
     x32, wp32, wn32, g32 = (as_kernel_f32(t) for t in (x, wpos, wneg, grad_out))
     ws = _workspace(lib.isa_ekv_exact_backward_workspace(M, K, O, int(need_grad_x), int(need_grad_w)), dev,
-                    workspace)
+                    workspace, ("exact_backward", M, K, O, 0, need_grad_x, need_grad_w))
     with _hip.on_device(dev):
         rc = lib.isa_ekv_exact_backward(_ptr(x32), _ptr(wp32), _ptr(wn32), _ptr(g32), M, K, O,
                                         _exact_params(params), float(v_sat), _ptr(gx), _ptr(gp), _ptr(gn),
@@ -419,7 +427,8 @@ def lut_layer_forward(x: torch.Tensor, wpos: torch.Tensor, wneg: torch.Tensor, f
         return out, idiff
     x32, wp32, wn32 = as_kernel_f32(x), as_kernel_f32(wpos), as_kernel_f32(wneg)
     glue = _glue_struct(aff, in_range, r, y_range, a_s, a_c, s_max, s_tot, r_ls, r_log_range)
-    ws = _workspace(lib.isa_ekv_layer_forward_workspace(M, K, O), dev, workspace)
+    ws = _workspace(lib.isa_ekv_forward_table_workspace(M, K, O, int(n_entries)), dev, workspace,
+                    ("forward", M, K, O, n_entries))
     with _hip.on_device(dev):
         rc = lib.isa_ekv_layer_forward(_ptr(x32), _ptr(wp32), _ptr(wn32), fwd_records.data_ptr(), M, K, O,
                                        int(n_entries), float(delta_min), float(delta_max), float(v_sat),
@@ -480,7 +489,7 @@ def lut_layer_backward(x: torch.Tensor, wpos: torch.Tensor, wneg: torch.Tensor, 
     x32, wp32, wn32, g32, id32 = (as_kernel_f32(t) for t in (x, wpos, wneg, grad_out, idiff))
     glue = _glue_struct(aff, in_range, r, y_range, a_s, a_c, r_log_scale=r_ls, r_log_range=r_log_range)
     ws = _workspace(lib.isa_ekv_layer_backward_workspace(M, K, O, int(n_entries), int(need_x), int(need_grad_w)), dev,
-                    workspace)
+                    workspace, ("layer_backward", M, K, O, n_entries, need_x, need_grad_w))
     with _hip.on_device(dev):
         rc = lib.isa_ekv_layer_backward(_ptr(x32), _ptr(wp32), _ptr(wn32), _ptr(g32), _ptr(id32),
                                         bwd_records.data_ptr(), M, K, O, int(n_entries), float(delta_min),

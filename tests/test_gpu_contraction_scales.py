@@ -201,7 +201,7 @@ def test_tokens_of_all_magnitudes(cuda_device, kind, entries, spread):
     g = g * torch.exp(-27.6 * torch.rand(M, 1, generator=gen)).cuda()
     print(f"[case] {kind} {entries} over {spread} V, tokens of all magnitudes", flush=True)
     got, cells = _run(kind, x, wp, wn, g, _tables(flash_cfg(entries)) if entries else None,
-                      (True, spread <= 0.31 or entries >= 6000))
+                      (True, kind == "formula" or spread <= 0.24 or entries >= 6000))
     ref, scale = _reference(x, wp, wn, g, cells)
     _check("out by token", got[0], ref[0], scale[0], 1, TOL[kind])
     _check("dX by token", got[1], ref[1], scale[1], 1, TOL[kind])
