@@ -329,7 +329,8 @@ int isa_ekv_plan_info(int which, int64_t M, int64_t K, int64_t O, int n_entries,
 
 /* Process-wide planning option (no reference counterpart; the reference has no plans).
  * Sets `option` to `value` and writes its former value to *previous (nullable); value < 0
- * only reads it. Options:
+ * only reads it. The options plan the table kernels: they have no effect on a call that the matrix
+ * cores take (path word 1 of isa_ekv_plan_info slot [10]). Options:
  *   ISA_EKV_OPT_COPY_MIN_CELLS: LUT calls of fewer cells M*K*O never use the second table
  *     copy, nor enqueue its assignment pass (default 2^28: below that the extra launch costs
  *     more than the copy saves). 0 lets every call consider it.

@@ -661,10 +661,12 @@ __device__ inline SepAt sep_at(const SepHead& h, float x) {
     return at;
 }
 
+// Four coefficients from the even j on (8-byte aligned: a class may begin at term 2).
 __device__ inline float4 sep_eval4(const float* tab, int R, const SepAt& at, int j) {
+    typedef float four __attribute__((ext_vector_type(4), aligned(8)));
     const float* p = tab + (size_t)at.i * R + j;
-    const float4 v0 = *reinterpret_cast<const float4*>(p), v1 = *reinterpret_cast<const float4*>(p + R);
-    const float4 v2 = *reinterpret_cast<const float4*>(p + 2 * R), v3 = *reinterpret_cast<const float4*>(p + 3 * R);
+    const four v0 = *reinterpret_cast<const four*>(p), v1 = *reinterpret_cast<const four*>(p + R);
+    const four v2 = *reinterpret_cast<const four*>(p + 2 * R), v3 = *reinterpret_cast<const four*>(p + 3 * R);
     float4 s;
     s.x = fmaf(at.w[3], v3.x, fmaf(at.w[2], v2.x, fmaf(at.w[1], v1.x, at.w[0] * v0.x)));
     s.y = fmaf(at.w[3], v3.y, fmaf(at.w[2], v2.y, fmaf(at.w[1], v1.y, at.w[0] * v0.y)));
@@ -1541,20 +1543,22 @@ __global__ __launch_bounds__(256) void sep_reduce_bwd_kernel(DxReduceArgs dx, Dx
 // ----------------------------------------------------------------------------------
 
 // Calls of fewer cells M K O run the per-cell kernels. A call that the contraction refuses pays for
-// the launches that return, 14 us where the sample refuses it (sep_sample_refuses; 5 us less for
-// tables, whose assignment passes are one launch), and the statistics, 11 us, where only they do:
-// the lines lie where that is 1% of the call. Measured (us, forward and backward, without the
-// contraction against refused): formula, 192 x 768 over 2 V at 2^27.2 cells 444 against 458, at
-// 2^28 over 4 V 804 against 820; tables over 5 V at 2^29 614 against 626, 768 -> 3072 -> 768 at
-// 2048 tokens (two calls of 2^32.2) 9125 against 9135. Taken calls gain from far smaller sizes on:
-// formula, 192 x 768 at 2^25.2 164 against 153, at 2^27.2 444 against 156.
+// the launches that return, 7 to 12 us (tables 1 to 5: their assignment passes are one launch) where the
+// sample refuses it (sep_sample_refuses), and the statistics, 10 to 20 us, where only they do (one threshold
+// or input far from the others). The lines lie where the first is 1% of the call; the second is then 2% of
+// it for the formula and up to 5% for tables. Measured (us, forward / backward, without the contraction
+// against refused): formula, 192 x 768 at 2^29 cells over 4 V 526 / 976 against 532 / 985, one outlier
+// 525 / 977 against 537 / 993; tables, 384 x 1536 at 2^30 over 5 V 376 / 801 against 380 / 803, one
+// outlier 347 / 738 against 366 / 761, 768 x 3072 at 4096 tokens 2256 / 5115 against 2278 / 5125. Taken
+// calls gain from far smaller sizes on: formula, 192 x 768 at 2^25.2 65 / 101 against 45 / 78, at 2^27.2
+// 157 / 288 against 52 / 106 (refused there 163 / 296).
 #ifndef ISA_EKV_CONTRACT_MIN_CELLS
 #define ISA_EKV_CONTRACT_MIN_CELLS (1 << 29)
 #endif
-// Table calls (us, forward / backward, per-cell kernels against the contraction, 4096 entries):
-// 384 x 1536 at 2^30 cells 334 / 557 against 137 / 261 at the initial thresholds, 344 / 740 against
-// 222 / 398 over 1 V (16 terms), 399 / 783 against 410 / 791 over 5 V (refused); at 2^29 224 / 329
-// against 98 / 200, 219 / 414 against 142 / 296, and 237 / 462 against 246 / 472.
+// Table calls (us, forward / backward, per-cell kernels against the contraction), 384 x 1536: at 2^30
+// cells 333 / 565 against 177 / 458 (4096 entries) and 339 / 606 against 160 / 414 (8192) at the initial
+// thresholds, over 1 V (16 terms) 343 against 242 (4096, forward) and 352 / 716 against 221 / 570 (8192);
+// at 2^29 222 / 331 against 122 / 271, and 227 / 408 against 234 / 409 over 5 V (refused).
 #ifndef ISA_EKV_CONTRACT_MIN_CELLS_LUT
 #define ISA_EKV_CONTRACT_MIN_CELLS_LUT (1 << 30)
 #endif
