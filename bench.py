@@ -9,7 +9,7 @@ parameters are resident in HBM before timing starts.
 value = cell-evals per second over the timed steps, counting M*K*O cells per CIM layer
 in the forward and again in the backward; the timed steps carry no instrumentation.
 `roofline` reports the dominant kernel (the backward main kernel) against its bound, the
-matrix cores' dense f16 peak where the calls run as contractions, else the VALU
+matrix cores' dense bf16 peak where the calls run as contractions, else the VALU
 lane-instruction peak, from HIP events the library records around each launch on its own
 stream in a second pass of the same steps; `cpu_baseline` times the reference's
 PyTorch CPU path (exact formula, chunked over 64 outputs, analytic backward) restated in
@@ -20,6 +20,7 @@ from __future__ import annotations
 
 import argparse
 import json
+import math
 import os
 import platform
 import statistics
@@ -35,8 +36,8 @@ for p in (str(ROOT / "isa-_amd"), str(ROOT)):
 
 # gfx950 VALU issue peak: 256 CUs x 64 lanes x 2.4 GHz (lane-instructions per second)
 VALU_PEAK = 256 * 64 * 2.4e9
-# dense f16 on the matrix cores (FLOP/s)
-MFMA_F16_PEAK = 2.5e15
+# dense bf16 on the matrix cores (FLOP/s)
+MFMA_PEAK = 2.5e15
 # lane-instructions per cell-eval (forward, backward). LUT path: the algorithmic count of
 # the interpolated lookup formulation. Exact path: the issued count of the exact kernels'
 # range-checked inner loops (4 log2 per cell forward; 4 log2 + 4 rcp backward, each with
@@ -207,21 +208,21 @@ def issued_valu_per_cell() -> dict:
 
 
 def contraction_roofline(exact: bool, entries: int, cells_launch: float, fwd_ms: float, bwd_ms: float) -> dict:
-    """The launches against the matrix cores' dense f16 peak, where the calls ran as contractions
-    (contraction.hpp) at the initial thresholds' 8 terms: products per cell-eval of the forward 4 terms
-    x 3 (pairs) + 4 (single f16), and 4 for each harmonic of a table's kinks (none above ~14000 entries,
-    one for the forward and dVth from ~3900 on and for dX from ~6000 on, else two); of the backward the
-    same for dX and for dVth (the formula's dVth: 8 x 3). Padding to tiles is not counted. The launch
-    times hold the operands' product, not the passes that expand the operands."""
-    harm, harm_dx = ((0, 0) if exact or entries > 14000 else
-                     (4 if entries > 3900 else 8, 4 if entries > 6000 else 8))
-    fwd = 16 + harm
-    bwd = 16 + 24 if exact else 32 + harm + harm_dx
+    """The launches against the matrix cores' dense bf16 peak, where the calls ran as contractions
+    (contraction.hpp) at the initial thresholds' 8 terms: products per cell-eval of the forward and of dX
+    2 terms x 6 (three bf16 parts) + 4 x 3 (two) + 2, of dVth 4 x 6 + 2 x 3 + 2, and 4 of each for every
+    harmonic of a table's kinks: as many as leave 7.7e-5 of a record of its growth from entry to entry.
+    Padding to tiles is not counted. The launch times hold the operands' product, not the passes that
+    expand the operands."""
+    growth = 0.0 if exact else math.expm1(13.0 / (4.1360 * 0.0259) / (entries - 1))
+    harmonics = next(h for h, left in ((0, 0.0373), (1, 0.0103), (2, 0.0050), (4, 0.0)) if left * growth <= 7.7e-5)
+    fwd = 26 + 4 * harmonics
+    bwd = 26 + 32 + 8 * harmonics
 
     def one(products: int, ms: float) -> dict:
         achieved = 2.0 * products * cells_launch / (ms * 1e-3) if ms else 0.0
         return {"products_per_cell": products, "avg_launch_ms": round(ms, 4),
-                "achieved": round(achieved / 1e12, 3), "frac": round(achieved / MFMA_F16_PEAK, 4)}
+                "achieved": round(achieved / 1e12, 3), "frac": round(achieved / MFMA_PEAK, 4)}
 
     return {"fwd": one(fwd, fwd_ms), "bwd": one(bwd, bwd_ms)}
 
@@ -590,7 +591,6 @@ def lds_roofline(model, cfg: dict, cells_launch: float, fwd_ms: float, bwd_ms: f
     output order. The kernels beat that rate where they spread a gather over the banks (the
     forward's windowed table copies, the ranked backward), so those fractions can pass 1;
     the conflict-free rate (one record per bank pair) bounds both."""
-    import math
 
     import torch
 
@@ -917,16 +917,16 @@ def main() -> int:
     if contracted:
         mfma = contraction_roofline(exact, args.lut_size, cells_launch, fwd_avg, bwd_avg)
         roofline = {
-            "bound": "mfma", "achieved": mfma["bwd"]["achieved"], "peak": round(MFMA_F16_PEAK / 1e12, 1),
+            "bound": "mfma", "achieved": mfma["bwd"]["achieved"], "peak": round(MFMA_PEAK / 1e12, 1),
             "unit": "TFLOP/s", "frac": mfma["bwd"]["frac"],
             "kernel": "sep_gemm_kernel (the backward's products, dominant)", "avg_launch_ms": round(bwd_avg, 4),
-            "work": f"{mfma['bwd']['products_per_cell']} f16 products per cell-eval x {cells_launch:.4e} cells per launch",
+            "work": f"{mfma['bwd']['products_per_cell']} bf16 products per cell-eval x {cells_launch:.4e} cells per launch",
             "forward_kernel": {"kernel": "sep_gemm_kernel (the forward's product) and sep_reduce_fwd_kernel",
                                **mfma["fwd"]},
             "traffic": None,
         }
         log(f"[bench] as contractions: forward product {fwd_avg:.3f} ms/launch ({mfma['fwd']['frac']:.3f} of the dense "
-            f"f16 peak), backward products {bwd_avg:.3f} ms/launch ({mfma['bwd']['frac']:.3f})")
+            f"bf16 peak), backward products {bwd_avg:.3f} ms/launch ({mfma['bwd']['frac']:.3f})")
     elif not exact:
         roofline["lds"] = lds_roofline(model, cfg, cells_launch, fwd_avg, bwd_avg, dev)
         clock = roofline["lds"].pop("_clock")
