@@ -66,7 +66,7 @@ constexpr int kSepStatG = 512;          // blocks of the largest |G|
 constexpr int kSepGridMax = 16384;      // x-table points, at most
 constexpr double kSepStep = 0.0148;     // x-table step in units of 2 n U_T
 constexpr int kSepMaxTerms = 16;
-constexpr int kSepLutMin = 3600, kSepLutMax = 65536;  // table entries: the kinks small enough, a thread per partial
+constexpr int kSepLutMin = 4000, kSepLutMax = 65536;  // table entries: the kinks small enough, a thread per partial
 constexpr int kSepMaxHarmonics = 4;
 
 // Widest threshold spread, in units of 2 n U_T, that R = 8 and 16 terms take: there the
@@ -485,7 +485,9 @@ __global__ __launch_bounds__(256) void sep_table_kernel(SepArgs a) {
             const double left = 7.7e-5;
             h.harmonics = 0.0373 * growth <= left ? 0 : 0.0103 * growth <= left ? 1 : 0.0050 * growth <= left ? 2 : 4;
             const double margin = 4.0 * step * a.lut_scale + 4.0;
-            ok = ok && s_info.x == 0.0f && growth > 1e-6 && 0.0021 * growth <= left &&
+            // (four to 3.1%: past it pairs of close thresholds far below threshold, where the per-cell
+            // kernels' coordinates are exact to 2^-14 of a record, are further off: 3600 entries 1.4 times)
+            ok = ok && s_info.x == 0.0f && growth > 1e-6 && growth <= 0.031 &&
                  ((double)xlo - (double)whi - a.lut_min) * a.lut_scale >= margin &&
                  ((double)xhi - (double)wlo - a.lut_min) * a.lut_scale <= (double)(a.lut_n - 1) - margin;
             h.lut_min = (float)a.lut_min;

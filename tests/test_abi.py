@@ -277,7 +277,7 @@ def test_plan_info_reports_the_call_plans():
 
 def test_plan_info_reports_the_matrix_cores_operands():
     """Slots 8 to 10: the per-cell plan's bytes, the bytes with the contraction's operands and the path
-    word, where a call considers it: from 2^29 cells (formula) and 2^30 (tables of 3600 to 65536
+    word, where a call considers it: from 2^29 cells (formula) and 2^30 (tables of 4000 to 65536
     entries)."""
     from isa.kernels.transformer_ffn import ops
 
@@ -288,7 +288,7 @@ def test_plan_info_reports_the_matrix_cores_operands():
         assert big["cell_bytes"] < big["contraction_bytes"], kind
         assert big["cell_bytes"] <= big["path_offset"] <= big["contraction_bytes"] - 4
         assert small["cell_bytes"] == small["contraction_bytes"] and small["path_offset"] == -1, kind
-    for n in (3599, 65537):
+    for n in (3999, 65537):
         assert ops.plan_info("forward", 8192, 768, 3072, n)["path_offset"] == -1
     assert ops.plan_info("exact_forward", 8192, 768, 3072, 0)["contraction_bytes"] == \
         lib.isa_ekv_exact_forward_workspace(8192, 768, 3072)

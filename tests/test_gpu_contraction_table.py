@@ -109,8 +109,8 @@ def _errors(got, ref):
 CASES = [
     (2048, 384, 1536, 4096, 0.2142),
     (2111, 389, 1533, 4096, 0.2142),
-    (515, 1031, 2051, 3700, 0.2142),
-    (2051, 513, 1031, 3700, 0.8),
+    (515, 1031, 2051, 4000, 0.2142),
+    (2051, 513, 1031, 4000, 0.8),
     (1999, 515, 1101, 4096, 0.3),
     (700, 770, 2003, 62000, 0.2142),
     (2053, 515, 1031, 5500, 0.2142),
