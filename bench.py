@@ -920,7 +920,8 @@ def main() -> int:
             "bound": "mfma", "achieved": mfma["bwd"]["achieved"], "peak": round(MFMA_PEAK / 1e12, 1),
             "unit": "TFLOP/s", "frac": mfma["bwd"]["frac"],
             "kernel": "sep_gemm_kernel (the backward's products, dominant)", "avg_launch_ms": round(bwd_avg, 4),
-            "work": f"{mfma['bwd']['products_per_cell']} bf16 products per cell-eval x {cells_launch:.4e} cells per launch",
+            "work": f"{mfma['bwd']['products_per_cell']} bf16 products per cell-eval (fp32 values as sums of up to "
+                    f"three bf16, fp32 sums) x {cells_launch:.4e} cells per launch",
             "forward_kernel": {"kernel": "sep_gemm_kernel (the forward's product) and sep_reduce_fwd_kernel",
                                **mfma["fwd"]},
             "traffic": None,
