@@ -88,3 +88,42 @@ def test_call_without_room_for_its_operands(cuda_device, monkeypatch, name):
     monkeypatch.setattr(torch, "empty", none)
     with pytest.raises(torch.OutOfMemoryError):
         call()
+
+
+@pytest.mark.parametrize("kind,tokens", [("forward", 21500), ("backward", 29000)])
+def test_operands_past_2_gib(cuda_device, kind, tokens):
+    """3072 -> 768 with as many tokens as the operands' limits take: offsets of up to 4 GiB. The first and
+    last tokens (and dVth, a sum over all of them) against the per-cell kernels: 1.5e-5 is what the two
+    paths' roundings (1e-5 and 4e-6) add up to."""
+    from isa.approximations.delta_lut import get_packed_tables, lut_range
+    from isa.kernels.transformer_ffn import ops
+
+    k, o = 3072, 768
+    cfg = flash_cfg(N)
+    lo, hi, n = lut_range(cfg)
+    fwd, bwd = get_packed_tables(cfg, torch.device("cuda"))
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.rand(tokens, k, generator=gen, device="cuda") * 4.0
+    wp, wn = (2.5 + 0.2142 * (torch.rand(o, k, generator=gen, device="cuda") - 0.5) for _ in range(2))
+    plan = ops.plan_info(kind, tokens, k, o, n)
+    assert plan["contraction_bytes"] - plan["cell_bytes"] > 4 << 30
+    print(f"[case] {kind} {tokens} x {k} -> {o}, {plan['contraction_bytes'] / 1e9:.1f} GB", flush=True)
+    if kind == "forward":
+        def call(ws):
+            return [ops.lut_forward(x, wp, wn, fwd, n, lo, hi, V_SAT, -1e30, 1e30, workspace=ws)]
+    else:
+        grad = torch.randn(tokens, o, generator=gen, device="cuda")
+
+        def call(ws):
+            return ops.lut_backward(x, wp, wn, grad, bwd, n, lo, hi, V_SAT, True, True, workspace=ws)
+
+    ws = torch.empty(plan["contraction_bytes"], dtype=torch.uint8, device="cuda")
+    got = call(ws)
+    torch.cuda.synchronize()
+    assert ops.took_contraction(ws, plan)
+    want = call(ws[:plan["cell_bytes"]])
+    for a, b in zip(got, want):
+        for rows in (slice(0, 300), slice(-300, None)):
+            e = float((a[rows] - b[rows]).norm() / b[rows].norm())
+            print(f"  {e:.2e}", flush=True)
+            assert e <= 1.5e-5, e
